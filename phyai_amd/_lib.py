@@ -95,6 +95,24 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+HOST_EXT_PATH = os.path.join(_PKG, "lib", "_phyai_host.so")
+
+
+def open_host_extension():
+    """The CPython extension that carries the eager call path (``csrc/host_ext.cpp``); not bound yet."""
+    import importlib.machinery
+    import importlib.util
+
+    import torch  # noqa: F401  - the extension links against torch's libraries, which this loads
+
+    if not os.path.exists(HOST_EXT_PATH):
+        raise Fp8LibraryError(f"{HOST_EXT_PATH} not found: build it with `make -C {CSRC_DIR}` (or phyai_amd._lib.build())")
+    loader = importlib.machinery.ExtensionFileLoader("_phyai_host", HOST_EXT_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_phyai_host", loader))
+    loader.exec_module(module)
+    return module
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().phyai_fp8_last_error()

@@ -1,0 +1,544 @@
+// CPython extension in front of the C ABI: the eager call path of the ops and of the fp8 linear layers.
+//
+// What bounds a small eager call is the host.  Checking tensors, asking torch for the stream and the
+// output, carving arguments and going through ctypes took 23 us per linear in Python where its one kernel
+// takes 4 - 6 us on the GPU (an MLP 34 us, a decoder layer 170 us); here the same steps are a few hundred
+// nanoseconds plus the launch itself.
+//
+// Every function either does the whole call and returns its result, or returns None having launched
+// nothing: the Python op then takes its own path, which checks the arguments one by one, handles the forms
+// this file leaves alone (copies of unaligned rows, empty inputs, another current device) and raises the
+// error a caller sees.  Nothing about results lives here: the kernels, their choice and the workspace
+// (phyai_amd.ops._workspaces, or the owner in scope while a graph is recorded) are those of the Python path.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <dlfcn.h>
+
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/phyai_fp8.h"
+
+namespace {
+
+// ---- what bind() was given -----------------------------------------------------------------------------
+struct Lib {
+    decltype(&phyai_fp8_linear) linear;
+    decltype(&phyai_fp8_linear_addcmul) linear_addcmul;
+    decltype(&phyai_fp8_gemm) gemm;
+    decltype(&phyai_fp8_gemm_addcmul) gemm_addcmul;
+    decltype(&phyai_fp8_mlp) mlp;
+    decltype(&phyai_fp8_linear_workspace_bytes) linear_ws;
+    decltype(&phyai_fp8_mlp_workspace_bytes) mlp_ws;
+    decltype(&phyai_fp8_quant_rowwise) quant_rowwise;
+    decltype(&phyai_fp8_quant_static) quant_static;
+    decltype(&phyai_fp8_rmsnorm_quant) rmsnorm;
+    decltype(&phyai_fp8_adarmsnorm_quant) adarmsnorm;
+} lib = {};
+
+struct Py {
+    PyObject *workspaces, *owner, *reserve, *epilogues, *layouts, *view_type, *per_channel, *per_tensor;
+} py = {};
+
+PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
+    *s_spec, *s_granularity;
+
+PyObject* declined() {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+}
+
+// ---- tensors ---------------------------------------------------------------------------------------------
+const at::Tensor* tensor(PyObject* o) { return o && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+PyObject* none_if_null(PyObject* o) { return o ? o : Py_None; }
+
+struct Rows {
+    const void* p;
+    int64_t M, K, ld;
+};
+// The [M, K] view of a tensor whose rows the kernels can read as they lie.
+bool rows_of(const at::Tensor& t, at::ScalarType dtype, Rows* r) {
+    if (!t.is_cuda() || t.scalar_type() != dtype || t.dim() < 1 || t.numel() == 0) return false;
+    const int64_t d = t.dim();
+    r->K = t.size(d - 1);
+    r->M = t.numel() / r->K;
+    if (t.stride(d - 1) != 1) return false;
+    if (t.is_contiguous()) r->ld = r->K;
+    else if (d == 2) r->ld = r->M > 1 ? t.stride(0) : r->K;
+    else return false;
+    r->p = t.const_data_ptr();
+    return r->ld >= r->K && r->ld % 8 == 0 && (reinterpret_cast<uintptr_t>(r->p) & 15) == 0;
+}
+bool codes_dtype(const at::Tensor& t) {
+    return t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kByte;
+}
+bool vector_of(const at::Tensor* t, at::ScalarType dtype, int64_t n) {
+    return t && t->is_cuda() && t->scalar_type() == dtype && t->numel() == n && t->is_contiguous();
+}
+
+// The device a call runs on and the stream of it; calls for another device than the current one are left
+// to the Python path.
+struct Where {
+    at::Device dev{at::kCUDA, 0};
+    hipStream_t stream = nullptr;
+};
+bool where(const at::Tensor& x, Where* w) {
+    const auto cur = c10::hip::current_device();
+    if (x.device().index() != cur) return false;
+    w->dev = x.device();
+    w->stream = c10::hip::getCurrentHIPStream(cur).stream();
+    return true;
+}
+
+// Fresh tensor shaped like `lead` with its last dimension replaced.
+at::Tensor fresh(const at::Tensor& lead, int64_t last, at::ScalarType dtype, const at::Device& dev) {
+    c10::SmallVector<int64_t, 6> shape(lead.sizes().begin(), lead.sizes().end());
+    shape.back() = last;
+    return at::Tensor(at::detail::empty_cuda(shape, dtype, dev, std::nullopt));
+}
+bool shaped(const at::Tensor* t, const at::Tensor& lead, int64_t last, at::ScalarType dtype) {
+    if (!t || !t->is_cuda() || t->scalar_type() != dtype || t->dim() != lead.dim() || !t->is_contiguous()) return false;
+    for (int64_t i = 0; i + 1 < lead.dim(); ++i)
+        if (t->size(i) != lead.size(i)) return false;
+    return t->size(lead.dim() - 1) == last;
+}
+
+// ---- workspace -----------------------------------------------------------------------------------------------
+struct Scratch {
+    void* p;
+    size_t n;
+};
+bool workspace(size_t need, const Where& w, Scratch* s) {
+    PyObject* owner = nullptr;
+    if (PyContextVar_Get(py.owner, nullptr, &owner) < 0) return false;
+    const bool shared = owner == nullptr || owner == Py_None;
+    Py_XDECREF(owner);
+    if (shared) {
+        PyObject* key = Py_BuildValue("iK", (int)w.dev.index(), (unsigned long long)reinterpret_cast<uintptr_t>(w.stream));
+        if (!key) return false;
+        const at::Tensor* t = tensor(PyDict_GetItemWithError(py.workspaces, key));
+        Py_DECREF(key);
+        if (t && (size_t)t->numel() >= need) {
+            *s = {t->mutable_data_ptr(), (size_t)t->numel()};
+            return true;
+        }
+    }
+    PyObject* o = PyObject_CallFunction(py.reserve, "K", (unsigned long long)need);
+    const at::Tensor* t = tensor(o);
+    if (t) *s = {t->mutable_data_ptr(), (size_t)t->numel()};
+    const bool ok = t != nullptr;
+    Py_XDECREF(o);   // its owner or the table of workspaces keeps it
+    return ok;
+}
+
+// ---- one linear -------------------------------------------------------------------------------------------------
+bool is_gated(int epi) { return epi >= PHYAI_FP8_EPI_GEGLU_TANH && epi <= PHYAI_FP8_EPI_SWIGLU; }
+
+// Epilogue (name, number or None) and the flag bits of the weight.
+bool epilogue_of(PyObject* o, int* epi) {
+    if (o == Py_None) { *epi = 0; return true; }
+    if (PyLong_CheckExact(o)) {
+        *epi = (int)PyLong_AsLong(o);
+        return *epi >= 0 && *epi <= PHYAI_FP8_EPI_GELU_ERF;
+    }
+    PyObject* v = PyDict_GetItemWithError(py.epilogues, o);
+    if (!v) return false;
+    *epi = (int)PyLong_AsLong(v);
+    return true;
+}
+bool flags_of(PyObject* layout, bool stream, int epi, int* flags) {
+    int f = 0;
+    if (layout != Py_None) {
+        PyObject* v = PyDict_GetItemWithError(py.layouts, layout);
+        if (!v) return false;
+        f = (int)PyLong_AsLong(v);
+        if (f && (f == PHYAI_FP8_FLAG_W_OPERAND_GATED) != is_gated(epi)) return false;
+    }
+    *flags = f | (stream ? PHYAI_FP8_FLAG_STREAM_WEIGHTS : 0);
+    return true;
+}
+
+struct Weight {
+    const void* w;
+    const float* scale;
+    const void* bias;
+    int64_t N;
+};
+bool weight_of(PyObject* w_, PyObject* s_, PyObject* b_, int64_t K, Weight* out) {
+    const at::Tensor *w = tensor(w_), *s = tensor(s_), *b = tensor(b_);
+    if (!w || !s || (b_ != Py_None && !b)) return false;
+    if (!w->is_cuda() || w->dim() != 2 || !codes_dtype(*w) || !w->is_contiguous() || w->size(1) != K) return false;
+    const int64_t N = w->size(0);
+    if (N == 0 || K % 16 != 0 || N % 16 != 0 || !vector_of(s, at::kFloat, N)) return false;
+    if (b && !vector_of(b, at::kBFloat16, N)) return false;
+    *out = {w->const_data_ptr(), s->const_data_ptr<float>(), b ? b->const_data_ptr() : nullptr, N};
+    return true;
+}
+
+struct Residual {
+    const void *residual, *gate;
+    int64_t ld_gate, gate_rows;
+};
+bool residual_of(PyObject* r_, PyObject* g_, const at::Tensor& x, int64_t M, int64_t N, int epi, Residual* out) {
+    *out = {nullptr, nullptr, 0, 0};
+    if (r_ == Py_None && g_ == Py_None) return true;
+    const at::Tensor *r = tensor(r_), *g = tensor(g_);
+    if (!r || !g || epi != 0 || !shaped(r, x, N, at::kBFloat16)) return false;
+    if (!g->is_cuda() || g->scalar_type() != at::kBFloat16 || g->dim() < 1 || g->size(g->dim() - 1) != N || g->numel() == 0) return false;
+    const int64_t rows = g->numel() / N;
+    if (!g->is_contiguous() || M % rows != 0) return false;
+    *out = {r->const_data_ptr(), g->const_data_ptr(), N, rows};
+    return true;
+}
+
+// bf16 rows `x_`, or codes `x_` with their scales `xs_` when that is given -> output tensor, null when declined.
+PyObject* linear_call(PyObject* x_, PyObject* xs_, PyObject* w_, PyObject* ws_, PyObject* b_, int epi, PyObject* layout,
+                      bool stream, PyObject* out_, PyObject* res_, PyObject* gate_) {
+    const at::Tensor* x = tensor(x_);
+    if (!x) return nullptr;
+    Rows r;
+    const bool codes = xs_ != nullptr;
+    if (codes ? !(codes_dtype(*x) && x->is_contiguous() && rows_of(*x, x->scalar_type(), &r)) : !rows_of(*x, at::kBFloat16, &r))
+        return nullptr;
+    Where at_;
+    Weight w;
+    int flags;
+    if (!where(*x, &at_) || !weight_of(w_, ws_, b_, r.K, &w) || !flags_of(layout, stream, epi, &flags)) return nullptr;
+    if (is_gated(epi) && w.N % 32 != 0) return nullptr;
+    const float* xs = nullptr;
+    int scalar = 0;
+    if (codes) {
+        const at::Tensor* s = tensor(xs_);
+        if (!s || !(vector_of(s, at::kFloat, r.M) || vector_of(s, at::kFloat, 1))) return nullptr;
+        xs = s->const_data_ptr<float>();
+        scalar = s->numel() == 1 && r.M != 1;
+    }
+    Residual rg;
+    if (!residual_of(res_, gate_, *x, r.M, w.N, epi, &rg)) return nullptr;
+    const int64_t n_out = is_gated(epi) ? w.N / 2 : w.N;
+    at::Tensor made;
+    void* out;
+    if (out_ == Py_None) {
+        made = fresh(*x, n_out, at::kBFloat16, at_.dev);
+        out = made.mutable_data_ptr();
+    } else {
+        const at::Tensor* o = tensor(out_);
+        if (!shaped(o, *x, n_out, at::kBFloat16)) return nullptr;
+        out = o->mutable_data_ptr();
+    }
+    Scratch ws;
+    if (!workspace(lib.linear_ws(r.M, w.N, r.K, epi), at_, &ws)) return nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    if (codes)
+        rc = rg.residual ? lib.gemm_addcmul(r.p, xs, scalar, w.w, w.scale, w.bias, rg.residual, w.N, rg.gate, rg.ld_gate, rg.gate_rows,
+                                            out, n_out, r.M, w.N, r.K, flags, ws.p, ws.n, at_.stream)
+                         : lib.gemm(r.p, xs, scalar, w.w, w.scale, w.bias, out, n_out, r.M, w.N, r.K, epi | flags, ws.p, ws.n, at_.stream);
+    else
+        rc = rg.residual ? lib.linear_addcmul(r.p, r.ld, w.w, w.scale, w.bias, rg.residual, w.N, rg.gate, rg.ld_gate, rg.gate_rows, out,
+                                              n_out, r.M, w.N, r.K, flags, ws.p, ws.n, at_.stream)
+                         : lib.linear(r.p, r.ld, w.w, w.scale, w.bias, out, n_out, r.M, w.N, r.K, epi | flags, ws.p, ws.n, at_.stream);
+    Py_END_ALLOW_THREADS
+    if (rc != 0) return nullptr;   // the Python path meets the same status and reports it
+    if (out_ != Py_None) {
+        Py_INCREF(out_);
+        return out_;
+    }
+    return THPVariable_Wrap(std::move(made));
+}
+
+// bf16 rows, one static scale for all of them: the codes live in a tensor of this call.
+PyObject* linear_static_call(PyObject* x_, PyObject* in_scale_, PyObject* w_, PyObject* ws_, PyObject* b_, int epi,
+                             PyObject* layout, bool stream, PyObject* res_, PyObject* gate_) {
+    const at::Tensor *x = tensor(x_), *s = tensor(in_scale_);
+    Rows r;
+    Where at_;
+    if (!x || !vector_of(s, at::kFloat, 1) || !rows_of(*x, at::kBFloat16, &r) || !where(*x, &at_)) return nullptr;
+    // what linear_call() would decline is declined before the quantizer is launched
+    Weight w;
+    int flags;
+    Residual rg;
+    if (!weight_of(w_, ws_, b_, r.K, &w) || !flags_of(layout, stream, epi, &flags) || (is_gated(epi) && w.N % 32 != 0) ||
+        !residual_of(res_, gate_, *x, r.M, w.N, epi, &rg))
+        return nullptr;
+    PyObject* xq = THPVariable_Wrap(fresh(*x, r.K, at::kFloat8_e4m3fn, at_.dev));
+    if (!xq) return nullptr;
+    int rc;
+    void* q = THPVariable_Unpack(xq).mutable_data_ptr();
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.quant_static(r.p, r.M, r.K, r.ld, s->const_data_ptr<float>(), q, at_.stream);
+    Py_END_ALLOW_THREADS
+    PyObject* y = rc == 0 ? linear_call(xq, in_scale_, w_, ws_, b_, epi, layout, stream, Py_None, res_, gate_) : nullptr;
+    Py_DECREF(xq);
+    return y;
+}
+
+// linear(x, weight, weight_scale, bias, epilogue, out, residual, gate, stream_weights, weight_layout)
+PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS   // e.g. torch out of memory
+    int epi;
+    if (n != 10 || !epilogue_of(a[4], &epi)) return declined();
+    PyObject* y = linear_call(a[0], nullptr, a[1], a[2], a[3], epi, a[9], PyObject_IsTrue(a[8]) == 1, a[5], a[6], a[7]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+// gemm(xq, x_scale, weight, weight_scale, bias, epilogue, out, residual, gate, stream_weights, weight_layout)
+PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    int epi;
+    if (n != 11 || !epilogue_of(a[5], &epi)) return declined();
+    PyObject* y = linear_call(a[0], a[1], a[2], a[3], a[4], epi, a[10], PyObject_IsTrue(a[9]) == 1, a[6], a[7], a[8]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- layers -------------------------------------------------------------------------------------------------------
+// What the HIP kernel needs of a linear layer, read from the module's own dictionaries (a module's
+// __getattr__ costs half a microsecond per parameter).  Borrowed references.
+struct Layer {
+    PyObject *weight, *scale, *input_scale, *layout, *granularity;
+    bool stream;
+};
+PyObject* plain_attr(PyObject* o, PyObject* dict, PyObject* name) {   // instance attribute, else the class's
+    PyObject* v = PyDict_GetItemWithError(dict, name);
+    return v ? v : _PyType_Lookup(Py_TYPE(o), name);
+}
+bool layer_of(PyObject* o, Layer* l) {
+    PyObject** dp = _PyObject_GetDictPtr(o);
+    if (!dp || !*dp) return false;
+    PyObject* params = PyDict_GetItemWithError(*dp, s_parameters);
+    PyObject* spec = PyDict_GetItemWithError(*dp, s_spec);
+    if (!params || !PyDict_Check(params) || !spec) return false;
+    l->weight = PyDict_GetItemWithError(params, s_weight);
+    l->scale = PyDict_GetItemWithError(params, s_weight_scale);
+    l->input_scale = PyDict_GetItemWithError(params, s_input_scale);
+    if (!l->weight || !l->scale) return false;
+    l->layout = none_if_null(plain_attr(o, *dp, s_weight_layout));
+    PyObject* st = plain_attr(o, *dp, s_stream_weights);
+    l->stream = st && PyObject_IsTrue(st) == 1;
+    PyObject* g = PyObject_GetAttr(spec, s_granularity);
+    if (!g) return false;
+    l->granularity = g;   // an enum member: its class keeps it
+    Py_DECREF(g);
+    return true;
+}
+
+// layer_apply(layer, x or ActivationView, bias, epilogue, residual, gate)
+PyObject* py_layer_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer l;
+    int epi;
+    if (n != 6 || !layer_of(a[0], &l) || !epilogue_of(a[3], &epi)) return declined();
+    PyObject* y = nullptr;
+    if (Py_TYPE(a[1]) == (PyTypeObject*)py.view_type) {
+        if (l.granularity != py.per_channel || PyTuple_GET_SIZE(a[1]) != 3 || PyTuple_GET_ITEM(a[1], 2) != py.per_channel) return declined();
+        y = linear_call(PyTuple_GET_ITEM(a[1], 0), PyTuple_GET_ITEM(a[1], 1), l.weight, l.scale, a[2], epi, l.layout, l.stream,
+                        Py_None, a[4], a[5]);
+    } else if (l.granularity == py.per_channel) {
+        y = linear_call(a[1], nullptr, l.weight, l.scale, a[2], epi, l.layout, l.stream, Py_None, a[4], a[5]);
+    } else if (l.granularity == py.per_tensor && l.input_scale) {
+        y = linear_static_call(a[1], l.input_scale, l.weight, l.scale, a[2], epi, l.layout, l.stream, a[4], a[5]);
+    }
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- MLP ------------------------------------------------------------------------------------------------------------
+PyObject* mlp_call(PyObject* x_, PyObject* w1_, PyObject* s1_, PyObject* b1_, PyObject* lay1, bool st1, PyObject* w2_,
+                   PyObject* s2_, PyObject* b2_, PyObject* lay2, bool st2, int epi, PyObject* out_, PyObject* res_,
+                   PyObject* gate_) {
+    const at::Tensor* x = tensor(x_);
+    Rows r;
+    Where at_;
+    Weight w1, w2;
+    int f1, f2;
+    Residual rg;
+    if (!x || epi == 0 || !rows_of(*x, at::kBFloat16, &r) || !where(*x, &at_) || !weight_of(w1_, s1_, b1_, r.K, &w1)) return nullptr;
+    if (is_gated(epi) && w1.N % 32 != 0) return nullptr;
+    const int64_t I = is_gated(epi) ? w1.N / 2 : w1.N;
+    if (!weight_of(w2_, s2_, b2_, I, &w2) || !flags_of(lay1, st1, epi, &f1) || !flags_of(lay2, st2, 0, &f2)) return nullptr;
+    if (!residual_of(res_, gate_, *x, r.M, w2.N, 0, &rg)) return nullptr;
+    at::Tensor made;
+    void* out;
+    if (out_ == Py_None) {
+        made = fresh(*x, w2.N, at::kBFloat16, at_.dev);
+        out = made.mutable_data_ptr();
+    } else {
+        const at::Tensor* o = tensor(out_);
+        if (!shaped(o, *x, w2.N, at::kBFloat16)) return nullptr;
+        out = o->mutable_data_ptr();
+    }
+    Scratch ws;
+    if (!workspace(lib.mlp_ws(r.M, r.K, I, w2.N, epi), at_, &ws)) return nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.mlp(r.p, r.ld, w1.w, w1.scale, w1.bias, f1, w2.w, w2.scale, w2.bias, f2, rg.residual, rg.residual ? w2.N : 0, rg.gate,
+                 rg.ld_gate, rg.gate_rows, out, w2.N, r.M, r.K, I, w2.N, epi, ws.p, ws.n, at_.stream);
+    Py_END_ALLOW_THREADS
+    if (rc != 0) return nullptr;
+    if (out_ != Py_None) {
+        Py_INCREF(out_);
+        return out_;
+    }
+    return THPVariable_Wrap(std::move(made));
+}
+
+// mlp(x, w1, s1, b1, w2, s2, b2, epilogue, out, residual, gate, stream1, stream2, layout1, layout2)
+PyObject* py_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    int epi;
+    if (n != 15 || !epilogue_of(a[7], &epi)) return declined();
+    PyObject* y = mlp_call(a[0], a[1], a[2], a[3], a[13], PyObject_IsTrue(a[11]) == 1, a[4], a[5], a[6], a[14],
+                           PyObject_IsTrue(a[12]) == 1, epi, a[8], a[9], a[10]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+// mlp_apply(first layer, second layer, x, bias1, bias2, epilogue, residual, gate): both per-channel layers
+PyObject* py_mlp_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer p, q;
+    int epi;
+    if (n != 8 || !layer_of(a[0], &p) || !layer_of(a[1], &q) || !epilogue_of(a[5], &epi) || p.granularity != py.per_channel ||
+        q.granularity != py.per_channel)
+        return declined();
+    PyObject* y = mlp_call(a[2], p.weight, p.scale, a[3], p.layout, p.stream, q.weight, q.scale, a[4], q.layout, q.stream, epi,
+                           Py_None, a[6], a[7]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- quantizers and norms ------------------------------------------------------------------------------------------
+// quant_rowwise(x) -> (codes, scale)
+PyObject* py_quant_rowwise(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* x = n == 1 ? tensor(a[0]) : nullptr;
+    Rows r;
+    Where at_;
+    if (!x || !rows_of(*x, at::kBFloat16, &r) || r.K % 8 != 0 || !where(*x, &at_)) return declined();
+    at::Tensor q = fresh(*x, r.K, at::kFloat8_e4m3fn, at_.dev), s = fresh(*x, 1, at::kFloat, at_.dev);
+    if (lib.quant_rowwise(r.p, r.M, r.K, r.ld, q.mutable_data_ptr(), s.mutable_data_ptr<float>(), at_.stream) != 0) return declined();
+    return Py_BuildValue("NN", THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(s)));
+    END_HANDLE_TH_ERRORS
+}
+
+struct NormOut {
+    at::Tensor out, xq, xs;
+    void* out_p() { return out.defined() ? out.mutable_data_ptr() : nullptr; }
+    void* xq_p() { return xq.defined() ? xq.mutable_data_ptr() : nullptr; }
+    float* xs_p() { return xs.defined() ? xs.mutable_data_ptr<float>() : nullptr; }
+};
+void make_norm_outputs(const at::Tensor& x, int64_t D, bool quantize, bool want_out, const Where& w, NormOut* o) {
+    if (want_out) o->out = fresh(x, D, at::kBFloat16, w.dev);
+    if (quantize) {
+        o->xq = fresh(x, D, at::kFloat8_e4m3fn, w.dev);
+        o->xs = fresh(x, 1, at::kFloat, w.dev);
+    }
+}
+PyObject* wrap_or_none(at::Tensor& t) {
+    if (t.defined()) return THPVariable_Wrap(std::move(t));
+    Py_RETURN_NONE;
+}
+
+// rmsnorm(x, weight, eps, gemma, quantize, want_out) -> (out, codes, scale)
+PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 6 ? tensor(a[0]) : nullptr, *w = n == 6 ? tensor(a[1]) : nullptr;
+    Rows r;
+    Where at_;
+    if (!x || !w || !rows_of(*x, at::kBFloat16, &r) || r.K % 8 != 0 || w->dim() != 1 || !vector_of(w, at::kBFloat16, r.K) || !where(*x, &at_))
+        return declined();
+    const double eps = PyFloat_AsDouble(a[2]);
+    if (eps == -1.0 && PyErr_Occurred()) return declined();
+    NormOut o;
+    make_norm_outputs(*x, r.K, a[4] == Py_True, a[5] == Py_True, at_, &o);
+    if (lib.rmsnorm(r.p, r.ld, w->const_data_ptr(), a[3] == Py_True, r.M, r.K, (float)eps, o.out_p(), r.K, o.xq_p(), o.xs_p(), at_.stream) != 0)
+        return declined();
+    return Py_BuildValue("NNN", wrap_or_none(o.out), wrap_or_none(o.xq), wrap_or_none(o.xs));
+    END_HANDLE_TH_ERRORS
+}
+
+// adarmsnorm(x, modulation, eps, quantize, want_out) -> (out, codes, scale, gate)
+PyObject* py_adarmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 5 ? tensor(a[0]) : nullptr, *m = n == 5 ? tensor(a[1]) : nullptr;
+    Rows r, q;
+    Where at_;
+    if (!x || !m || !rows_of(*x, at::kBFloat16, &r) || !rows_of(*m, at::kBFloat16, &q) || r.K % 8 != 0 || q.K != 3 * r.K ||
+        r.M % q.M != 0 || !where(*x, &at_))
+        return declined();
+    const double eps = PyFloat_AsDouble(a[2]);
+    if (eps == -1.0 && PyErr_Occurred()) return declined();
+    NormOut o;
+    make_norm_outputs(*x, r.K, a[3] == Py_True, a[4] == Py_True, at_, &o);
+    at::Tensor gate = fresh(*m, r.K, at::kBFloat16, at_.dev);
+    if (lib.adarmsnorm(r.p, r.ld, q.p, q.M > 1 ? q.ld : q.K, q.M, r.M, r.K, (float)eps, o.out_p(), r.K, gate.mutable_data_ptr(), r.K,
+                       o.xq_p(), o.xs_p(), at_.stream) != 0)
+        return declined();
+    return Py_BuildValue("NNNN", wrap_or_none(o.out), wrap_or_none(o.xq), wrap_or_none(o.xs), THPVariable_Wrap(std::move(gate)));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- module --------------------------------------------------------------------------------------------------------
+// bind(library path, workspaces, owner variable, reserve, epilogues, layouts, ActivationView, PER_CHANNEL, PER_TENSOR)
+PyObject* py_bind(PyObject*, PyObject* args) {
+    const char* path;
+    Py p = {};
+    if (!PyArg_ParseTuple(args, "sOOOOOOOO", &path, &p.workspaces, &p.owner, &p.reserve, &p.epilogues, &p.layouts, &p.view_type,
+                          &p.per_channel, &p.per_tensor))
+        return nullptr;
+    void* h = dlopen(path, RTLD_NOW | RTLD_LOCAL);   // the library that is loaded already: one more reference to it
+    if (!h) return PyErr_Format(PyExc_RuntimeError, "%s", dlerror());
+    Lib l = {};
+    bool ok = true;
+    auto get = [&](auto& fn, const char* name) {
+        fn = reinterpret_cast<std::decay_t<decltype(fn)>>(dlsym(h, name));
+        ok = ok && fn != nullptr;
+    };
+    get(l.linear, "phyai_fp8_linear");
+    get(l.linear_addcmul, "phyai_fp8_linear_addcmul");
+    get(l.gemm, "phyai_fp8_gemm");
+    get(l.gemm_addcmul, "phyai_fp8_gemm_addcmul");
+    get(l.mlp, "phyai_fp8_mlp");
+    get(l.linear_ws, "phyai_fp8_linear_workspace_bytes");
+    get(l.mlp_ws, "phyai_fp8_mlp_workspace_bytes");
+    get(l.quant_rowwise, "phyai_fp8_quant_rowwise");
+    get(l.quant_static, "phyai_fp8_quant_static");
+    get(l.rmsnorm, "phyai_fp8_rmsnorm_quant");
+    get(l.adarmsnorm, "phyai_fp8_adarmsnorm_quant");
+    if (!ok) return PyErr_Format(PyExc_RuntimeError, "%s lacks an entry point this extension binds", path);
+    for (PyObject* o : {p.workspaces, p.owner, p.reserve, p.epilogues, p.layouts, p.view_type, p.per_channel, p.per_tensor}) Py_INCREF(o);
+    lib = l;
+    py = p;
+    Py_RETURN_NONE;
+}
+
+#define PHYAI_FAST(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    {"bind", py_bind, METH_VARARGS, nullptr},
+    PHYAI_FAST("linear", py_linear),
+    PHYAI_FAST("gemm", py_gemm),
+    PHYAI_FAST("mlp", py_mlp),
+    PHYAI_FAST("layer_apply", py_layer_apply),
+    PHYAI_FAST("mlp_apply", py_mlp_apply),
+    PHYAI_FAST("quant_rowwise", py_quant_rowwise),
+    PHYAI_FAST("rmsnorm", py_rmsnorm),
+    PHYAI_FAST("adarmsnorm", py_adarmsnorm),
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_phyai_host", "Eager call path of phyai_amd.ops and of the fp8 layers.", -1, methods,
+                      nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__phyai_host() {
+    const struct { PyObject** at; const char* text; } names[] = {
+        {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_weight_scale, "weight_scale"}, {&s_input_scale, "input_scale"},
+        {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
+        {&s_granularity, "granularity"}};
+    for (const auto& e : names)
+        if (!(*e.at = PyUnicode_InternFromString(e.text))) return nullptr;
+    return PyModule_Create(&module);
+}

@@ -32,6 +32,9 @@ class KernelDispatcher:
         self.policy: Policy = policy if policy is not None else (ForcedPolicy(forced) if forced else DefaultPolicy())
         self._cache: dict[tuple[Any, ...], LinearKernel] = {}
         self._sm = sm_arch()
+        # Counts clear_cache() calls: a layer that remembers its selections (LinearBase._kernel_for)
+        # drops them when this has moved.
+        self.generation = 0
 
     def select(self, *, spec_id: str, M: int, N: int, K: int, in_dtype: torch.dtype,
                out_dtype: torch.dtype) -> LinearKernel:
@@ -54,6 +57,7 @@ class KernelDispatcher:
 
     def clear_cache(self) -> None:
         self._cache.clear()
+        self.generation += 1
 
 
 _dispatcher: KernelDispatcher | None = None

@@ -17,6 +17,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
+from phyai_amd import ops
 from phyai_amd.linear.backend import KernelProbe
 from phyai_amd.linear.registry import register_linear_kernel
 from phyai_amd.quant.types import ActivationView, Granularity
@@ -48,8 +49,9 @@ class HipFp8Kernel:
         """``epilogue`` / ``residual`` + ``gate`` are extensions over the reference protocol:
         ``DenseMLP`` passes the gated activation here so that it runs inside the GEMM kernel, and a
         decoder layer its ``addcmul(residual, out, gate)`` (``forward_addcmul`` of the layers)."""
-        from phyai_amd import ops
-
+        y = ops._native().layer_apply(layer, x, bias, epilogue, residual, gate)
+        if y is not None:
+            return y
         # set by phyai_amd.cache_plan.plan_weight_streaming on the layers whose weights should
         # pass the Infinity Cache by
         stream = bool(getattr(layer, "stream_weights", False))

@@ -24,16 +24,14 @@ import torch.nn as nn
 from phyai_amd.linear.dispatch import get_linear_dispatcher
 from phyai_amd.quant import AllocationRequest, Bf16Spec
 from phyai_amd.quant.types import ActivationView
+from phyai_amd.state import current_mode
 
 
 def _M_of(x) -> int:
+    """Number of token rows: product of every dim but the last."""
     if isinstance(x, ActivationView):
         x = x.x
-    """Number of token rows: product of every dim but the last."""
-    m = 1
-    for s in x.shape[:-1]:
-        m *= int(s)
-    return m
+    return x.numel() // (x.shape[-1] or 1) if x.dim() != 2 else x.shape[0]
 
 
 def _max_of_legs(layer: nn.Module):
@@ -143,20 +141,32 @@ class LinearBase(nn.Module):
     def _run(self, x, add_bias: bool = True, **kernel_kwargs) -> torch.Tensor:
         """``x`` is the bf16 activations or, for an fp8 layer, an ``ActivationView`` that a norm
         already quantized per token (``phyai_amd.norm``): then the layer's own quantizer is skipped."""
-        quantized = isinstance(x, ActivationView)
-        if quantized and not getattr(self.spec, "needs_act_quant", False):
+        if isinstance(x, ActivationView) and not getattr(self.spec, "needs_act_quant", False):
             raise RuntimeError(f"{type(self).__name__}: got quantized activations but spec "
                                f"{self.spec.spec_id!r} does not quantize its input")
-        kernel = get_linear_dispatcher().select(
-            spec_id=self.spec.spec_id, M=_M_of(x), N=self.output_size_per_partition,
-            K=self.input_size_per_partition, in_dtype=self.params_dtype if quantized else x.dtype,
-            out_dtype=self.params_dtype)
-        bias = self.bias if (add_bias and not self.skip_bias_add) else None
-        return kernel.apply(self, x, bias, **kernel_kwargs)
+        bias = self._parameters["bias"] if (add_bias and not self.skip_bias_add) else None
+        return self._kernel_for(x).apply(self, x, bias, **kernel_kwargs)
+
+    def _kernel_for(self, x):
+        """The dispatcher's choice for this input.  Remembered per layer under what can change between two
+        calls - token count bucket, input type, eager or capturing - as long as dispatcher, spec and parameter
+        type are the ones it was made for: building the dispatcher's full key takes longer than a launch."""
+        d = get_linear_dispatcher()
+        dtype = self.params_dtype if isinstance(x, ActivationView) else x.dtype
+        M = _M_of(x)
+        key = (M.bit_length(), dtype, current_mode())
+        memo = self.__dict__.get("_selected")
+        if memo is None or memo[0] is not d or memo[1] != d.generation or memo[2] is not self.spec or memo[3] is not self.params_dtype:
+            memo = self.__dict__["_selected"] = (d, d.generation, self.spec, self.params_dtype, {})
+        kernel = memo[4].get(key)
+        if kernel is None:
+            kernel = memo[4][key] = d.select(spec_id=self.spec.spec_id, M=M, N=self.output_size_per_partition,
+                                             K=self.input_size_per_partition, in_dtype=dtype, out_dtype=self.params_dtype)
+        return kernel
 
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor | None]:
         y = self._run(x)
-        return y, (self.bias if self.skip_bias_add else None)
+        return y, (self._parameters["bias"] if self.skip_bias_add else None)
 
     def forward_fused(self, x: torch.Tensor, epilogue: str) -> torch.Tensor:
         """Run the linear with an activation fused into the GEMM epilogue.  Only kernels
@@ -175,11 +185,7 @@ class LinearBase(nn.Module):
         return torch.addcmul(residual, y, gate)
 
     def supports_fused_epilogue(self, x) -> bool:
-        kernel = get_linear_dispatcher().select(
-            spec_id=self.spec.spec_id, M=_M_of(x), N=self.output_size_per_partition,
-            K=self.input_size_per_partition,
-            in_dtype=self.params_dtype if isinstance(x, ActivationView) else x.dtype, out_dtype=self.params_dtype)
-        return getattr(kernel, "name", "") == "hip_fp8" and not self.skip_bias_add
+        return getattr(self._kernel_for(x), "name", "") == "hip_fp8" and not self.skip_bias_add
 
 
 class ReplicatedLinear(LinearBase):

@@ -22,7 +22,9 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from phyai_amd import ops
 from phyai_amd.linear import ColumnParallelLinear, MergedColumnParallelLinear, RowParallelLinear
+from phyai_amd.quant.types import Granularity
 
 _GATED_ACTS = ("silu", "gelu", "gelu_tanh")
 _PLAIN_ACTS = ("gelu", "gelu_tanh")
@@ -104,20 +106,21 @@ class DenseMLP(nn.Module):
         MLP is then one library call (``ops.fp8_mlp``), which lets the first kernel hand its output's row
         maxima to the second."""
         return (self.fuse_activation and isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16
-                and getattr(first.spec, "spec_id", "") == "fp8_per_channel"
-                and getattr(second.spec, "spec_id", "") == "fp8_per_channel"
-                and not first.skip_bias_add and not second.skip_bias_add
+                and getattr(first.spec, "granularity", None) is Granularity.PER_CHANNEL
+                and getattr(second.spec, "granularity", None) is Granularity.PER_CHANNEL
                 and first.supports_fused_epilogue(x) and second.supports_fused_epilogue(x))
 
     def forward(self, x: torch.Tensor, *, residual: torch.Tensor | None = None,
                 gate: torch.Tensor | None = None) -> torch.Tensor:
         """``residual`` / ``gate``: ``torch.addcmul(residual, mlp(x), gate)`` in the second GEMM's epilogue
         (the decoder layer's gated residual, reference ``models/pi05/modeling_pi05.py:835``)."""
-        first = self.gate_up_proj if self.gated else self.fc1
-        second = self.down_proj if self.gated else self.fc2
+        mods = self._modules
+        first, second = (mods["gate_up_proj"], mods["down_proj"]) if self.gated else (mods["fc1"], mods["fc2"])
         if self._one_call(first, second, x):
-            from phyai_amd import ops
-
+            y = ops._native().mlp_apply(first, second, x, first._parameters["bias"], second._parameters["bias"], self._epilogue,
+                                        residual, gate)
+            if y is not None:
+                return y
             return ops.fp8_mlp(x, first.weight, first.weight_scale, first.bias, second.weight, second.weight_scale,
                                second.bias, epilogue=self._epilogue, residual=residual, gate=gate,
                                stream_weights1=bool(getattr(first, "stream_weights", False)),

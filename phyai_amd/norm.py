@@ -15,6 +15,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
+from phyai_amd import ops
 from phyai_amd.quant.types import ActivationView, Granularity
 
 
@@ -48,15 +49,11 @@ class RMSNorm(nn.Module):
         return torch.ones(hidden_size, dtype=dtype, device=device)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from phyai_amd import ops
-
         fn = ops.gemma_rmsnorm if self._gemma else ops.rmsnorm
-        return fn(x, self.weight.data, self.variance_epsilon)
+        return fn(x, self._parameters["weight"], self.variance_epsilon)
 
     def forward_fp8(self, x: torch.Tensor) -> ActivationView:
-        from phyai_amd import ops
-
-        xq, xs = ops.rmsnorm_fp8(x, self.weight.data, self.variance_epsilon, gemma=self._gemma)
+        xq, xs = ops.rmsnorm_fp8(x, self._parameters["weight"], self.variance_epsilon, gemma=self._gemma)
         return ActivationView(xq, xs, Granularity.PER_CHANNEL)
 
     def extra_repr(self) -> str:
@@ -128,14 +125,10 @@ class AdaRMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor, cond: torch.Tensor | None = None, *,
                 modulation: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
-        from phyai_amd import ops
-
         return ops.adarmsnorm(x, self._modulation(x, cond, modulation), self.variance_epsilon)
 
     def forward_fp8(self, x: torch.Tensor, cond: torch.Tensor | None = None, *,
                     modulation: torch.Tensor | None = None) -> tuple[ActivationView, torch.Tensor]:
-        from phyai_amd import ops
-
         xq, xs, gate = ops.adarmsnorm_fp8(x, self._modulation(x, cond, modulation), self.variance_epsilon)
         return ActivationView(xq, xs, Granularity.PER_CHANNEL), gate
 

@@ -108,6 +108,25 @@ def workspace_owner(owner: WorkspaceOwner):
         _owner.reset(token)
 
 
+# The eager call path in C++ (csrc/host_ext.cpp), bound on first use to the library, to the tables above and
+# to the names of this module.  Its functions return None, with nothing launched, for a call they leave to
+# the Python code below: every check and every error message stays here.
+_host = None
+
+
+def _native():
+    global _host
+    if _host is None:
+        from phyai_amd.quant.types import ActivationView, Granularity
+
+        _lib.load()
+        ext = _lib.open_host_extension()
+        ext.bind(_lib.LIB_PATH, _workspaces, _owner, reserve_workspace, EPILOGUES, WEIGHT_LAYOUTS, ActivationView,
+                 Granularity.PER_CHANNEL, Granularity.PER_TENSOR)
+        _host = ext
+    return _host
+
+
 def workspace_bytes(M: int, N: int, K: int, epilogue=EPI_NONE) -> int:
     return int(_lib.load().phyai_fp8_linear_workspace_bytes(M, N, K, _epi("workspace_bytes", epilogue)))
 
@@ -176,6 +195,8 @@ def fp8_quant_rowwise(x: torch.Tensor, *, out: torch.Tensor | None = None,
     with ``Fp8Spec.quantize_activation`` (reference ``layers/quant/fp8.py:150-155``).
     """
     op = "fp8_quant_rowwise"
+    if out is None and scale_out is None and (got := _native().quant_rowwise(x)) is not None:
+        return got
     x2 = _as_rows(op, x, "x", torch.bfloat16)
     M, K = x2.shape
     if K % 8 != 0:
@@ -213,6 +234,8 @@ def _norm_outputs(op: str, x: torch.Tensor, out, quantize: bool, want_out: bool)
 
 
 def _rmsnorm(op: str, x, weight, eps, out, gemma: bool, quantize: bool, want_out: bool):
+    if out is None and (got := _native().rmsnorm(x, weight, eps, gemma, quantize, want_out)) is not None:
+        return got
     x2 = _as_rows(op, x, "x", torch.bfloat16)
     M, D = x2.shape
     if not (isinstance(weight, torch.Tensor) and weight.is_cuda and weight.dtype == torch.bfloat16
@@ -256,6 +279,8 @@ def rmsnorm_fp8(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, *, gem
 
 
 def _adarmsnorm(op: str, x, modulation, eps, out, gate_out, quantize: bool, want_out: bool):
+    if out is None and gate_out is None and (got := _native().adarmsnorm(x, modulation, eps, quantize, want_out)) is not None:
+        return got
     if not (isinstance(modulation, torch.Tensor) and modulation.is_cuda):
         raise _err(op, "tensors must live on the GPU")
     if x.shape[-1] * 3 != modulation.shape[-1]:
@@ -476,6 +501,9 @@ def fp8_gemm(xq: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor, weig
     ``layers/linear/backends/torch.py:166-175`` (and ``:145-152``).
     """
     op = "fp8_gemm"
+    y = _native().gemm(xq, x_scale, weight, weight_scale, bias, epilogue, out, residual, gate, stream_weights, weight_layout)
+    if y is not None:
+        return y
     epi = _epi(op, epilogue)
     if not (isinstance(xq, torch.Tensor) and xq.is_cuda and xq.dtype in (torch.float8_e4m3fn, torch.uint8)):
         raise _err(op, "xq must be a float8_e4m3fn GPU tensor")
@@ -526,6 +554,9 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     (``layers/mlp/dense_mlp.py:256-261``).
     """
     op = "fp8_linear"
+    y = _native().linear(x, weight, weight_scale, bias, epilogue, out, residual, gate, stream_weights, weight_layout)
+    if y is not None:
+        return y
     epi = _epi(op, epilogue)
     x2 = _as_rows(op, x, "x", torch.bfloat16)
     M, K = x2.shape
@@ -580,6 +611,10 @@ def fp8_mlp(x: torch.Tensor, weight1: torch.Tensor, weight1_scale: torch.Tensor,
 
     Replaces ``DenseMLP.forward`` of the reference (``layers/mlp/dense_mlp.py:256-265``)."""
     op = "fp8_mlp"
+    y = _native().mlp(x, weight1, weight1_scale, bias1, weight2, weight2_scale, bias2, epilogue, out, residual, gate,
+                      stream_weights1, stream_weights2, weight1_layout, weight2_layout)
+    if y is not None:
+        return y
     epi = _epi(op, epilogue)
     if epi == EPI_NONE:
         raise _err(op, "epilogue must be the first projection's activation")
