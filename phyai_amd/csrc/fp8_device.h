@@ -97,6 +97,26 @@ __device__ __forceinline__ void copy16_to_lds_nt(const uint8_t* base, uint32_t l
                  :: "v"(lane_offset), "s"(base), "s"(lds_wave_base) : "memory", "m0");
 }
 
+// Copies out of a matrix whose row length K is not a multiple of the 128-byte K step.  In the last step the chunks
+// past the row's end must arrive as zeros: they would otherwise be the head of the next row (a NaN there would
+// reach this row's sums) or lie outside the matrix.  The copy goes through a buffer resource that knows the
+// matrix's size, and the lanes of those chunks carry an offset beyond it (kCopyNothing), which the hardware
+// answers with zeros and no access to memory.  Matrices are smaller than 2^31 bytes.
+constexpr uint32_t kCopyNothing = 0x80000000u;
+__device__ __forceinline__ v4i copy_source(const uint8_t* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    v4i r;
+    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+    r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xFFFF);   // stride 0: raw bytes
+    r[2] = __builtin_amdgcn_readfirstlane((int)bytes);
+    r[3] = 0x00020000;
+    return r;
+}
+__device__ __forceinline__ void copy16_to_lds_checked(v4i source, uint32_t lane_offset, uint32_t offset, uint32_t lds_wave_base) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(lane_offset), "s"(source), "s"(offset), "s"(lds_wave_base) : "memory", "m0");
+}
+
 // s_waitcnt vmcnt(N) with a compile-time N: at most N of this wavefront's copies still in flight.
 template <int N>
 __device__ __forceinline__ void wait_copies() {

@@ -46,8 +46,11 @@
 //
 // Gated epilogues: within a wavefront's 32*TN columns the first half are gate columns and the
 // second half the matching up columns, so the pair sits in the same lane of two accumulators.
-// Requires K % 128 == 0 and K >= 512 per split (stage-loads are never partial and must fill the
-// ring).
+// Requires K >= 512 per split (the stage-loads must fill the ring).  K that is not a multiple of 128 (RAGGED
+// instantiations, weights staged row-major): the last stage-load is partial, its missing chunks arrive as zeros
+// (copy16_to_lds_checked), one extra VALU instruction per copy and nothing in the MFMA loop.  Such widths used to go
+// to the generic tile kernel: the MLP 1168 -> 4304 -> 1168 at M = 777 took 43 + 37 us of GEMM there, 85 us in all;
+// 38 us in all here.
 #include "fp8_device.h"
 #include "launch.h"
 #include "tuning.h"
@@ -202,7 +205,7 @@ __host__ __device__ constexpr bool big_two_per_cu(int tm, int tn, int depth, int
 // unit * 2 KB + c * 256 + (l32 % 16) * 16.  2: operand order and WGM == 1, so that a wavefront's weight
 // blocks are its own: they go global -> registers, DEPTH stage-loads ahead through a ring of register
 // sets, and LDS carries the activations only.
-template <int TM, int TN, int DEPTH, int EPI, bool SPLIT, int WGM = 2, int WGN = 2, int WMODE = 0>
+template <int TM, int TN, int DEPTH, int EPI, bool SPLIT, int WGM = 2, int WGN = 2, int WMODE = 0, bool RAGGED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1)))
 void gemm_fp8_big_kernel(
     const uint8_t* __restrict__ a_a, const uint8_t* __restrict__ a_b, int a_K, int a_M, int a_N, int a_m_tiles,
@@ -222,6 +225,7 @@ void gemm_fp8_big_kernel(
     constexpr bool GATED = epi_is_gated(EPI);
     constexpr bool OPW = WMODE != 0, BDIRECT = WMODE == 2;
     static_assert(WGM * WGN == 4, "four wavefronts per workgroup");
+    static_assert(!RAGGED || WMODE == 0, "operand order exists for whole K steps only");
     static_assert(!BDIRECT || (WGM == 1 && (DEPTH == 4 || DEPTH == 8)), "weights go straight to registers only where a wavefront owns them");
     constexpr int BM = WGM * 32 * TM, BN = WGN * 32 * TN;   // workgroup tile
     constexpr int WM = 32 * TM, WN = 32 * TN;        // wavefront tile
@@ -331,9 +335,24 @@ void gemm_fp8_big_kernel(
             ob = operand_offset_plain((uint32_t)rb, (uint32_t)p.K);
         }
         const uint32_t chunk = (uint32_t)((lane & 7) ^ big_swizzle(jj));
-        boff[i] = p.operand_w ? ob + chunk * kOperandChunkBytes : (uint32_t)rb * (uint32_t)p.K + (chunk << 4);
+        boff[i] = !RAGGED && p.operand_w ? ob + chunk * kOperandChunkBytes : (uint32_t)rb * (uint32_t)p.K + (chunk << 4);
     }
     const int k_begin = SPLIT ? split_z * p.k_per_split : 0;
+    // RAGGED: the last stage-load of the matrix holds K % 128 bytes per row; kCopyNothing for the lanes whose chunk is
+    // not among them.  The chunk of a lane depends on its row's swizzle, which repeats every two 8-row groups.
+    uint32_t a_gone[2] = {0, 0}, b_gone[2] = {0, 0};
+    v4i a_source = {0, 0, 0, 0}, b_source = {0, 0, 0, 0};
+    if constexpr (RAGGED) {
+        const int tail = p.K & (BIG_BK - 1);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int ra = (wave * CA + e) * 8 + (lane >> 3), rb = (wave * CB + e) * 8 + (lane >> 3);
+            a_gone[e] = (((lane & 7) ^ big_swizzle(ra)) << 4) >= tail ? kCopyNothing : 0u;
+            b_gone[e] = (((lane & 7) ^ big_swizzle(rb)) << 4) >= tail ? kCopyNothing : 0u;
+        }
+        a_source = copy_source(p.a, (uint32_t)p.M * (uint32_t)p.K);
+        b_source = copy_source(p.b, (uint32_t)p.N * (uint32_t)p.K);
+    }
     const int b_step_shift = (OPW || p.operand_w) ? 4 : 0;   // a K step of operand-order weights is 2 KB away, not 128 bytes
     // BDIRECT: this lane's 16 bytes of chunk h of row l32 of weight block j, K step 0; chunk c of the same row
     // is c * 256 further, the next K step 2 KB
@@ -354,6 +373,12 @@ void gemm_fp8_big_kernel(
     auto issue = [&](int d, int c, auto slot) {
         const int k = k_begin + d * BIG_BK;
         const uint32_t stage_off = (d % DEPTH) * STAGE_BYTES;
+        if constexpr (RAGGED) {
+            const uint32_t last = k + BIG_BK > p.K ? ~0u : 0u;   // (uniform)
+            if (c < CA) copy16_to_lds_checked(a_source, aoff[c] | (a_gone[c & 1] & last), k, wave_a + stage_off + c * 1024);
+            else copy16_to_lds_checked(b_source, boff[c - CA] | (b_gone[(c - CA) & 1] & last), k, wave_b + stage_off + (c - CA) * 1024);
+            return;
+        }
         if (c < CA) {
             if (!(PHYAI_FP8_ABLATE & 16) || d < LEAD) copy16_to_lds(p.a + k, aoff[c], wave_a + stage_off + c * 1024);
         } else if constexpr (BDIRECT) {
@@ -367,7 +392,10 @@ void gemm_fp8_big_kernel(
     };
     using Slot0 = std::integral_constant<int, 0>;
 
-    const int n_loads = (SPLIT ? p.k_per_split : p.K) / BIG_BK;   // stage-loads in all, >= DEPTH
+    // stage-loads in all, >= DEPTH
+    const int n_loads = RAGGED && SPLIT ? ((k_begin + p.k_per_split < p.K ? p.k_per_split : p.K - k_begin) + BIG_BK - 1) / BIG_BK
+                        : RAGGED        ? (p.K + BIG_BK - 1) / BIG_BK
+                                        : (SPLIT ? p.k_per_split : p.K) / BIG_BK;
     const int arow = wm * WM + l32, brow = wn * WN + l32;
     auto stage_ptr = [&](int d) -> const uint8_t* { return lds + (d % DEPTH) * STAGE_BYTES; };
     // weight block with first row `row` - l32 out of the staged B rows, K half kh
@@ -872,7 +900,8 @@ static double big_fill(int tiles, int slots) {
 
 BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     BigPlan pl = {0, 0, 1, 0, 0, 0};
-    if (K % 128 != 0 || K < 512) return pl;   // slabs come in pairs and must fill the ring
+    if (K < 512) return pl;   // the stage-loads must fill the ring
+    const bool ragged = K % 128 != 0;
     int forced = -1;
     if (const char* e = tuning_env("PHYAI_FP8_BIG")) forced = atoi(e);   // "0": never; "256"/"192"/"128": force
     if (forced == 0) return pl;
@@ -959,7 +988,7 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     } else if (pl.tile == 128) {
         // Measured at M = 816: splitting pays for K = 16384 (67 -> 49 us with two splits) and
         // costs for K = 2048 (19 -> 25 us): the partial-sum round trip is worth about 6 us.
-        if (tiles < 200 && K >= 8192 && K % 256 == 0) pl.splits = 2;
+        if (tiles < 200 && K >= 8192 && (K % 256 == 0 || ragged)) pl.splits = 2;
         // With more tiles than CUs a ring of two stages lets two workgroups share a CU instead of
         // queueing behind each other (800 x 8192 x 1024, 448 tiles: 17.5 -> 14.4 us; 1632 x 2560 x 2048,
         // 260 tiles: 23.3 -> 18.3 us); up to one tile per CU the deeper ring hides more latency
@@ -968,7 +997,7 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     }
     if (const char* e = tuning_env("PHYAI_FP8_BIG_SPLITS")) {
         const int s = atoi(e);
-        if (pl.tile == 128 && pl.cols == 128 && s >= 1 && K % (s * 128) == 0 && K / s >= 512 && tiles * s <= 4096) pl.splits = s;
+        if (pl.tile == 128 && pl.cols == 128 && s >= 1 && (K % (s * 128) == 0 || (ragged && s <= 2)) && K / s >= 512 && tiles * s <= 4096) pl.splits = s;
     }
     if (const char* e = tuning_env("PHYAI_FP8_BIG_DEPTH")) {
         const int d = atoi(e);
@@ -995,7 +1024,7 @@ size_t big_partial_bytes(int M, int N, int epilogue, const BigPlan& pl) {
     return (size_t)big_tiles(M, N, epilogue, pl.tile, bn) * pl.splits * pl.tile * bn * sizeof(float);
 }
 
-template <int TM, int TN, int DEPTH, int EPI, int WGM = 2, int WGN = 2, int WMODE = 0>
+template <int TM, int TN, int DEPTH, int EPI, int WGM = 2, int WGN = 2, int WMODE = 0, bool RAGGED = false>
 static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t st) {
     const bool gated = epi_is_gated(EPI);
     constexpr int BM = WGM * 32 * TM, BN = WGN * 32 * TN;
@@ -1055,33 +1084,33 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
         // not built with them: its 256 accumulators leave the gather no registers, and a kernel that spills has
         // vector-memory instructions of the compiler's among the copies that the waits count by hand.)
         if constexpr ((TM == TN && TM == 2 && DEPTH == 4) || (WMODE == 2 && TN == 1 && !big_two_per_cu(TM, TN, DEPTH, WMODE)))
-            hipLaunchKernelGGL((gemm_fp8_big_kernel<TM, TN, DEPTH, EPI, true, WGM, WGN, WMODE>), grid, dim3(256), 0, st, PHYAI_BIG_ARGS);
+            hipLaunchKernelGGL((gemm_fp8_big_kernel<TM, TN, DEPTH, EPI, true, WGM, WGN, WMODE, RAGGED>), grid, dim3(256), 0, st, PHYAI_BIG_ARGS);
     } else {
-        hipLaunchKernelGGL((gemm_fp8_big_kernel<TM, TN, DEPTH, EPI, false, WGM, WGN, WMODE>), grid, dim3(256), 0, st, PHYAI_BIG_ARGS);
+        hipLaunchKernelGGL((gemm_fp8_big_kernel<TM, TN, DEPTH, EPI, false, WGM, WGN, WMODE, RAGGED>), grid, dim3(256), 0, st, PHYAI_BIG_ARGS);
     }
 #undef PHYAI_BIG_ARGS
 }
 
-template <int TM, int TN, int DEPTH, int WGM = 2, int WGN = 2, int WMODE = 0>
+template <int TM, int TN, int DEPTH, int WGM = 2, int WGN = 2, int WMODE = 0, bool RAGGED = false>
 static int big_launch_epi(const BigArgs& a, const GemmProblem& g, int splits, hipStream_t st) {
     switch (g.epilogue) {
-    case EPI_NONE: big_launch<TM, TN, DEPTH, EPI_NONE, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_GEGLU_TANH: big_launch<TM, TN, DEPTH, EPI_GEGLU_TANH, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_GEGLU_ERF: big_launch<TM, TN, DEPTH, EPI_GEGLU_ERF, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_SWIGLU: big_launch<TM, TN, DEPTH, EPI_SWIGLU, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_GELU_TANH: big_launch<TM, TN, DEPTH, EPI_GELU_TANH, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_GELU_ERF: big_launch<TM, TN, DEPTH, EPI_GELU_ERF, WGM, WGN, WMODE>(a, g, splits, st); return 0;
+    case EPI_NONE: big_launch<TM, TN, DEPTH, EPI_NONE, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_GEGLU_TANH: big_launch<TM, TN, DEPTH, EPI_GEGLU_TANH, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_GEGLU_ERF: big_launch<TM, TN, DEPTH, EPI_GEGLU_ERF, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_SWIGLU: big_launch<TM, TN, DEPTH, EPI_SWIGLU, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_GELU_TANH: big_launch<TM, TN, DEPTH, EPI_GELU_TANH, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_GELU_ERF: big_launch<TM, TN, DEPTH, EPI_GELU_ERF, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
     default: return -2;
     }
 }
 
 // (tiles with one column block per wavefront cannot hold a gate / up pair: plain epilogues only)
-template <int TM, int TN, int DEPTH, int WGM = 2, int WGN = 2, int WMODE = 0>
+template <int TM, int TN, int DEPTH, int WGM = 2, int WGN = 2, int WMODE = 0, bool RAGGED = false>
 static int big_launch_plain(const BigArgs& a, const GemmProblem& g, int splits, hipStream_t st) {
     switch (g.epilogue) {
-    case EPI_NONE: big_launch<TM, TN, DEPTH, EPI_NONE, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_GELU_TANH: big_launch<TM, TN, DEPTH, EPI_GELU_TANH, WGM, WGN, WMODE>(a, g, splits, st); return 0;
-    case EPI_GELU_ERF: big_launch<TM, TN, DEPTH, EPI_GELU_ERF, WGM, WGN, WMODE>(a, g, splits, st); return 0;
+    case EPI_NONE: big_launch<TM, TN, DEPTH, EPI_NONE, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_GELU_TANH: big_launch<TM, TN, DEPTH, EPI_GELU_TANH, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
+    case EPI_GELU_ERF: big_launch<TM, TN, DEPTH, EPI_GELU_ERF, WGM, WGN, WMODE, RAGGED>(a, g, splits, st); return 0;
     default: return -2;
     }
 }
@@ -1090,6 +1119,7 @@ static int big_launch_plain(const BigArgs& a, const GemmProblem& g, int splits, 
 // operand order as they lie.
 template <int TM, int TN, int DEPTH, int WGM = 2, int WGN = 2>
 static int big_launch_layout(const BigArgs& a, const GemmProblem& g, int splits, hipStream_t st) {
+    if (g.K % BIG_BK != 0) return big_launch_epi<TM, TN, DEPTH, WGM, WGN, 0, true>(a, g, splits, st);
     if (a.operand_w && !tuning_env("PHYAI_FP8_BIG_GATHER")) return big_launch_epi<TM, TN, DEPTH, WGM, WGN, 1>(a, g, splits, st);
     return big_launch_epi<TM, TN, DEPTH, WGM, WGN, 0>(a, g, splits, st);
 }
@@ -1113,7 +1143,8 @@ int launch_gemm_big(const GemmProblem& g, const BigPlan& pl, hipStream_t st) {
     a.a_scale_scalar = g.x_scale_is_scalar;
     a.res = residual_of(g);
     a.operand_w = g.weight_layout != W_ROW_MAJOR;
-    a.k_per_split = g.K / pl.splits;
+    // (K that is no multiple of 128: the ranges end on whole K steps, the last one is the shorter)
+    a.k_per_split = g.K % BIG_BK == 0 ? g.K / pl.splits : big_ceil_div(big_ceil_div(g.K, BIG_BK), pl.splits) * BIG_BK;
     a.counters = static_cast<int*>(g.workspace);
     a.partials = g.workspace ? reinterpret_cast<float*>(static_cast<uint8_t*>(g.workspace) + kGemmHeaderBytes) : nullptr;
     if (pl.splits > 1 && (g.workspace == nullptr ||
@@ -1129,10 +1160,12 @@ int launch_gemm_big(const GemmProblem& g, const BigPlan& pl, hipStream_t st) {
     if (pl.tile == 192 && pl.splits == 1) return big_launch_layout<3, 2, 2>(a, g, 1, st);
     if (pl.tile == 96) {   // 96 rows x 128 columns: wavefronts 1 x 4, three row blocks each; plain epilogues
         if (pl.splits != 1) return -2;
+        if (g.K % BIG_BK != 0) return big_launch_plain<3, 1, 4, 1, 4, 0, true>(a, g, 1, st);
         return a.operand_w ? big_launch_plain<3, 1, 4, 1, 4, 1>(a, g, 1, st) : big_launch_plain<3, 1, 4, 1, 4, 0>(a, g, 1, st);
     }
     if (pl.tile == 128 && pl.cols == 64) {
         if (pl.splits != 1) return -2;
+        if (g.K % BIG_BK != 0) return big_launch_plain<2, 1, 4, 2, 2, 0, true>(a, g, 1, st);
         return a.operand_w ? big_launch_plain<2, 1, 4, 2, 2, 1>(a, g, 1, st) : big_launch_plain<2, 1, 4, 2, 2, 0>(a, g, 1, st);
     }
     if (pl.tile == 128 && pl.depth == 4 && pl.regs == 8) return big_launch_plain<4, 1, 8, 1, 4, 2>(a, g, pl.splits, st);

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
         const uint32_t u = blockIdx.x * NT + nt;
         return u < w_units ? u : w_units - 1;
     };
-    p.rounds = (((a_K >> 7) + SK_WAVES - 1) / SK_WAVES + KPW - 1) / KPW;
+    p.rounds = ((((a_K + 127) >> 7) + SK_WAVES - 1) / SK_WAVES + KPW - 1) / KPW;
     p.res = a_res;
     constexpr bool GATED = epi_is_gated(EPI);
     constexpr int COLS_PER_TILE = GATED ? 8 : 16;  // output columns per 16-row weight tile
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
     const int half_n = p.N / 2;
     const int n_out_total = GATED ? half_n : p.N;
     const int col0 = blockIdx.x * (COLS_PER_TILE * NT);  // first output column of the workgroup
-    const int total_steps = p.K >> 7;
+    const int total_steps = (p.K + 127) >> 7;   // the last one is partial where K is not a multiple of 128 (STAGED only)
     const int m_base = blockIdx.y * (MB * 16);
 
     // ---- epilogue roles of this thread and their operands (requested first) --------------------
@@ -282,6 +282,12 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) xoff[mb][hf] = __umul24((uint32_t)x_row(mb, r16), (uint32_t)p.K) + chunk;
         }
+        // K not a multiple of 128: kCopyNothing for this lane's chunk in the last K step, see copy16_to_lds_checked
+        const bool ragged = (p.K & 127) != 0;
+        uint32_t gone[2];
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+            gone[hf] = ((c_slot ^ (((hf * 8 + c_row) >> 1) & 7)) << 4) >= (p.K & 127) ? kCopyNothing : 0u;
         const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wave * PER_WAVE);
         const uint8_t* my_stage = smem + wave * PER_WAVE;
         const int swz = (l16 >> 1) & 7;
@@ -297,6 +303,20 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
                 const int s = __builtin_amdgcn_readfirstlane((rnd * KPW + j) * SK_WAVES + wave);
                 if (s < total_steps) {
                     const uint32_t dst = lds_wave + j * (BLOCKS * 2048);
+                    if (ragged && s == total_steps - 1) {
+                        const v4i ws = copy_source(p.w, (uint32_t)p.N * (uint32_t)p.K), xs = copy_source(p.xq, (uint32_t)p.M * (uint32_t)p.K);
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                            for (int hf = 0; hf < 2; ++hf)
+                                copy16_to_lds_checked(ws, woff[nt][hf] | gone[hf], (uint32_t)s << 7, dst + (nt * 2 + hf) * 1024);
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                            for (int hf = 0; hf < 2; ++hf)
+                                copy16_to_lds_checked(xs, xoff[mb][hf] | gone[hf], (uint32_t)s << 7, dst + ((NT + mb) * 2 + hf) * 1024);
+                        continue;
+                    }
                     // one branch per K step: the weights of this call either pass the caches by or not
                     if (stream_w) {
 #pragma unroll
@@ -409,15 +429,25 @@ static int skinny_max_m() {
     return 1024;
 }
 
+// K that is not a multiple of 128 (staged form only).  Few token rows: always, from two K steps on - the generic
+// kernel's K splits cost it a round trip through memory.  More rows: as for whole K steps, but not below 1024 output
+// columns, where the generic kernel's splits are what fills the chip.
+static bool skinny_takes_ragged(int M, int N, int K) {
+    static const bool staged = []() { const char* e = tuning_env("PHYAI_FP8_SKINNY_STAGED"); return !(e && atoi(e) == 0); }();
+    if (!staged || (int64_t)K * (N > M ? N : M) >= ((int64_t)1 << 31) || K >= (1 << 24)) return false;
+    return K > 256 && (M <= 64 || N >= 1024);
+}
+
 bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo) {
-    if (M > skinny_max_m() || K % 128 != 0 || ldo % 4 != 0) return false;
+    if (M > skinny_max_m() || ldo % 4 != 0) return false;
+    if (K % 128 != 0 && !skinny_takes_ragged(M, N, K)) return false;
     if (epi_is_gated(epilogue)) return (N / 2) % 8 == 0;
     return N % 8 == 0;
 }
 
 // K steps a wavefront stages per round: up to 4, as many as K offers and the LDS holds
 static int skinny_steps_per_round(int K, int nt, int mb) {
-    const int per_wave = sk_ceil_div(K / 128, SK_WAVES);
+    const int per_wave = sk_ceil_div(sk_ceil_div(K, 128), SK_WAVES);
     int kpw = per_wave >= 4 ? 4 : (per_wave >= 2 ? 2 : 1);
     while (kpw > 1 && SK_WAVES * kpw * (nt + mb) * 2048 > 160 * 1024) kpw /= 2;
     return kpw;
@@ -463,7 +493,7 @@ SkinnyPlan skinny_plan(int M, int N, int K, int epilogue) {
     // staging of 8 wavefronts x kpw steps x (nt + mb) blocks of 2 KB must fit the 160 KB of LDS:
     // more rounds of fewer steps beat the unstaged form (down 50..400 x 1024 x 4096: 12 -> 7 us)
     pl.kpw = skinny_steps_per_round(K, pl.nt, pl.mb);
-    pl.rounds = sk_ceil_div(sk_ceil_div(K / 128, SK_WAVES), pl.kpw);
+    pl.rounds = sk_ceil_div(sk_ceil_div(sk_ceil_div(K, 128), SK_WAVES), pl.kpw);
     return pl;
 }
 
