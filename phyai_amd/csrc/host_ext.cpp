@@ -18,6 +18,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -43,7 +44,11 @@ struct Lib {
 struct Py {
     PyObject *workspaces, *owner, *reserve, *epilogues, *layouts, *view_type, *per_channel, *per_tensor;
 } py = {};
+struct PyLayers {
+    PyObject *dispatch_dict, *mode, *kernel_type;
+} pl = {};
 
+PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bias_add, *s_bias;
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
     *s_spec, *s_granularity;
 
@@ -327,22 +332,79 @@ bool layer_of(PyObject* o, Layer* l) {
     return true;
 }
 
+PyObject* layer_call(const Layer& l, PyObject* x, PyObject* bias, int epi, PyObject* residual, PyObject* gate) {
+    if (Py_TYPE(x) == (PyTypeObject*)py.view_type) {
+        if (l.granularity != py.per_channel || PyTuple_GET_SIZE(x) != 3 || PyTuple_GET_ITEM(x, 2) != py.per_channel) return nullptr;
+        return linear_call(PyTuple_GET_ITEM(x, 0), PyTuple_GET_ITEM(x, 1), l.weight, l.scale, bias, epi, l.layout, l.stream, Py_None,
+                           residual, gate);
+    }
+    if (l.granularity == py.per_channel)
+        return linear_call(x, nullptr, l.weight, l.scale, bias, epi, l.layout, l.stream, Py_None, residual, gate);
+    if (l.granularity == py.per_tensor && l.input_scale)
+        return linear_static_call(x, l.input_scale, l.weight, l.scale, bias, epi, l.layout, l.stream, residual, gate);
+    return nullptr;
+}
+
 // layer_apply(layer, x or ActivationView, bias, epilogue, residual, gate)
 PyObject* py_layer_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Layer l;
     int epi;
     if (n != 6 || !layer_of(a[0], &l) || !epilogue_of(a[3], &epi)) return declined();
-    PyObject* y = nullptr;
-    if (Py_TYPE(a[1]) == (PyTypeObject*)py.view_type) {
-        if (l.granularity != py.per_channel || PyTuple_GET_SIZE(a[1]) != 3 || PyTuple_GET_ITEM(a[1], 2) != py.per_channel) return declined();
-        y = linear_call(PyTuple_GET_ITEM(a[1], 0), PyTuple_GET_ITEM(a[1], 1), l.weight, l.scale, a[2], epi, l.layout, l.stream,
-                        Py_None, a[4], a[5]);
-    } else if (l.granularity == py.per_channel) {
-        y = linear_call(a[1], nullptr, l.weight, l.scale, a[2], epi, l.layout, l.stream, Py_None, a[4], a[5]);
-    } else if (l.granularity == py.per_tensor && l.input_scale) {
-        y = linear_static_call(a[1], l.input_scale, l.weight, l.scale, a[2], epi, l.layout, l.stream, a[4], a[5]);
-    }
+    PyObject* y = layer_call(l, a[1], a[2], epi, a[4], a[5]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+
+// Whether the dispatcher's remembered choice (LinearBase._kernel_for, which fills the memory this reads) for
+// this layer and input is the HIP kernel.  False also where nothing is remembered yet.
+bool hip_kernel_remembered(PyObject* layer, PyObject* x) {
+    PyObject** dp = _PyObject_GetDictPtr(layer);
+    if (!dp || !*dp || !pl.mode) return false;
+    PyObject* memo = PyDict_GetItemWithError(*dp, s_selected);   // (dispatcher, generation, spec, params_dtype, {key: kernel})
+    if (!memo || !PyTuple_CheckExact(memo) || PyTuple_GET_SIZE(memo) != 5) return false;
+    PyObject* d = PyDict_GetItemWithError(pl.dispatch_dict, s_dispatcher);
+    if (!d || d != PyTuple_GET_ITEM(memo, 0)) return false;
+    PyObject** dd = _PyObject_GetDictPtr(d);
+    PyObject* gen = dd && *dd ? PyDict_GetItemWithError(*dd, s_generation) : nullptr;
+    if (!gen || PyObject_RichCompareBool(gen, PyTuple_GET_ITEM(memo, 1), Py_EQ) != 1) return false;
+    PyObject* params_dtype = PyDict_GetItemWithError(*dp, s_params_dtype);
+    if (PyDict_GetItemWithError(*dp, s_spec) != PyTuple_GET_ITEM(memo, 2) || params_dtype != PyTuple_GET_ITEM(memo, 3)) return false;
+    const bool view = Py_TYPE(x) == (PyTypeObject*)py.view_type;
+    const at::Tensor* t = tensor(view && PyTuple_GET_SIZE(x) == 3 ? PyTuple_GET_ITEM(x, 0) : x);
+    if (!t || t->dim() < 1 || t->numel() == 0) return false;
+    const uint64_t M = (uint64_t)(t->numel() / t->size(t->dim() - 1));
+    PyObject* mode = nullptr;
+    if (PyContextVar_Get(pl.mode, nullptr, &mode) < 0 || !mode) return false;
+    PyObject* bits = PyLong_FromLong(64 - __builtin_clzll(M));
+    PyObject* key = PyTuple_Pack(3, bits, view ? params_dtype : (PyObject*)torch::getTHPDtype(t->scalar_type()), mode);
+    Py_XDECREF(bits);
+    Py_DECREF(mode);
+    if (!key) return false;
+    PyObject* kernel = PyDict_GetItemWithError(PyTuple_GET_ITEM(memo, 4), key);
+    Py_DECREF(key);
+    return kernel && Py_TYPE(kernel) == (PyTypeObject*)pl.kernel_type;
+}
+bool bias_of(PyObject* layer, PyObject** bias) {   // what the layer adds: None with skip_bias_add
+    PyObject** dp = _PyObject_GetDictPtr(layer);
+    PyObject* skip = PyDict_GetItemWithError(*dp, s_skip_bias_add);
+    PyObject* b = PyDict_GetItemWithError(PyDict_GetItemWithError(*dp, s_parameters), s_bias);
+    if (!skip || !b) return false;
+    *bias = skip == Py_False ? b : Py_None;
+    return skip == Py_False || skip == Py_True;
+}
+
+// layer_forward(layer, x or ActivationView, epilogue, residual, gate): selection and call in one
+PyObject* py_layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer l;
+    int epi;
+    PyObject* bias;
+    if (n != 5 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || !bias_of(a[0], &bias) || !epilogue_of(a[2], &epi))
+        return declined();
+    if (bias == Py_None && PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[0]), s_skip_bias_add) == Py_True && (epi != 0 || a[3] != Py_None))
+        return declined();   // fused forms exist for layers that add their own bias
+    PyObject* y = layer_call(l, a[1], bias, epi, a[3], a[4]);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -397,16 +459,20 @@ PyObject* py_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
-// mlp_apply(first layer, second layer, x, bias1, bias2, epilogue, residual, gate): both per-channel layers
-PyObject* py_mlp_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
+// mlp_forward(first layer, second layer, x, epilogue, residual, gate): both per-channel layers that add their own bias
+PyObject* py_mlp_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Layer p, q;
     int epi;
-    if (n != 8 || !layer_of(a[0], &p) || !layer_of(a[1], &q) || !epilogue_of(a[5], &epi) || p.granularity != py.per_channel ||
-        q.granularity != py.per_channel)
+    PyObject *b1, *b2;
+    if (n != 6 || !tensor(a[2]) || !hip_kernel_remembered(a[0], a[2]) || !hip_kernel_remembered(a[1], a[2]) || !layer_of(a[0], &p) ||
+        !layer_of(a[1], &q) || !epilogue_of(a[3], &epi) || p.granularity != py.per_channel || q.granularity != py.per_channel ||
+        !bias_of(a[0], &b1) || !bias_of(a[1], &b2))
         return declined();
-    PyObject* y = mlp_call(a[2], p.weight, p.scale, a[3], p.layout, p.stream, q.weight, q.scale, a[4], q.layout, q.stream, epi,
-                           Py_None, a[6], a[7]);
+    for (int i = 0; i < 2; ++i)
+        if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[i]), s_skip_bias_add) != Py_False) return declined();
+    PyObject* y = mlp_call(a[2], p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None,
+                           a[4], a[5]);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -461,10 +527,21 @@ PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+PyObject* view_of(at::Tensor& xq, at::Tensor& xs) {
+    PyObject *q = THPVariable_Wrap(std::move(xq)), *s = THPVariable_Wrap(std::move(xs));
+    PyObject* v = q && s ? PyObject_CallFunctionObjArgs(py.view_type, q, s, py.per_channel, nullptr) : nullptr;
+    Py_XDECREF(q);
+    Py_XDECREF(s);
+    return v;
+}
+
 // adarmsnorm(x, modulation, eps, quantize, want_out) -> (out, codes, scale, gate)
+// adarmsnorm(x, modulation, eps, True, False, hidden size) -> (ActivationView, gate), the rows of x and modulation
+// checked against the hidden size and (B, 3D) modulation rows serving the (S, D) rows of each item of the batch
 PyObject* py_adarmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    const at::Tensor *x = n == 5 ? tensor(a[0]) : nullptr, *m = n == 5 ? tensor(a[1]) : nullptr;
+    const at::Tensor *x = n >= 5 ? tensor(a[0]) : nullptr, *m = n >= 5 ? tensor(a[1]) : nullptr;
+    if (n == 6 && (!x || !m || x->dim() != 2 || m->dim() != 2 || x->size(1) != PyLong_AsLong(a[5]))) return declined();
     Rows r, q;
     Where at_;
     if (!x || !m || !rows_of(*x, at::kBFloat16, &r) || !rows_of(*m, at::kBFloat16, &q) || r.K % 8 != 0 || q.K != 3 * r.K ||
@@ -478,6 +555,7 @@ PyObject* py_adarmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (lib.adarmsnorm(r.p, r.ld, q.p, q.M > 1 ? q.ld : q.K, q.M, r.M, r.K, (float)eps, o.out_p(), r.K, gate.mutable_data_ptr(), r.K,
                        o.xq_p(), o.xs_p(), at_.stream) != 0)
         return declined();
+    if (n == 6) return Py_BuildValue("NN", view_of(o.xq, o.xs), THPVariable_Wrap(std::move(gate)));
     return Py_BuildValue("NNNN", wrap_or_none(o.out), wrap_or_none(o.xq), wrap_or_none(o.xs), THPVariable_Wrap(std::move(gate)));
     END_HANDLE_TH_ERRORS
 }
@@ -516,14 +594,27 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
+// bind_layers(phyai_amd.linear.dispatch's dictionary, mode variable, HipFp8Kernel)
+PyObject* py_bind_layers(PyObject*, PyObject* args) {
+    PyLayers p = {};
+    if (!PyArg_ParseTuple(args, "O!OO", &PyDict_Type, &p.dispatch_dict, &p.mode, &p.kernel_type)) return nullptr;
+    Py_INCREF(p.dispatch_dict);
+    Py_INCREF(p.mode);
+    Py_INCREF(p.kernel_type);
+    pl = p;
+    Py_RETURN_NONE;
+}
+
 #define PHYAI_FAST(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", py_bind, METH_VARARGS, nullptr},
+    {"bind_layers", py_bind_layers, METH_VARARGS, nullptr},
     PHYAI_FAST("linear", py_linear),
     PHYAI_FAST("gemm", py_gemm),
     PHYAI_FAST("mlp", py_mlp),
     PHYAI_FAST("layer_apply", py_layer_apply),
-    PHYAI_FAST("mlp_apply", py_mlp_apply),
+    PHYAI_FAST("layer_forward", py_layer_forward),
+    PHYAI_FAST("mlp_forward", py_mlp_forward),
     PHYAI_FAST("quant_rowwise", py_quant_rowwise),
     PHYAI_FAST("rmsnorm", py_rmsnorm),
     PHYAI_FAST("adarmsnorm", py_adarmsnorm),
@@ -537,7 +628,8 @@ PyMODINIT_FUNC PyInit__phyai_host() {
     const struct { PyObject** at; const char* text; } names[] = {
         {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_weight_scale, "weight_scale"}, {&s_input_scale, "input_scale"},
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
-        {&s_granularity, "granularity"}};
+        {&s_granularity, "granularity"}, {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
+        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}};
     for (const auto& e : names)
         if (!(*e.at = PyUnicode_InternFromString(e.text))) return nullptr;
     return PyModule_Create(&module);

@@ -21,6 +21,7 @@ from typing import Mapping, Sequence
 import torch
 import torch.nn as nn
 
+from phyai_amd import ops
 from phyai_amd.linear.dispatch import get_linear_dispatcher
 from phyai_amd.quant import AllocationRequest, Bf16Spec
 from phyai_amd.quant.types import ActivationView
@@ -138,14 +139,19 @@ class LinearBase(nn.Module):
             hook(self)
 
     # -- the hot call -----------------------------------------------------------------
-    def _run(self, x, add_bias: bool = True, **kernel_kwargs) -> torch.Tensor:
+    def _run(self, x, *, epilogue=None, residual=None, gate=None) -> torch.Tensor:
         """``x`` is the bf16 activations or, for an fp8 layer, an ``ActivationView`` that a norm
         already quantized per token (``phyai_amd.norm``): then the layer's own quantizer is skipped."""
+        if getattr(self.spec, "needs_act_quant", False):
+            y = ops._native().layer_forward(self, x, epilogue, residual, gate)
+            if y is not None:
+                return y
         if isinstance(x, ActivationView) and not getattr(self.spec, "needs_act_quant", False):
             raise RuntimeError(f"{type(self).__name__}: got quantized activations but spec "
                                f"{self.spec.spec_id!r} does not quantize its input")
-        bias = self._parameters["bias"] if (add_bias and not self.skip_bias_add) else None
-        return self._kernel_for(x).apply(self, x, bias, **kernel_kwargs)
+        bias = None if self.skip_bias_add else self._parameters["bias"]
+        extra = {k: v for k, v in (("epilogue", epilogue), ("residual", residual), ("gate", gate)) if v is not None}
+        return self._kernel_for(x).apply(self, x, bias, **extra)
 
     def _kernel_for(self, x):
         """The dispatcher's choice for this input.  Remembered per layer under what can change between two
@@ -179,6 +185,10 @@ class LinearBase(nn.Module):
         (the gated residual after ``o_proj`` / ``down_proj``, reference
         ``models/pi05/modeling_pi05.py:826,835``).  Falls back to the separate op for kernels
         without the extension."""
+        if getattr(self.spec, "needs_act_quant", False):
+            y = ops._native().layer_forward(self, x, None, residual, gate)
+            if y is not None:
+                return y
         if self.supports_fused_epilogue(x):
             return self._run(x, residual=residual, gate=gate)
         y, _ = self.forward(x)

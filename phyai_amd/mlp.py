@@ -116,11 +116,11 @@ class DenseMLP(nn.Module):
         (the decoder layer's gated residual, reference ``models/pi05/modeling_pi05.py:835``)."""
         mods = self._modules
         first, second = (mods["gate_up_proj"], mods["down_proj"]) if self.gated else (mods["fc1"], mods["fc2"])
-        if self._one_call(first, second, x):
-            y = ops._native().mlp_apply(first, second, x, first._parameters["bias"], second._parameters["bias"], self._epilogue,
-                                        residual, gate)
+        if self.fuse_activation and getattr(first.spec, "needs_act_quant", False):
+            y = ops._native().mlp_forward(first, second, x, self._epilogue, residual, gate)
             if y is not None:
                 return y
+        if self._one_call(first, second, x):
             return ops.fp8_mlp(x, first.weight, first.weight_scale, first.bias, second.weight, second.weight_scale,
                                second.bias, epilogue=self._epilogue, residual=residual, gate=gate,
                                stream_weights1=bool(getattr(first, "stream_weights", False)),

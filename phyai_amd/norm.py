@@ -129,6 +129,8 @@ class AdaRMSNorm(nn.Module):
 
     def forward_fp8(self, x: torch.Tensor, cond: torch.Tensor | None = None, *,
                     modulation: torch.Tensor | None = None) -> tuple[ActivationView, torch.Tensor]:
+        if cond is None and (got := ops._native().adarmsnorm(x, modulation, self.variance_epsilon, True, False, self.hidden_size)) is not None:
+            return got
         xq, xs, gate = ops.adarmsnorm_fp8(x, self._modulation(x, cond, modulation), self.variance_epsilon)
         return ActivationView(xq, xs, Granularity.PER_CHANNEL), gate
 

@@ -116,13 +116,17 @@ _host = None
 
 def _native():
     global _host
-    if _host is None:
+    if _host is None:   # (bound in full before anyone sees it: another thread may be in here as well)
         from phyai_amd.quant.types import ActivationView, Granularity
 
         _lib.load()
         ext = _lib.open_host_extension()
         ext.bind(_lib.LIB_PATH, _workspaces, _owner, reserve_workspace, EPILOGUES, WEIGHT_LAYOUTS, ActivationView,
                  Granularity.PER_CHANNEL, Granularity.PER_TENSOR)
+        from phyai_amd import state
+        from phyai_amd.linear import dispatch, kernels
+
+        ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel)
         _host = ext
     return _host
 

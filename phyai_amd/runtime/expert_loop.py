@@ -100,12 +100,14 @@ class ExpertLayer(nn.Module):
                 variant: str = "fused") -> torch.Tensor:
         residual = h
         if variant == "fused":
-            view, gate_attn = self.input_layernorm.forward_fp8(h, modulation=modulation.input_ln)
-            fused, _ = self.qkv_proj(view)
-            h = self.o_proj.forward_addcmul(attend(fused, index), residual, gate_attn)
-            view, gate_mlp = self.post_attention_layernorm.forward_fp8(h, modulation=modulation.post_attention_ln)
-            act = self.mlp.gate_up_proj.forward_fused(view, "geglu_tanh")
-            return self.mlp.down_proj.forward_addcmul(act, h, gate_mlp)
+            mods = self._modules   # (a module's attributes go through its __getattr__, a third of a microsecond each)
+            mlp = mods["mlp"]._modules
+            view, gate_attn = mods["input_layernorm"].forward_fp8(h, modulation=modulation.input_ln)
+            fused, _ = mods["qkv_proj"](view)
+            h = mods["o_proj"].forward_addcmul(attend(fused, index), residual, gate_attn)
+            view, gate_mlp = mods["post_attention_layernorm"].forward_fp8(h, modulation=modulation.post_attention_ln)
+            act = mlp["gate_up_proj"].forward_fused(view, "geglu_tanh")
+            return mlp["down_proj"].forward_addcmul(act, h, gate_mlp)
         if variant == "unfused":
             n, gate_attn = self.input_layernorm(h, modulation=modulation.input_ln)
             fused, _ = self.qkv_proj(n)
