@@ -214,6 +214,23 @@ int phyai_fp8_mlp(const void *x, int64_t ldx, const void *w1, const float *w1_sc
                   const void *residual, int64_t ld_res, const void *gate, int64_t ld_gate,
                   int64_t gate_rows, void *out, int64_t ldo, int64_t M, int64_t H, int64_t I,
                   int64_t O, int epilogue, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * phyai_fp8_linear / phyai_fp8_mlp on the output of an adaptive RMSNorm (phyai_fp8_adarmsnorm_quant's norm, bit for
+ * bit): x is the norm's input, modulation [mod_rows, >= 3 K (H)] bf16 = scale | shift | gate, the gate part not read.
+ * Up to 128 token rows, K (H) <= 2048, one modulation row, epilogue NONE or GEGLU_TANH, and a workgroup shape whose grid
+ * fits the chip: the norm runs inside the linear's one launch.  Otherwise the norm + quantizer kernel runs first.
+ */
+int phyai_fp8_adarmsnorm_linear(const void *x, int64_t ldx, const void *modulation, int64_t ld_mod, int64_t mod_rows,
+                                float eps, const void *w, const float *w_scale, const void *bias, void *out, int64_t ldo,
+                                int64_t M, int64_t N, int64_t K, int epilogue, void *workspace, size_t workspace_bytes,
+                                void *stream);
+int phyai_fp8_adarmsnorm_mlp(const void *x, int64_t ldx, const void *modulation, int64_t ld_mod, int64_t mod_rows,
+                             float eps, const void *w1, const float *w1_scale, const void *bias1, int flags1,
+                             const void *w2, const float *w2_scale, const void *bias2, int flags2, const void *residual,
+                             int64_t ld_res, const void *gate, int64_t ld_gate, int64_t gate_rows, void *out, int64_t ldo,
+                             int64_t M, int64_t H, int64_t I, int64_t O, int epilogue, void *workspace,
+                             size_t workspace_bytes, void *stream);
 /* "row maxima handed over: <first> | <second>" or "<first> | <second>", each part as
  * phyai_fp8_describe_linear_plan reports it.  Host only.  Row-major weights, or - with
  * PHYAI_FP8_FLAG_W_OPERAND_ORDER or-ed into `epilogue` - both matrices in operand order. */

@@ -274,37 +274,79 @@ int run_gemm(const char* fn, const void* xq, const float* x_scale, int x_scale_i
     return launch_prepared(fn, g, stream);
 }
 
+// An adaptive RMSNorm in front of a linear (phyai_fp8_adarmsnorm_linear / _mlp): modulation rows of scale | shift | gate.
+struct NormSpec {
+    const void* modulation;
+    int64_t ld_mod, mod_rows;
+    float eps;
+};
+int check_norm_spec(const char* fn, const NormSpec& n, int64_t M, int64_t D) {
+    if (D % 8 != 0 || D > (1 << 20)) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: D=%lld must be a multiple of 8 up to 2^20", fn, (long long)D);
+    if (!n.modulation || !aligned(n.modulation, 16) || n.ld_mod < 3 * D || n.ld_mod % 8 != 0)
+        return fail(PHYAI_FP8_EINVAL, "%s: modulation must be 16-byte aligned with row stride >= 3*D, a multiple of 8", fn);
+    if (n.mod_rows <= 0 || M % n.mod_rows != 0)
+        return fail(PHYAI_FP8_EINVAL, "%s: M=%lld must be a non-zero multiple of the modulation rows (%lld)", fn, (long long)M, (long long)n.mod_rows);
+    return 0;
+}
+// What turns bf16 rows into the codes at g.xq / g.x_scale in front of the GEMM `g`, unless the kernel that serves g does
+// that itself: the quantizer, or the norm with the quantizer behind it (g.x_bf16 is then dropped: those rows are not
+// what the GEMM multiplies).
+int launch_producer(const char* fn, const NormSpec* norm, phyai::GemmProblem* g, int64_t M, int64_t K, void* stream) {
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    uint8_t* xq = const_cast<uint8_t*>(g->xq);
+    float* xs = const_cast<float*>(g->x_scale);
+    if (norm == nullptr) {
+        if (phyai::gemm_quantizes_itself(*g)) return 0;
+        phyai::launch_quant_rowwise(g->x_bf16, M, K, g->ldx, xq, xs, st);
+        return check_launch(fn);
+    }
+    if (phyai::gemm_normalises_itself(*g)) return 0;
+    phyai::NormQuantArgs a = {};
+    a.x = g->x_bf16; a.ldx = g->ldx; a.D = (int)K; a.eps = norm->eps;
+    a.mod = static_cast<const uint16_t*>(norm->modulation); a.ld_mod = norm->ld_mod; a.group = (int)(M / norm->mod_rows);
+    a.xq = xq; a.scale = xs;
+    g->x_bf16 = nullptr;
+    g->norm_mod = nullptr;
+    if (phyai::launch_norm_quant(a, M, true, st) != 0) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: no norm kernel for D=%lld", fn, (long long)K);
+    return check_launch(fn);
+}
+void set_norm(const NormSpec* norm, phyai::GemmProblem* g) {
+    if (norm == nullptr || norm->mod_rows != 1) return;   // (the GEMM kernel takes one modulation row for all token rows)
+    g->norm_mod = static_cast<const uint16_t*>(norm->modulation);
+    g->norm_eps = norm->eps;
+}
+
 // Quantizer + GEMM with the codes and scales staged at xq / xs and the GEMM's own scratch at
 // gemm_ws.  Every argument of both launches is checked before the first one is enqueued.
 int run_linear_at(const char* fn, const void* x, int64_t ldx, const void* w, const float* w_scale, const void* bias,
                   const ResidualSpec& res, void* out, int64_t ldo, int64_t M, int64_t N, int64_t K, int epilogue,
-                  void* xq, float* xs, void* gemm_ws, size_t gemm_ws_bytes, void* stream) {
+                  void* xq, float* xs, void* gemm_ws, size_t gemm_ws_bytes, void* stream, const NormSpec* norm = nullptr) {
     if (int rc = check_quant_args(fn, x, M, K, ldx, xq)) return rc;
     phyai::GemmProblem g;
     if (int rc = prepare_gemm(fn, xq, xs, 0, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, gemm_ws,
                               gemm_ws_bytes, &g, x, ldx))
         return rc;
     // small token counts: one kernel quantizes its rows and multiplies them; otherwise two launches
-    if (!phyai::gemm_quantizes_itself(g)) {
-        phyai::launch_quant_rowwise(x, M, K, ldx, xq, xs, static_cast<hipStream_t>(stream));
-        if (int rc = check_launch(fn)) return rc;
-    }
+    set_norm(norm, &g);
+    if (int rc = launch_producer(fn, norm, &g, M, K, stream)) return rc;
     return launch_prepared(fn, g, stream);
 }
 
 int run_linear(const char* fn, const void* x, int64_t ldx, const void* w, const float* w_scale, const void* bias,
                const ResidualSpec& res, void* out, int64_t ldo, int64_t M, int64_t N, int64_t K, int epilogue,
-               void* workspace, size_t workspace_bytes, void* stream) {
+               void* workspace, size_t workspace_bytes, void* stream, const NormSpec* norm = nullptr) {
     if (M < 0 || N <= 0 || K <= 0)
         return fail(PHYAI_FP8_EINVAL, "%s: bad shape M=%lld N=%lld K=%lld", fn, (long long)M, (long long)N, (long long)K);
     if (M == 0) return PHYAI_FP8_OK;
+    if (norm)
+        if (int rc = check_norm_spec(fn, *norm, M, K)) return rc;
     const LinearCarve c = carve(M, N, K, epilogue & PHYAI_FP8_EPILOGUE_MASK);
     if (!workspace || workspace_bytes < c.total) {
         // The kernel that quantizes its own rows touches neither staged codes nor GEMM scratch: a call
         // that it serves needs no workspace at all (x stands in for the code and scale pointers, which
         // are never dereferenced then).
         phyai::GemmProblem g;
-        if (x && check_quant_args(fn, x, M, K, ldx, x) == 0 &&
+        if (!norm && x && check_quant_args(fn, x, M, K, ldx, x) == 0 &&
             prepare_gemm(fn, x, static_cast<const float*>(x), 0, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, nullptr,
                          0, &g, x, ldx) == 0 &&
             phyai::gemm_quantizes_itself(g))
@@ -315,7 +357,7 @@ int run_linear(const char* fn, const void* x, int64_t ldx, const void* w, const 
     if (!aligned(workspace, 256)) return fail(PHYAI_FP8_EINVAL, "%s: workspace must be 256-byte aligned", fn);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     return run_linear_at(fn, x, ldx, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, ws + c.xq_off,
-                         reinterpret_cast<float*>(ws + c.xs_off), workspace, c.gemm_bytes, stream);
+                         reinterpret_cast<float*>(ws + c.xs_off), workspace, c.gemm_bytes, stream, norm);
 }
 }  // namespace
 
@@ -380,11 +422,11 @@ size_t phyai_fp8_mlp_workspace_bytes(int64_t M, int64_t H, int64_t I, int64_t O,
     return mlp_carve(M, H, I, O, epilogue & PHYAI_FP8_EPILOGUE_MASK).total;
 }
 
-int phyai_fp8_mlp(const void* x, int64_t ldx, const void* w1, const float* w1_scale, const void* bias1, int flags1,
+namespace {
+int run_mlp(const char* fn, const NormSpec* norm, const void* x, int64_t ldx, const void* w1, const float* w1_scale, const void* bias1, int flags1,
                   const void* w2, const float* w2_scale, const void* bias2, int flags2, const void* residual,
                   int64_t ld_res, const void* gate, int64_t ld_gate, int64_t gate_rows, void* out, int64_t ldo, int64_t M,
                   int64_t H, int64_t I, int64_t O, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
-    const char* fn = "phyai_fp8_mlp";
     if (M < 0 || H <= 0 || I <= 0 || O <= 0)
         return fail(PHYAI_FP8_EINVAL, "%s: bad shape M=%lld H=%lld I=%lld O=%lld", fn, (long long)M, (long long)H, (long long)I, (long long)O);
     if ((epilogue & ~PHYAI_FP8_EPILOGUE_MASK) || epilogue <= PHYAI_FP8_EPI_NONE || epilogue > PHYAI_FP8_EPI_GELU_ERF)
@@ -392,6 +434,8 @@ int phyai_fp8_mlp(const void* x, int64_t ldx, const void* w1, const float* w1_sc
     if ((flags1 | flags2) & PHYAI_FP8_EPILOGUE_MASK) return fail(PHYAI_FP8_EINVAL, "%s: flags carry an epilogue", fn);
     if ((residual == nullptr) != (gate == nullptr)) return fail(PHYAI_FP8_EINVAL, "%s: residual and gate go together", fn);
     if (M == 0) return PHYAI_FP8_OK;
+    if (norm)
+        if (int rc = check_norm_spec(fn, *norm, M, H)) return rc;
     const MlpCarve c = mlp_carve(M, H, I, O, epilogue);
     if (!workspace || workspace_bytes < c.total)
         return fail(PHYAI_FP8_EWORKSPACE, "%s: workspace of %zu bytes is too small, need %zu", fn,
@@ -411,24 +455,48 @@ int phyai_fp8_mlp(const void* x, int64_t ldx, const void* w1, const float* w1_sc
     if (int rc = prepare_gemm(fn, ws + c.second.xq_off, reinterpret_cast<float*>(ws + c.second.xs_off), 0, w2, w2_scale, bias2,
                               res, out, ldo, M, O, I, PHYAI_FP8_EPI_NONE | flags2, workspace, c.second.gemm_bytes, &g2, h, I))
         return rc;
-    const int slots = phyai::gemm_row_maxima_slots(g1);
+    set_norm(norm, &g1);
+    if (norm && g1.norm_mod && !phyai::gemm_normalises_itself(g1)) g1.norm_mod = nullptr;
+    const bool first_on_codes = norm && !g1.norm_mod;   // the norm's own launch: no row maxima from a GEMM on ready codes
+    const int slots = first_on_codes ? 0 : phyai::gemm_row_maxima_slots(g1);
     if (slots > 0) {
         g2.amax_in = table;
         g2.amax_parts = slots;
         if (phyai::gemm_takes_row_maxima(g2)) g1.amax_out = table;
         else g2.amax_in = nullptr;
     }
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    if (!phyai::gemm_quantizes_itself(g1)) {
-        phyai::launch_quant_rowwise(x, M, H, ldx, ws + c.first.xq_off, reinterpret_cast<float*>(ws + c.first.xs_off), st);
-        if (int rc = check_launch(fn)) return rc;
-    }
+    if (int rc = launch_producer(fn, norm, &g1, M, H, stream)) return rc;
     if (int rc = launch_prepared(fn, g1, stream)) return rc;
-    if (!phyai::gemm_quantizes_itself(g2)) {
-        phyai::launch_quant_rowwise(h, M, I, I, ws + c.second.xq_off, reinterpret_cast<float*>(ws + c.second.xs_off), st);
-        if (int rc = check_launch(fn)) return rc;
-    }
+    if (int rc = launch_producer(fn, nullptr, &g2, M, I, stream)) return rc;
     return launch_prepared(fn, g2, stream);
+}
+}  // namespace
+
+int phyai_fp8_mlp(const void* x, int64_t ldx, const void* w1, const float* w1_scale, const void* bias1, int flags1,
+                  const void* w2, const float* w2_scale, const void* bias2, int flags2, const void* residual,
+                  int64_t ld_res, const void* gate, int64_t ld_gate, int64_t gate_rows, void* out, int64_t ldo, int64_t M,
+                  int64_t H, int64_t I, int64_t O, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
+    return run_mlp("phyai_fp8_mlp", nullptr, x, ldx, w1, w1_scale, bias1, flags1, w2, w2_scale, bias2, flags2, residual, ld_res, gate,
+                   ld_gate, gate_rows, out, ldo, M, H, I, O, epilogue, workspace, workspace_bytes, stream);
+}
+
+int phyai_fp8_adarmsnorm_mlp(const void* x, int64_t ldx, const void* modulation, int64_t ld_mod, int64_t mod_rows, float eps,
+                             const void* w1, const float* w1_scale, const void* bias1, int flags1, const void* w2,
+                             const float* w2_scale, const void* bias2, int flags2, const void* residual, int64_t ld_res,
+                             const void* gate, int64_t ld_gate, int64_t gate_rows, void* out, int64_t ldo, int64_t M,
+                             int64_t H, int64_t I, int64_t O, int epilogue, void* workspace, size_t workspace_bytes,
+                             void* stream) {
+    const NormSpec norm = {modulation, ld_mod, mod_rows, eps};
+    return run_mlp("phyai_fp8_adarmsnorm_mlp", &norm, x, ldx, w1, w1_scale, bias1, flags1, w2, w2_scale, bias2, flags2, residual, ld_res,
+                   gate, ld_gate, gate_rows, out, ldo, M, H, I, O, epilogue, workspace, workspace_bytes, stream);
+}
+
+int phyai_fp8_adarmsnorm_linear(const void* x, int64_t ldx, const void* modulation, int64_t ld_mod, int64_t mod_rows, float eps,
+                                const void* w, const float* w_scale, const void* bias, void* out, int64_t ldo, int64_t M,
+                                int64_t N, int64_t K, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
+    const NormSpec norm = {modulation, ld_mod, mod_rows, eps};
+    return run_linear("phyai_fp8_adarmsnorm_linear", x, ldx, w, w_scale, bias, ResidualSpec{}, out, ldo, M, N, K, epilogue, workspace,
+                      workspace_bytes, stream, &norm);
 }
 
 int phyai_fp8_linear_static(const void* x, int64_t ldx, const void* w, const float* w_scale, const void* bias,

@@ -113,14 +113,14 @@ def check_kernel(kernel: str, younger_loads_are_rows: int) -> list[str]:
 
 def rows_loaded(name: str) -> int:
     """Invisible loads of an instantiation, from its template arguments in the mangled name:
-    <ROWS, NT, KPW, EPI, STREAM, DIRECT, AMAX_IN>: KPW x ceil(ROWS / 4) row loads (at most 4 per 16-row block)
-    plus ceil(ROWS / 8) loads of handed-over maxima."""
-    m = re.search(r"ILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb([01])ELb([01])ELb([01])E", name)
+    <ROWS, NT, KPW, EPI, STREAM, DIRECT, AMAX_IN, NORM>: KPW x ceil(ROWS / 4) row loads (at most 4 per 16-row block)
+    plus ceil(ROWS / 8) loads of handed-over maxima or 2 x KPW loads of modulation."""
+    m = re.search(r"ILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb([01])ELb([01])ELb([01])ELb([01])E", name)
     if not m:
         raise AssertionError(f"cannot read the template arguments of {name}")
-    rows, _, kpw, _, _, _, amax_in = (int(g) for g in m.groups())
+    rows, _, kpw, _, _, _, amax_in, norm = (int(g) for g in m.groups())
     per_step = sum(min(4, (min(16, rows - 16 * mb) + 3) // 4) for mb in range((rows + 15) // 16))
-    return kpw * per_step + (((rows + 7) // 8) if amax_in else 0)
+    return kpw * per_step + (((rows + 7) // 8) if amax_in else 0) + (2 * kpw if norm else 0)
 
 
 def check_text(asm_text: str, min_kernels: int = 100) -> list[str]:

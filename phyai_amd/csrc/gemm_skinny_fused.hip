@@ -100,7 +100,15 @@ struct AmaxOut {
 //
 // AMAX_IN: the row maxima come from the producer of the activations (AmaxOut of an earlier launch)
 // instead of being found here: no table of per-wavefront maxima, no barrier before the conversions.
-template <int ROWS, int NT, int KPW, int EPI, bool STREAM, bool DIRECT, bool AMAX_IN>
+//
+// NORM: the rows are the input of an adaptive RMSNorm whose output the linear takes; every workgroup normalises the
+// rows it multiplies between their arrival and the search for their maxima.  One modulation row (scale | shift) serves
+// all token rows: a_amax_in is its address, a_amax_parts the bits of eps.  Costs a second table (sums of squares) and a
+// barrier, about 0.7 us, and saves the norm's own launch, 2.4 us with its node floor: the qkv_proj and gate_up_proj of
+// the expert layer at M = 50 take one launch each instead of two.  Bit-equal to norm_quant_kernel followed by this
+// kernel's other form: sums of squares are added in that kernel's order (8 elements of a lane, the 16 lanes of a K
+// step, K steps in fours, then the fours), everything after them element by element in the same operations.
+template <int ROWS, int NT, int KPW, int EPI, bool STREAM, bool DIRECT, bool AMAX_IN, bool NORM>
 __global__ __launch_bounds__(FQ_THREADS) void gemm_fp8_fusedq_kernel(
     const uint8_t* __restrict__ a_w, const uint8_t* __restrict__ a_x, int a_K, int a_N, int a_M, int a_ldx_bytes,
     const uint8_t* __restrict__ a_amax_in, int a_amax_parts, const float* __restrict__ a_w_scale,
@@ -122,11 +130,13 @@ __global__ __launch_bounds__(FQ_THREADS) void gemm_fp8_fusedq_kernel(
     // leaves no room: then it lies over the first wavefront's code block of K step 0, which nobody
     // writes before a second barrier has seen every wavefront read the table.
     constexpr int TBL_ROWS = ROWS < 64 ? ROWS : 64;
-    constexpr bool TBL_ALIASED = !AMAX_IN && FQ_WAVES * PER_WAVE + FQ_WAVES * 64 * 4 > 160 * 1024;
+    constexpr int SS_BYTES = NORM ? FQ_WAVES * KPW * ROWS * 4 : 0;    // sums of squares per K step and row
+    constexpr bool TBL_ALIASED = !AMAX_IN && FQ_WAVES * PER_WAVE + FQ_WAVES * 64 * 4 + SS_BYTES > 160 * 1024;
     static_assert(!TBL_ALIASED || FQ_WAVES * TBL_ROWS * 4 <= XB, "aliased table does not fit a code block");
     static_assert(ROWS == 8 || ROWS % 16 == 0, "token rows per workgroup");   // (4-row workgroups were measured: slower)
     static_assert(FQ_WAVES * PER_WAVE + ((TBL_ALIASED || AMAX_IN) ? 0 : FQ_WAVES * 64 * 4) <= 160 * 1024, "staging does not fit the LDS");
     static_assert(!AMAX_IN || (ROWS <= 16 && EPI == EPI_NONE), "row maxima are handed to plain projections of up to 16 rows per workgroup");
+    static_assert(!NORM || (!AMAX_IN && !TBL_ALIASED && ROWS <= 16 && KPW <= 2), "rows are normalised in blocks of up to 16, K <= 2048");
     constexpr int ROLE_ROUNDS = (NT * MB + FQ_WAVES - 1) / FQ_WAVES;
     constexpr int AL = AMAX_IN ? (ROWS + 7) / 8 : 0;  // loads of handed-over maxima per lane: 8 rows x 8 lanes x 16 bytes each
     constexpr int YOUNGER = KPW * NT * 2;             // weight requests issued behind the row loads
@@ -135,6 +145,7 @@ __global__ __launch_bounds__(FQ_THREADS) void gemm_fp8_fusedq_kernel(
     __shared__ __attribute__((aligned(1024))) uint8_t smem[FQ_WAVES * PER_WAVE];
     __shared__ uint32_t amax_own[(TBL_ALIASED || AMAX_IN) ? 1 : FQ_WAVES * 64];
     constexpr bool MAKES_AMAX = EPI != EPI_NONE;      // AmaxOut exists for the epilogues an MLP's first projection has
+    __shared__ float ss_tbl[NORM ? FQ_WAVES * KPW * ROWS : 1];   // NORM: [K step][row]
     __shared__ uint32_t amax_made[MAKES_AMAX ? 64 : 1];   // AmaxOut: maxima of this workgroup's outputs per token row
     uint32_t* amax_tbl = TBL_ALIASED ? reinterpret_cast<uint32_t*>(smem + WB) : amax_own;   // [wavefront][TBL_ROWS]
     auto red = [&](int w, int nt, int mb, int l) -> v4f& {
@@ -164,6 +175,17 @@ __global__ __launch_bounds__(FQ_THREADS) void gemm_fp8_fusedq_kernel(
             int r = m_base + a * 8 + (lane >> 3);
             r = r < M ? r : M - 1;
             am[a] = fq_load16_async(a_amax_in, (uint32_t)r * (kAmaxSlots * 2) + (lane & 7) * 16);
+        }
+    }
+    // (NORM: in front of the rows, this lane's 8 columns of scale and shift of every K step)
+    v4i mod_scale[NORM ? KPW : 1], mod_shift[NORM ? KPW : 1];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < KPW; ++j) {
+            const int s = __builtin_amdgcn_readfirstlane(j * FQ_WAVES + wave);
+            const uint8_t* at = a_amax_in + ((size_t)(s < total_steps ? s : total_steps - 1) << 8);
+            mod_scale[j] = fq_load16_async(at, xc * 16);
+            mod_shift[j] = fq_load16_async(at + (size_t)K * 2, xc * 16);
         }
     }
     v4i xv[KPW][MB][4];
@@ -291,6 +313,13 @@ __global__ __launch_bounds__(FQ_THREADS) void gemm_fp8_fusedq_kernel(
 #pragma unroll
         for (int a = 0; a < AL; ++a) fq_landed<YOUNGER>(am[a]);
     }
+    if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < KPW; ++j) {
+            fq_landed<YOUNGER>(mod_scale[j]);
+            fq_landed<YOUNGER>(mod_shift[j]);
+        }
+    }
 #pragma unroll
     for (int j = 0; j < KPW; ++j)
 #pragma unroll
@@ -300,6 +329,69 @@ __global__ __launch_bounds__(FQ_THREADS) void gemm_fp8_fusedq_kernel(
                 if (4 * i < rows_in_block(mb)) fq_landed<YOUNGER>(xv[j][mb][i]);
 
     PHYAI_STAMP(1)
+    if constexpr (NORM) {
+        auto unpack8 = [](v4i v, float* f) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                f[2 * i] = __uint_as_float((uint32_t)v[i] << 16);
+                f[2 * i + 1] = __uint_as_float((uint32_t)v[i] & 0xFFFF0000u);
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < KPW; ++j)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (4 * i >= rows_in_block(mb)) continue;
+                    float f[8], ss = 0.f;
+                    unpack8(xv[j][mb][i], f);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+                    ss += __uint_as_float(dpp_move_u32<0xB1>(__float_as_uint(ss)));      // the 16 lanes of a row
+                    ss += __uint_as_float(dpp_move_u32<0x4E>(__float_as_uint(ss)));
+                    ss += __uint_as_float(dpp_move_u32<0x141>(__float_as_uint(ss)));
+                    ss += __uint_as_float(dpp_move_u32<0x140>(__float_as_uint(ss)));
+                    if (xc == 0) ss_tbl[(j * FQ_WAVES + wave) * ROWS + mb * 16 + 4 * i + xr] = ss;
+                }
+        __syncthreads();
+        float rstd = 0.f;   // lane l: of row l
+        if (lane < ROWS) {
+            auto part = [&](int s) { return s < total_steps ? ss_tbl[s * ROWS + lane] : 0.f; };
+            float ss = 0.f;
+#pragma unroll
+            for (int g = 0; g < 2 * KPW; ++g) {
+                const float four = (part(4 * g) + part(4 * g + 1)) + (part(4 * g + 2) + part(4 * g + 3));
+                ss = g == 0 ? four : ss + four;
+            }
+            rstd = 1.0f / sqrtf(ss / (float)K + __uint_as_float((uint32_t)a_amax_parts));
+        }
+        float rstd_of[MB][4];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rstd_of[mb][i] = 4 * i < rows_in_block(mb) ? fq_bpermute(rstd, mb * 16 + 4 * i + xr) : 0.f;
+#pragma unroll
+        for (int j = 0; j < KPW; ++j) {
+            float sc[8], sh[8];
+            unpack8(mod_scale[j], sc);
+            unpack8(mod_shift[j], sh);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sc[e] = 1.0f + sc[e];
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (4 * i >= rows_in_block(mb)) continue;
+                    float f[8];
+                    unpack8(xv[j][mb][i], f);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) f[e] = (f[e] * rstd_of[mb][i]) * sc[e] + sh[e];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) xv[j][mb][i][e] = (int)pack_bf16x2(f[2 * e], f[2 * e + 1]);
+                }
+        }
+    }
     // ---- row scales: lane l holds the scale of "its" row and the reciprocal ----------------------------
     // own maxima: lane l <-> row l, every wavefront derives all scales from the table; handed-over maxima:
     // lanes 8 r .. 8 r + 7 of register set a <-> row 8 a + r
@@ -579,12 +671,13 @@ static int fq_ceil_div(int a, int b) { return (a + b - 1) / b; }
 // LDS of a workgroup shape, as the kernel lays it out (the table of row maxima has its own 2 KB unless
 // only the staging fits, see the kernel; none with handed-over maxima; weights that go straight to
 // registers are not staged).
-static constexpr bool fq_fits(int rows, int nt, int kpw, bool direct, bool amax_in, bool act_epilogue) {
+static constexpr bool fq_fits(int rows, int nt, int kpw, bool direct, bool amax_in, bool act_epilogue, bool norm = false) {
     const int mb = (rows + 15) / 16;
     const int xb = rows < 16 ? rows * 128 : 2048;
     const int stage = kpw * ((direct ? 0 : nt * 2048) + mb * xb), redb = nt * mb * 1024;
     const int waves = FQ_WAVES * (stage > redb ? stage : redb) + (act_epilogue ? 256 : 0);   // + the table of AmaxOut
     if (amax_in) return rows <= 16 && waves <= 160 * 1024;
+    if (norm) return rows <= 16 && kpw <= 2 && waves + FQ_WAVES * 64 * 4 + FQ_WAVES * kpw * rows * 4 <= 160 * 1024;
     if (waves + FQ_WAVES * 64 * 4 <= 160 * 1024) return true;
     return waves <= 160 * 1024 && FQ_WAVES * (rows < 64 ? rows : 64) * 4 <= xb;
 }
@@ -604,11 +697,15 @@ static constexpr bool fq_amax_in_shape(int rows, int nt) {
     return (rows == 8 && (nt == 2 || nt == 4)) || (rows == 16 && (nt == 1 || nt == 2));
 }
 
-FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout, bool amax_in) {
+// Rows normalised in the kernel (NORM): the epilogues that follow an adaptive norm in a decoder layer.
+static constexpr bool fq_norm_epilogue(int epi) { return epi == EPI_NONE || epi == EPI_GEGLU_TANH; }
+
+FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout, bool amax_in, bool norm) {
     FusedPlan pl = {0, 0, 0, 0, 0};
     if (const char* e = tuning_env("PHYAI_FP8_FUSED")) { if (atoi(e) == 0) return pl; }
     if (M < 1 || M > kFusedMaxM || K % 128 != 0 || K > 4096 || ldo % 4 != 0) return pl;
     if (amax_in && epilogue != EPI_NONE) return pl;
+    if (norm && (amax_in || K > 2048 || !fq_norm_epilogue(epilogue))) return pl;
     const bool gated = epi_is_gated(epilogue);
     const bool direct = weight_layout != W_ROW_MAJOR;
     const int cols = gated ? N / 2 : N;
@@ -632,7 +729,7 @@ FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_
     const bool long_k_alone = K > 2048 && !amax_in && !forced_rows;
     for (const auto& sh : kFusedShapes) {
         const int rows = sh[0], nt = sh[1];
-        if (!fq_fits(rows, nt, kpw, direct, amax_in, epilogue != EPI_NONE) || !fq_regs_ok(rows, nt, kpw, direct)) continue;
+        if (!fq_fits(rows, nt, kpw, direct, amax_in, epilogue != EPI_NONE, norm) || !fq_regs_ok(rows, nt, kpw, direct)) continue;
         if (amax_in && !fq_amax_in_shape(rows, nt)) continue;
         if (long_k_alone && (rows != 8 || nt != 2)) continue;
         if (forced_rows && (rows != forced_rows || nt != forced_nt)) continue;
@@ -641,7 +738,7 @@ FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_
             if (rows > 16 && (rows >= 2 * M || M > 64)) continue;              // blocks that do not exist; see kFusedMaxM
             if ((int64_t)tiles * msplit > 256) continue;
         }
-        const double conv = (double)rows * K * 5.5 / 64.0;                      // cycles of VALU per workgroup
+        const double conv = (double)rows * K * (norm ? 11.0 : 5.5) / 64.0;                      // cycles of VALU per workgroup
         const double pull = (double)(nt * 16 + rows * 2) * K / 50.0;           // bytes through the vector cache
         // workgroups that share a weight tile sit on one XCD (and fetch the tile from HBM once) only when
         // the tile count is a multiple of 8: 27 tiles instead of 32 made qkv 1.6 x slower
@@ -653,21 +750,25 @@ FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_
     return pl;
 }
 
-template <int ROWS, int NT, int KPW, int EPI, bool DIRECT, bool AMAX_IN>
+template <int ROWS, int NT, int KPW, int EPI, bool DIRECT, bool AMAX_IN, bool NORM = false>
 static int fq_launch_one(const GemmProblem& g, const FusedPlan& pl, hipStream_t st) {
     if constexpr (!fq_fits(ROWS, NT, KPW, DIRECT, AMAX_IN, EPI != EPI_NONE) || !fq_regs_ok(ROWS, NT, KPW, DIRECT) ||
-                  (AMAX_IN && (EPI != EPI_NONE || !fq_amax_in_shape(ROWS, NT)))) {
+                  (AMAX_IN && (EPI != EPI_NONE || !fq_amax_in_shape(ROWS, NT))) ||
+                  (NORM && (!fq_norm_epilogue(EPI) || !fq_fits(ROWS, NT, KPW, DIRECT, AMAX_IN, EPI != EPI_NONE, true)))) {
         return -2;
     } else {
         const AmaxOut made = {EPI != EPI_NONE ? g.amax_out : nullptr};
         const int m_flags = g.M;   // (weights in operand order take the DIRECT kernels)
+        const uint8_t* handed = reinterpret_cast<const uint8_t*>(NORM ? g.norm_mod : g.amax_in);
+        int parts = g.amax_parts;
+        if (NORM) __builtin_memcpy(&parts, &g.norm_eps, sizeof(parts));
 #define PHYAI_FQ_ARGS g.w, reinterpret_cast<const uint8_t*>(g.x_bf16), g.K, g.N, m_flags, (int)(g.ldx * 2),                     \
-                      reinterpret_cast<const uint8_t*>(g.amax_in), g.amax_parts, g.w_scale, g.bias, g.out, g.ldo, residual_of(g), made
+                      handed, parts, g.w_scale, g.bias, g.out, g.ldo, residual_of(g), made
         if (g.stream_weights)
-            hipLaunchKernelGGL((gemm_fp8_fusedq_kernel<ROWS, NT, KPW, EPI, true, DIRECT, AMAX_IN>), dim3(pl.tiles, pl.msplit),
+            hipLaunchKernelGGL((gemm_fp8_fusedq_kernel<ROWS, NT, KPW, EPI, true, DIRECT, AMAX_IN, NORM>), dim3(pl.tiles, pl.msplit),
                                dim3(FQ_THREADS), 0, st, PHYAI_FQ_ARGS);
         else
-            hipLaunchKernelGGL((gemm_fp8_fusedq_kernel<ROWS, NT, KPW, EPI, false, DIRECT, AMAX_IN>), dim3(pl.tiles, pl.msplit),
+            hipLaunchKernelGGL((gemm_fp8_fusedq_kernel<ROWS, NT, KPW, EPI, false, DIRECT, AMAX_IN, NORM>), dim3(pl.tiles, pl.msplit),
                                dim3(FQ_THREADS), 0, st, PHYAI_FQ_ARGS);
 #undef PHYAI_FQ_ARGS
         return 0;
@@ -677,6 +778,15 @@ static int fq_launch_one(const GemmProblem& g, const FusedPlan& pl, hipStream_t 
 template <int ROWS, int NT, int KPW, int EPI>
 static int fq_launch_variant(const GemmProblem& g, const FusedPlan& pl, hipStream_t st) {
     const bool direct = g.weight_layout != W_ROW_MAJOR;
+    if (g.norm_mod != nullptr) {
+        if constexpr (fq_norm_epilogue(EPI) && ROWS <= 16 && KPW <= 2) {
+            if (g.amax_in != nullptr) return -2;
+            return direct ? fq_launch_one<ROWS, NT, KPW, EPI, true, false, true>(g, pl, st)
+                          : fq_launch_one<ROWS, NT, KPW, EPI, false, false, true>(g, pl, st);
+        } else {
+            return -2;
+        }
+    }
     if (g.amax_in != nullptr) {
         if constexpr (EPI == EPI_NONE) {
             return direct ? fq_launch_one<ROWS, NT, KPW, EPI, true, true>(g, pl, st)

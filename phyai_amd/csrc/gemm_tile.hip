@@ -382,8 +382,13 @@ struct GemmChoice {
 // have_x: the bf16 activations are at hand (whole-linear entry points), so a kernel that quantizes
 // its own rows may serve the call.
 static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
-                              int layout = W_ROW_MAJOR, bool amax_in = false) {
+                              int layout = W_ROW_MAJOR, bool amax_in = false, bool norm = false) {
     GemmChoice c = {};
+    if (norm) {   // rows still to be normalised: one kernel does it or the caller launches the norm itself
+        c.kind = GemmChoice::FUSED;
+        if (have_x && vec_ok) c.fq = fused_plan(M, N, K, epilogue, ldo, layout, false, true);
+        return c;
+    }
     if (have_x && vec_ok) {
         if (amax_in) {
             c.fq = fused_plan(M, N, K, epilogue, ldo, layout, true);
@@ -427,7 +432,12 @@ static GemmChoice choose_gemm(const GemmProblem& g) {
                         g.K < (1 << 24) && g.N < (1 << 24) && !g.x_scale_is_scalar;
     return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout,
                        g.amax_in != nullptr && g.amax_parts >= 1 && g.amax_parts <= kRowAmaxSlots &&
-                           (reinterpret_cast<uintptr_t>(g.amax_in) & 15) == 0);
+                           (reinterpret_cast<uintptr_t>(g.amax_in) & 15) == 0,
+                       g.norm_mod != nullptr);
+}
+
+bool gemm_normalises_itself(const GemmProblem& g) {
+    return g.M != 0 && g.N != 0 && g.norm_mod != nullptr && (reinterpret_cast<uintptr_t>(g.norm_mod) & 15) == 0 && choose_gemm(g).fq.rows != 0;
 }
 
 int gemm_row_maxima_slots(const GemmProblem& g) {
@@ -509,6 +519,7 @@ int launch_gemm(const GemmProblem& g, hipStream_t st) {
     const GemmChoice ch = choose_gemm(g);
     if (ch.need > 0 && (g.workspace == nullptr || g.workspace_bytes < ch.need)) return -3;
     if (ch.kind == GemmChoice::FUSED) {
+        if (ch.fq.rows == 0) return -2;
         if (g.amax_in != nullptr && !ch.takes_amax) {   // the plan finds the row maxima itself
             GemmProblem own = g;
             own.amax_in = nullptr;

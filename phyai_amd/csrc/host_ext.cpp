@@ -33,6 +33,8 @@ struct Lib {
     decltype(&phyai_fp8_gemm) gemm;
     decltype(&phyai_fp8_gemm_addcmul) gemm_addcmul;
     decltype(&phyai_fp8_mlp) mlp;
+    decltype(&phyai_fp8_adarmsnorm_linear) norm_linear;
+    decltype(&phyai_fp8_adarmsnorm_mlp) norm_mlp;
     decltype(&phyai_fp8_linear_workspace_bytes) linear_ws;
     decltype(&phyai_fp8_mlp_workspace_bytes) mlp_ws;
     decltype(&phyai_fp8_quant_rowwise) quant_rowwise;
@@ -200,9 +202,32 @@ bool residual_of(PyObject* r_, PyObject* g_, const at::Tensor& x, int64_t M, int
     return true;
 }
 
+// Rows of scale | shift | gate of an adaptive norm of width D.
+struct Modulation {
+    const uint8_t* p;
+    int64_t rows, ld, D;
+    double eps;
+};
+bool modulation_of(PyObject* m_, PyObject* eps, int64_t D, int64_t M, Modulation* out) {
+    const at::Tensor* m = tensor(m_);
+    Rows q;
+    if (!m || m->dim() != 2 || !rows_of(*m, at::kBFloat16, &q) || q.K != 3 * D || D % 8 != 0 || M % q.M != 0) return false;
+    *out = {static_cast<const uint8_t*>(q.p), q.M, q.M > 1 ? q.ld : q.K, D, eps ? PyFloat_AsDouble(eps) : 0.0};
+    return !PyErr_Occurred();
+}
+// residual + gate part of a modulation row (one row per group of token rows)
+bool residual_gated_by(PyObject* r_, PyObject* m_, const at::Tensor& x, int64_t M, int64_t N, Residual* out) {
+    const at::Tensor* r = tensor(r_);
+    Modulation m;
+    if (!r || !shaped(r, x, N, at::kBFloat16) || !modulation_of(m_, nullptr, N, M, &m)) return false;
+    *out = {r->const_data_ptr(), m.p + 4 * N, m.ld, m.rows};
+    return true;
+}
+
 // bf16 rows `x_`, or codes `x_` with their scales `xs_` when that is given -> output tensor, null when declined.
 PyObject* linear_call(PyObject* x_, PyObject* xs_, PyObject* w_, PyObject* ws_, PyObject* b_, int epi, PyObject* layout,
-                      bool stream, PyObject* out_, PyObject* res_, PyObject* gate_) {
+                      bool stream, PyObject* out_, PyObject* res_, PyObject* gate_, bool gate_in_modulation = false,
+                      PyObject* mod_ = nullptr, PyObject* eps_ = nullptr) {
     const at::Tensor* x = tensor(x_);
     if (!x) return nullptr;
     Rows r;
@@ -223,7 +248,10 @@ PyObject* linear_call(PyObject* x_, PyObject* xs_, PyObject* w_, PyObject* ws_, 
         scalar = s->numel() == 1 && r.M != 1;
     }
     Residual rg;
-    if (!residual_of(res_, gate_, *x, r.M, w.N, epi, &rg)) return nullptr;
+    if (gate_in_modulation ? epi != 0 || !residual_gated_by(res_, gate_, *x, r.M, w.N, &rg) : !residual_of(res_, gate_, *x, r.M, w.N, epi, &rg))
+        return nullptr;
+    Modulation mod = {};
+    if (mod_ && (codes || rg.residual || !modulation_of(mod_, eps_, r.K, r.M, &mod))) return nullptr;
     const int64_t n_out = is_gated(epi) ? w.N / 2 : w.N;
     at::Tensor made;
     void* out;
@@ -239,7 +267,10 @@ PyObject* linear_call(PyObject* x_, PyObject* xs_, PyObject* w_, PyObject* ws_, 
     if (!workspace(lib.linear_ws(r.M, w.N, r.K, epi), at_, &ws)) return nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    if (codes)
+    if (mod_)
+        rc = lib.norm_linear(r.p, r.ld, mod.p, mod.ld, mod.rows, (float)mod.eps, w.w, w.scale, w.bias, out, n_out, r.M, w.N, r.K,
+                             epi | flags, ws.p, ws.n, at_.stream);
+    else if (codes)
         rc = rg.residual ? lib.gemm_addcmul(r.p, xs, scalar, w.w, w.scale, w.bias, rg.residual, w.N, rg.gate, rg.ld_gate, rg.gate_rows,
                                             out, n_out, r.M, w.N, r.K, flags, ws.p, ws.n, at_.stream)
                          : lib.gemm(r.p, xs, scalar, w.w, w.scale, w.bias, out, n_out, r.M, w.N, r.K, epi | flags, ws.p, ws.n, at_.stream);
@@ -412,7 +443,7 @@ PyObject* py_layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // ---- MLP ------------------------------------------------------------------------------------------------------------
 PyObject* mlp_call(PyObject* x_, PyObject* w1_, PyObject* s1_, PyObject* b1_, PyObject* lay1, bool st1, PyObject* w2_,
                    PyObject* s2_, PyObject* b2_, PyObject* lay2, bool st2, int epi, PyObject* out_, PyObject* res_,
-                   PyObject* gate_) {
+                   PyObject* gate_, PyObject* mod_ = nullptr, PyObject* eps_ = nullptr) {
     const at::Tensor* x = tensor(x_);
     Rows r;
     Where at_;
@@ -423,7 +454,9 @@ PyObject* mlp_call(PyObject* x_, PyObject* w1_, PyObject* s1_, PyObject* b1_, Py
     if (is_gated(epi) && w1.N % 32 != 0) return nullptr;
     const int64_t I = is_gated(epi) ? w1.N / 2 : w1.N;
     if (!weight_of(w2_, s2_, b2_, I, &w2) || !flags_of(lay1, st1, epi, &f1) || !flags_of(lay2, st2, 0, &f2)) return nullptr;
-    if (!residual_of(res_, gate_, *x, r.M, w2.N, 0, &rg)) return nullptr;
+    Modulation mod = {};
+    if (mod_ && !modulation_of(mod_, eps_, r.K, r.M, &mod)) return nullptr;
+    if (mod_ ? !residual_gated_by(res_, mod_, *x, r.M, w2.N, &rg) : !residual_of(res_, gate_, *x, r.M, w2.N, 0, &rg)) return nullptr;
     at::Tensor made;
     void* out;
     if (out_ == Py_None) {
@@ -438,8 +471,12 @@ PyObject* mlp_call(PyObject* x_, PyObject* w1_, PyObject* s1_, PyObject* b1_, Py
     if (!workspace(lib.mlp_ws(r.M, r.K, I, w2.N, epi), at_, &ws)) return nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.mlp(r.p, r.ld, w1.w, w1.scale, w1.bias, f1, w2.w, w2.scale, w2.bias, f2, rg.residual, rg.residual ? w2.N : 0, rg.gate,
-                 rg.ld_gate, rg.gate_rows, out, w2.N, r.M, r.K, I, w2.N, epi, ws.p, ws.n, at_.stream);
+    if (mod_)
+        rc = lib.norm_mlp(r.p, r.ld, mod.p, mod.ld, mod.rows, (float)mod.eps, w1.w, w1.scale, w1.bias, f1, w2.w, w2.scale, w2.bias, f2,
+                          rg.residual, w2.N, rg.gate, rg.ld_gate, rg.gate_rows, out, w2.N, r.M, r.K, I, w2.N, epi, ws.p, ws.n, at_.stream);
+    else
+        rc = lib.mlp(r.p, r.ld, w1.w, w1.scale, w1.bias, f1, w2.w, w2.scale, w2.bias, f2, rg.residual, rg.residual ? w2.N : 0, rg.gate,
+                     rg.ld_gate, rg.gate_rows, out, w2.N, r.M, r.K, I, w2.N, epi, ws.p, ws.n, at_.stream);
     Py_END_ALLOW_THREADS
     if (rc != 0) return nullptr;
     if (out_ != Py_None) {
@@ -473,6 +510,49 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[i]), s_skip_bias_add) != Py_False) return declined();
     PyObject* y = mlp_call(a[2], p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None,
                            a[4], a[5]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- a decoder layer's three calls: adaptive norm + linear, linear + gated residual, adaptive norm + MLP + gated residual
+// norm_linear(layer, x, modulation, eps): layer(norm(x)), x in rows of the layer's input width
+PyObject* py_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer l;
+    PyObject* bias;
+    if (n != 4 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || l.granularity != py.per_channel || !bias_of(a[0], &bias) ||
+        PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[0]), s_skip_bias_add) != Py_False)
+        return declined();
+    PyObject* y = linear_call(a[1], nullptr, l.weight, l.scale, bias, 0, l.layout, l.stream, Py_None, Py_None, Py_None, false, a[2], a[3]);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+// linear_residual(layer, x, residual, modulation): residual + layer(x) * gate part of the modulation
+PyObject* py_linear_residual(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer l;
+    PyObject* bias;
+    if (n != 4 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || l.granularity != py.per_channel || !bias_of(a[0], &bias) ||
+        PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[0]), s_skip_bias_add) != Py_False)
+        return declined();
+    PyObject* y = linear_call(a[1], nullptr, l.weight, l.scale, bias, 0, l.layout, l.stream, Py_None, a[2], a[3], true);
+    return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+// norm_mlp(first layer, second layer, x, modulation, eps, epilogue): x + mlp(norm(x)) * gate part of the modulation
+PyObject* py_norm_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer p, q;
+    int epi;
+    PyObject *b1, *b2;
+    if (n != 6 || !tensor(a[2]) || !hip_kernel_remembered(a[0], a[2]) || !hip_kernel_remembered(a[1], a[2]) || !layer_of(a[0], &p) ||
+        !layer_of(a[1], &q) || !epilogue_of(a[5], &epi) || p.granularity != py.per_channel || q.granularity != py.per_channel ||
+        !bias_of(a[0], &b1) || !bias_of(a[1], &b2))
+        return declined();
+    for (int i = 0; i < 2; ++i)
+        if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[i]), s_skip_bias_add) != Py_False) return declined();
+    PyObject* y = mlp_call(a[2], p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None,
+                           a[2], nullptr, a[3], a[4]);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -581,6 +661,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     get(l.gemm, "phyai_fp8_gemm");
     get(l.gemm_addcmul, "phyai_fp8_gemm_addcmul");
     get(l.mlp, "phyai_fp8_mlp");
+    get(l.norm_linear, "phyai_fp8_adarmsnorm_linear");
+    get(l.norm_mlp, "phyai_fp8_adarmsnorm_mlp");
     get(l.linear_ws, "phyai_fp8_linear_workspace_bytes");
     get(l.mlp_ws, "phyai_fp8_mlp_workspace_bytes");
     get(l.quant_rowwise, "phyai_fp8_quant_rowwise");
@@ -615,6 +697,9 @@ PyMethodDef methods[] = {
     PHYAI_FAST("layer_apply", py_layer_apply),
     PHYAI_FAST("layer_forward", py_layer_forward),
     PHYAI_FAST("mlp_forward", py_mlp_forward),
+    PHYAI_FAST("norm_linear", py_norm_linear),
+    PHYAI_FAST("linear_residual", py_linear_residual),
+    PHYAI_FAST("norm_mlp", py_norm_mlp),
     PHYAI_FAST("quant_rowwise", py_quant_rowwise),
     PHYAI_FAST("rmsnorm", py_rmsnorm),
     PHYAI_FAST("adarmsnorm", py_adarmsnorm),

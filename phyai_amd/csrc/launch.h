@@ -77,6 +77,10 @@ struct GemmProblem {
     uint16_t* amax_out;
     const uint16_t* amax_in;
     int amax_parts;
+    // x_bf16 is the input of an adaptive RMSNorm (eps norm_eps) and this its modulation row, scale | shift of K bf16
+    // each, for all token rows: the one-launch small-M kernel normalises the rows itself (fused_plan with norm).
+    const uint16_t* norm_mod;
+    float norm_eps;
 };
 
 // What the kernels need of the above, by value.
@@ -103,6 +107,8 @@ int launch_gemm(const GemmProblem& p, hipStream_t st);
 // True when launch_gemm would serve this problem (x_bf16 set) with the kernel that quantizes its own
 // rows: the caller then skips the quantizer launch.
 bool gemm_quantizes_itself(const GemmProblem& p);
+// True when launch_gemm would serve this problem (x_bf16 and norm_mod set) with the kernel that normalises its rows too.
+bool gemm_normalises_itself(const GemmProblem& p);
 // Row maxima handed from one linear to the next (GemmProblem::amax_out / amax_in).  Slots per token row
 // that launch_gemm would write for this producer (x_bf16 set, an activation epilogue), 0 when the kernel
 // that serves it cannot; whether launch_gemm would serve this consumer (amax_in, amax_parts set) with
@@ -134,7 +140,7 @@ struct FusedPlan {
     int tiles;   // workgroups along N
     int msplit;  // workgroups along M
 };
-FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout = 0, bool amax_in = false);
+FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout = 0, bool amax_in = false, bool norm = false);
 constexpr int kRowAmaxSlots = 64;   // slots per token row of a table of handed-over row maxima
 int launch_gemm_fused(const GemmProblem& p, const FusedPlan& pl, hipStream_t st);
 

@@ -16,9 +16,10 @@ not a kernel of this package.
 
 Three forms of the layer run on the same weights:
 
-``fused``    norm + quantizer in one kernel, GEMM on its codes, attention, GEMM with the gated
-             residual in its epilogue, norm + quantizer, GEMM + GeGLU epilogue, GEMM + gated
-             residual: 8 kernels of this library per layer;
+``fused``    norm + quantizer + GEMM, attention, quantizer + GEMM with the gated residual in its epilogue,
+             norm + quantizer + GEMM + GeGLU epilogue, quantizer + GEMM + gated residual: four kernels
+             of this library per layer up to 128 token rows (each norm and quantizer runs inside the
+             linear behind it), 8 beyond;
 ``unfused``  the reference's structure on this library's kernels: norm, quantized linear,
              attention, quantized linear, ``torch.addcmul``, norm, MLP, ``torch.addcmul``
              (12 kernels per layer).  Bit-equal to ``fused``;
@@ -36,6 +37,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from phyai_amd import ops
 from phyai_amd.linear import QKVParallelLinear, ReplicatedLinear, RowParallelLinear
 from phyai_amd.mlp import DenseMLP
 from phyai_amd.norm import AdaRMSNorm
@@ -102,6 +104,9 @@ class ExpertLayer(nn.Module):
         if variant == "fused":
             mods = self._modules   # (a module's attributes go through its __getattr__, a third of a microsecond each)
             mlp = mods["mlp"]._modules
+            out = self._three_calls(mods, mlp, h, attend, index, modulation)
+            if out is not None:
+                return out
             view, gate_attn = mods["input_layernorm"].forward_fp8(h, modulation=modulation.input_ln)
             fused, _ = mods["qkv_proj"](view)
             h = mods["o_proj"].forward_addcmul(attend(fused, index), residual, gate_attn)
@@ -123,6 +128,33 @@ class ExpertLayer(nn.Module):
             act = _torch_fp8_linear(m, self.mlp.gate_up_proj, act=True)
             return torch.addcmul(h, _torch_fp8_linear(act, self.mlp.down_proj), gate_mlp)
         raise ValueError(f"unknown variant {variant!r}; expected one of {VARIANTS}")
+
+
+    def _three_calls(self, mods, mlp, h, attend: Attend, index: int, modulation: ExpertLayerModulation):
+        """The layer as three library calls around attention: norm + qkv_proj, o_proj + gated residual, norm + MLP +
+        gated residual; for few token rows each norm runs inside the linear that follows it.  The gates are read where
+        they lie in the modulation rows.  Same bits as the calls below; None when this form does not serve the input."""
+        if h.dim() != 2 or h.shape[1] != self.hidden_size:
+            return None
+        native, qkv, o = ops._native(), mods["qkv_proj"], mods["o_proj"]
+        first, second = mlp["gate_up_proj"], mlp["down_proj"]
+        fused = native.norm_linear(qkv, h, modulation.input_ln, mods["input_layernorm"].variance_epsilon)
+        if fused is None:
+            if not all(lin.supports_fused_epilogue(h) for lin in (qkv, o, first, second)):
+                return None
+            # (the dispatcher's choice for this token count and mode is remembered now)
+            fused = native.norm_linear(qkv, h, modulation.input_ln, mods["input_layernorm"].variance_epsilon)
+            if fused is None:
+                return None
+        a = attend(fused, index)
+        r = native.linear_residual(o, a, h, modulation.input_ln)
+        if r is None:
+            r = o.forward_addcmul(a, h, modulation.input_ln[:, 2 * self.hidden_size:].contiguous())
+        out = native.norm_mlp(first, second, r, modulation.post_attention_ln, mods["post_attention_layernorm"].variance_epsilon, "geglu_tanh")
+        if out is None:
+            view, gate_mlp = mods["post_attention_layernorm"].forward_fp8(r, modulation=modulation.post_attention_ln)
+            out = second.forward_addcmul(first.forward_fused(view, "geglu_tanh"), r, gate_mlp)
+        return out
 
 
 class PrefixAttentionStandIn:
