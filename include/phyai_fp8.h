@@ -216,6 +216,16 @@ int phyai_fp8_mlp(const void *x, int64_t ldx, const void *w1, const float *w1_sc
                   int64_t O, int epilogue, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * phyai_fp8_quant_static + phyai_fp8_gemm (x_scale_is_scalar = 1) as one call: a linear whose activations have one
+ * static scale (layers/linear/backends/torch.py:123-153).  residual / gate as for phyai_fp8_linear_addcmul, or both
+ * null.  Up to 48 token rows and K = 16384 it is one launch where the grid fits the chip.
+ */
+int phyai_fp8_linear_per_tensor(const void *x, int64_t ldx, const float *input_scale, const void *w, const float *w_scale,
+                                const void *bias, const void *residual, int64_t ld_res, const void *gate, int64_t ld_gate,
+                                int64_t gate_rows, void *out, int64_t ldo, int64_t M, int64_t N, int64_t K, int epilogue,
+                                void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * phyai_fp8_linear / phyai_fp8_mlp on the output of an adaptive RMSNorm (phyai_fp8_adarmsnorm_quant's norm, bit for
  * bit): x is the norm's input, modulation [mod_rows, >= 3 K (H)] bf16 = scale | shift | gate, the gate part not read.
  * Up to 128 token rows, K (H) <= 2048, one modulation row, epilogue NONE or GEGLU_TANH, and a workgroup shape whose grid

@@ -36,6 +36,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "phyai_fp8_mlp_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
     "phyai_fp8_mlp": (_int, [_vp, _i64, _vp, _vp, _vp, _int, _vp, _vp, _vp, _int, _vp, _i64, _vp, _i64, _i64, _vp, _i64,
                              _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
+    "phyai_fp8_linear_per_tensor": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64,
+                                           _int, _vp, _sz, _vp]),
     "phyai_fp8_adarmsnorm_linear": (_int, [_vp, _i64, _vp, _i64, _i64, ctypes.c_float, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
                                            _int, _vp, _sz, _vp]),
     "phyai_fp8_adarmsnorm_mlp": (_int, [_vp, _i64, _vp, _i64, _i64, ctypes.c_float, _vp, _vp, _vp, _int, _vp, _vp, _vp, _int, _vp,

@@ -388,6 +388,32 @@ int phyai_fp8_linear(const void* x, int64_t ldx, const void* w, const float* w_s
                       workspace, workspace_bytes, stream);
 }
 
+int phyai_fp8_linear_per_tensor(const void* x, int64_t ldx, const float* input_scale, const void* w, const float* w_scale,
+                                const void* bias, const void* residual, int64_t ld_res, const void* gate, int64_t ld_gate,
+                                int64_t gate_rows, void* out, int64_t ldo, int64_t M, int64_t N, int64_t K, int epilogue,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "phyai_fp8_linear_per_tensor";
+    if (M < 0 || N <= 0 || K <= 0)
+        return fail(PHYAI_FP8_EINVAL, "%s: bad shape M=%lld N=%lld K=%lld", fn, (long long)M, (long long)N, (long long)K);
+    if (M == 0) return PHYAI_FP8_OK;
+    if (!input_scale) return fail(PHYAI_FP8_EINVAL, "%s: null input_scale", fn);
+    const LinearCarve c = carve(M, N, K, epilogue & PHYAI_FP8_EPILOGUE_MASK);
+    if (!workspace || workspace_bytes < c.total)
+        return fail(PHYAI_FP8_EWORKSPACE, "%s: workspace of %zu bytes is too small, need %zu", fn, workspace ? workspace_bytes : (size_t)0, c.total);
+    if (!aligned(workspace, 256)) return fail(PHYAI_FP8_EINVAL, "%s: workspace must be 256-byte aligned", fn);
+    void* xq = static_cast<uint8_t*>(workspace) + c.xq_off;
+    if (int rc = check_quant_args(fn, x, M, K, ldx, xq)) return rc;
+    const ResidualSpec res = {residual, ld_res, gate, ld_gate, gate_rows};
+    phyai::GemmProblem g;
+    if (int rc = prepare_gemm(fn, xq, input_scale, 1, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, workspace, c.gemm_bytes, &g, x, ldx))
+        return rc;
+    if (!phyai::gemm_quantizes_itself(g)) {
+        phyai::launch_quant_static(x, M, K, ldx, input_scale, xq, static_cast<hipStream_t>(stream));
+        if (int rc = check_launch(fn)) return rc;
+    }
+    return launch_prepared(fn, g, stream);
+}
+
 int phyai_fp8_linear_addcmul(const void* x, int64_t ldx, const void* w, const float* w_scale,
                              const void* bias, const void* residual, int64_t ld_res, const void* gate,
                              int64_t ld_gate, int64_t gate_rows, void* out, int64_t ldo, int64_t M,
@@ -400,7 +426,7 @@ int phyai_fp8_linear_addcmul(const void* x, int64_t ldx, const void* w, const fl
 }
 
 namespace {
-// Workspace of phyai_fp8_mlp: [scratch of either linear][h: M x I bf16][row maxima: M x 64 x 16 bit].
+// Workspace of phyai_fp8_mlp: [scratch of either linear][h: M x I bf16][row maxima, M <= 128: M x 256 x 16 bit].
 struct MlpCarve {
     size_t linear_bytes, h_off, amax_off, total;
     LinearCarve first, second;
@@ -413,7 +439,8 @@ MlpCarve mlp_carve(int64_t M, int64_t H, int64_t I, int64_t O, int epilogue) {
     c.linear_bytes = c.first.total > c.second.total ? c.first.total : c.second.total;
     c.h_off = c.linear_bytes;
     c.amax_off = c.h_off + align_up((size_t)(M > 0 ? M : 0) * (size_t)(I > 0 ? I : 0) * 2, 256);
-    c.total = c.amax_off + align_up((size_t)(M > 0 ? M : 0) * phyai::kRowAmaxSlots * 2, 256);
+    // (row maxima pass between kernels of up to 128 token rows only)
+    c.total = c.amax_off + (M > 0 && M <= 128 ? align_up((size_t)M * phyai::kRowAmaxSlots * 2, 256) : 0);
     return c;
 }
 }  // namespace
@@ -458,7 +485,7 @@ int run_mlp(const char* fn, const NormSpec* norm, const void* x, int64_t ldx, co
     set_norm(norm, &g1);
     if (norm && g1.norm_mod && !phyai::gemm_normalises_itself(g1)) g1.norm_mod = nullptr;
     const bool first_on_codes = norm && !g1.norm_mod;   // the norm's own launch: no row maxima from a GEMM on ready codes
-    const int slots = first_on_codes ? 0 : phyai::gemm_row_maxima_slots(g1);
+    const int slots = first_on_codes || M > 128 ? 0 : phyai::gemm_row_maxima_slots(g1);
     if (slots > 0) {
         g2.amax_in = table;
         g2.amax_parts = slots;

@@ -423,19 +423,19 @@ static int sk_ceil_div(int a, int b) { return (a + b - 1) / b; }
 // Largest M served here.  Every group of token rows re-reads the weight tiles from L2, so with
 // enough output tiles the LDS-staged tile kernels win; the dispatcher prefers those as soon as
 // their grid is large enough (see launch_gemm) and falls back to this kernel up to here
-// (N = 1024: ahead of the 128 x 128 tile kernel up to M = 1000, 11.0 against 17.5 us at 800 x 1024 x 4096).
+// (N = 1024: ahead of the 128 x 128 tile kernel up to M = 1000, 11.0 against 17.5 us at 800 x 1024 x 4096; beyond
+// M = 1024 where the tile kernels have fewer than 64 tiles, i.e. few columns: 1548 x 256 x 6016 47.9 -> 21.4 us).
 static int skinny_max_m() {
     if (const char* e = tuning_env("PHYAI_FP8_SKINNY_MAXM")) return atoi(e);
-    return 1024;
+    return 4096;
 }
 
-// K that is not a multiple of 128 (staged form only).  Few token rows: always, from two K steps on - the generic
-// kernel's K splits cost it a round trip through memory.  More rows: as for whole K steps, but not below 1024 output
-// columns, where the generic kernel's splits are what fills the chip.
+// K that is not a multiple of 128 (staged form only): from three K steps on (ten with
+// more than 64 rows and few columns), the generic kernel's K splits cost it a round trip through memory (184 x 896 x 2256: 31.3 -> 9.1 us, 353 x 384 x 3216: 35.9 -> 9.0 us).
 static bool skinny_takes_ragged(int M, int N, int K) {
     static const bool staged = []() { const char* e = tuning_env("PHYAI_FP8_SKINNY_STAGED"); return !(e && atoi(e) == 0); }();
     if (!staged || (int64_t)K * (N > M ? N : M) >= ((int64_t)1 << 31) || K >= (1 << 24)) return false;
-    return K > 256 && (M <= 64 || N >= 1024);
+    return K > 256 && (M <= 64 || N >= 1024 || K >= 1280);
 }
 
 bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo) {

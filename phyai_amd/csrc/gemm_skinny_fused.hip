@@ -75,10 +75,10 @@ __device__ __forceinline__ float fq_bpermute(float v, int src_lane) {
 }
 
 // Row maxima handed from one linear to the next (the gate | up projection of an MLP to its down
-// projection): table[M][64] of bf16 bit patterns of |value| maxima, one slot per workgroup column of
+// projection): table[M][kAmaxSlots] of bf16 bit patterns of |value| maxima, one slot per workgroup column of
 // the producer; the consumer takes the maximum over the first `parts` slots of a row.  Plain stores
 // and loads, no atomics, nothing to reset between calls.
-constexpr int kAmaxSlots = 64;   // slots (16-bit) per token row: 128 bytes
+constexpr int kAmaxSlots = kRowAmaxSlots;   // slots (16-bit) per token row; the consumer below reads the first kFusedAmaxSlots
 struct AmaxOut {
     uint16_t* table;   // null: do not produce
 };
@@ -838,7 +838,7 @@ int launch_set_stamp_sink_fused(unsigned long long* buf, unsigned int records) {
 
 int launch_gemm_fused(const GemmProblem& g, const FusedPlan& pl, hipStream_t st) {
     if (g.amax_out != nullptr && pl.tiles > kAmaxSlots) return -2;   // one slot per workgroup column
-    if (g.amax_in != nullptr && (g.amax_parts < 1 || g.amax_parts > kAmaxSlots)) return -2;
+    if (g.amax_in != nullptr && (g.amax_parts < 1 || g.amax_parts > kFusedAmaxSlots)) return -2;
     switch (g.epilogue) {
     case EPI_NONE: return fq_launch_epi<EPI_NONE>(g, pl, st);
     case EPI_GEGLU_TANH: return fq_launch_epi<EPI_GEGLU_TANH>(g, pl, st);

@@ -359,13 +359,15 @@ static int launch_epi(const TileArgs& a, const TileConfig& c, dim3 grid, hipStre
 
 // launch_gemm's choice of kernel for one problem, and the scratch that choice needs.
 struct GemmChoice {
-    enum Kind { SKINNY, BIG, GENERIC, FUSED } kind;
+    enum Kind { SKINNY, BIG, GENERIC, FUSED, SELFQ } kind;
     FusedPlan fq;
+    SelfqPlan sq;
+    int sq_source;
     SkinnyPlan sk;
     BigPlan big;
     TileConfig tc;
     size_t need;   // workspace bytes (header + split-K partial sums), 0 if the kernel uses none
-    bool takes_amax;   // FUSED: the plan is the one for handed-over row maxima
+    bool takes_amax;   // FUSED, SELFQ: the plan is the one for handed-over row maxima
 };
 
 // Kernel choice (measured on the expert and prefill shapes, M = 50 .. 13056):
@@ -380,9 +382,10 @@ struct GemmChoice {
 // accesses; out16: the output is 16-byte addressable (pointer and row stride), which the pipelined
 // tile kernel's epilogue needs.
 // have_x: the bf16 activations are at hand (whole-linear entry points), so a kernel that quantizes
-// its own rows may serve the call.
+// its own rows may serve the call (one_scale: with one static scale for all of them; amax_parts > 0: with
+// row maxima in that many slots per row): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
 static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
-                              int layout = W_ROW_MAJOR, bool amax_in = false, bool norm = false) {
+                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false) {
     GemmChoice c = {};
     if (norm) {   // rows still to be normalised: one kernel does it or the caller launches the norm itself
         c.kind = GemmChoice::FUSED;
@@ -390,12 +393,26 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
         return c;
     }
     if (have_x && vec_ok) {
-        if (amax_in) {
-            c.fq = fused_plan(M, N, K, epilogue, ldo, layout, true);
-            if (c.fq.rows) { c.kind = GemmChoice::FUSED; c.need = 0; c.takes_amax = true; return c; }
+        auto selfq = [&](int source) {
+            c.sq = selfq_plan(M, N, K, epilogue, ldo, layout, source);
+            c.sq_source = source;
+            if (c.sq.rg == 0) return false;
+            c.kind = GemmChoice::SELFQ;
+            c.takes_amax = source == SELFQ_FROM_MAXIMA;
+            return true;
+        };
+        if (one_scale) {
+            if (selfq(SELFQ_FROM_SCALAR)) return c;
+        } else {
+            if (amax_parts > 0) {
+                if (amax_parts <= kFusedAmaxSlots) c.fq = fused_plan(M, N, K, epilogue, ldo, layout, true);
+                if (c.fq.rows) { c.kind = GemmChoice::FUSED; c.need = 0; c.takes_amax = true; return c; }
+                if (selfq(SELFQ_FROM_MAXIMA)) return c;
+            }
+            c.fq = fused_plan(M, N, K, epilogue, ldo, layout, false);
+            if (c.fq.rows) { c.kind = GemmChoice::FUSED; c.need = 0; return c; }
+            if (selfq(SELFQ_FROM_ROWS)) return c;
         }
-        c.fq = fused_plan(M, N, K, epilogue, ldo, layout, false);
-        if (c.fq.rows) { c.kind = GemmChoice::FUSED; c.need = 0; return c; }
     }
     const bool skinny_ok = vec_ok && skinny_applicable(M, N, K, epilogue, ldo);
     auto small = [&]() {
@@ -429,11 +446,11 @@ static GemmChoice choose_gemm(const GemmProblem& g) {
     const bool out16 = g.ldo % 8 == 0 && (reinterpret_cast<uintptr_t>(g.out) & 15) == 0;
     const bool have_x = g.x_bf16 != nullptr && (reinterpret_cast<uintptr_t>(g.x_bf16) & 15) == 0 && g.ldx % 8 == 0 &&
                         (int64_t)g.M * g.ldx * 2 < ((int64_t)1 << 32) && (int64_t)g.N * g.K < ((int64_t)1 << 32) &&
-                        g.K < (1 << 24) && g.N < (1 << 24) && !g.x_scale_is_scalar;
-    return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout,
-                       g.amax_in != nullptr && g.amax_parts >= 1 && g.amax_parts <= kRowAmaxSlots &&
-                           (reinterpret_cast<uintptr_t>(g.amax_in) & 15) == 0,
-                       g.norm_mod != nullptr);
+                        g.K < (1 << 24) && g.N < (1 << 24);
+    const bool maxima = g.amax_in != nullptr && g.amax_parts >= 1 && g.amax_parts <= kRowAmaxSlots &&
+                        (reinterpret_cast<uintptr_t>(g.amax_in) & 15) == 0;
+    return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, maxima ? g.amax_parts : 0,
+                       g.norm_mod != nullptr, g.x_scale_is_scalar != 0);
 }
 
 bool gemm_normalises_itself(const GemmProblem& g) {
@@ -443,18 +460,19 @@ bool gemm_normalises_itself(const GemmProblem& g) {
 int gemm_row_maxima_slots(const GemmProblem& g) {
     if (g.M == 0 || g.N == 0 || g.epilogue == EPI_NONE) return 0;
     const GemmChoice c = choose_gemm(g);
-    return (c.kind == GemmChoice::FUSED && c.fq.tiles <= kRowAmaxSlots) ? c.fq.tiles : 0;
+    const int tiles = c.kind == GemmChoice::FUSED ? c.fq.tiles : c.kind == GemmChoice::SELFQ ? c.sq.tiles : 0;
+    return tiles <= kRowAmaxSlots ? tiles : 0;
 }
 
 bool gemm_takes_row_maxima(const GemmProblem& g) {
     if (g.M == 0 || g.N == 0) return false;
-    const GemmChoice c = choose_gemm(g);
-    return c.kind == GemmChoice::FUSED && c.takes_amax;
+    return choose_gemm(g).takes_amax;
 }
 
 bool gemm_quantizes_itself(const GemmProblem& g) {
     if (g.M == 0 || g.N == 0) return false;
-    return choose_gemm(g).kind == GemmChoice::FUSED;
+    const GemmChoice c = choose_gemm(g);
+    return c.kind == GemmChoice::FUSED || c.kind == GemmChoice::SELFQ;
 }
 
 size_t gemm_scratch_need(const GemmProblem& g) {
@@ -485,6 +503,8 @@ int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n,
     const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout);
     if (c.kind == GemmChoice::FUSED)
         return snprintf(buf, n, "one launch: small-m rows=%d nt=%d kpw=%d grid=%dx%d", c.fq.rows, c.fq.nt, c.fq.kpw, c.fq.tiles, c.fq.msplit);
+    if (c.kind == GemmChoice::SELFQ)
+        return snprintf(buf, n, "one launch: rows in registers, rows=%d nt=%d steps=%d grid=%dx%d", 4 * c.sq.rg, c.sq.nt, c.sq.steps, c.sq.tiles, c.sq.msplit);
     const int len = snprintf(buf, n, "quantizer + ");
     if (len < 0 || (size_t)len >= n) return len;
     return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout);
@@ -495,19 +515,20 @@ int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_
     const int lay1 = !operand_order ? W_ROW_MAJOR : (epi_is_gated(epilogue) ? W_OPERAND_GATED : W_OPERAND_PLAIN);
     const int lay2 = operand_order ? W_OPERAND_PLAIN : W_ROW_MAJOR;
     const GemmChoice a = choose_gemm(M, n1, H, epilogue, I, true, I % 8 == 0, true, lay1);
-    bool handed = false;
-    if (a.kind == GemmChoice::FUSED && a.fq.tiles <= kRowAmaxSlots) {
-        const GemmChoice b = choose_gemm(M, O, I, EPI_NONE, O, true, O % 8 == 0, true, lay2, true);
-        handed = b.kind == GemmChoice::FUSED && b.takes_amax;
-    }
+    const int parts = a.kind == GemmChoice::FUSED ? a.fq.tiles : a.kind == GemmChoice::SELFQ ? a.sq.tiles : 0;
+    const bool some = parts > 0 && parts <= kRowAmaxSlots;
+    const GemmChoice b = choose_gemm(M, O, I, EPI_NONE, O, true, O % 8 == 0, true, lay2, some ? parts : 0);
+    const bool handed = some && b.takes_amax;
     int len = handed ? snprintf(buf, n, "row maxima handed over: ") : 0;
     if (len < 0 || (size_t)len >= n) return len;
     len += describe_linear_plan(M, n1, H, epilogue, buf + len, n - len, lay1);
     if ((size_t)len >= n) return len;
     len += snprintf(buf + len, n - len, " | ");
     if ((size_t)len >= n) return len;
+    if (handed && b.kind == GemmChoice::SELFQ)
+        return len + snprintf(buf + len, n - len, "one launch: rows in registers, rows=%d nt=%d steps=%d grid=%dx%d", 4 * b.sq.rg, b.sq.nt,
+                              b.sq.steps, b.sq.tiles, b.sq.msplit);
     if (handed) {
-        const GemmChoice b = choose_gemm(M, O, I, EPI_NONE, O, true, O % 8 == 0, true, lay2, true);
         return len + snprintf(buf + len, n - len, "one launch: small-m rows=%d nt=%d kpw=%d grid=%dx%d", b.fq.rows, b.fq.nt,
                               b.fq.kpw, b.fq.tiles, b.fq.msplit);
     }
@@ -518,6 +539,7 @@ int launch_gemm(const GemmProblem& g, hipStream_t st) {
     if (g.M == 0 || g.N == 0) return 0;
     const GemmChoice ch = choose_gemm(g);
     if (ch.need > 0 && (g.workspace == nullptr || g.workspace_bytes < ch.need)) return -3;
+    if (ch.kind == GemmChoice::SELFQ) return launch_gemm_selfq(g, ch.sq, ch.sq_source, st);
     if (ch.kind == GemmChoice::FUSED) {
         if (ch.fq.rows == 0) return -2;
         if (g.amax_in != nullptr && !ch.takes_amax) {   // the plan finds the row maxima itself

@@ -38,7 +38,7 @@ struct Lib {
     decltype(&phyai_fp8_linear_workspace_bytes) linear_ws;
     decltype(&phyai_fp8_mlp_workspace_bytes) mlp_ws;
     decltype(&phyai_fp8_quant_rowwise) quant_rowwise;
-    decltype(&phyai_fp8_quant_static) quant_static;
+    decltype(&phyai_fp8_linear_per_tensor) per_tensor;
     decltype(&phyai_fp8_rmsnorm_quant) rmsnorm;
     decltype(&phyai_fp8_adarmsnorm_quant) adarmsnorm;
 } lib = {};
@@ -287,30 +287,28 @@ PyObject* linear_call(PyObject* x_, PyObject* xs_, PyObject* w_, PyObject* ws_, 
     return THPVariable_Wrap(std::move(made));
 }
 
-// bf16 rows, one static scale for all of them: the codes live in a tensor of this call.
+// bf16 rows, one static scale for all of them
 PyObject* linear_static_call(PyObject* x_, PyObject* in_scale_, PyObject* w_, PyObject* ws_, PyObject* b_, int epi,
                              PyObject* layout, bool stream, PyObject* res_, PyObject* gate_) {
     const at::Tensor *x = tensor(x_), *s = tensor(in_scale_);
     Rows r;
     Where at_;
-    if (!x || !vector_of(s, at::kFloat, 1) || !rows_of(*x, at::kBFloat16, &r) || !where(*x, &at_)) return nullptr;
-    // what linear_call() would decline is declined before the quantizer is launched
     Weight w;
     int flags;
     Residual rg;
-    if (!weight_of(w_, ws_, b_, r.K, &w) || !flags_of(layout, stream, epi, &flags) || (is_gated(epi) && w.N % 32 != 0) ||
-        !residual_of(res_, gate_, *x, r.M, w.N, epi, &rg))
+    if (!x || !vector_of(s, at::kFloat, 1) || !rows_of(*x, at::kBFloat16, &r) || !where(*x, &at_) || !weight_of(w_, ws_, b_, r.K, &w) ||
+        !flags_of(layout, stream, epi, &flags) || (is_gated(epi) && w.N % 32 != 0) || !residual_of(res_, gate_, *x, r.M, w.N, epi, &rg))
         return nullptr;
-    PyObject* xq = THPVariable_Wrap(fresh(*x, r.K, at::kFloat8_e4m3fn, at_.dev));
-    if (!xq) return nullptr;
+    const int64_t n_out = is_gated(epi) ? w.N / 2 : w.N;
+    at::Tensor made = fresh(*x, n_out, at::kBFloat16, at_.dev);
+    Scratch ws;
+    if (!workspace(lib.linear_ws(r.M, w.N, r.K, epi), at_, &ws)) return nullptr;
     int rc;
-    void* q = THPVariable_Unpack(xq).mutable_data_ptr();
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.quant_static(r.p, r.M, r.K, r.ld, s->const_data_ptr<float>(), q, at_.stream);
+    rc = lib.per_tensor(r.p, r.ld, s->const_data_ptr<float>(), w.w, w.scale, w.bias, rg.residual, w.N, rg.gate, rg.ld_gate, rg.gate_rows,
+                        made.mutable_data_ptr(), n_out, r.M, w.N, r.K, epi | flags, ws.p, ws.n, at_.stream);
     Py_END_ALLOW_THREADS
-    PyObject* y = rc == 0 ? linear_call(xq, in_scale_, w_, ws_, b_, epi, layout, stream, Py_None, res_, gate_) : nullptr;
-    Py_DECREF(xq);
-    return y;
+    return rc == 0 ? THPVariable_Wrap(std::move(made)) : nullptr;
 }
 
 // linear(x, weight, weight_scale, bias, epilogue, out, residual, gate, stream_weights, weight_layout)
@@ -666,7 +664,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     get(l.linear_ws, "phyai_fp8_linear_workspace_bytes");
     get(l.mlp_ws, "phyai_fp8_mlp_workspace_bytes");
     get(l.quant_rowwise, "phyai_fp8_quant_rowwise");
-    get(l.quant_static, "phyai_fp8_quant_static");
+    get(l.per_tensor, "phyai_fp8_linear_per_tensor");
     get(l.rmsnorm, "phyai_fp8_rmsnorm_quant");
     get(l.adarmsnorm, "phyai_fp8_adarmsnorm_quant");
     if (!ok) return PyErr_Format(PyExc_RuntimeError, "%s lacks an entry point this extension binds", path);

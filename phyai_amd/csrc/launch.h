@@ -141,8 +141,25 @@ struct FusedPlan {
     int msplit;  // workgroups along M
 };
 FusedPlan fused_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout = 0, bool amax_in = false, bool norm = false);
-constexpr int kRowAmaxSlots = 64;   // slots per token row of a table of handed-over row maxima
+constexpr int kRowAmaxSlots = 256;  // slots per token row of a table of handed-over row maxima (one per workgroup column of the producer)
+constexpr int kFusedAmaxSlots = 64; // ... that the consumer of gemm_skinny_fused.hip reads (that of gemm_selfq.h: all)
 int launch_gemm_fused(const GemmProblem& p, const FusedPlan& pl, hipStream_t st);
+
+// Small-M linear that quantizes its own rows at any K up to 16384 (gemm_selfq.h).  rg == 0: does not apply.
+struct SelfqPlan {
+    int rg;      // groups of four token rows per workgroup (1 or 2)
+    int nt;      // 16-row weight tiles per workgroup
+    int steps;   // K steps per wavefront
+    int tiles;   // workgroups along N
+    int msplit;  // workgroups along M
+};
+enum SelfqSource : int { SELFQ_FROM_ROWS = 0, SELFQ_FROM_MAXIMA = 1, SELFQ_FROM_SCALAR = 2 };   // of the row scales
+SelfqPlan selfq_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout, int source);
+int launch_gemm_selfq(const GemmProblem& p, const SelfqPlan& pl, int source, hipStream_t st);
+int launch_selfq_own(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
+int launch_selfq_own_act(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
+int launch_selfq_handed(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
+int launch_selfq_static(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
 
 // Pipelined tile kernel for large M (gemm_big.hip), 256 x 256 or 128 x 128 tiles; the small
 // tiles may be split along K (partials in the workspace, as for the generic tile kernel).
