@@ -125,6 +125,11 @@ int phyai_fp8_weight_to_operand_order(const void *w, int64_t N, int64_t K, int g
                                       void *stream);
 
 /*
+ * The plain (not gated) form in place.  K <= 16384.
+ */
+int phyai_fp8_weight_to_operand_order_inplace(void *w, int64_t N, int64_t K, void *stream);
+
+/*
  * Bytes of workspace phyai_fp8_linear / phyai_fp8_gemm need for this shape.
  * The workspace must be 256-byte aligned and its first
  * PHYAI_FP8_WORKSPACE_HEADER_BYTES must be zero before the first call that uses

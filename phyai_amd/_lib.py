@@ -30,6 +30,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "phyai_fp8_quant_static": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp]),
     "phyai_fp8_weight_quant_rowwise": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp]),
     "phyai_fp8_weight_to_operand_order": (_int, [_vp, _i64, _i64, _int, _vp, _vp]),
+    "phyai_fp8_weight_to_operand_order_inplace": (_int, [_vp, _i64, _i64, _vp]),
     "phyai_fp8_linear_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "phyai_fp8_gemm": (_int, [_vp, _vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "phyai_fp8_linear": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),

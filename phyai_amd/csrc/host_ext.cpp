@@ -38,6 +38,9 @@ struct Lib {
     decltype(&phyai_fp8_linear_workspace_bytes) linear_ws;
     decltype(&phyai_fp8_mlp_workspace_bytes) mlp_ws;
     decltype(&phyai_fp8_quant_rowwise) quant_rowwise;
+    decltype(&phyai_fp8_weight_quant_rowwise) weight_quant;
+    decltype(&phyai_fp8_weight_to_operand_order) relay;
+    decltype(&phyai_fp8_weight_to_operand_order_inplace) relay_inplace;
     decltype(&phyai_fp8_linear_per_tensor) per_tensor;
     decltype(&phyai_fp8_rmsnorm_quant) rmsnorm;
     decltype(&phyai_fp8_adarmsnorm_quant) adarmsnorm;
@@ -512,6 +515,41 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- loading -------------------------------------------------------------------------------------------------------
+// quantize_weight(layer, bf16 [N, K]): codes and scales into the layer's parameters -> True, or None
+PyObject* py_quantize_weight(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer l;
+    if (n != 2 || !layer_of(a[0], &l) || l.granularity != py.per_channel) return declined();
+    const at::Tensor *x = tensor(a[1]), *w = tensor(l.weight), *s = tensor(l.scale);
+    Where at_;
+    if (!x || !w || !s || x->dim() != 2 || w->dim() != 2 || !x->is_cuda() || !w->is_cuda() || x->scalar_type() != at::kBFloat16 || !codes_dtype(*w) ||
+        !x->is_contiguous() || !w->is_contiguous() || x->size(0) != w->size(0) || x->size(1) != w->size(1) || x->numel() == 0 ||
+        x->size(1) % 8 != 0 || !vector_of(s, at::kFloat, w->size(0)) || x->device() != w->device() || s->device() != w->device() || !where(*x, &at_))
+        return declined();
+    if (lib.weight_quant(x->const_data_ptr(), x->size(0), x->size(1), x->size(1), w->mutable_data_ptr(), s->mutable_data_ptr<float>(), at_.stream) != 0)
+        return declined();
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+// relay_weight(weight, gated): the matrix re-laid in MFMA operand order, in its own storage -> True, or None
+PyObject* py_relay_weight(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = n == 2 ? tensor(a[0]) : nullptr;
+    Where at_;
+    if (!w || !w->is_cuda() || w->dim() != 2 || !codes_dtype(*w) || !w->is_contiguous() || w->numel() == 0 || !where(*w, &at_)) return declined();
+    const int64_t N = w->size(0), K = w->size(1);
+    const bool gated = a[1] == Py_True;
+    void* p = w->mutable_data_ptr();
+    if (!gated && lib.relay_inplace(p, N, K, at_.stream) == 0) Py_RETURN_TRUE;
+    at::Tensor t = at::Tensor(at::detail::empty_cuda(w->sizes(), w->scalar_type(), at_.dev, std::nullopt));
+    // (a plain copy first and the re-lay back: the allocator's stream order covers the temporary)
+    if (hipMemcpyAsync(t.mutable_data_ptr(), p, (size_t)(N * K), hipMemcpyDeviceToDevice, at_.stream) != hipSuccess) return declined();
+    if (lib.relay(t.const_data_ptr(), N, K, gated, p, at_.stream) != 0) return declined();
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
 // ---- a decoder layer's three calls: adaptive norm + linear, linear + gated residual, adaptive norm + MLP + gated residual
 // norm_linear(layer, x, modulation, eps): layer(norm(x)), x in rows of the layer's input width
 PyObject* py_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -664,6 +702,9 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     get(l.linear_ws, "phyai_fp8_linear_workspace_bytes");
     get(l.mlp_ws, "phyai_fp8_mlp_workspace_bytes");
     get(l.quant_rowwise, "phyai_fp8_quant_rowwise");
+    get(l.weight_quant, "phyai_fp8_weight_quant_rowwise");
+    get(l.relay, "phyai_fp8_weight_to_operand_order");
+    get(l.relay_inplace, "phyai_fp8_weight_to_operand_order_inplace");
     get(l.per_tensor, "phyai_fp8_linear_per_tensor");
     get(l.rmsnorm, "phyai_fp8_rmsnorm_quant");
     get(l.adarmsnorm, "phyai_fp8_adarmsnorm_quant");
@@ -695,6 +736,8 @@ PyMethodDef methods[] = {
     PHYAI_FAST("layer_apply", py_layer_apply),
     PHYAI_FAST("layer_forward", py_layer_forward),
     PHYAI_FAST("mlp_forward", py_mlp_forward),
+    PHYAI_FAST("quantize_weight", py_quantize_weight),
+    PHYAI_FAST("relay_weight", py_relay_weight),
     PHYAI_FAST("norm_linear", py_norm_linear),
     PHYAI_FAST("linear_residual", py_linear_residual),
     PHYAI_FAST("norm_mlp", py_norm_mlp),

@@ -16,6 +16,8 @@ int launch_quant_static(const void* x, int64_t M, int64_t K, int64_t ldx, const 
 int launch_debug_cast(const float* v, int64_t n, void* codes, hipStream_t st);
 // Row-major fp8 weights -> MFMA operand order (weight_layout.hip); gated: the fused gate | up form.
 int launch_weight_to_operand_order(const void* w, int64_t N, int64_t K, int gated, void* out, hipStream_t st);
+// The plain form in place, K <= 16384 (-2 beyond).
+int launch_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, hipStream_t st);
 // fp8 MFMA issue-rate probe (probe_kernels.hip): out holds 2 x workgroups 64-bit counters.
 int launch_mfma_rate(int workgroups, int iters, unsigned long long* out, float* sink, hipStream_t st);
 

@@ -113,14 +113,15 @@ class Fp8Spec:
         checkpoint loader, ``quantize_weight_``) clears ``weight_layout`` first."""
         from phyai_amd import ops
 
-        w = layer.weight
+        w = layer._parameters["weight"]
         if getattr(layer, "weight_layout", None):
             return True
         gated = bool(getattr(layer, "gated_pairs", False))
         n, k = w.shape
         if not w.is_cuda or k % 128 != 0 or n % (32 if gated else 16) != 0:
             return False
-        w.data.copy_(ops.fp8_weight_to_operand_order(w.data, gated=gated))
+        if ops._native().relay_weight(w, gated) is None:
+            w.data.copy_(ops.fp8_weight_to_operand_order(w.data, gated=gated))
         layer.weight_layout = "operand_gated" if gated else "operand"
         return True
 
@@ -144,9 +145,11 @@ class Fp8Spec:
 
         if self.granularity is not Granularity.PER_CHANNEL:
             raise RuntimeError("quantize_weight_ is defined for PER_CHANNEL only")
-        if tuple(w_bf16.shape) != tuple(layer.weight.shape):
+        if w_bf16.shape != layer.weight.shape:
             raise ValueError(f"weight shape {tuple(w_bf16.shape)} != {tuple(layer.weight.shape)}")
         layer.weight_layout = None   # row-major again until process_after_loading re-lays it
+        if ops._native().quantize_weight(layer, w_bf16) is not None:
+            return
         ops.fp8_weight_quant(w_bf16.to(device=layer.weight.device, dtype=torch.bfloat16).contiguous(),
                              out=layer.weight.data, scale_out=layer.weight_scale.data)
 

@@ -1,6 +1,6 @@
 """Small-M linears that quantize their own rows at any K (csrc/gemm_selfq.h) against quantizer + GEMM, bit for bit:
 partial and missing K steps, row groups of four, every number of weight tiles, own / handed-over / static scales, NaN and
-Inf in rows; and the reciprocal form of the static and weight quantizers against the division on the CPU."""
+Inf in rows; the reciprocal form of the static and weight quantizers against the division on the CPU; and weights re-laid in place."""
 
 from __future__ import annotations
 
@@ -93,3 +93,13 @@ def test_weight_quantizer_equals_the_division(dev):
     want_s = w.float().abs().amax(1) / 448.0
     assert torch.equal(s.cpu(), want_s)
     assert torch.equal(q.view(torch.uint8).cpu(), (w.float() / want_s[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8))
+
+
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 1024), (1040, 1152), (32, 2176), (64, 8192), (48, 8320), (16, 16384)])
+def test_weights_relaid_in_place(dev, N, K):
+    from phyai_amd import ops
+
+    w = torch.randint(0, 256, (N, K), dtype=torch.uint8, generator=torch.Generator().manual_seed(N + K)).to(dev)
+    want = ops.fp8_weight_to_operand_order(w.view(torch.float8_e4m3fn)).view(torch.uint8)
+    assert ops._native().relay_weight(w, False) is True
+    assert torch.equal(w, want)
