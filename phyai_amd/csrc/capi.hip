@@ -8,6 +8,7 @@
 
 #include "../../include/phyai_fp8.h"
 #include "fp8_device.h"
+#include "call_memo.h"
 #include "launch.h"
 #include "weight_layout.h"
 
@@ -52,7 +53,7 @@ int check_epilogue(int epilogue, int64_t N) {
 struct LinearCarve {
     size_t gemm_bytes, xq_off, xs_off, total;
 };
-LinearCarve carve(int64_t M, int64_t N, int64_t K, int epilogue) {
+LinearCarve make_carve(int64_t M, int64_t N, int64_t K, int epilogue) {
     LinearCarve c;
     {
         const int64_t n_out = phyai::epi_is_gated(epilogue) ? N / 2 : N;
@@ -65,6 +66,11 @@ LinearCarve carve(int64_t M, int64_t N, int64_t K, int epilogue) {
     c.xs_off = c.xq_off + align_up((size_t)(M > 0 ? M : 0) * (size_t)(K > 0 ? K : 0), 256);
     c.total = c.xs_off + align_up((size_t)(M > 0 ? M : 0) * sizeof(float), 256);
     return c;
+}
+
+LinearCarve carve(int64_t M, int64_t N, int64_t K, int epilogue) {
+    static thread_local phyai::CallMemo<LinearCarve, 128> memo;
+    return memo.get(M, N, K, epilogue, [&]() { return make_carve(M, N, K, epilogue); });
 }
 
 int check_quant_args(const char* fn, const void* x, int64_t M, int64_t K, int64_t ldx, const void* xq) {

@@ -24,6 +24,7 @@
 // results are reproducible - and runs the epilogue.  It then resets the
 // counter, which keeps the workspace header zero between calls.
 #include "fp8_device.h"
+#include "call_memo.h"
 #include "launch.h"
 #include "tuning.h"
 #include "splitk.h"
@@ -439,7 +440,7 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
     return c;
 }
 
-static GemmChoice choose_gemm(const GemmProblem& g) {
+static const GemmChoice& choose_gemm(const GemmProblem& g) {
     const bool vec_ok = (reinterpret_cast<uintptr_t>(g.w_scale) % 16 == 0) &&
                         (reinterpret_cast<uintptr_t>(g.bias) % 8 == 0) &&
                         (reinterpret_cast<uintptr_t>(g.out) % 8 == 0);
@@ -449,8 +450,14 @@ static GemmChoice choose_gemm(const GemmProblem& g) {
                         g.K < (1 << 24) && g.N < (1 << 24);
     const bool maxima = g.amax_in != nullptr && g.amax_parts >= 1 && g.amax_parts <= kRowAmaxSlots &&
                         (reinterpret_cast<uintptr_t>(g.amax_in) & 15) == 0;
-    return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, maxima ? g.amax_parts : 0,
-                       g.norm_mod != nullptr, g.x_scale_is_scalar != 0);
+    const int parts = maxima ? g.amax_parts : 0;
+    const bool norm = g.norm_mod != nullptr, one_scale = g.x_scale_is_scalar != 0;
+    const int64_t how = (int64_t)g.epilogue | (int64_t)vec_ok << 8 | (int64_t)out16 << 9 | (int64_t)have_x << 10 | (int64_t)norm << 11 |
+                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)parts << 16;
+    static thread_local CallMemo<GemmChoice, 128> memo;
+    return memo.get((int64_t)g.M | how << 32, g.N, g.K, g.ldo, [&]() {
+        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale);
+    });
 }
 
 bool gemm_normalises_itself(const GemmProblem& g) {
@@ -459,7 +466,7 @@ bool gemm_normalises_itself(const GemmProblem& g) {
 
 int gemm_row_maxima_slots(const GemmProblem& g) {
     if (g.M == 0 || g.N == 0 || g.epilogue == EPI_NONE) return 0;
-    const GemmChoice c = choose_gemm(g);
+    const GemmChoice& c = choose_gemm(g);
     const int tiles = c.kind == GemmChoice::FUSED ? c.fq.tiles : c.kind == GemmChoice::SELFQ ? c.sq.tiles : 0;
     return tiles <= kRowAmaxSlots ? tiles : 0;
 }
@@ -471,7 +478,7 @@ bool gemm_takes_row_maxima(const GemmProblem& g) {
 
 bool gemm_quantizes_itself(const GemmProblem& g) {
     if (g.M == 0 || g.N == 0) return false;
-    const GemmChoice c = choose_gemm(g);
+    const GemmChoice& c = choose_gemm(g);
     return c.kind == GemmChoice::FUSED || c.kind == GemmChoice::SELFQ;
 }
 
@@ -537,7 +544,7 @@ int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_
 
 int launch_gemm(const GemmProblem& g, hipStream_t st) {
     if (g.M == 0 || g.N == 0) return 0;
-    const GemmChoice ch = choose_gemm(g);
+    const GemmChoice& ch = choose_gemm(g);
     if (ch.need > 0 && (g.workspace == nullptr || g.workspace_bytes < ch.need)) return -3;
     if (ch.kind == GemmChoice::SELFQ) return launch_gemm_selfq(g, ch.sq, ch.sq_source, st);
     if (ch.kind == GemmChoice::FUSED) {

@@ -52,8 +52,15 @@ struct Py {
 struct PyLayers {
     PyObject *dispatch_dict, *mode, *kernel_type;
 } pl = {};
+// what the calls of modules need: phyai_amd.ops's dictionary, this extension, nn.Module.__call__, the tables of hooks that
+// apply to every module, and the forward methods that the calls below stand for
+struct PyModules {
+    PyObject *ops_dict, *self, *module_call, *global_hooks, *linear_forward, *mlp_forward;
+} pm = {};
 
 PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bias_add, *s_bias;
+PyObject *s_host, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
+    *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
     *s_spec, *s_granularity;
 
@@ -497,20 +504,22 @@ PyObject* py_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
-// mlp_forward(first layer, second layer, x, epilogue, residual, gate): both per-channel layers that add their own bias
+// both projections per-channel layers that add their own bias
+PyObject* mlp_native(PyObject* first, PyObject* second, PyObject* x, int epi, PyObject* residual, PyObject* gate) {
+    Layer p, q;
+    PyObject *b1, *b2;
+    if (!tensor(x) || !hip_kernel_remembered(first, x) || !hip_kernel_remembered(second, x) || !layer_of(first, &p) || !layer_of(second, &q) ||
+        p.granularity != py.per_channel || q.granularity != py.per_channel || !bias_of(first, &b1) || !bias_of(second, &b2))
+        return nullptr;
+    for (PyObject* layer : {first, second})
+        if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(layer), s_skip_bias_add) != Py_False) return nullptr;
+    return mlp_call(x, p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None, residual, gate);
+}
+// mlp_forward(first layer, second layer, x, epilogue, residual, gate)
 PyObject* py_mlp_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    Layer p, q;
     int epi;
-    PyObject *b1, *b2;
-    if (n != 6 || !tensor(a[2]) || !hip_kernel_remembered(a[0], a[2]) || !hip_kernel_remembered(a[1], a[2]) || !layer_of(a[0], &p) ||
-        !layer_of(a[1], &q) || !epilogue_of(a[3], &epi) || p.granularity != py.per_channel || q.granularity != py.per_channel ||
-        !bias_of(a[0], &b1) || !bias_of(a[1], &b2))
-        return declined();
-    for (int i = 0; i < 2; ++i)
-        if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[i]), s_skip_bias_add) != Py_False) return declined();
-    PyObject* y = mlp_call(a[2], p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None,
-                           a[4], a[5]);
+    PyObject* y = n == 6 && epilogue_of(a[3], &epi) ? mlp_native(a[0], a[1], a[2], epi, a[4], a[5]) : nullptr;
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -590,6 +599,75 @@ PyObject* py_norm_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyObject* y = mlp_call(a[2], p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None,
                            a[2], nullptr, a[3], a[4]);
     return y ? y : declined();
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- modules: __call__ of the linear layers and of the MLP ---------------------------------------------------------
+// nn.Module.__call__ and the two Python frames behind it take 0.9 us.  These go straight to the native call when nothing
+// stands in between - no hooks, no compiled or replaced forward - and to nn.Module.__call__ otherwise.
+bool plain_call(PyObject* self, PyObject* dict, PyObject* forward) {
+    if (!pm.self || PyDict_GetItemWithError(pm.ops_dict, s_host) != pm.self) return false;
+    if (_PyType_Lookup(Py_TYPE(self), s_forward) != forward || PyDict_GetItemWithError(dict, s_forward) || PyDict_GetItemWithError(dict, s_compiled))
+        return false;
+    for (PyObject* name : s_hooks) {
+        PyObject* h = PyDict_GetItemWithError(dict, name);
+        if (!h || !PyDict_Check(h) || PyDict_GET_SIZE(h) != 0) return false;
+    }
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(pm.global_hooks); ++i)
+        if (PyDict_GET_SIZE(PyTuple_GET_ITEM(pm.global_hooks, i)) != 0) return false;
+    return true;
+}
+PyObject* module_call(PyObject* args, PyObject* kwargs) {
+    PyErr_Clear();
+    return PyObject_Call(pm.module_call, args, kwargs);
+}
+// linear(x) -> (output, bias left to the caller or None)
+PyObject* py_linear_call(PyObject*, PyObject* args, PyObject* kwargs) {
+    HANDLE_TH_ERRORS
+    if (PyTuple_GET_SIZE(args) == 2 && (!kwargs || PyDict_GET_SIZE(kwargs) == 0)) {
+        PyObject *self = PyTuple_GET_ITEM(args, 0), *x = PyTuple_GET_ITEM(args, 1);
+        PyObject** dp = _PyObject_GetDictPtr(self);
+        Layer l;
+        PyObject* bias;
+        if (dp && *dp && plain_call(self, *dp, pm.linear_forward) && hip_kernel_remembered(self, x) && layer_of(self, &l) && bias_of(self, &bias)) {
+            PyObject* y = layer_call(l, x, bias, 0, Py_None, Py_None);
+            if (y) {
+                PyObject* left = Py_None;
+                if (PyDict_GetItemWithError(*dp, s_skip_bias_add) == Py_True) left = PyDict_GetItemWithError(PyDict_GetItemWithError(*dp, s_parameters), s_bias);
+                PyObject* r = left ? PyTuple_Pack(2, y, left) : nullptr;
+                Py_DECREF(y);
+                return r;
+            }
+        }
+    }
+    return module_call(args, kwargs);
+    END_HANDLE_TH_ERRORS
+}
+// mlp(x, residual=, gate=)
+PyObject* py_mlp_call(PyObject*, PyObject* args, PyObject* kwargs) {
+    HANDLE_TH_ERRORS
+    if (PyTuple_GET_SIZE(args) == 2) {
+        PyObject *self = PyTuple_GET_ITEM(args, 0), *x = PyTuple_GET_ITEM(args, 1), *residual = Py_None, *gate = Py_None;
+        Py_ssize_t known = 0;
+        if (kwargs) {
+            if (PyObject* r = PyDict_GetItemWithError(kwargs, s_residual)) { residual = r; ++known; }
+            if (PyObject* g = PyDict_GetItemWithError(kwargs, s_gate)) { gate = g; ++known; }
+        }
+        PyObject** dp = _PyObject_GetDictPtr(self);
+        if ((!kwargs || known == PyDict_GET_SIZE(kwargs)) && dp && *dp && plain_call(self, *dp, pm.mlp_forward) &&
+            PyDict_GetItemWithError(*dp, s_fuse_activation) == Py_True) {
+            PyObject *mods = PyDict_GetItemWithError(*dp, s_modules), *epilogue = PyDict_GetItemWithError(*dp, s_epilogue);
+            const bool gated = PyDict_GetItemWithError(*dp, s_gated) == Py_True;
+            PyObject* first = mods ? PyDict_GetItemWithError(mods, gated ? s_gate_up : s_fc1) : nullptr;
+            PyObject* second = mods ? PyDict_GetItemWithError(mods, gated ? s_down : s_fc2) : nullptr;
+            int epi;
+            if (first && second && epilogue && epilogue_of(epilogue, &epi)) {
+                PyObject* y = mlp_native(first, second, x, epi, residual, gate);
+                if (y) return y;
+            }
+        }
+    }
+    return module_call(args, kwargs);
     END_HANDLE_TH_ERRORS
 }
 
@@ -726,10 +804,31 @@ PyObject* py_bind_layers(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
+PyMethodDef linear_call_def = {"__call__", (PyCFunction)(void (*)(void))py_linear_call, METH_VARARGS | METH_KEYWORDS, nullptr};
+PyMethodDef mlp_call_def = {"__call__", (PyCFunction)(void (*)(void))py_mlp_call, METH_VARARGS | METH_KEYWORDS, nullptr};
+// bind_modules(phyai_amd.ops's dictionary, this module, nn.Module.__call__, tuple of global hook tables,
+//              LinearBase.forward, DenseMLP.forward) -> (LinearBase.__call__, DenseMLP.__call__)
+PyObject* py_bind_modules(PyObject*, PyObject* args) {
+    PyModules m = {};
+    if (!PyArg_ParseTuple(args, "O!OOO!OO", &PyDict_Type, &m.ops_dict, &m.self, &m.module_call, &PyTuple_Type, &m.global_hooks,
+                          &m.linear_forward, &m.mlp_forward))
+        return nullptr;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(m.global_hooks); ++i)
+        if (!PyDict_Check(PyTuple_GET_ITEM(m.global_hooks, i))) return PyErr_Format(PyExc_TypeError, "hook tables are dictionaries");
+    for (PyObject* o : {m.ops_dict, m.self, m.module_call, m.global_hooks, m.linear_forward, m.mlp_forward}) Py_INCREF(o);
+    pm = m;
+    PyObject *a = PyCFunction_New(&linear_call_def, nullptr), *b = PyCFunction_New(&mlp_call_def, nullptr);
+    PyObject *ma = a ? PyInstanceMethod_New(a) : nullptr, *mb = b ? PyInstanceMethod_New(b) : nullptr;
+    Py_XDECREF(a);
+    Py_XDECREF(b);
+    return ma && mb ? Py_BuildValue("NN", ma, mb) : nullptr;
+}
+
 #define PHYAI_FAST(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", py_bind, METH_VARARGS, nullptr},
     {"bind_layers", py_bind_layers, METH_VARARGS, nullptr},
+    {"bind_modules", py_bind_modules, METH_VARARGS, nullptr},
     PHYAI_FAST("linear", py_linear),
     PHYAI_FAST("gemm", py_gemm),
     PHYAI_FAST("mlp", py_mlp),
@@ -755,7 +854,11 @@ PyMODINIT_FUNC PyInit__phyai_host() {
         {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_weight_scale, "weight_scale"}, {&s_input_scale, "input_scale"},
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
         {&s_granularity, "granularity"}, {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
-        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}};
+        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_forward, "forward"},
+        {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
+        {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},
+        {&s_compiled, "_compiled_call_impl"}, {&s_hooks[0], "_forward_hooks"}, {&s_hooks[1], "_forward_pre_hooks"},
+        {&s_hooks[2], "_backward_hooks"}, {&s_hooks[3], "_backward_pre_hooks"}};
     for (const auto& e : names)
         if (!(*e.at = PyUnicode_InternFromString(e.text))) return nullptr;
     return PyModule_Create(&module);

@@ -127,6 +127,14 @@ def _native():
         from phyai_amd.linear import dispatch, kernels
 
         ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel)
+        from torch.nn.modules import module as m
+
+        from phyai_amd.linear.layers import LinearBase
+        from phyai_amd.mlp import DenseMLP
+
+        hooks = (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks)
+        LinearBase.__call__, DenseMLP.__call__ = ext.bind_modules(globals(), ext, torch.nn.Module.__call__, hooks,
+                                                                  LinearBase.forward, DenseMLP.forward)
         _host = ext
     return _host
 
