@@ -154,33 +154,25 @@ static int big_grid_ids(int m_tiles, int n_tiles, int band_rows) {
 // rows of equal parity among 16 consecutive ones must land in different chunk columns.
 __device__ __forceinline__ int big_swizzle(int row) { return (row >> 1) & 7; }
 
-// Operand block of v_mfma_f32_32x32x64 for K half kh (bytes [64 kh, 64 kh + 64) of the row): lane
-// (l32, h) supplies 32 of the 64 K-bytes.  Which 32 is free as long as A and B agree; chunks h
-// and 2+h of the half are taken so that the two halves of a wavefront never meet in a chunk
-// column either.
-__device__ __forceinline__ v8i big_frag(const uint8_t* buf, int row, int h, int kh) {
-    const int sw = big_swizzle(row);
-    const uint8_t* r = buf + row * BIG_BK;
-    const v4i lo = *reinterpret_cast<const v4i*>(r + (((4 * kh + h) ^ sw) << 4));
-    const v4i hi = *reinterpret_cast<const v4i*>(r + (((4 * kh + 2 + h) ^ sw) << 4));
-    v8i f;
-    f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
-    f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];
-    return f;
-}
-
+// Operand block of v_mfma_f32_16x16x128: 16 rows x 128 bytes of K; lane (l16, q) supplies 32 of the 128 bytes of row
+// l16.  Which 32 is free as long as A and B agree: chunks q and 4 + q, so that a quarter of a wavefront reads one chunk
+// column.  `row`: the block's first row plus l16.
 __device__ __forceinline__ v8i big_join(v4i lo, v4i hi) {
     v8i f;
     f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
     f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];
     return f;
 }
-// The same block out of weights staged in operand order (WMODE 1): `row` is the block's first row plus l32;
-// chunk c of it lies at unit * 2 KB + c * 256 + (row % 16) * 16.  Sixteen consecutive lanes read 256 bytes in a
-// row: no bank conflicts.
-__device__ __forceinline__ v8i big_frag_operand(const uint8_t* buf, int row, int h, int kh) {
-    const uint8_t* r = buf + (row >> 4) * 2048 + (row & 15) * 16;
-    return big_join(*reinterpret_cast<const v4i*>(r + (4 * kh + h) * 256), *reinterpret_cast<const v4i*>(r + (4 * kh + 2 + h) * 256));
+__device__ __forceinline__ v8i big_frag(const uint8_t* buf, int row, int q) {
+    const int sw = big_swizzle(row);
+    const uint8_t* r = buf + row * BIG_BK;
+    return big_join(*reinterpret_cast<const v4i*>(r + ((q ^ sw) << 4)), *reinterpret_cast<const v4i*>(r + (((4 + q) ^ sw) << 4)));
+}
+// The same block out of weights staged in operand order (WMODE 1): chunk c of row r of a unit lies at c * 256 + r * 16, so
+// the lanes read 1 KB in a row, twice.
+__device__ __forceinline__ v8i big_frag_operand(const uint8_t* buf, int row, int q) {
+    const uint8_t* r = buf + (row >> 4) * 2048 + (row & 15) * 16 + q * 256;
+    return big_join(*reinterpret_cast<const v4i*>(r), *reinterpret_cast<const v4i*>(r + 1024));
 }
 
 // Variants held to the register and LDS budget of two workgroups per CU (two wavefronts per SIMD).
@@ -201,8 +193,8 @@ __host__ __device__ constexpr bool big_two_per_cu(int tm, int tn, int depth, int
 // WMODE: how the weights are laid out and reach the MFMA.  0: row-major [N, K] (or operand order, gathered
 // row by row into the same LDS layout: the slow way, kept for shapes without a dedicated variant), staged
 // through LDS in 128-byte rows.  1: MFMA operand order (weight_layout.h), staged through LDS as they lie:
-// a copy instruction moves 1 KB in a row, and lane (l32, h) finds chunk c of its row at
-// unit * 2 KB + c * 256 + (l32 % 16) * 16.  2: operand order and WGM == 1, so that a wavefront's weight
+// a copy instruction moves 1 KB in a row, and lane (l16, q) finds chunk c of its row at
+// unit * 2 KB + c * 256 + l16 * 16.  2: operand order and WGM == 1, so that a wavefront's weight
 // blocks are its own: they go global -> registers, DEPTH stage-loads ahead through a ring of register
 // sets, and LDS carries the activations only.
 template <int TM, int TN, int DEPTH, int EPI, bool SPLIT, int WGM = 2, int WGN = 2, int WMODE = 0, bool RAGGED = false>
@@ -233,7 +225,8 @@ void gemm_fp8_big_kernel(
     constexpr int CA = BM / 32, CB = BDIRECT ? 0 : BN / 32;   // copy instructions (8 rows each) per wavefront per stage
     constexpr int BL = BDIRECT ? TN * 4 : 0;         // 16-byte weight loads per lane per stage: TN blocks x 2 K halves x 2
     constexpr int COPIES = CA + CB + BL;             // vector-memory instructions per wavefront per stage-load
-    constexpr int SLOTS_PER_STAGE = 2 * TM * TN;     // MFMAs of a wavefront per stage
+    constexpr int SLOTS_PER_STAGE = 4 * TM * TN;     // MFMAs of a wavefront per stage
+    constexpr int SLOTS_AFTER = BDIRECT ? 2 * (TM - 1) * TN : (2 * TN - 1) * TM;   // ... behind its barrier / hand-over
     // Requests of a stage-load are numbered; request n goes out behind MFMA n / CPS counted from the barrier of
     // the stage that frees its target: CPS per MFMA, so that they are out by mid-stage.
     // LEAD: the barrier of stage d frees the target of stage-load d + LEAD.  Staged operands: LEAD = DEPTH - the
@@ -245,13 +238,13 @@ void gemm_fp8_big_kernel(
     // Weights in registers, ring of eight (one column block per wavefront, stages of 8 MFMAs or fewer): LEAD = 6, so
     // that a wavefront may run two stages ahead of the slowest (see the hand-over below) with its weight loads six
     // stages and its activation copies three stages old when they are needed.
-    constexpr int CPS = BDIRECT ? (COPIES + (TM - 1) * TN - 1) / ((TM - 1) * TN) : (COPIES * 2 + SLOTS_PER_STAGE - 1) / SLOTS_PER_STAGE;
+    constexpr int CPS = BDIRECT ? (COPIES + SLOTS_AFTER - 1) / SLOTS_AFTER : (COPIES * 2 + SLOTS_PER_STAGE - 1) / SLOTS_PER_STAGE;
     constexpr int LEAD = BDIRECT ? (DEPTH == 8 ? 6 : DEPTH - 1) : DEPTH;
     // (weights in registers) progress word d of a wavefront vouches for its activation copies up to stage-load
     // d + CLAIM; SLACK: how many stages a wavefront may be ahead of the slowest one
     constexpr int CLAIM = DEPTH == 8 ? 3 : 2;
     constexpr int SLACK = CLAIM - 1 < DEPTH - LEAD ? CLAIM - 1 : DEPTH - LEAD;
-    constexpr int LATE = (TM - 1) * TN * CPS;        // first request number that falls into the next stage
+    constexpr int LATE = SLOTS_AFTER * CPS;          // first request number that falls into the next stage
     constexpr int IDX_END = COPIES;
     static_assert(!BDIRECT || COPIES <= LATE, "with weights in registers every request goes out behind the barrier");
     static_assert((TM == TN && TM % 2 == 0) || (TM == 3 && TN == 2) || (TM == 7 && TN == 2) || (TM == 2 && TN == 1 && !GATED) ||
@@ -266,7 +259,7 @@ void gemm_fp8_big_kernel(
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WGN, wn = wave % WGN;
-    const int l32 = lane & 31, h = lane >> 5;
+    const int l16 = lane & 15, q = lane >> 4;
     (void)wm;
     const int half_n = p.N / 2;
     BigTile tile_id;
@@ -291,13 +284,20 @@ void gemm_fp8_big_kernel(
     const int m0 = tile_id.m * BM;
     const int n0 = GATED ? tile_id.n * (BN / 2) : tile_id.n * BN;
 
-    v16f acc[TM][TN];
+    // acc[i][j][p][b]: rows 32 i + 16 p .., columns 32 j + 16 b .. of the wavefront's tile
+    v4f acc[TM][TN][2][2];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int e = 0; e < TM * TN * 4; ++e) acc[e / (TN * 4)][e / 4 % TN][e / 2 % 2][e % 2] = v4f{0.f, 0.f, 0.f, 0.f};
+    // The multiply in inline assembly, with the sum in place: left to the compiler, a sum may land in other registers than
+    // it came from, and with 96 - 256 of them live that ends in copies and spills (3 x 2 blocks: 174 registers this way,
+    // 256 the other; 7 x 2 did not fit).  AGPRs where a wavefront has its SIMD to itself.  The s_nop covers a VALU write of
+    // an operand just before (the hazards inside an asm are not the compiler's).
+    constexpr bool ACC_IN_AGPR = !big_two_per_cu(TM, TN, DEPTH, WMODE);
+    auto multiply = [&](v8i w, v8i x, v4f& c) {
+        if constexpr (ACC_IN_AGPR) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
+        else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+v"(c) : "v"(w), "v"(x));
+    };
+    auto acc_of = [&](int blk, int e) -> float { return acc[blk / TN][blk % TN][e >> 3][(e >> 2) & 1][e & 3]; };   // e: 0 .. 15
 
     // ---- copy geometry: wavefront w moves 8-row groups w*CA .. of A and w*CB .. of B; lane i
     // fills slot i%8 of row i/8 of its group with the chunk that the swizzle assigns to it ------
@@ -354,16 +354,19 @@ void gemm_fp8_big_kernel(
         b_source = copy_source(p.b, (uint32_t)p.N * (uint32_t)p.K);
     }
     const int b_step_shift = (OPW || p.operand_w) ? 4 : 0;   // a K step of operand-order weights is 2 KB away, not 128 bytes
-    // BDIRECT: this lane's 16 bytes of chunk h of row l32 of weight block j, K step 0; chunk c of the same row
-    // is c * 256 further, the next K step 2 KB
-    const uint8_t* bsrc[BDIRECT ? TN : 1];
-    v4i bring[BDIRECT ? DEPTH : 1][BDIRECT ? TN : 1][2][2];   // [stage-load % DEPTH][block][K half][chunk pair]
+    // BDIRECT: unit b of weight block j, K step 0 (the same for the whole wavefront); lane i takes bytes 16 i of its first
+    // KB (chunk q of row l16: the units' own order) and of its second, the next K step is 2 KB further
+    const uint32_t lane16 = (uint32_t)lane * 16;
+    const uint8_t* bsrc[BDIRECT ? TN : 1][2];
+    v4i bring[BDIRECT ? DEPTH : 1][BDIRECT ? TN : 1][2][2];   // [stage-load % DEPTH][block][unit][chunk pair]
     if constexpr (BDIRECT) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const uint32_t u = unit0 + (uint32_t)(wn * (WN / 16) + 2 * j) + ((uint32_t)l32 >> 4);
-            bsrc[j] = p.b + (size_t)(u < units ? u : units - 1) * ((size_t)p.K << 4) + ((size_t)k_begin << 4) + h * 256 + (l32 & 15) * 16;
-        }
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const uint32_t u = unit0 + (uint32_t)(__builtin_amdgcn_readfirstlane(wn) * (WN / 16) + 2 * j + b);
+                bsrc[j][b] = p.b + (size_t)(u < units ? u : units - 1) * ((size_t)p.K << 4) + ((size_t)k_begin << 4);
+            }
     }
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
     const uint32_t wave_a = __builtin_amdgcn_readfirstlane(lds_base + wave * (CA * 1024));
@@ -372,7 +375,7 @@ void gemm_fp8_big_kernel(
     // (slot: d % DEPTH as a compile-time value, needed where the target is a register set)
     auto issue = [&](int d, int c, auto slot) {
         const int k = k_begin + d * BIG_BK;
-        const uint32_t stage_off = (d % DEPTH) * STAGE_BYTES;
+        const uint32_t stage_off = __builtin_amdgcn_readfirstlane((d % DEPTH) * STAGE_BYTES);   // (goes into m0: a scalar)
         if constexpr (RAGGED) {
             const uint32_t last = k + BIG_BK > p.K ? ~0u : 0u;   // (uniform)
             if (c < CA) copy16_to_lds_checked(a_source, aoff[c] | (a_gone[c & 1] & last), k, wave_a + stage_off + c * 1024);
@@ -384,8 +387,8 @@ void gemm_fp8_big_kernel(
         } else if constexpr (BDIRECT) {
             constexpr int S = decltype(slot)::value;
             if ((PHYAI_FP8_ABLATE & 8) && d >= LEAD) return;
-            const int e = c - CA, j = e >> 2, kh = (e >> 1) & 1, pr = e & 1;   // chunk 4 kh + 2 pr + h of block j
-            bring[S][j][kh][pr] = *reinterpret_cast<const v4i*>(bsrc[j] + ((size_t)d << 11) + (4 * kh + 2 * pr) * 256);
+            const int e = c - CA, j = e >> 2, b = (e >> 1) & 1, pr = e & 1;   // half pr of unit b of block j
+            bring[S][j][b][pr] = *reinterpret_cast<const v4i*>(bsrc[j][b] + ((size_t)d << 11) + pr * 1024 + lane16);
         } else {
             copy16_to_lds(p.b + ((size_t)k << b_step_shift), boff[c - CA], wave_b + stage_off + (c - CA) * 1024);
         }
@@ -396,12 +399,13 @@ void gemm_fp8_big_kernel(
     const int n_loads = RAGGED && SPLIT ? ((k_begin + p.k_per_split < p.K ? p.k_per_split : p.K - k_begin) + BIG_BK - 1) / BIG_BK
                         : RAGGED        ? (p.K + BIG_BK - 1) / BIG_BK
                                         : (SPLIT ? p.k_per_split : p.K) / BIG_BK;
-    const int arow = wm * WM + l32, brow = wn * WN + l32;
+    const int arow = wm * WM + l16, brow = wn * WN + l16;
     auto stage_ptr = [&](int d) -> const uint8_t* { return lds + (d % DEPTH) * STAGE_BYTES; };
-    // weight block with first row `row` - l32 out of the staged B rows, K half kh
-    auto read_b = [&](const uint8_t* bbuf, int row, int kh) -> v8i {
-        if constexpr (WMODE == 1) return big_frag_operand(bbuf, row, h, kh);
-        else return big_frag(bbuf, row, h, kh);
+    // 16-row block jj of the wavefront's staged weight rows
+    auto read_b = [&](const uint8_t* stage, int jj) -> v8i {
+        const uint8_t* bbuf = stage + BM * BIG_BK;
+        if constexpr (WMODE == 1) return big_frag_operand(bbuf, brow + jj * 16, q);
+        else return big_frag(bbuf, brow + jj * 16, q);
     };
 
     // Weights in registers: LDS carries the activations only, and the wavefronts hand its stages to each other
@@ -438,22 +442,20 @@ void gemm_fp8_big_kernel(
         }
     };
 
-    // Operand blocks read one K half ahead: those of the current half (cur) and of the next one
-    // (nxt); the two sets swap roles every half.  All B blocks and the first A block - or all A
-    // blocks when there are only two row groups, which are too short to hide an LDS read.
-    constexpr bool A_AHEAD = TM == 2;
-    constexpr int NA = A_AHEAD ? TM : 1;             // A blocks read a half ahead
-    v8i fa_cur[TM], fa_nxt[TM], fb_cur[TN], fb_nxt[TN];
+    // A stage-load is multiplied in two halves, each with one 16-row half (p) of the wavefront's 32-row activation blocks
+    // and all of its weights: TM x 2 TN MFMAs.  Activation blocks of half p are in fa[p]; staged weights (fb) are read
+    // once per stage-load, block by block into the registers that its predecessor's last MFMA has just left.
+    // Weights in registers: only the block that opens a half is read ahead of it (fa[p][0]), the others behind its first
+    // MFMAs (the ring of weight sets leaves no room for two sets of activation blocks).
+    // (224-row tiles with staged weights read only the first three of a half's activation blocks ahead, the others where
+    // the last group of MFMAs leaves their predecessors' registers: two whole sets of seven do not fit)
+    constexpr int NA = BDIRECT ? 1 : TM;             // activation blocks of stage-load 0 read in front of the loop
+    constexpr int AHEAD_BLOCKS = TM == 7 ? 3 : TM;
+    v8i fa[2][TM], fb[BDIRECT ? 1 : 2 * TN];
 
-// One K half (64 bytes, TM*TN MFMAs per wavefront) of stage-load D.  KH: which half.  FA0/FB: its
-// opening blocks (in registers); NFA0/NFB receive those of the half that follows (the other half
-// of the same stage, or half 0 of stage-load D+1).  NEXT: that half exists.
+// LDS reads are issued long before their MFMAs: a batch of 128-bit reads takes several hundred cycles to land.
 //
-// LDS reads are issued long before their MFMAs: a batch of 128-bit reads takes several hundred
-// cycles to land, a row group of four MFMAs 256.  Row group 0 requests the remaining A blocks of
-// this half, row groups 1.. the opening blocks of the next half (B0 and A0 first).
-//
-// One barrier per stage-load, in half 1 after row group 0: by then a wavefront has issued every
+// One barrier per stage-load, in half 1 after the first group of MFMAs: by then a wavefront has issued every
 // LDS read of stage-load D, so the barrier both publishes stage-load D+1 (own copies awaited
 // first: AHEAD later stage-loads may stay in flight) and releases D's stage, which load D+DEPTH
 // then refills.  Its copies are requested one or two at a time between the MFMAs that follow - a
@@ -461,70 +463,94 @@ void gemm_fp8_big_kernel(
 // MFMA pipe runs dry.  ISSUE: load D+DEPTH exists (requests after the barrier); ISSUE_P: load
 // D-1+DEPTH exists (requests still being spread before the barrier).  All flags are literals, so
 // the steady-state loop body is straight-line code.
-#define PHYAI_RUN_HALF(D, SLOT, KH, NEXT, AHEAD, ISSUE_P, ISSUE, FA0, FB, NFA0, NFB)                           \
+//
+// PHYAI_MFMA_SLOT: one MFMA and the requests that go out behind it; SLOT_: MFMAs since the last barrier.
+#define PHYAI_MFMA_SLOT(FB, FA, ACC, SLOT_)                                                                    \
+    {                                                                                                          \
+        multiply(FB, FA, ACC);                                                                                 \
+        _Pragma("unroll") for (int c_ = 0; c_ < CPS; ++c_)                                                     \
+            if (req_ && (SLOT_) * CPS + c_ < IDX_END && !(PHYAI_FP8_ABLATE & 1)) {                             \
+                /* (register set of the load: its number modulo DEPTH) */                                      \
+                if (after_) issue(load_, (SLOT_) * CPS + c_, std::integral_constant<int, (stage_slot_ + LEAD) % DEPTH>{});     \
+                else issue(load_, (SLOT_) * CPS + c_, std::integral_constant<int, (stage_slot_ + LEAD - 1) % DEPTH>{}); \
+            }                                                                                                  \
+        __builtin_amdgcn_sched_barrier(0);                                                                     \
+    }
+// Half P of stage-load D with staged weights: weight block after weight block, so that a block's registers are free for
+// the next stage-load's as soon as its own MFMAs are issued.
+#define PHYAI_RUN_HALF_STAGED(D, SLOT, P, NEXT, AHEAD, ISSUE_P, ISSUE)                                         \
     {                                                                                                          \
         const int d_ = (D);                                                                                    \
-        const uint8_t* abuf_ = stage_ptr(d_);                                                                  \
-        const uint8_t* nbuf_ = (KH) == 0 ? abuf_ : stage_ptr(d_ + 1);                                          \
-        v8i fa_[TM];                                                                                           \
-        v4i seen_ = {0, 0, 0, 0};                                                                              \
-        if constexpr (BDIRECT) if ((KH) == 1 && (NEXT)) seen_ = progress_words();                              \
-        _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) fa_[i_] = FA0[A_AHEAD ? i_ : 0];                     \
-        _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) {                                                    \
-            if (!A_AHEAD && i_ == 0) {                                                                         \
-                _Pragma("unroll") for (int a_ = 1; a_ < TM; ++a_)                                              \
-                    fa_[a_] = (PHYAI_FP8_ABLATE & 2) ? fa_[0] : big_frag(abuf_, arow + a_ * 32, h, KH);        \
-            }                                                                                                  \
-            if (i_ >= 1 && (NEXT)) {                                                                           \
-                /* item 0: B0; items 1..NA: the A blocks; then B1..: spread over row groups 1..TM-1 */         \
-                _Pragma("unroll") for (int q_ = 0; q_ < TN + NA; ++q_) {                                       \
-                    if (q_ * (TM - 1) / (TN + NA) != i_ - 1) continue;                                         \
-                    if (q_ >= 1 && q_ <= NA) NFA0[q_ - 1] = big_frag(nbuf_, arow + (q_ - 1) * 32, h, 1 - (KH)); \
-                    else if constexpr (!BDIRECT) {                                                             \
-                        const int j_ = q_ == 0 ? 0 : q_ - NA;                                                  \
-                        NFB[j_] = read_b(nbuf_ + BM * BIG_BK, brow + j_ * 32, 1 - (KH));                       \
-                    }                                                                                          \
-                }                                                                                              \
-            }                                                                                                  \
-            const bool after_ = (KH) == 1 && i_ >= 1;   /* past this stage-load's barrier */                   \
+        constexpr int stage_slot_ = (SLOT);                                                                    \
+        const uint8_t* nbuf_ = (P) == 0 ? stage_ptr(d_) : stage_ptr(d_ + 1);                                   \
+        if ((P) == 0) {                                                                                        \
+            _Pragma("unroll") for (int a_ = 0; a_ < AHEAD_BLOCKS; ++a_)                                        \
+                fa[1][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[0][a_] : big_frag(nbuf_, arow + a_ * 32 + 16, q);      \
+        }                                                                                                      \
+        _Pragma("unroll") for (int jj_ = 0; jj_ < 2 * TN; ++jj_) {                                             \
+            const bool after_ = (P) == 1 && jj_ >= 1;   /* past this stage-load's barrier */                   \
             const bool req_ = after_ ? (ISSUE) : (ISSUE_P);                                                    \
             const int load_ = after_ ? d_ + LEAD : d_ - 1 + LEAD;                                              \
-            /* MFMAs since the last barrier */                                                                 \
-            const int slot0_ = after_ ? (i_ - 1) * TN : (TM - 1) * TN + ((KH) * TM + i_) * TN;                 \
-            _Pragma("unroll") for (int j_ = 0; j_ < TN; ++j_) {                                                \
-                v8i fb_;                                                                                       \
-                if constexpr (BDIRECT) fb_ = big_join(bring[SLOT][j_][KH][0], bring[SLOT][j_][KH][1]);         \
-                else fb_ = FB[j_];                                                                             \
-                acc[i_][j_] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb_, fa_[i_], acc[i_][j_],       \
-                                                                               0, 0, 0, 0, 0, 0);              \
-                _Pragma("unroll") for (int c_ = 0; c_ < CPS; ++c_)                                             \
-                    if (req_ && (slot0_ + j_) * CPS + c_ < IDX_END && !(PHYAI_FP8_ABLATE & 1)) {               \
-                        /* (register set of the load: its number modulo DEPTH) */                              \
-                        if (after_) issue(load_, (slot0_ + j_) * CPS + c_, std::integral_constant<int, ((SLOT) + LEAD) % DEPTH>{});     \
-                        else issue(load_, (slot0_ + j_) * CPS + c_, std::integral_constant<int, ((SLOT) + LEAD - 1) % DEPTH>{}); \
-                    }                                                                                          \
-                __builtin_amdgcn_sched_barrier(0);                                                             \
+            const int slot0_ = after_ ? (jj_ - 1) * TM : SLOTS_AFTER + ((P) * 2 * TN + jj_) * TM;              \
+            _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) {                                                \
+                PHYAI_MFMA_SLOT(fb[jj_], fa[P][i_], acc[i_][jj_ >> 1][P][jj_ & 1], slot0_ + i_)                \
+                if (i_ >= AHEAD_BLOCKS && jj_ == 2 * TN - 1 && ((P) == 0 || (NEXT)))                           \
+                    fa[1 - (P)][i_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][i_] : big_frag(nbuf_, arow + i_ * 32 + 16 * (1 - (P)), q); \
             }                                                                                                  \
-            if ((KH) == 1 && i_ == 0 && (NEXT)) {                                                              \
-                if constexpr (BDIRECT) {                                                                       \
-                    /* my activation copies of D+CLAIM have landed (AHEAD: the stage-loads from that one on  */ \
-                    /* that have been requested: its weight loads, which follow its copies, and all of the   */ \
-                    /* later ones may be in flight); published, and everybody's of D+1 awaited               */ \
-                    wait_copies<(AHEAD) == 0 ? 0 : ((AHEAD) - 1) * COPIES + (COPIES - CA)>();                  \
-                    if (!(PHYAI_FP8_ABLATE & 4)) hand_over(d_, seen_);                                                \
-                    asm volatile("" ::: "memory");                                                             \
-                } else {                                                                                       \
+            if ((P) == 1 && (NEXT)) {                                                                          \
+                if (jj_ == 0) {                                                                                \
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* my reads of stage-load D have landed */ \
                     wait_copies<COPIES * (AHEAD)>();               /* ... my copies of D+1 too ... */          \
                     if (!(PHYAI_FP8_ABLATE & 4)) __syncthreads();  /* ... and so have everybody's */           \
                 }                                                                                              \
+                fb[jj_] = read_b(nbuf_, jj_);                                                                  \
+                /* the activation blocks of the next half 0: one or two behind each of the first groups */     \
+                _Pragma("unroll") for (int a_ = 0; a_ < AHEAD_BLOCKS; ++a_)                                    \
+                    if (a_ * TN / TM == jj_) fa[0][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[1][a_] : big_frag(nbuf_, arow + a_ * 32, q); \
             }                                                                                                  \
         }                                                                                                      \
     }
-// a whole stage-load: half 0 with the cur register set, half 1 with the nxt set
+// Half P of stage-load D with weights in registers: row block after row block.
+#define PHYAI_RUN_HALF_DIRECT(D, SLOT, P, NEXT, AHEAD, ISSUE_P, ISSUE)                                         \
+    {                                                                                                          \
+        const int d_ = (D);                                                                                    \
+        constexpr int stage_slot_ = (SLOT);                                                                    \
+        const uint8_t* abuf_ = stage_ptr(d_);                                                                  \
+        const uint8_t* nbuf_ = (P) == 0 ? abuf_ : stage_ptr(d_ + 1);                                           \
+        v4i seen_ = {0, 0, 0, 0};                                                                              \
+        if ((P) == 1 && (NEXT)) seen_ = progress_words();                                                      \
+        _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) {                                                    \
+            if (i_ == 0) {                                                                                     \
+                _Pragma("unroll") for (int a_ = 1; a_ < TM; ++a_)                                              \
+                    fa[P][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][0] : big_frag(abuf_, arow + a_ * 32 + 16 * (P), q); \
+            }                                                                                                  \
+            if (i_ == 1 + (TM - 1) / (TN + 1) && (NEXT)) fa[1 - (P)][0] = big_frag(nbuf_, arow + 16 * (1 - (P)), q); \
+            const bool after_ = (P) == 1 && i_ >= 1;   /* past this stage-load's hand-over */                  \
+            const bool req_ = after_ ? (ISSUE) : (ISSUE_P);                                                    \
+            const int load_ = after_ ? d_ + LEAD : d_ - 1 + LEAD;                                              \
+            const int slot0_ = after_ ? (i_ - 1) * 2 * TN : SLOTS_AFTER + ((P) * TM + i_) * 2 * TN;            \
+            _Pragma("unroll") for (int jj_ = 0; jj_ < 2 * TN; ++jj_)                                           \
+                PHYAI_MFMA_SLOT(big_join(bring[SLOT][jj_ >> 1][jj_ & 1][0], bring[SLOT][jj_ >> 1][jj_ & 1][1]), \
+                                fa[P][i_], acc[i_][jj_ >> 1][P][jj_ & 1], slot0_ + jj_)                        \
+            if ((P) == 1 && i_ == 0 && (NEXT)) {                                                               \
+                /* my activation copies of D+CLAIM have landed (AHEAD: the stage-loads from that one on  */     \
+                /* that have been requested: its weight loads, which follow its copies, and all of the   */     \
+                /* later ones may be in flight); published, and everybody's of D+1 awaited               */     \
+                wait_copies<(AHEAD) == 0 ? 0 : ((AHEAD) - 1) * COPIES + (COPIES - CA)>();                      \
+                if (!(PHYAI_FP8_ABLATE & 4)) hand_over(d_, seen_);                                             \
+                asm volatile("" ::: "memory");                                                                 \
+            }                                                                                                  \
+        }                                                                                                      \
+    }
+// a whole stage-load
 #define PHYAI_RUN_STAGE(D, SLOT, NEXT, AHEAD, ISSUE_P, ISSUE)                                                  \
-    PHYAI_RUN_HALF(D, SLOT, 0, 1, 0, ISSUE_P, 0, fa_cur, fb_cur, fa_nxt, fb_nxt)                               \
-    PHYAI_RUN_HALF(D, SLOT, 1, NEXT, AHEAD, ISSUE_P, ISSUE, fa_nxt, fb_nxt, fa_cur, fb_cur)
+    if constexpr (BDIRECT) {                                                                                   \
+        PHYAI_RUN_HALF_DIRECT(D, SLOT, 0, 1, 0, ISSUE_P, 0)                                                    \
+        PHYAI_RUN_HALF_DIRECT(D, SLOT, 1, NEXT, AHEAD, ISSUE_P, ISSUE)                                         \
+    } else {                                                                                                   \
+        PHYAI_RUN_HALF_STAGED(D, SLOT, 0, 1, 0, ISSUE_P, 0)                                                    \
+        PHYAI_RUN_HALF_STAGED(D, SLOT, 1, NEXT, AHEAD, ISSUE_P, ISSUE)                                         \
+    }
 
     // prologue: stage-loads 0 .. DEPTH-2 and the copies of load DEPTH-1 that the row groups after
     // a barrier would have requested in flight (the rest of it is spread over stage-load 0 like
@@ -566,9 +592,7 @@ void gemm_fp8_big_kernel(
     // compiler they are zeroed behind the wait, 1 - 2 k cycles in which nothing else happens)
     if constexpr (TM * TN >= 14) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
+        for (int e = 0; e < TM * TN * 4; ++e) asm volatile("" : "+a"(acc[e / (TN * 4)][e / 4 % TN][e / 2 % 2][e % 2]));
     }
     if constexpr (BDIRECT) {
         // stage-load 0 and the activations up to stage-load CLAIM - 1 have landed (what progress word -1 stands for)
@@ -579,11 +603,12 @@ void gemm_fp8_big_kernel(
     }
     __syncthreads();
     PHYAI_STAMP(1)
+    if constexpr (!BDIRECT) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-        if constexpr (!BDIRECT) fb_cur[j] = read_b(lds + BM * BIG_BK, brow + j * 32, 0);
+        for (int jj = 0; jj < 2 * TN; ++jj) fb[jj] = read_b(lds, jj);
+    }
 #pragma unroll
-    for (int i = 0; i < (A_AHEAD ? TM : 1); ++i) fa_cur[i] = big_frag(lds, arow + i * 32, h, 0);
+    for (int i = 0; i < NA; ++i) fa[0][i] = big_frag(lds, arow + i * 32, q);
     int d = 0;
     if constexpr (BDIRECT) {
         // the register sets are named at compile time: DEPTH stage-loads per trip (the launcher sees to it
@@ -634,7 +659,18 @@ void gemm_fp8_big_kernel(
         PHYAI_RUN_STAGE(d + 3, 3, 0, 0, 0, 0)
     }
 #undef PHYAI_RUN_STAGE
-#undef PHYAI_RUN_HALF
+#undef PHYAI_RUN_HALF_STAGED
+#undef PHYAI_RUN_HALF_DIRECT
+#undef PHYAI_MFMA_SLOT
+    // the last MFMAs' results, before anything else reads them (24 wait states; every sum passes behind them)
+    asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+    for (int e = 0; e < TM * TN * 4; ++e) {
+        v4f& c = acc[e / (TN * 4)][e / 4 % TN][e / 2 % 2][e % 2];
+        if constexpr (ACC_IN_AGPR) asm volatile("" : "+a"(c));
+        else asm volatile("" : "+v"(c));
+    }
+    __builtin_amdgcn_sched_barrier(0);
     PHYAI_STAMP(2)
 
     // ---- split-K: publish partial sums; the last split to arrive adds them in split order --
@@ -653,7 +689,7 @@ void gemm_fp8_big_kernel(
             for (int c = 0; c < TM * TN / 2; ++c) {
                 float frag[CHUNK];
 #pragma unroll
-                for (int r = 0; r < 32; ++r) frag[r] = acc[(2 * c) / TN][(2 * c) % TN + r / 16][r % 16];
+                for (int r = 0; r < 32; ++r) frag[r] = acc_of(2 * c + r / 16, r % 16);
                 splitk_publish_part<FRAG, 256, CHUNK>(p.partials, tile, S, split_z, c * CHUNK, frag);
             }
             wait_own_stores();
@@ -681,7 +717,8 @@ void gemm_fp8_big_kernel(
 #pragma unroll
                 for (int r = 0; r < GCH; ++r) {
                     const int blk = (c * GCH + r) / 16;
-                    acc[blk / TN][blk % TN][r % 16] = frag[r];
+                    const int e = r % 16;
+                    acc[blk / TN][blk % TN][e >> 3][(e >> 2) & 1][e & 3] = frag[r];
                 }
             }
         }
@@ -690,8 +727,8 @@ void gemm_fp8_big_kernel(
 
     PHYAI_STAMP(3)
     // ---- epilogue ------------------------------------------------------------------------
-    // The weight block is the MFMA's first operand, so accumulator r of lane (l32, h) of block
-    // (i, j) is the output at token row i*32 + l32, column j*32 + 8*(r/4) + 4*h + r%4: a lane
+    // The weight block is the MFMA's first operand, so accumulator r of lane (l16, q) of block
+    // (i, j, p, b) is the output at token row i*32 + 16*p + l16, column j*32 + 16*b + 4*q + r: a lane
     // owns runs of four consecutive columns of one row.  A run becomes four bf16 with two packed
     // converts and goes to the wavefront's slice of the (now idle) LDS as one 8-byte write; the
     // staged tile leaves row-wise, 16 bytes per lane, whole row segments per instruction.  The
@@ -727,11 +764,11 @@ void gemm_fp8_big_kernel(
             }
         }
     };
-    float sa[TM];
+    float sa[TM][2];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int m = m0 + wm * WM + i * 32 + l32;
-        sa[i] = p.a_scale[p.a_scale_scalar ? 0 : (m < p.M ? m : p.M - 1)];
+    for (int e = 0; e < 2 * TM; ++e) {
+        const int m = m0 + wm * WM + e * 16 + l16;
+        sa[e >> 1][e & 1] = p.a_scale[p.a_scale_scalar ? 0 : (m < p.M ? m : p.M - 1)];
     }
     __syncthreads();  // every wavefront is done reading operands from LDS
     uint8_t* stg = lds + wave * STG_BYTES;
@@ -744,69 +781,67 @@ void gemm_fp8_big_kernel(
     // accumulator r of a block, with the other half where there is one (a + b: the sum in split order either way)
     auto summed = [&](float a, const float* po, int r) { return SPLIT && add_other ? a + po[r] : a; };
     if constexpr (OPW && GATED) {
-        // Weights in the gated operand order: rows 4p .. 4p+3 of a 16-row unit are gate columns 2p, 2p+1 and up
-        // columns 2p, 2p+1.  Accumulator 4k + e of lane (l32, h) of block j is block row 8k + 4h + e, i.e. with
-        // e = 2t + b: gate (t = 0) / up (t = 1) of output column 16 j + 4 k + 2 h + b of the wavefront - a lane
-        // holds both halves of two neighbouring output columns per k.  Same arithmetic as below, operation for
-        // operation.
+        // Weights in the gated operand order: rows 4q .. 4q+3 of a 16-row unit are gate columns 2q, 2q+1 and up
+        // columns 2q, 2q+1 of the unit's 8.  Accumulator 2t + c of lane (l16, q) of unit b of block j is gate (t = 0) /
+        // up (t = 1) of output column 16 j + 8 b + 2 q + c of the wavefront - a lane holds both halves of two
+        // neighbouring output columns per unit.  Same arithmetic as below, operation for operation.
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            float sgk[4][2], suk[4][2], bgk[4][2], buk[4][2];
+            float sgk[2][2], suk[2][2], bgk[2][2], buk[2][2];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int n = nbase + 16 * j + 4 * k + 2 * h;
+            for (int b = 0; b < 2; ++b) {
+                const int n = nbase + 16 * j + 8 * b + 2 * q;
                 const int n_safe = n < n_lim ? n : 0;
 #pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    sgk[k][b] = p.b_scale[n_safe + b];
-                    suk[k][b] = p.b_scale[half_n + n_safe + b];
-                    bgk[k][b] = p.bias ? bf16_bits_to_f32(p.bias[n_safe + b]) : 0.f;
-                    buk[k][b] = p.bias ? bf16_bits_to_f32(p.bias[half_n + n_safe + b]) : 0.f;
+                for (int c = 0; c < 2; ++c) {
+                    sgk[b][c] = p.b_scale[n_safe + c];
+                    suk[b][c] = p.b_scale[half_n + n_safe + c];
+                    bgk[b][c] = p.bias ? bf16_bits_to_f32(p.bias[n_safe + c]) : 0.f;
+                    buk[b][c] = p.bias ? bf16_bits_to_f32(p.bias[half_n + n_safe + c]) : 0.f;
                 }
             }
             float pn[16] = {};
             other_half(0, j, pn);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                const int row = i * 32 + l32;
-                const int sw = (row / ROWS_PER_PASS) & (SLOTS - 1);
                 float po[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) po[r] = pn[r];
                 if (i + 1 < TM) other_half(i + 1, j, pn);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float g0 = __builtin_fmaf(summed(acc[i][j][4 * k + 0], po, 4 * k + 0), sa[i] * sgk[k][0], bgk[k][0]);
-                    const float g1 = __builtin_fmaf(summed(acc[i][j][4 * k + 1], po, 4 * k + 1), sa[i] * sgk[k][1], bgk[k][1]);
-                    const float u0 = __builtin_fmaf(summed(acc[i][j][4 * k + 2], po, 4 * k + 2), sa[i] * suk[k][0], buk[k][0]);
-                    const float u1 = __builtin_fmaf(summed(acc[i][j][4 * k + 3], po, 4 * k + 3), sa[i] * suk[k][1], buk[k][1]);
+                for (int pb = 0; pb < 4; ++pb) {
+                    const int half = pb >> 1, b = pb & 1, row = i * 32 + 16 * half + l16;
+                    const int sw = (row / ROWS_PER_PASS) & (SLOTS - 1);
+                    const v4f& a = acc[i][j][half][b];
+                    const float s = sa[i][half];
+                    const float g0 = __builtin_fmaf(summed(a[0], po, 4 * pb + 0), s * sgk[b][0], bgk[b][0]);
+                    const float g1 = __builtin_fmaf(summed(a[1], po, 4 * pb + 1), s * sgk[b][1], bgk[b][1]);
+                    const float u0 = __builtin_fmaf(summed(a[2], po, 4 * pb + 2), s * suk[b][0], buk[b][0]);
+                    const float u1 = __builtin_fmaf(summed(a[3], po, 4 * pb + 3), s * suk[b][1], buk[b][1]);
                     // gate and up pass through bf16 first, as the two-launch form materialises them
                     const uint32_t g01 = pack_bf16x2(g0, g1), u01 = pack_bf16x2(u0, u1);
                     const float o0 = apply_act<EPI>(__uint_as_float(g01 << 16)) * __uint_as_float(u01 << 16);
                     const float o1 = apply_act<EPI>(__uint_as_float(g01 & 0xFFFF0000u)) * __uint_as_float(u01 & 0xFFFF0000u);
-                    const int slot = (2 * j + (k >> 1)) ^ sw;
-                    *reinterpret_cast<uint32_t*>(stg + row * ROWB + slot * 16 + 8 * (k & 1) + 4 * h) = pack_bf16x2(o0, o1);
+                    *reinterpret_cast<uint32_t*>(stg + row * ROWB + ((2 * j + b) ^ sw) * 16 + 4 * q) = pack_bf16x2(o0, o1);
                 }
             }
         }
     } else {
 #pragma unroll
     for (int j = 0; j < TNO; ++j) {
-        v4f sg[4], bg[4], su[4], bu[4];
+        v4f sg[2], bg[2], su[2], bu[2];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int n = nbase + j * 32 + 8 * g + 4 * h;
+        for (int b = 0; b < 2; ++b) {
+            const int n = nbase + j * 32 + 16 * b + 4 * q;
             const int n_safe = n < n_lim ? n : 0;
-            load_cols(n_safe, sg[g], bg[g]);
-            if constexpr (GATED) load_cols(half_n + n_safe, su[g], bu[g]);
+            load_cols(n_safe, sg[b], bg[b]);
+            if constexpr (GATED) load_cols(half_n + n_safe, su[b], bu[b]);
         }
         float pn[16] = {}, un[16] = {};
         other_half(0, j, pn);
         if constexpr (GATED) other_half(0, j + TN / 2, un);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            const int row = i * 32 + l32;
-            const int sw = (row / ROWS_PER_PASS) & (SLOTS - 1);
             float po[16], pu[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) { po[r] = pn[r]; pu[r] = un[r]; }
@@ -815,14 +850,17 @@ void gemm_fp8_big_kernel(
                 if constexpr (GATED) other_half(i + 1, j + TN / 2, un);
             }
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
+            for (int pb = 0; pb < 4; ++pb) {
+                const int half = pb >> 1, b = pb & 1, row = i * 32 + 16 * half + l16;
+                const int sw = (row / ROWS_PER_PASS) & (SLOTS - 1);
+                const float s = sa[i][half];
                 float o[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(summed(acc[i][j][4 * g + e], po, 4 * g + e), sa[i] * sg[g][e], bg[g][e]);
+                for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(summed(acc[i][j][half][b][e], po, 4 * pb + e), s * sg[b][e], bg[b][e]);
                 if constexpr (GATED) {
                     float u[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) u[e] = __builtin_fmaf(summed(acc[i][j + TN / 2][4 * g + e], pu, 4 * g + e), sa[i] * su[g][e], bu[g][e]);
+                    for (int e = 0; e < 4; ++e) u[e] = __builtin_fmaf(summed(acc[i][j + TN / 2][half][b][e], pu, 4 * pb + e), s * su[b][e], bu[b][e]);
                     // gate and up pass through bf16 first, as the two-launch form materialises them
                     const uint32_t g01 = pack_bf16x2(o[0], o[1]), g23 = pack_bf16x2(o[2], o[3]);
                     const uint32_t u01 = pack_bf16x2(u[0], u[1]), u23 = pack_bf16x2(u[2], u[3]);
@@ -839,7 +877,7 @@ void gemm_fp8_big_kernel(
                 } else {
                     if (p.res.residual != nullptr) {       // out = residual + bf16(linear) * gate
                         const int m = m0 + wm * WM + row;
-                        const int n = nbase + j * 32 + 8 * g + 4 * h;
+                        const int n = nbase + j * 32 + 16 * b + 4 * q;
                         if (m < p.M && n < n_lim) {
                             const uint2 rs = *reinterpret_cast<const uint2*>(p.res.residual + (int64_t)m * p.res.ld_res + n);
                             const uint2 gt = *reinterpret_cast<const uint2*>(
@@ -851,8 +889,7 @@ void gemm_fp8_big_kernel(
                 uint2 w;
                 w.x = pack_bf16x2(o[0], o[1]);
                 w.y = pack_bf16x2(o[2], o[3]);
-                const int slot = (j * 4 + g) ^ sw;
-                *reinterpret_cast<uint2*>(stg + row * ROWB + slot * 16 + h * 8) = w;
+                *reinterpret_cast<uint2*>(stg + row * ROWB + ((j * 4 + 2 * b + (q >> 1)) ^ sw) * 16 + (q & 1) * 8) = w;
             }
         }
     }
