@@ -226,9 +226,9 @@ void gemm_fp8_big_kernel(
     constexpr int BL = BDIRECT ? TN * 4 : 0;         // 16-byte weight loads per lane per stage: TN blocks x 2 K halves x 2
     constexpr int COPIES = CA + CB + BL;             // vector-memory instructions per wavefront per stage-load
     constexpr int SLOTS_PER_STAGE = 4 * TM * TN;     // MFMAs of a wavefront per stage
-    constexpr int SLOTS_AFTER = BDIRECT ? 2 * (TM - 1) * TN : (2 * TN - 1) * TM;   // ... behind its barrier / hand-over
+    constexpr int SLOTS_AFTER = BDIRECT ? 2 * (TM == 4 ? TM : TM - 1) * TN : (2 * TN - 1) * TM;   // ... behind its barrier / hand-over
     // Requests of a stage-load are numbered; request n goes out behind MFMA n / CPS counted from the barrier of
-    // the stage that frees its target: CPS per MFMA, so that they are out by mid-stage.
+    // the stage that frees its target: CPS per MFMA.
     // LEAD: the barrier of stage d frees the target of stage-load d + LEAD.  Staged operands: LEAD = DEPTH - the
     // barrier waits for this wavefront's LDS reads of stage d, whose stage is then refilled.  Weights in registers:
     // LEAD = DEPTH - 1 - the targets (LDS stage and register set of stage d - 1) were last read by MFMAs that
@@ -238,7 +238,7 @@ void gemm_fp8_big_kernel(
     // Weights in registers, ring of eight (one column block per wavefront, stages of 8 MFMAs or fewer): LEAD = 6, so
     // that a wavefront may run two stages ahead of the slowest (see the hand-over below) with its weight loads six
     // stages and its activation copies three stages old when they are needed.
-    constexpr int CPS = BDIRECT ? (COPIES + SLOTS_AFTER - 1) / SLOTS_AFTER : (COPIES * 2 + SLOTS_PER_STAGE - 1) / SLOTS_PER_STAGE;
+    constexpr int CPS = BDIRECT ? (COPIES + SLOTS_AFTER - 1) / SLOTS_AFTER : 1;
     constexpr int LEAD = BDIRECT ? (DEPTH == 8 ? 6 : DEPTH - 1) : DEPTH;
     // (weights in registers) progress word d of a wavefront vouches for its activation copies up to stage-load
     // d + CLAIM; SLACK: how many stages a wavefront may be ahead of the slowest one
@@ -246,6 +246,7 @@ void gemm_fp8_big_kernel(
     constexpr int SLACK = CLAIM - 1 < DEPTH - LEAD ? CLAIM - 1 : DEPTH - LEAD;
     constexpr int LATE = SLOTS_AFTER * CPS;          // first request number that falls into the next stage
     constexpr int IDX_END = COPIES;
+    static_assert(BDIRECT || COPIES <= SLOTS_PER_STAGE, "a stage-load's requests are out before the next barrier");
     static_assert(!BDIRECT || COPIES <= LATE, "with weights in registers every request goes out behind the barrier");
     static_assert((TM == TN && TM % 2 == 0) || (TM == 3 && TN == 2) || (TM == 7 && TN == 2) || (TM == 2 && TN == 1 && !GATED) ||
                   (TM == 3 && TN == 1 && !GATED) || (TM == 4 && TN == 1 && !GATED && BDIRECT), "supported wavefront tiles");
@@ -449,7 +450,8 @@ void gemm_fp8_big_kernel(
     // MFMAs (the ring of weight sets leaves no room for two sets of activation blocks).
     // (224-row tiles with staged weights read only the first three of a half's activation blocks ahead, the others where
     // the last group of MFMAs leaves their predecessors' registers: two whole sets of seven do not fit)
-    constexpr int NA = BDIRECT ? 1 : TM;             // activation blocks of stage-load 0 read in front of the loop
+    constexpr bool A_ALL_AHEAD = !BDIRECT || TM == 4;
+    constexpr int NA = A_ALL_AHEAD ? TM : 1;         // activation blocks of stage-load 0 read in front of the loop
     constexpr int AHEAD_BLOCKS = TM == 7 ? 3 : TM;
     v8i fa[2][TM], fb[BDIRECT ? 1 : 2 * TN];
 
@@ -510,41 +512,49 @@ void gemm_fp8_big_kernel(
             }                                                                                                  \
         }                                                                                                      \
     }
-// Half P of stage-load D with weights in registers: row block after row block.
+// My activation copies of D+CLAIM have landed (AHEAD: the stage-loads from that one on that have been requested: its
+// weight loads, which follow its copies, and all of the later ones may be in flight); published, and everybody's of D+1
+// awaited.
+#define PHYAI_HAND_OVER(D_, AHEAD)                                                                             \
+    {                                                                                                          \
+        wait_copies<(AHEAD) == 0 ? 0 : ((AHEAD) - 1) * COPIES + (COPIES - CA)>();                              \
+        if (!(PHYAI_FP8_ABLATE & 4)) hand_over(D_, seen_);                                                     \
+        asm volatile("" ::: "memory");                                                                         \
+    }
+// Half P of stage-load D with weights in registers: row block after row block.  Four row blocks: all of a half's blocks are
+// read during the half before, one behind each pair of MFMAs, so that the hand-over can open half 1 and the requests have
+// all of it.  Seven: see above; the hand-over comes behind the first row block of half 1.
 #define PHYAI_RUN_HALF_DIRECT(D, SLOT, P, NEXT, AHEAD, ISSUE_P, ISSUE)                                         \
     {                                                                                                          \
         const int d_ = (D);                                                                                    \
         constexpr int stage_slot_ = (SLOT);                                                                    \
         const uint8_t* abuf_ = stage_ptr(d_);                                                                  \
         const uint8_t* nbuf_ = (P) == 0 ? abuf_ : stage_ptr(d_ + 1);                                           \
-        v4i seen_ = {0, 0, 0, 0};                                                                              \
-        if ((P) == 1 && (NEXT)) seen_ = progress_words();                                                      \
+        if ((P) == 1 && (NEXT) && !A_ALL_AHEAD) seen_ = progress_words();                                      \
+        if ((P) == 1 && (NEXT) && A_ALL_AHEAD) PHYAI_HAND_OVER(d_, AHEAD)                                      \
         _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) {                                                    \
-            if (i_ == 0) {                                                                                     \
+            if (i_ == 0 && !A_ALL_AHEAD) {                                                                     \
                 _Pragma("unroll") for (int a_ = 1; a_ < TM; ++a_)                                              \
                     fa[P][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][0] : big_frag(abuf_, arow + a_ * 32 + 16 * (P), q); \
             }                                                                                                  \
-            if (i_ == 1 + (TM - 1) / (TN + 1) && (NEXT)) fa[1 - (P)][0] = big_frag(nbuf_, arow + 16 * (1 - (P)), q); \
-            const bool after_ = (P) == 1 && i_ >= 1;   /* past this stage-load's hand-over */                  \
+            if (A_ALL_AHEAD && (P) == 0 && i_ == TM - 1) seen_ = progress_words();                             \
+            if (A_ALL_AHEAD && (NEXT))                                                                         \
+                fa[1 - (P)][i_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][i_] : big_frag(nbuf_, arow + i_ * 32 + 16 * (1 - (P)), q); \
+            if (i_ == 1 + (TM - 1) / (TN + 1) && !A_ALL_AHEAD && (NEXT)) fa[1 - (P)][0] = big_frag(nbuf_, arow + 16 * (1 - (P)), q); \
+            const bool after_ = (P) == 1 && (i_ >= 1 || A_ALL_AHEAD);   /* past this stage-load's hand-over */ \
             const bool req_ = after_ ? (ISSUE) : (ISSUE_P);                                                    \
             const int load_ = after_ ? d_ + LEAD : d_ - 1 + LEAD;                                              \
-            const int slot0_ = after_ ? (i_ - 1) * 2 * TN : SLOTS_AFTER + ((P) * TM + i_) * 2 * TN;            \
+            const int slot0_ = after_ ? (A_ALL_AHEAD ? i_ : i_ - 1) * 2 * TN : SLOTS_AFTER + ((P) * TM + i_) * 2 * TN; \
             _Pragma("unroll") for (int jj_ = 0; jj_ < 2 * TN; ++jj_)                                           \
                 PHYAI_MFMA_SLOT(big_join(bring[SLOT][jj_ >> 1][jj_ & 1][0], bring[SLOT][jj_ >> 1][jj_ & 1][1]), \
                                 fa[P][i_], acc[i_][jj_ >> 1][P][jj_ & 1], slot0_ + jj_)                        \
-            if ((P) == 1 && i_ == 0 && (NEXT)) {                                                               \
-                /* my activation copies of D+CLAIM have landed (AHEAD: the stage-loads from that one on  */     \
-                /* that have been requested: its weight loads, which follow its copies, and all of the   */     \
-                /* later ones may be in flight); published, and everybody's of D+1 awaited               */     \
-                wait_copies<(AHEAD) == 0 ? 0 : ((AHEAD) - 1) * COPIES + (COPIES - CA)>();                      \
-                if (!(PHYAI_FP8_ABLATE & 4)) hand_over(d_, seen_);                                             \
-                asm volatile("" ::: "memory");                                                                 \
-            }                                                                                                  \
+            if ((P) == 1 && i_ == 0 && (NEXT) && !A_ALL_AHEAD) PHYAI_HAND_OVER(d_, AHEAD)                      \
         }                                                                                                      \
     }
 // a whole stage-load
 #define PHYAI_RUN_STAGE(D, SLOT, NEXT, AHEAD, ISSUE_P, ISSUE)                                                  \
     if constexpr (BDIRECT) {                                                                                   \
+        v4i seen_ = {0, 0, 0, 0};                                                                              \
         PHYAI_RUN_HALF_DIRECT(D, SLOT, 0, 1, 0, ISSUE_P, 0)                                                    \
         PHYAI_RUN_HALF_DIRECT(D, SLOT, 1, NEXT, AHEAD, ISSUE_P, ISSUE)                                         \
     } else {                                                                                                   \
@@ -661,6 +671,7 @@ void gemm_fp8_big_kernel(
 #undef PHYAI_RUN_STAGE
 #undef PHYAI_RUN_HALF_STAGED
 #undef PHYAI_RUN_HALF_DIRECT
+#undef PHYAI_HAND_OVER
 #undef PHYAI_MFMA_SLOT
     // the last MFMAs' results, before anything else reads them (24 wait states; every sum passes behind them)
     asm volatile("s_nop 15\n\ts_nop 7");
