@@ -223,7 +223,7 @@ int phyai_fp8_mlp(const void *x, int64_t ldx, const void *w1, const float *w1_sc
 /*
  * phyai_fp8_quant_static + phyai_fp8_gemm (x_scale_is_scalar = 1) as one call: a linear whose activations have one
  * static scale (layers/linear/backends/torch.py:123-153).  residual / gate as for phyai_fp8_linear_addcmul, or both
- * null.  Up to 48 token rows and K = 16384 it is one launch where the grid fits the chip.
+ * null.  Up to 128 token rows and K = 16384 it is one launch where the grid fits the chip.
  */
 int phyai_fp8_linear_per_tensor(const void *x, int64_t ldx, const float *input_scale, const void *w, const float *w_scale,
                                 const void *bias, const void *residual, int64_t ld_res, const void *gate, int64_t ld_gate,

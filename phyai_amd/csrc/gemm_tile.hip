@@ -426,7 +426,14 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
     if (!tuning_env("PHYAI_FP8_TILE")) {
         const BigPlan bp = big_plan(M, N, K, epilogue, layout != W_ROW_MAJOR);
         const bool few_small_tiles = bp.tile == 128 && bp.cols == 128 && bp.tiles <= 64 && !tuning_env("PHYAI_FP8_BIG");
-        if (bp.tile && out16 && !(few_small_tiles && skinny_ok)) {
+        // ... and its 128 x 64 tiles lose to one round of weight-streaming workgroups on long K (777 x 1168 x 4304: 17.4
+        // against 15.0 us; level at K = 4096, 700 x 1408; 7.6 against 8.4 at K = 2048)
+        bool one_round = false;
+        if (bp.tile == 128 && bp.cols == 64 && K > 4096 && skinny_ok && !tuning_env("PHYAI_FP8_BIG")) {
+            const SkinnyPlan sp = skinny_plan(M, N, K, epilogue);
+            one_round = sp.tiles * sp.msplit <= 256;
+        }
+        if (bp.tile && out16 && !((few_small_tiles || one_round) && skinny_ok)) {
             c.kind = GemmChoice::BIG;
             c.big = bp;
             c.need = bp.splits > 1 ? kHeaderBytes + big_partial_bytes(M, N, epilogue, bp) : 0;

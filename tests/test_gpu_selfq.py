@@ -23,7 +23,7 @@ def _same(a, b):
 
 
 @pytest.mark.parametrize("K", [16, 144, 1040, 1392, 2064, 4224, 6016, 8192, 12160, 16384])
-@pytest.mark.parametrize("M,N,layout", [(1, 48, None), (3, 1040, "operand"), (8, 4112, None), (13, 3072, "operand"), (48, 208, None)])
+@pytest.mark.parametrize("M,N,layout", [(1, 48, None), (3, 1040, "operand"), (8, 4112, None), (13, 3072, "operand"), (48, 208, None), (125, 1040, "operand")])
 @pytest.mark.parametrize("source", ["rows", "scalar"])
 def test_linear(dev, monkeypatch, source, M, N, layout, K):
     from phyai_amd import ops
