@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import contextlib
 import contextvars
+import threading
 
 import torch
 
@@ -112,11 +113,19 @@ def workspace_owner(owner: WorkspaceOwner):
 # to the names of this module.  Its functions return None, with nothing launched, for a call they leave to
 # the Python code below: every check and every error message stays here.
 _host = None
+_host_lock = threading.Lock()
 
 
 def _native():
+    return _host if _host is not None else _bind_native()
+
+
+def _bind_native():
+    """Bound once, and in full before anyone sees it: several threads may make their first call at the same time."""
     global _host
-    if _host is None:   # (bound in full before anyone sees it: another thread may be in here as well)
+    with _host_lock:
+        if _host is not None:
+            return _host
         from phyai_amd.quant.types import ActivationView, Granularity
 
         _lib.load()
@@ -136,7 +145,7 @@ def _native():
         LinearBase.__call__, DenseMLP.__call__ = ext.bind_modules(globals(), ext, torch.nn.Module.__call__, hooks,
                                                                   LinearBase.forward, DenseMLP.forward)
         _host = ext
-    return _host
+        return _host
 
 
 def workspace_bytes(M: int, N: int, K: int, epilogue=EPI_NONE) -> int:
