@@ -341,10 +341,27 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- layers -------------------------------------------------------------------------------------------------------
+// A reference of its own.  The dictionaries that a module's parameters are read from belong to the program: another
+// thread (the GIL is released around a launch) or Python code that a call runs into (a property of the spec, the
+// workspace's allocation) may put something else there before the launch has used the addresses it was given.
+struct Ref {
+    PyObject* p = nullptr;
+    Ref() = default;
+    Ref(const Ref&) = delete;
+    Ref& operator=(const Ref&) = delete;
+    ~Ref() { Py_XDECREF(p); }
+    void set(PyObject* borrowed) {
+        Py_XINCREF(borrowed);
+        Py_XDECREF(p);
+        p = borrowed;
+    }
+    operator PyObject*() const { return p; }
+};
+
 // What the HIP kernel needs of a linear layer, read from the module's own dictionaries (a module's
-// __getattr__ costs half a microsecond per parameter).  Borrowed references.
+// __getattr__ costs half a microsecond per parameter) and held until the call returns.
 struct Layer {
-    PyObject *weight, *scale, *input_scale, *layout, *granularity;
+    Ref weight, scale, input_scale, layout, granularity, bias;
     bool stream;
 };
 PyObject* plain_attr(PyObject* o, PyObject* dict, PyObject* name) {   // instance attribute, else the class's
@@ -357,18 +374,18 @@ bool layer_of(PyObject* o, Layer* l) {
     PyObject* params = PyDict_GetItemWithError(*dp, s_parameters);
     PyObject* spec = PyDict_GetItemWithError(*dp, s_spec);
     if (!params || !PyDict_Check(params) || !spec) return false;
-    l->weight = PyDict_GetItemWithError(params, s_weight);
-    l->scale = PyDict_GetItemWithError(params, s_weight_scale);
-    l->input_scale = PyDict_GetItemWithError(params, s_input_scale);
+    l->weight.set(PyDict_GetItemWithError(params, s_weight));
+    l->scale.set(PyDict_GetItemWithError(params, s_weight_scale));
+    l->input_scale.set(PyDict_GetItemWithError(params, s_input_scale));
+    l->bias.set(PyDict_GetItemWithError(params, s_bias));
     if (!l->weight || !l->scale) return false;
-    l->layout = none_if_null(plain_attr(o, *dp, s_weight_layout));
-    PyObject* st = plain_attr(o, *dp, s_stream_weights);
+    l->layout.set(none_if_null(plain_attr(o, *dp, s_weight_layout)));
+    Ref st, held_spec;
+    held_spec.set(spec);
+    st.set(plain_attr(o, *dp, s_stream_weights));
     l->stream = st && PyObject_IsTrue(st) == 1;
-    PyObject* g = PyObject_GetAttr(spec, s_granularity);
-    if (!g) return false;
-    l->granularity = g;   // an enum member: its class keeps it
-    Py_DECREF(g);
-    return true;
+    l->granularity.p = PyObject_GetAttr(held_spec, s_granularity);
+    return l->granularity.p != nullptr;
 }
 
 PyObject* layer_call(const Layer& l, PyObject* x, PyObject* bias, int epi, PyObject* residual, PyObject* gate) {
@@ -424,13 +441,12 @@ bool hip_kernel_remembered(PyObject* layer, PyObject* x) {
     Py_DECREF(key);
     return kernel && Py_TYPE(kernel) == (PyTypeObject*)pl.kernel_type;
 }
-bool bias_of(PyObject* layer, PyObject** bias) {   // what the layer adds: None with skip_bias_add
-    PyObject** dp = _PyObject_GetDictPtr(layer);
-    PyObject* skip = PyDict_GetItemWithError(*dp, s_skip_bias_add);
-    PyObject* b = PyDict_GetItemWithError(PyDict_GetItemWithError(*dp, s_parameters), s_bias);
-    if (!skip || !b) return false;
-    *bias = skip == Py_False ? b : Py_None;
-    return skip == Py_False || skip == Py_True;
+// Whether the layer adds its own bias (None counts as one) or, with skip_bias_add, leaves it to the caller.
+enum BiasUse { BIAS_UNKNOWN, BIAS_ADDED, BIAS_LEFT };
+BiasUse bias_use(PyObject* layer, const Layer& l) {
+    PyObject* skip = PyDict_GetItemWithError(*_PyObject_GetDictPtr(layer), s_skip_bias_add);
+    if (!skip || !l.bias) return BIAS_UNKNOWN;
+    return skip == Py_False ? BIAS_ADDED : skip == Py_True ? BIAS_LEFT : BIAS_UNKNOWN;
 }
 
 // layer_forward(layer, x or ActivationView, epilogue, residual, gate): selection and call in one
@@ -438,12 +454,11 @@ PyObject* py_layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Layer l;
     int epi;
-    PyObject* bias;
-    if (n != 5 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || !bias_of(a[0], &bias) || !epilogue_of(a[2], &epi))
-        return declined();
-    if (bias == Py_None && PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[0]), s_skip_bias_add) == Py_True && (epi != 0 || a[3] != Py_None))
+    if (n != 5 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || !epilogue_of(a[2], &epi)) return declined();
+    const BiasUse use = bias_use(a[0], l);
+    if (use == BIAS_UNKNOWN || (use == BIAS_LEFT && (epi != 0 || a[3] != Py_None)))
         return declined();   // fused forms exist for layers that add their own bias
-    PyObject* y = layer_call(l, a[1], bias, epi, a[3], a[4]);
+    PyObject* y = layer_call(l, a[1], use == BIAS_ADDED ? l.bias.p : Py_None, epi, a[3], a[4]);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -507,13 +522,10 @@ PyObject* py_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // both projections per-channel layers that add their own bias
 PyObject* mlp_native(PyObject* first, PyObject* second, PyObject* x, int epi, PyObject* residual, PyObject* gate) {
     Layer p, q;
-    PyObject *b1, *b2;
     if (!tensor(x) || !hip_kernel_remembered(first, x) || !hip_kernel_remembered(second, x) || !layer_of(first, &p) || !layer_of(second, &q) ||
-        p.granularity != py.per_channel || q.granularity != py.per_channel || !bias_of(first, &b1) || !bias_of(second, &b2))
+        p.granularity != py.per_channel || q.granularity != py.per_channel || bias_use(first, p) != BIAS_ADDED || bias_use(second, q) != BIAS_ADDED)
         return nullptr;
-    for (PyObject* layer : {first, second})
-        if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(layer), s_skip_bias_add) != Py_False) return nullptr;
-    return mlp_call(x, p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None, residual, gate);
+    return mlp_call(x, p.weight, p.scale, p.bias, p.layout, p.stream, q.weight, q.scale, q.bias, q.layout, q.stream, epi, Py_None, residual, gate);
 }
 // mlp_forward(first layer, second layer, x, epilogue, residual, gate)
 PyObject* py_mlp_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -564,11 +576,9 @@ PyObject* py_relay_weight(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Layer l;
-    PyObject* bias;
-    if (n != 4 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || l.granularity != py.per_channel || !bias_of(a[0], &bias) ||
-        PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[0]), s_skip_bias_add) != Py_False)
+    if (n != 4 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || l.granularity != py.per_channel || bias_use(a[0], l) != BIAS_ADDED)
         return declined();
-    PyObject* y = linear_call(a[1], nullptr, l.weight, l.scale, bias, 0, l.layout, l.stream, Py_None, Py_None, Py_None, false, a[2], a[3]);
+    PyObject* y = linear_call(a[1], nullptr, l.weight, l.scale, l.bias, 0, l.layout, l.stream, Py_None, Py_None, Py_None, false, a[2], a[3]);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -576,11 +586,9 @@ PyObject* py_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_linear_residual(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Layer l;
-    PyObject* bias;
-    if (n != 4 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || l.granularity != py.per_channel || !bias_of(a[0], &bias) ||
-        PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[0]), s_skip_bias_add) != Py_False)
+    if (n != 4 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || l.granularity != py.per_channel || bias_use(a[0], l) != BIAS_ADDED)
         return declined();
-    PyObject* y = linear_call(a[1], nullptr, l.weight, l.scale, bias, 0, l.layout, l.stream, Py_None, a[2], a[3], true);
+    PyObject* y = linear_call(a[1], nullptr, l.weight, l.scale, l.bias, 0, l.layout, l.stream, Py_None, a[2], a[3], true);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
 }
@@ -589,14 +597,11 @@ PyObject* py_norm_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Layer p, q;
     int epi;
-    PyObject *b1, *b2;
     if (n != 6 || !tensor(a[2]) || !hip_kernel_remembered(a[0], a[2]) || !hip_kernel_remembered(a[1], a[2]) || !layer_of(a[0], &p) ||
         !layer_of(a[1], &q) || !epilogue_of(a[5], &epi) || p.granularity != py.per_channel || q.granularity != py.per_channel ||
-        !bias_of(a[0], &b1) || !bias_of(a[1], &b2))
+        bias_use(a[0], p) != BIAS_ADDED || bias_use(a[1], q) != BIAS_ADDED)
         return declined();
-    for (int i = 0; i < 2; ++i)
-        if (PyDict_GetItemWithError(*_PyObject_GetDictPtr(a[i]), s_skip_bias_add) != Py_False) return declined();
-    PyObject* y = mlp_call(a[2], p.weight, p.scale, b1, p.layout, p.stream, q.weight, q.scale, b2, q.layout, q.stream, epi, Py_None,
+    PyObject* y = mlp_call(a[2], p.weight, p.scale, p.bias, p.layout, p.stream, q.weight, q.scale, q.bias, q.layout, q.stream, epi, Py_None,
                            a[2], nullptr, a[3], a[4]);
     return y ? y : declined();
     END_HANDLE_TH_ERRORS
@@ -628,13 +633,11 @@ PyObject* py_linear_call(PyObject*, PyObject* args, PyObject* kwargs) {
         PyObject *self = PyTuple_GET_ITEM(args, 0), *x = PyTuple_GET_ITEM(args, 1);
         PyObject** dp = _PyObject_GetDictPtr(self);
         Layer l;
-        PyObject* bias;
-        if (dp && *dp && plain_call(self, *dp, pm.linear_forward) && hip_kernel_remembered(self, x) && layer_of(self, &l) && bias_of(self, &bias)) {
-            PyObject* y = layer_call(l, x, bias, 0, Py_None, Py_None);
+        if (dp && *dp && plain_call(self, *dp, pm.linear_forward) && hip_kernel_remembered(self, x) && layer_of(self, &l)) {
+            const BiasUse use = bias_use(self, l);
+            PyObject* y = use == BIAS_UNKNOWN ? nullptr : layer_call(l, x, use == BIAS_ADDED ? l.bias.p : Py_None, 0, Py_None, Py_None);
             if (y) {
-                PyObject* left = Py_None;
-                if (PyDict_GetItemWithError(*dp, s_skip_bias_add) == Py_True) left = PyDict_GetItemWithError(PyDict_GetItemWithError(*dp, s_parameters), s_bias);
-                PyObject* r = left ? PyTuple_Pack(2, y, left) : nullptr;
+                PyObject* r = PyTuple_Pack(2, y, use == BIAS_LEFT ? l.bias.p : Py_None);
                 Py_DECREF(y);
                 return r;
             }
@@ -658,8 +661,9 @@ PyObject* py_mlp_call(PyObject*, PyObject* args, PyObject* kwargs) {
             PyDict_GetItemWithError(*dp, s_fuse_activation) == Py_True) {
             PyObject *mods = PyDict_GetItemWithError(*dp, s_modules), *epilogue = PyDict_GetItemWithError(*dp, s_epilogue);
             const bool gated = PyDict_GetItemWithError(*dp, s_gated) == Py_True;
-            PyObject* first = mods ? PyDict_GetItemWithError(mods, gated ? s_gate_up : s_fc1) : nullptr;
-            PyObject* second = mods ? PyDict_GetItemWithError(mods, gated ? s_down : s_fc2) : nullptr;
+            Ref first, second;
+            first.set(mods ? PyDict_GetItemWithError(mods, gated ? s_gate_up : s_fc1) : nullptr);
+            second.set(mods ? PyDict_GetItemWithError(mods, gated ? s_down : s_fc2) : nullptr);
             int epi;
             if (first && second && epilogue && epilogue_of(epilogue, &epi)) {
                 PyObject* y = mlp_native(first, second, x, epi, residual, gate);

@@ -53,3 +53,34 @@ def test_two_threads_bind_the_native_path_once(monkeypatch):
     for t in threads:
         t.join()
     assert len(opened) == 1 and got[0] is got[1] is ops._host
+
+
+def test_a_native_call_keeps_the_parameters_it_read():
+    """Python code that runs in the middle of a call (a property of the spec, another thread while the GIL is released)
+    may give the layer another weight: the call goes on with the tensors it read, and they live until it returns."""
+    native, alive = ops._native(), []
+
+    class Swapping(Fp8Spec):
+        @property
+        def granularity(self):
+            if hasattr(self, "layer"):
+                layer, self.__dict__["layer"] = self.layer, None
+                if layer is not None:
+                    layer.weight = nn.Parameter(torch.empty_like(layer.weight), requires_grad=False)
+            return Granularity.PER_CHANNEL
+
+        @granularity.setter
+        def granularity(self, value):
+            pass
+
+    class Epilogue:   # looked up in a dictionary behind the layer's parameters
+        def __hash__(self):
+            alive.append(old() is not None)
+            return 0
+
+    lin = L.ColumnParallelLinear(128, 64, bias=False, params_dtype=torch.bfloat16, spec=Swapping(), device="cpu")
+    old = weakref.ref(lin.weight)
+    lin.spec.layer = lin
+    assert native.layer_apply(lin, torch.zeros(4, 128, dtype=torch.bfloat16), None, Epilogue(), None, None) is None
+    assert alive == [True]
+    assert old() is None, "and no longer"
