@@ -52,14 +52,14 @@ struct Py {
 struct PyLayers {
     PyObject *dispatch_dict, *mode, *kernel_type;
 } pl = {};
-// what the calls of modules need: phyai_amd.ops's dictionary, this extension, nn.Module.__call__, the tables of hooks that
-// apply to every module, and the forward methods that the calls below stand for
+// what the calls of modules need: phyai_amd.ops's dictionary, this extension, nn.Module and its __call__, the tables of
+// hooks that apply to every module, and the forward methods that the calls below stand for
 struct PyModules {
-    PyObject *ops_dict, *self, *module_call, *global_hooks, *linear_forward, *mlp_forward;
+    PyObject *ops_dict, *self, *module_type, *module_call, *global_hooks, *linear_forward, *mlp_forward;
 } pm = {};
 
 PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bias_add, *s_bias;
-PyObject *s_host, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
+PyObject *s_host, *s_call, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
     *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
     *s_spec, *s_granularity;
@@ -612,6 +612,7 @@ PyObject* py_norm_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // stands in between - no hooks, no compiled or replaced forward - and to nn.Module.__call__ otherwise.
 bool plain_call(PyObject* self, PyObject* dict, PyObject* forward) {
     if (!pm.self || PyDict_GetItemWithError(pm.ops_dict, s_host) != pm.self) return false;
+    if (_PyType_Lookup((PyTypeObject*)pm.module_type, s_call) != pm.module_call) return false;   // replaced, as torch.fx does while it traces
     if (_PyType_Lookup(Py_TYPE(self), s_forward) != forward || PyDict_GetItemWithError(dict, s_forward) || PyDict_GetItemWithError(dict, s_compiled))
         return false;
     for (PyObject* name : s_hooks) {
@@ -622,9 +623,11 @@ bool plain_call(PyObject* self, PyObject* dict, PyObject* forward) {
         if (PyDict_GET_SIZE(PyTuple_GET_ITEM(pm.global_hooks, i)) != 0) return false;
     return true;
 }
-PyObject* module_call(PyObject* args, PyObject* kwargs) {
+PyObject* module_call(PyObject* args, PyObject* kwargs) {   // nn.Module.__call__ as it is now
     PyErr_Clear();
-    return PyObject_Call(pm.module_call, args, kwargs);
+    Ref call;
+    call.p = PyObject_GetAttr(pm.module_type, s_call);
+    return call ? PyObject_Call(call, args, kwargs) : nullptr;
 }
 // linear(x) -> (output, bias left to the caller or None)
 PyObject* py_linear_call(PyObject*, PyObject* args, PyObject* kwargs) {
@@ -810,16 +813,16 @@ PyObject* py_bind_layers(PyObject*, PyObject* args) {
 
 PyMethodDef linear_call_def = {"__call__", (PyCFunction)(void (*)(void))py_linear_call, METH_VARARGS | METH_KEYWORDS, nullptr};
 PyMethodDef mlp_call_def = {"__call__", (PyCFunction)(void (*)(void))py_mlp_call, METH_VARARGS | METH_KEYWORDS, nullptr};
-// bind_modules(phyai_amd.ops's dictionary, this module, nn.Module.__call__, tuple of global hook tables,
+// bind_modules(phyai_amd.ops's dictionary, this module, nn.Module, its own __call__, tuple of global hook tables,
 //              LinearBase.forward, DenseMLP.forward) -> (LinearBase.__call__, DenseMLP.__call__)
 PyObject* py_bind_modules(PyObject*, PyObject* args) {
     PyModules m = {};
-    if (!PyArg_ParseTuple(args, "O!OOO!OO", &PyDict_Type, &m.ops_dict, &m.self, &m.module_call, &PyTuple_Type, &m.global_hooks,
-                          &m.linear_forward, &m.mlp_forward))
+    if (!PyArg_ParseTuple(args, "O!OO!OO!OO", &PyDict_Type, &m.ops_dict, &m.self, &PyType_Type, &m.module_type, &m.module_call, &PyTuple_Type,
+                          &m.global_hooks, &m.linear_forward, &m.mlp_forward))
         return nullptr;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(m.global_hooks); ++i)
         if (!PyDict_Check(PyTuple_GET_ITEM(m.global_hooks, i))) return PyErr_Format(PyExc_TypeError, "hook tables are dictionaries");
-    for (PyObject* o : {m.ops_dict, m.self, m.module_call, m.global_hooks, m.linear_forward, m.mlp_forward}) Py_INCREF(o);
+    for (PyObject* o : {m.ops_dict, m.self, m.module_type, m.module_call, m.global_hooks, m.linear_forward, m.mlp_forward}) Py_INCREF(o);
     pm = m;
     PyObject *a = PyCFunction_New(&linear_call_def, nullptr), *b = PyCFunction_New(&mlp_call_def, nullptr);
     PyObject *ma = a ? PyInstanceMethod_New(a) : nullptr, *mb = b ? PyInstanceMethod_New(b) : nullptr;
@@ -858,7 +861,7 @@ PyMODINIT_FUNC PyInit__phyai_host() {
         {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_weight_scale, "weight_scale"}, {&s_input_scale, "input_scale"},
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
         {&s_granularity, "granularity"}, {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
-        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_forward, "forward"},
+        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward, "forward"},
         {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
         {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},
         {&s_compiled, "_compiled_call_impl"}, {&s_hooks[0], "_forward_hooks"}, {&s_hooks[1], "_forward_pre_hooks"},

@@ -114,6 +114,7 @@ def workspace_owner(owner: WorkspaceOwner):
 # the Python code below: every check and every error message stays here.
 _host = None
 _host_lock = threading.Lock()
+_module_call = torch.nn.Module.__call__   # (as it was on import: the first call may come while a tracer has replaced it)
 
 
 def _native():
@@ -142,7 +143,7 @@ def _bind_native():
         from phyai_amd.mlp import DenseMLP
 
         hooks = (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks)
-        LinearBase.__call__, DenseMLP.__call__ = ext.bind_modules(globals(), ext, torch.nn.Module.__call__, hooks,
+        LinearBase.__call__, DenseMLP.__call__ = ext.bind_modules(globals(), ext, torch.nn.Module, _module_call, hooks,
                                                                   LinearBase.forward, DenseMLP.forward)
         _host = ext
         return _host

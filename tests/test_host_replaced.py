@@ -84,3 +84,29 @@ def test_a_native_call_keeps_the_parameters_it_read():
     assert native.layer_apply(lin, torch.zeros(4, 128, dtype=torch.bfloat16), None, Epilogue(), None, None) is None
     assert alive == [True]
     assert old() is None, "and no longer"
+
+
+def test_a_replaced_module_call_is_called(monkeypatch):
+    """torch.fx records calls of modules by replacing nn.Module.__call__ while it traces."""
+    ops._native()
+    lin = _bf16_linear()
+
+    class Leaves(torch.fx.Tracer):
+        def is_leaf_module(self, m, name):
+            return isinstance(m, (L.ColumnParallelLinear, DenseMLP))
+
+    class Model(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.lin = lin
+            self.mlp = DenseMLP(16, 32, params_dtype=torch.bfloat16)
+
+        def forward(self, x):
+            return self.mlp(self.lin(x)[0])
+
+    graph = Leaves().trace(Model())
+    assert [n.target for n in graph.nodes if n.op == "call_module"] == ["lin", "mlp"]
+    seen, own = [], nn.Module.__call__
+    monkeypatch.setattr(nn.Module, "__call__", lambda self, *a, **k: (seen.append(type(self)), own(self, *a, **k))[1])
+    lin(torch.zeros(2, 32, dtype=torch.bfloat16))
+    assert seen == [L.ColumnParallelLinear]
