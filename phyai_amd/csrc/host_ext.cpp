@@ -50,7 +50,7 @@ struct Py {
     PyObject *workspaces, *owner, *reserve, *epilogues, *layouts, *view_type, *per_channel, *per_tensor;
 } py = {};
 struct PyLayers {
-    PyObject *dispatch_dict, *mode, *kernel_type;
+    PyObject *dispatch_dict, *mode, *kernel_type, *kernel_apply;
 } pl = {};
 // what the calls of modules need: phyai_amd.ops's dictionary, this extension, nn.Module and its __call__, the tables of
 // hooks that apply to every module, and the forward methods that the calls below stand for
@@ -62,7 +62,7 @@ PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bia
 PyObject *s_host, *s_call, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
     *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
-    *s_spec, *s_granularity;
+    *s_spec, *s_granularity, *s_apply;
 
 PyObject* declined() {
     PyErr_Clear();
@@ -364,6 +364,11 @@ struct Layer {
     Ref weight, scale, input_scale, layout, granularity, bias;
     bool stream;
 };
+// Whether calling o.name() would run `fn`: the class's own method, not overridden by the instance.
+bool has_method(PyObject* o, PyObject* name, PyObject* fn) {
+    PyObject** dp = _PyObject_GetDictPtr(o);
+    return _PyType_Lookup(Py_TYPE(o), name) == fn && !(dp && *dp && PyDict_GetItemWithError(*dp, name));
+}
 PyObject* plain_attr(PyObject* o, PyObject* dict, PyObject* name) {   // instance attribute, else the class's
     PyObject* v = PyDict_GetItemWithError(dict, name);
     return v ? v : _PyType_Lookup(Py_TYPE(o), name);
@@ -413,7 +418,8 @@ PyObject* py_layer_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // Whether the dispatcher's remembered choice (LinearBase._kernel_for, which fills the memory this reads) for
-// this layer and input is the HIP kernel.  False also where nothing is remembered yet.
+// this layer and input is the HIP kernel with its own apply, which the native calls stand for.  False also where nothing
+// is remembered yet.
 bool hip_kernel_remembered(PyObject* layer, PyObject* x) {
     PyObject** dp = _PyObject_GetDictPtr(layer);
     if (!dp || !*dp || !pl.mode) return false;
@@ -439,7 +445,7 @@ bool hip_kernel_remembered(PyObject* layer, PyObject* x) {
     if (!key) return false;
     PyObject* kernel = PyDict_GetItemWithError(PyTuple_GET_ITEM(memo, 4), key);
     Py_DECREF(key);
-    return kernel && Py_TYPE(kernel) == (PyTypeObject*)pl.kernel_type;
+    return kernel && Py_TYPE(kernel) == (PyTypeObject*)pl.kernel_type && has_method(kernel, s_apply, pl.kernel_apply);
 }
 // Whether the layer adds its own bias (None counts as one) or, with skip_bias_add, leaves it to the caller.
 enum BiasUse { BIAS_UNKNOWN, BIAS_ADDED, BIAS_LEFT };
@@ -800,13 +806,11 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
-// bind_layers(phyai_amd.linear.dispatch's dictionary, mode variable, HipFp8Kernel)
+// bind_layers(phyai_amd.linear.dispatch's dictionary, mode variable, HipFp8Kernel, its apply)
 PyObject* py_bind_layers(PyObject*, PyObject* args) {
     PyLayers p = {};
-    if (!PyArg_ParseTuple(args, "O!OO", &PyDict_Type, &p.dispatch_dict, &p.mode, &p.kernel_type)) return nullptr;
-    Py_INCREF(p.dispatch_dict);
-    Py_INCREF(p.mode);
-    Py_INCREF(p.kernel_type);
+    if (!PyArg_ParseTuple(args, "O!OOO", &PyDict_Type, &p.dispatch_dict, &p.mode, &p.kernel_type, &p.kernel_apply)) return nullptr;
+    for (PyObject* o : {p.dispatch_dict, p.mode, p.kernel_type, p.kernel_apply}) Py_INCREF(o);
     pl = p;
     Py_RETURN_NONE;
 }
@@ -860,7 +864,7 @@ PyMODINIT_FUNC PyInit__phyai_host() {
     const struct { PyObject** at; const char* text; } names[] = {
         {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_weight_scale, "weight_scale"}, {&s_input_scale, "input_scale"},
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
-        {&s_granularity, "granularity"}, {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
+        {&s_granularity, "granularity"}, {&s_apply, "apply"}, {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
         {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward, "forward"},
         {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
         {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},

@@ -76,6 +76,9 @@ class HipFp8Kernel:
         raise RuntimeError(f"HipFp8Kernel got unhandled spec_id={spec_id!r}")
 
 
+HIP_FP8_APPLY = HipFp8Kernel.apply   # what the native calls of csrc/host_ext.cpp stand for; another apply is called
+
+
 @register_linear_kernel()
 class TorchBf16Kernel:
     name = "torch"

@@ -136,7 +136,7 @@ def _bind_native():
         from phyai_amd import state
         from phyai_amd.linear import dispatch, kernels
 
-        ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel)
+        ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel, kernels.HIP_FP8_APPLY)
         from torch.nn.modules import module as m
 
         from phyai_amd.linear.layers import LinearBase
