@@ -50,7 +50,7 @@ struct Py {
     PyObject *workspaces, *owner, *reserve, *epilogues, *layouts, *view_type, *per_channel, *per_tensor;
 } py = {};
 struct PyLayers {
-    PyObject *dispatch_dict, *mode, *kernel_type, *kernel_apply;
+    PyObject *dispatch_dict, *mode, *kernel_type, *kernel_apply, *quantize_activation;
 } pl = {};
 // what the calls of modules need: phyai_amd.ops's dictionary, this extension, nn.Module and its __call__, the tables of
 // hooks that apply to every module, and the forward methods that the calls below stand for
@@ -62,7 +62,7 @@ PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bia
 PyObject *s_host, *s_call, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
     *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
-    *s_spec, *s_granularity, *s_apply;
+    *s_spec, *s_granularity, *s_apply, *s_quantize;
 
 PyObject* declined() {
     PyErr_Clear();
@@ -361,7 +361,7 @@ struct Ref {
 // What the HIP kernel needs of a linear layer, read from the module's own dictionaries (a module's
 // __getattr__ costs half a microsecond per parameter) and held until the call returns.
 struct Layer {
-    Ref weight, scale, input_scale, layout, granularity, bias;
+    Ref weight, scale, input_scale, layout, granularity, bias, spec;
     bool stream;
 };
 // Whether calling o.name() would run `fn`: the class's own method, not overridden by the instance.
@@ -385,11 +385,11 @@ bool layer_of(PyObject* o, Layer* l) {
     l->bias.set(PyDict_GetItemWithError(params, s_bias));
     if (!l->weight || !l->scale) return false;
     l->layout.set(none_if_null(plain_attr(o, *dp, s_weight_layout)));
-    Ref st, held_spec;
-    held_spec.set(spec);
+    l->spec.set(spec);
+    Ref st;
     st.set(plain_attr(o, *dp, s_stream_weights));
     l->stream = st && PyObject_IsTrue(st) == 1;
-    l->granularity.p = PyObject_GetAttr(held_spec, s_granularity);
+    l->granularity.p = PyObject_GetAttr(l->spec, s_granularity);
     return l->granularity.p != nullptr;
 }
 
@@ -401,7 +401,8 @@ PyObject* layer_call(const Layer& l, PyObject* x, PyObject* bias, int epi, PyObj
     }
     if (l.granularity == py.per_channel)
         return linear_call(x, nullptr, l.weight, l.scale, bias, epi, l.layout, l.stream, Py_None, residual, gate);
-    if (l.granularity == py.per_tensor && l.input_scale)
+    // (a spec that makes these codes in another way is asked for them, by the Python path)
+    if (l.granularity == py.per_tensor && l.input_scale && has_method(l.spec, s_quantize, pl.quantize_activation))
         return linear_static_call(x, l.input_scale, l.weight, l.scale, bias, epi, l.layout, l.stream, residual, gate);
     return nullptr;
 }
@@ -806,11 +807,12 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
-// bind_layers(phyai_amd.linear.dispatch's dictionary, mode variable, HipFp8Kernel, its apply)
+// bind_layers(phyai_amd.linear.dispatch's dictionary, mode variable, HipFp8Kernel, its apply, Fp8Spec.quantize_activation)
 PyObject* py_bind_layers(PyObject*, PyObject* args) {
     PyLayers p = {};
-    if (!PyArg_ParseTuple(args, "O!OOO", &PyDict_Type, &p.dispatch_dict, &p.mode, &p.kernel_type, &p.kernel_apply)) return nullptr;
-    for (PyObject* o : {p.dispatch_dict, p.mode, p.kernel_type, p.kernel_apply}) Py_INCREF(o);
+    if (!PyArg_ParseTuple(args, "O!OOOO", &PyDict_Type, &p.dispatch_dict, &p.mode, &p.kernel_type, &p.kernel_apply, &p.quantize_activation))
+        return nullptr;
+    for (PyObject* o : {p.dispatch_dict, p.mode, p.kernel_type, p.kernel_apply, p.quantize_activation}) Py_INCREF(o);
     pl = p;
     Py_RETURN_NONE;
 }
@@ -864,7 +866,8 @@ PyMODINIT_FUNC PyInit__phyai_host() {
     const struct { PyObject** at; const char* text; } names[] = {
         {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_weight_scale, "weight_scale"}, {&s_input_scale, "input_scale"},
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
-        {&s_granularity, "granularity"}, {&s_apply, "apply"}, {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
+        {&s_granularity, "granularity"}, {&s_apply, "apply"}, {&s_quantize, "quantize_activation"},
+        {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
         {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward, "forward"},
         {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
         {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},

@@ -135,8 +135,9 @@ def _bind_native():
                  Granularity.PER_CHANNEL, Granularity.PER_TENSOR)
         from phyai_amd import state
         from phyai_amd.linear import dispatch, kernels
+        from phyai_amd.quant import specs
 
-        ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel, kernels.HIP_FP8_APPLY)
+        ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel, kernels.HIP_FP8_APPLY, specs.FP8_QUANTIZE_ACTIVATION)
         from torch.nn.modules import module as m
 
         from phyai_amd.linear.layers import LinearBase

@@ -154,4 +154,6 @@ class Fp8Spec:
                              out=layer.weight.data, scale_out=layer.weight_scale.data)
 
 
+FP8_QUANTIZE_ACTIVATION = Fp8Spec.quantize_activation   # what csrc/host_ext.cpp stands for; another one is called
+
 __all__ = ["Bf16Spec", "Fp8Spec"]

@@ -32,6 +32,28 @@ def _fill(lin, seed):
     return lin
 
 
+def test_an_overridden_activation_quantizer_is_called(dev, linear):
+    """Static scales: the layer's spec makes the codes (the reference's kernels call it, linear/backends/torch.py:132)."""
+    L = linear
+
+    class Halved(L.Fp8Spec):
+        def quantize_activation(self, x, layer):
+            return super().quantize_activation(x * 0.5, layer)
+
+    def made(spec):
+        return _fill(L.ColumnParallelLinear(H, 256, bias=False, params_dtype=torch.bfloat16, spec=spec), 30)
+
+    x = seeded((M, H), 31).to(dev)
+    plain, halved = made(L.Fp8Spec(granularity=L.Granularity.PER_TENSOR)), made(Halved(granularity=L.Granularity.PER_TENSOR))
+    want = plain(x * 0.5)[0]
+    assert not torch.equal(plain(x)[0], want)
+    assert torch.equal(halved(x)[0], want)
+    patched = made(L.Fp8Spec(granularity=L.Granularity.PER_TENSOR))
+    own = patched.spec.quantize_activation
+    patched.spec.quantize_activation = lambda x, layer: own(x * 0.5, layer)
+    assert torch.equal(patched(x)[0], want)
+
+
 @pytest.mark.parametrize("where", ["class", "instance"])
 def test_an_instrumented_kernel_is_called(dev, linear, monkeypatch, where):
     from phyai_amd.linear.dispatch import get_linear_dispatcher
