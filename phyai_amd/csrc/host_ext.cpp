@@ -55,11 +55,12 @@ struct PyLayers {
 // what the calls of modules need: phyai_amd.ops's dictionary, this extension, nn.Module and its __call__, the tables of
 // hooks that apply to every module, and the forward methods that the calls below stand for
 struct PyModules {
-    PyObject *ops_dict, *self, *module_type, *module_call, *global_hooks, *linear_forward, *mlp_forward;
+    PyObject *ops_dict, *self, *module_type, *module_call, *global_hooks, *linear_forward, *mlp_forward, *linear_forward_fused,
+        *linear_forward_addcmul, *norm_forward_fp8, *linear_call;
 } pm = {};
 
 PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bias_add, *s_bias;
-PyObject *s_host, *s_call, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
+PyObject *s_host, *s_call, *s_forward_fused, *s_forward_addcmul, *s_forward_fp8, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
     *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
     *s_spec, *s_granularity, *s_apply, *s_quantize;
@@ -636,6 +637,19 @@ PyObject* module_call(PyObject* args, PyObject* kwargs) {   // nn.Module.__call_
     call.p = PyObject_GetAttr(pm.module_type, s_call);
     return call ? PyObject_Call(call, args, kwargs) : nullptr;
 }
+// decoder_layer_plain(qkv_proj, o_proj, gate_up_proj, down_proj, first norm, second norm): whether the three calls above
+// do what these parts' own methods would - qkv_proj called as a module (hooks, a replaced forward, a wrapper around
+// it), the others through the methods that a decoder layer uses of them
+PyObject* py_decoder_layer_plain(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "six parts");
+    PyObject** dp = _PyObject_GetDictPtr(a[0]);
+    const bool plain = pm.self && dp && *dp && _PyType_Lookup(Py_TYPE(a[0]), s_call) == pm.linear_call && plain_call(a[0], *dp, pm.linear_forward) &&
+                       has_method(a[1], s_forward_addcmul, pm.linear_forward_addcmul) && has_method(a[2], s_forward_fused, pm.linear_forward_fused) &&
+                       has_method(a[3], s_forward_addcmul, pm.linear_forward_addcmul) && has_method(a[4], s_forward_fp8, pm.norm_forward_fp8) &&
+                       has_method(a[5], s_forward_fp8, pm.norm_forward_fp8);
+    if (PyErr_Occurred()) return nullptr;
+    return PyBool_FromLong(plain);
+}
 // linear(x) -> (output, bias left to the caller or None)
 PyObject* py_linear_call(PyObject*, PyObject* args, PyObject* kwargs) {
     HANDLE_TH_ERRORS
@@ -820,20 +834,26 @@ PyObject* py_bind_layers(PyObject*, PyObject* args) {
 PyMethodDef linear_call_def = {"__call__", (PyCFunction)(void (*)(void))py_linear_call, METH_VARARGS | METH_KEYWORDS, nullptr};
 PyMethodDef mlp_call_def = {"__call__", (PyCFunction)(void (*)(void))py_mlp_call, METH_VARARGS | METH_KEYWORDS, nullptr};
 // bind_modules(phyai_amd.ops's dictionary, this module, nn.Module, its own __call__, tuple of global hook tables,
-//              LinearBase.forward, DenseMLP.forward) -> (LinearBase.__call__, DenseMLP.__call__)
+//              LinearBase.forward, DenseMLP.forward, LinearBase.forward_fused, .forward_addcmul, AdaRMSNorm.forward_fp8)
+//   -> (LinearBase.__call__, DenseMLP.__call__)
 PyObject* py_bind_modules(PyObject*, PyObject* args) {
     PyModules m = {};
-    if (!PyArg_ParseTuple(args, "O!OO!OO!OO", &PyDict_Type, &m.ops_dict, &m.self, &PyType_Type, &m.module_type, &m.module_call, &PyTuple_Type,
-                          &m.global_hooks, &m.linear_forward, &m.mlp_forward))
+    if (!PyArg_ParseTuple(args, "O!OO!OO!OOOOO", &PyDict_Type, &m.ops_dict, &m.self, &PyType_Type, &m.module_type, &m.module_call, &PyTuple_Type,
+                          &m.global_hooks, &m.linear_forward, &m.mlp_forward, &m.linear_forward_fused, &m.linear_forward_addcmul,
+                          &m.norm_forward_fp8))
         return nullptr;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(m.global_hooks); ++i)
         if (!PyDict_Check(PyTuple_GET_ITEM(m.global_hooks, i))) return PyErr_Format(PyExc_TypeError, "hook tables are dictionaries");
-    for (PyObject* o : {m.ops_dict, m.self, m.module_type, m.module_call, m.global_hooks, m.linear_forward, m.mlp_forward}) Py_INCREF(o);
-    pm = m;
+    for (PyObject* o : {m.ops_dict, m.self, m.module_type, m.module_call, m.global_hooks, m.linear_forward, m.mlp_forward, m.linear_forward_fused,
+                        m.linear_forward_addcmul, m.norm_forward_fp8})
+        Py_INCREF(o);
     PyObject *a = PyCFunction_New(&linear_call_def, nullptr), *b = PyCFunction_New(&mlp_call_def, nullptr);
     PyObject *ma = a ? PyInstanceMethod_New(a) : nullptr, *mb = b ? PyInstanceMethod_New(b) : nullptr;
     Py_XDECREF(a);
     Py_XDECREF(b);
+    Py_XINCREF(ma);
+    m.linear_call = ma;
+    pm = m;
     return ma && mb ? Py_BuildValue("NN", ma, mb) : nullptr;
 }
 
@@ -853,6 +873,7 @@ PyMethodDef methods[] = {
     PHYAI_FAST("norm_linear", py_norm_linear),
     PHYAI_FAST("linear_residual", py_linear_residual),
     PHYAI_FAST("norm_mlp", py_norm_mlp),
+    PHYAI_FAST("decoder_layer_plain", py_decoder_layer_plain),
     PHYAI_FAST("quant_rowwise", py_quant_rowwise),
     PHYAI_FAST("rmsnorm", py_rmsnorm),
     PHYAI_FAST("adarmsnorm", py_adarmsnorm),
@@ -868,7 +889,8 @@ PyMODINIT_FUNC PyInit__phyai_host() {
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
         {&s_granularity, "granularity"}, {&s_apply, "apply"}, {&s_quantize, "quantize_activation"},
         {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
-        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward, "forward"},
+        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward_fused, "forward_fused"}, {&s_forward_addcmul, "forward_addcmul"},
+        {&s_forward_fp8, "forward_fp8"}, {&s_forward, "forward"},
         {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
         {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},
         {&s_compiled, "_compiled_call_impl"}, {&s_hooks[0], "_forward_hooks"}, {&s_hooks[1], "_forward_pre_hooks"},

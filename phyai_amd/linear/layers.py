@@ -198,6 +198,10 @@ class LinearBase(nn.Module):
         return getattr(self._kernel_for(x), "name", "") == "hip_fp8" and not self.skip_bias_add
 
 
+# The methods that the native calls of csrc/host_ext.cpp stand for; others in their place are called.
+LINEAR_METHODS = (LinearBase.forward, LinearBase.forward_fused, LinearBase.forward_addcmul)
+
+
 class ReplicatedLinear(LinearBase):
     """Full weight on every rank (reference ``layers.py:126-198``)."""
 

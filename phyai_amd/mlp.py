@@ -145,4 +145,6 @@ class DenseMLP(nn.Module):
                 f"activation={self.activation!r}, gated={self.gated}, bias={self.bias_enabled}")
 
 
+MLP_FORWARD = DenseMLP.forward   # what the native call of csrc/host_ext.cpp stands for; another one is called
+
 __all__ = ["DenseMLP"]

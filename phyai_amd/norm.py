@@ -136,3 +136,6 @@ class AdaRMSNorm(nn.Module):
 
     def extra_repr(self) -> str:
         return f"{self.hidden_size}, cond_dim={self.cond_dim}, eps={self.variance_epsilon}, backend={self.backend!r}"
+
+
+ADA_FORWARD_FP8 = AdaRMSNorm.forward_fp8   # what the native calls of csrc/host_ext.cpp stand for; another one is called

@@ -140,12 +140,14 @@ def _bind_native():
         ext.bind_layers(dispatch.__dict__, state._MODE, kernels.HipFp8Kernel, kernels.HIP_FP8_APPLY, specs.FP8_QUANTIZE_ACTIVATION)
         from torch.nn.modules import module as m
 
-        from phyai_amd.linear.layers import LinearBase
-        from phyai_amd.mlp import DenseMLP
+        from phyai_amd.linear.layers import LINEAR_METHODS, LinearBase
+        from phyai_amd.mlp import MLP_FORWARD, DenseMLP
+        from phyai_amd.norm import ADA_FORWARD_FP8
 
         hooks = (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks)
-        LinearBase.__call__, DenseMLP.__call__ = ext.bind_modules(globals(), ext, torch.nn.Module, _module_call, hooks,
-                                                                  LinearBase.forward, DenseMLP.forward)
+        forward, *fused = LINEAR_METHODS
+        LinearBase.__call__, DenseMLP.__call__ = ext.bind_modules(globals(), ext, torch.nn.Module, _module_call, hooks, forward,
+                                                                  MLP_FORWARD, *fused, ADA_FORWARD_FP8)
         _host = ext
         return _host
 

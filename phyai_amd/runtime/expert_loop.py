@@ -102,17 +102,15 @@ class ExpertLayer(nn.Module):
                 variant: str = "fused") -> torch.Tensor:
         residual = h
         if variant == "fused":
-            mods = self._modules   # (a module's attributes go through its __getattr__, a third of a microsecond each)
-            mlp = mods["mlp"]._modules
-            out = self._three_calls(mods, mlp, h, attend, index, modulation)
+            out = self._three_calls(h, attend, index, modulation)
             if out is not None:
                 return out
-            view, gate_attn = mods["input_layernorm"].forward_fp8(h, modulation=modulation.input_ln)
-            fused, _ = mods["qkv_proj"](view)
-            h = mods["o_proj"].forward_addcmul(attend(fused, index), residual, gate_attn)
-            view, gate_mlp = mods["post_attention_layernorm"].forward_fp8(h, modulation=modulation.post_attention_ln)
-            act = mlp["gate_up_proj"].forward_fused(view, "geglu_tanh")
-            return mlp["down_proj"].forward_addcmul(act, h, gate_mlp)
+            view, gate_attn = self.input_layernorm.forward_fp8(h, modulation=modulation.input_ln)
+            fused, _ = self.qkv_proj(view)
+            h = self.o_proj.forward_addcmul(attend(fused, index), residual, gate_attn)
+            view, gate_mlp = self.post_attention_layernorm.forward_fp8(h, modulation=modulation.post_attention_ln)
+            act = self.mlp.gate_up_proj.forward_fused(view, "geglu_tanh")
+            return self.mlp.down_proj.forward_addcmul(act, h, gate_mlp)
         if variant == "unfused":
             n, gate_attn = self.input_layernorm(h, modulation=modulation.input_ln)
             fused, _ = self.qkv_proj(n)
@@ -129,30 +127,34 @@ class ExpertLayer(nn.Module):
             return torch.addcmul(h, _torch_fp8_linear(act, self.mlp.down_proj), gate_mlp)
         raise ValueError(f"unknown variant {variant!r}; expected one of {VARIANTS}")
 
-
-    def _three_calls(self, mods, mlp, h, attend: Attend, index: int, modulation: ExpertLayerModulation):
+    def _three_calls(self, h, attend: Attend, index: int, modulation: ExpertLayerModulation):
         """The layer as three library calls around attention: norm + qkv_proj, o_proj + gated residual, norm + MLP +
         gated residual; for few token rows each norm runs inside the linear that follows it.  The gates are read where
-        they lie in the modulation rows.  Same bits as the calls below; None when this form does not serve the input."""
+        they lie in the modulation rows.  Same bits as the calls they stand for; None when this form does not serve the
+        input, or when a part is not the package's own or has something attached that those calls would run."""
         if h.dim() != 2 or h.shape[1] != self.hidden_size:
             return None
-        native, qkv, o = ops._native(), mods["qkv_proj"], mods["o_proj"]
-        first, second = mlp["gate_up_proj"], mlp["down_proj"]
-        fused = native.norm_linear(qkv, h, modulation.input_ln, mods["input_layernorm"].variance_epsilon)
+        mods = self._modules   # (a module's attributes go through its __getattr__, a third of a microsecond each)
+        mlp = getattr(mods.get("mlp"), "_modules", None) or {}
+        native, qkv, o, first, second = ops._native(), mods.get("qkv_proj"), mods.get("o_proj"), mlp.get("gate_up_proj"), mlp.get("down_proj")
+        norm1, norm2 = mods.get("input_layernorm"), mods.get("post_attention_layernorm")
+        if not native.decoder_layer_plain(qkv, o, first, second, norm1, norm2):
+            return None
+        fused = native.norm_linear(qkv, h, modulation.input_ln, norm1.variance_epsilon)
         if fused is None:
             if not all(lin.supports_fused_epilogue(h) for lin in (qkv, o, first, second)):
                 return None
             # (the dispatcher's choice for this token count and mode is remembered now)
-            fused = native.norm_linear(qkv, h, modulation.input_ln, mods["input_layernorm"].variance_epsilon)
+            fused = native.norm_linear(qkv, h, modulation.input_ln, norm1.variance_epsilon)
             if fused is None:
                 return None
         a = attend(fused, index)
         r = native.linear_residual(o, a, h, modulation.input_ln)
         if r is None:
             r = o.forward_addcmul(a, h, modulation.input_ln[:, 2 * self.hidden_size:].contiguous())
-        out = native.norm_mlp(first, second, r, modulation.post_attention_ln, mods["post_attention_layernorm"].variance_epsilon, "geglu_tanh")
+        out = native.norm_mlp(first, second, r, modulation.post_attention_ln, norm2.variance_epsilon, "geglu_tanh")
         if out is None:
-            view, gate_mlp = mods["post_attention_layernorm"].forward_fp8(r, modulation=modulation.post_attention_ln)
+            view, gate_mlp = norm2.forward_fp8(r, modulation=modulation.post_attention_ln)
             out = second.forward_addcmul(first.forward_fused(view, "geglu_tanh"), r, gate_mlp)
         return out
 

@@ -32,6 +32,75 @@ def _fill(lin, seed):
     return lin
 
 
+@pytest.fixture
+def expert(dev, linear):
+    """(layer, call): call() is one pass of a small decoder layer in the fused form, its output."""
+    from phyai_amd.runtime.expert_loop import ExpertLayer, ExpertLayerModulation
+
+    layer = ExpertLayer(H, HEAD, HEADS, 1, I, H)
+    for j, lin in enumerate((layer.qkv_proj, layer.o_proj, layer.mlp.gate_up_proj, layer.mlp.down_proj)):
+        _fill(lin, 10 + j)
+    mod = ExpertLayerModulation(seeded((1, 3 * H), 20, 0.1).to(dev), seeded((1, 3 * H), 21, 0.1).to(dev))
+    x = seeded((M, H), 22).to(dev)
+    return layer, lambda: layer(x, lambda fused, index: fused[:, :HEAD * HEADS], 0, mod)
+
+
+def test_hooks_of_qkv_proj_run(expert):
+    layer, call = expert
+    want, seen = call(), []
+    handle = layer.qkv_proj.register_forward_hook(lambda mod, args, out: seen.append("after"))
+    before = layer.qkv_proj.register_forward_pre_hook(lambda mod, args: seen.append("before"))
+    assert torch.equal(call(), want) and seen == ["before", "after"]
+    handle.remove()
+    before.remove()
+    assert torch.equal(call(), want) and len(seen) == 2
+
+
+@pytest.mark.parametrize("what", ["instance", "class", "wrapper", "not a registered module"])
+def test_a_replaced_qkv_proj_is_called(expert, what):
+    layer, call = expert
+    want, own, seen = call(), layer.qkv_proj, []
+    if what == "instance":
+        forward = own.forward
+        own.forward = lambda x: (seen.append(1), forward(x))[1]
+    elif what == "class":
+        class Watched(type(own)):
+            def forward(self, x):
+                seen.append(1)
+                return super().forward(x)
+
+        own.__class__ = Watched
+    else:
+        class Wrapper(torch.nn.Module):
+            def __init__(self):
+                super().__init__()
+                self.inner = own
+
+            def forward(self, x):
+                seen.append(1)
+                return self.inner(x)
+
+        wrapper = Wrapper()
+        if what == "wrapper":
+            layer.qkv_proj = wrapper
+        else:
+            del layer.qkv_proj
+            layer.__dict__["qkv_proj"] = wrapper
+    assert torch.equal(call(), want) and seen == [1]
+
+
+@pytest.mark.parametrize("name,method", [("input_layernorm", "forward_fp8"), ("post_attention_layernorm", "forward_fp8"),
+                                         ("o_proj", "forward_addcmul"), ("mlp.gate_up_proj", "forward_fused"),
+                                         ("mlp.down_proj", "forward_addcmul")])
+def test_replaced_methods_of_the_other_parts_are_called(expert, name, method):
+    layer, call = expert
+    want, seen = call(), []
+    part = layer.get_submodule(name)
+    own = getattr(part, method)
+    setattr(part, method, lambda *a, **k: (seen.append(1), own(*a, **k))[1])
+    assert torch.equal(call(), want) and seen == [1]
+
+
 def test_an_overridden_activation_quantizer_is_called(dev, linear):
     """Static scales: the layer's spec makes the codes (the reference's kernels call it, linear/backends/torch.py:132)."""
     L = linear
