@@ -56,11 +56,11 @@ struct PyLayers {
 // hooks that apply to every module, and the forward methods that the calls below stand for
 struct PyModules {
     PyObject *ops_dict, *self, *module_type, *module_call, *global_hooks, *linear_forward, *mlp_forward, *linear_forward_fused,
-        *linear_forward_addcmul, *norm_forward_fp8, *linear_call;
+        *linear_forward_addcmul, *norm_forward_fp8, *linear_supports, *linear_call;
 } pm = {};
 
 PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bias_add, *s_bias;
-PyObject *s_host, *s_call, *s_forward_fused, *s_forward_addcmul, *s_forward_fp8, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
+PyObject *s_host, *s_call, *s_forward_fused, *s_forward_addcmul, *s_forward_fp8, *s_supports, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
     *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
     *s_spec, *s_granularity, *s_apply, *s_quantize;
@@ -419,6 +419,8 @@ PyObject* py_layer_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// Fused epilogues are for layers that say so themselves.
+bool own_supports(PyObject* layer) { return has_method(layer, s_supports, pm.linear_supports); }
 // Whether the dispatcher's remembered choice (LinearBase._kernel_for, which fills the memory this reads) for
 // this layer and input is the HIP kernel with its own apply, which the native calls stand for.  False also where nothing
 // is remembered yet.
@@ -464,7 +466,7 @@ PyObject* py_layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int epi;
     if (n != 5 || !hip_kernel_remembered(a[0], a[1]) || !layer_of(a[0], &l) || !epilogue_of(a[2], &epi)) return declined();
     const BiasUse use = bias_use(a[0], l);
-    if (use == BIAS_UNKNOWN || (use == BIAS_LEFT && (epi != 0 || a[3] != Py_None)))
+    if (use == BIAS_UNKNOWN || (use == BIAS_LEFT && (epi != 0 || a[3] != Py_None)) || (a[3] != Py_None && !own_supports(a[0])))
         return declined();   // fused forms exist for layers that add their own bias
     PyObject* y = layer_call(l, a[1], use == BIAS_ADDED ? l.bias.p : Py_None, epi, a[3], a[4]);
     return y ? y : declined();
@@ -531,7 +533,8 @@ PyObject* py_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* mlp_native(PyObject* first, PyObject* second, PyObject* x, int epi, PyObject* residual, PyObject* gate) {
     Layer p, q;
     if (!tensor(x) || !hip_kernel_remembered(first, x) || !hip_kernel_remembered(second, x) || !layer_of(first, &p) || !layer_of(second, &q) ||
-        p.granularity != py.per_channel || q.granularity != py.per_channel || bias_use(first, p) != BIAS_ADDED || bias_use(second, q) != BIAS_ADDED)
+        p.granularity != py.per_channel || q.granularity != py.per_channel || bias_use(first, p) != BIAS_ADDED || bias_use(second, q) != BIAS_ADDED ||
+        !own_supports(first) || !own_supports(second))
         return nullptr;
     return mlp_call(x, p.weight, p.scale, p.bias, p.layout, p.stream, q.weight, q.scale, q.bias, q.layout, q.stream, epi, Py_None, residual, gate);
 }
@@ -646,7 +649,7 @@ PyObject* py_decoder_layer_plain(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const bool plain = pm.self && dp && *dp && _PyType_Lookup(Py_TYPE(a[0]), s_call) == pm.linear_call && plain_call(a[0], *dp, pm.linear_forward) &&
                        has_method(a[1], s_forward_addcmul, pm.linear_forward_addcmul) && has_method(a[2], s_forward_fused, pm.linear_forward_fused) &&
                        has_method(a[3], s_forward_addcmul, pm.linear_forward_addcmul) && has_method(a[4], s_forward_fp8, pm.norm_forward_fp8) &&
-                       has_method(a[5], s_forward_fp8, pm.norm_forward_fp8);
+                       has_method(a[5], s_forward_fp8, pm.norm_forward_fp8) && own_supports(a[1]) && own_supports(a[3]);
     if (PyErr_Occurred()) return nullptr;
     return PyBool_FromLong(plain);
 }
@@ -834,18 +837,19 @@ PyObject* py_bind_layers(PyObject*, PyObject* args) {
 PyMethodDef linear_call_def = {"__call__", (PyCFunction)(void (*)(void))py_linear_call, METH_VARARGS | METH_KEYWORDS, nullptr};
 PyMethodDef mlp_call_def = {"__call__", (PyCFunction)(void (*)(void))py_mlp_call, METH_VARARGS | METH_KEYWORDS, nullptr};
 // bind_modules(phyai_amd.ops's dictionary, this module, nn.Module, its own __call__, tuple of global hook tables,
-//              LinearBase.forward, DenseMLP.forward, LinearBase.forward_fused, .forward_addcmul, AdaRMSNorm.forward_fp8)
+//              LinearBase.forward, DenseMLP.forward, LinearBase.forward_fused, .forward_addcmul,
+//              .supports_fused_epilogue, AdaRMSNorm.forward_fp8)
 //   -> (LinearBase.__call__, DenseMLP.__call__)
 PyObject* py_bind_modules(PyObject*, PyObject* args) {
     PyModules m = {};
-    if (!PyArg_ParseTuple(args, "O!OO!OO!OOOOO", &PyDict_Type, &m.ops_dict, &m.self, &PyType_Type, &m.module_type, &m.module_call, &PyTuple_Type,
+    if (!PyArg_ParseTuple(args, "O!OO!OO!OOOOOO", &PyDict_Type, &m.ops_dict, &m.self, &PyType_Type, &m.module_type, &m.module_call, &PyTuple_Type,
                           &m.global_hooks, &m.linear_forward, &m.mlp_forward, &m.linear_forward_fused, &m.linear_forward_addcmul,
-                          &m.norm_forward_fp8))
+                          &m.linear_supports, &m.norm_forward_fp8))
         return nullptr;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(m.global_hooks); ++i)
         if (!PyDict_Check(PyTuple_GET_ITEM(m.global_hooks, i))) return PyErr_Format(PyExc_TypeError, "hook tables are dictionaries");
     for (PyObject* o : {m.ops_dict, m.self, m.module_type, m.module_call, m.global_hooks, m.linear_forward, m.mlp_forward, m.linear_forward_fused,
-                        m.linear_forward_addcmul, m.norm_forward_fp8})
+                        m.linear_forward_addcmul, m.linear_supports, m.norm_forward_fp8})
         Py_INCREF(o);
     PyObject *a = PyCFunction_New(&linear_call_def, nullptr), *b = PyCFunction_New(&mlp_call_def, nullptr);
     PyObject *ma = a ? PyInstanceMethod_New(a) : nullptr, *mb = b ? PyInstanceMethod_New(b) : nullptr;
@@ -890,7 +894,7 @@ PyMODINIT_FUNC PyInit__phyai_host() {
         {&s_granularity, "granularity"}, {&s_apply, "apply"}, {&s_quantize, "quantize_activation"},
         {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
         {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward_fused, "forward_fused"}, {&s_forward_addcmul, "forward_addcmul"},
-        {&s_forward_fp8, "forward_fp8"}, {&s_forward, "forward"},
+        {&s_forward_fp8, "forward_fp8"}, {&s_supports, "supports_fused_epilogue"}, {&s_forward, "forward"},
         {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
         {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},
         {&s_compiled, "_compiled_call_impl"}, {&s_hooks[0], "_forward_hooks"}, {&s_hooks[1], "_forward_pre_hooks"},

@@ -199,7 +199,7 @@ class LinearBase(nn.Module):
 
 
 # The methods that the native calls of csrc/host_ext.cpp stand for; others in their place are called.
-LINEAR_METHODS = (LinearBase.forward, LinearBase.forward_fused, LinearBase.forward_addcmul)
+LINEAR_METHODS = (LinearBase.forward, LinearBase.forward_fused, LinearBase.forward_addcmul, LinearBase.supports_fused_epilogue)
 
 
 class ReplicatedLinear(LinearBase):

@@ -139,3 +139,23 @@ def test_an_instrumented_kernel_is_called(dev, linear, monkeypatch, where):
         own = kernel.apply
         monkeypatch.setattr(kernel, "apply", lambda *a, **k: (seen.append(1), own(*a, **k))[1], raising=False)
     assert torch.equal(lin(x)[0], want) and seen == [1]
+
+
+@pytest.mark.parametrize("gated,which", [(True, "gate_up_proj"), (True, "down_proj"), (False, "fc1")])
+def test_a_projection_that_refuses_fused_epilogues_gets_none(dev, linear, gated, which):
+    """supports_fused_epilogue is the question that DenseMLP and forward_addcmul ask; an override answers it."""
+    from phyai_amd.mlp import DenseMLP
+
+    mlp = DenseMLP(H, I, activation="gelu_tanh", gated=gated, params_dtype=torch.bfloat16, spec_in=linear.Fp8Spec(), spec_out=linear.Fp8Spec())
+    for j, name in enumerate(("gate_up_proj", "down_proj") if gated else ("fc1", "fc2")):
+        _fill(getattr(mlp, name), 50 + j)
+    x, gate = seeded((M, H), 52).to(dev), seeded((1, H), 53).to(dev)
+    want, asked = mlp(x), []
+    part = getattr(mlp, which)
+    part.supports_fused_epilogue = lambda x: bool(asked.append(1))
+    got = mlp(x)
+    assert asked and torch.allclose(got.float(), want.float(), rtol=2e-2, atol=1e-2 * want.float().abs().max().item())
+    if which == "down_proj":
+        h, asked[:] = part(mlp.gate_up_proj.forward_fused(x, "geglu_tanh"))[0], []
+        got = part.forward_addcmul(mlp.gate_up_proj.forward_fused(x, "geglu_tanh"), x, gate)
+        assert asked and torch.equal(got, torch.addcmul(x, h, gate))
