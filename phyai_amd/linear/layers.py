@@ -149,7 +149,7 @@ class LinearBase(nn.Module):
         if isinstance(x, ActivationView) and not getattr(self.spec, "needs_act_quant", False):
             raise RuntimeError(f"{type(self).__name__}: got quantized activations but spec "
                                f"{self.spec.spec_id!r} does not quantize its input")
-        bias = None if self.skip_bias_add else self._parameters["bias"]
+        bias = None if self.skip_bias_add else self.bias
         extra = {k: v for k, v in (("epilogue", epilogue), ("residual", residual), ("gate", gate)) if v is not None}
         return self._kernel_for(x).apply(self, x, bias, **extra)
 
@@ -172,7 +172,7 @@ class LinearBase(nn.Module):
 
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor | None]:
         y = self._run(x)
-        return y, (self._parameters["bias"] if self.skip_bias_add else None)
+        return y, (self.bias if self.skip_bias_add else None)
 
     def forward_fused(self, x: torch.Tensor, epilogue: str) -> torch.Tensor:
         """Run the linear with an activation fused into the GEMM epilogue.  Only kernels

@@ -114,8 +114,7 @@ class DenseMLP(nn.Module):
                 gate: torch.Tensor | None = None) -> torch.Tensor:
         """``residual`` / ``gate``: ``torch.addcmul(residual, mlp(x), gate)`` in the second GEMM's epilogue
         (the decoder layer's gated residual, reference ``models/pi05/modeling_pi05.py:835``)."""
-        mods = self._modules
-        first, second = (mods["gate_up_proj"], mods["down_proj"]) if self.gated else (mods["fc1"], mods["fc2"])
+        first, second = (self.gate_up_proj, self.down_proj) if self.gated else (self.fc1, self.fc2)
         if self.fuse_activation and getattr(first.spec, "needs_act_quant", False):
             y = ops._native().mlp_forward(first, second, x, self._epilogue, residual, gate)
             if y is not None:

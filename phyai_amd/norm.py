@@ -50,10 +50,10 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         fn = ops.gemma_rmsnorm if self._gemma else ops.rmsnorm
-        return fn(x, self._parameters["weight"], self.variance_epsilon)
+        return fn(x, self.weight, self.variance_epsilon)
 
     def forward_fp8(self, x: torch.Tensor) -> ActivationView:
-        xq, xs = ops.rmsnorm_fp8(x, self._parameters["weight"], self.variance_epsilon, gemma=self._gemma)
+        xq, xs = ops.rmsnorm_fp8(x, self.weight, self.variance_epsilon, gemma=self._gemma)
         return ActivationView(xq, xs, Granularity.PER_CHANNEL)
 
     def extra_repr(self) -> str:

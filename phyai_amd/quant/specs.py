@@ -113,7 +113,7 @@ class Fp8Spec:
         checkpoint loader, ``quantize_weight_``) clears ``weight_layout`` first."""
         from phyai_amd import ops
 
-        w = layer._parameters["weight"]
+        w = layer.weight
         if getattr(layer, "weight_layout", None):
             return True
         gated = bool(getattr(layer, "gated_pairs", False))

@@ -110,3 +110,42 @@ def test_a_replaced_module_call_is_called(monkeypatch):
     monkeypatch.setattr(nn.Module, "__call__", lambda self, *a, **k: (seen.append(type(self)), own(self, *a, **k))[1])
     lin(torch.zeros(2, 32, dtype=torch.bfloat16))
     assert seen == [L.ColumnParallelLinear]
+
+
+def test_parameters_that_are_plain_attributes():
+    """A bias or weight replaced by a plain tensor (merged, shared, parametrized) is still the layer's bias or weight."""
+    x = torch.randn(3, 32).to(torch.bfloat16)
+    for skip in (False, True):
+        lin = _bf16_linear(bias=True, skip_bias_add=skip)
+        lin.bias.data.normal_()
+        want = lin(x)
+        bias = lin.bias.data
+        del lin.bias
+        lin.bias = bias
+        got = lin(x)
+        assert torch.equal(got[0], want[0]) and (got[1] is bias if skip else got[1] is None)
+    spec = Fp8Spec(operand_order=True)
+    lin = L.ColumnParallelLinear(128, 64, bias=False, params_dtype=torch.bfloat16, spec=spec, device="cpu")
+    weight = lin.weight.data
+    del lin.weight
+    lin.weight = weight
+    assert spec.to_operand_order_(lin) is False                       # a weight on the CPU is left alone
+    norm = GemmaRMSNorm(32, device="cpu")
+    weight = norm.weight.data
+    del norm.weight
+    norm.weight = weight
+    for call in (norm, norm.forward_fp8):
+        with pytest.raises(RuntimeError, match="must live on the GPU"):
+            call(x)
+
+
+def test_projections_that_are_not_registered_modules():
+    """An MLP whose projection is shared with another owner and held as a plain attribute."""
+    mlp = DenseMLP(32, 64, activation="gelu", gated=False, params_dtype=torch.bfloat16)
+    for p in mlp.parameters():
+        nn.init.normal_(p, std=0.1)
+    x = torch.randn(3, 32).to(torch.bfloat16)
+    want, shared = mlp(x), mlp.fc1
+    del mlp.fc1
+    mlp.__dict__["fc1"] = shared
+    assert torch.equal(mlp(x), want)
