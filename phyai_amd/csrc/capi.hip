@@ -171,8 +171,9 @@ int phyai_fp8_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, voi
     if (N < 0 || K <= 0) return fail(PHYAI_FP8_EINVAL, "%s: bad shape N=%lld K=%lld", fn, (long long)N, (long long)K);
     if (N == 0) return PHYAI_FP8_OK;
     if (!w || !aligned(w, 16)) return fail(PHYAI_FP8_EINVAL, "%s: w must be a 16-byte aligned pointer", fn);
-    if (K % 128 != 0 || N % 16 != 0 || K > 16384 || N >= kMaxElems)
+    if (K % 128 != 0 || N % 16 != 0 || K > 16384)
         return fail(PHYAI_FP8_EUNSUPPORTED, "%s: needs K %% 128 == 0, K <= 16384 and N %% 16 == 0, got N=%lld K=%lld", fn, (long long)N, (long long)K);
+    if (N >= kMaxElems || N * K >= kMaxElems) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: matrix larger than 2^31 elements", fn);
     if (phyai::launch_weight_to_operand_order_inplace(w, N, K, static_cast<hipStream_t>(stream)) != 0)
         return fail(PHYAI_FP8_EUNSUPPORTED, "%s: no kernel", fn);
     return check_launch(fn);

@@ -75,6 +75,21 @@ def test_workspace_query_and_argument_validation_without_gpu():
     assert b"workspace" in lib.phyai_fp8_last_error()
 
 
+def test_in_place_relay_refuses_what_no_kernel_could_read():
+    """The GEMM entry points take matrices of less than 2^31 elements: a larger one must not be re-laid and marked."""
+    from phyai_amd import _lib
+
+    lib, buf = _lib.load(), (ctypes.c_char * 64)()
+    at = (ctypes.addressof(buf) + 15) // 16 * 16
+    for n, k in ((1 << 17, 16384), (1 << 24, 128), (1 << 20, 8192)):
+        assert lib.phyai_fp8_weight_to_operand_order(at, n, k, 0, at + 16, None) == -2
+        assert lib.phyai_fp8_weight_to_operand_order_inplace(at, n, k, None) == -2
+        assert b"2^31" in lib.phyai_fp8_last_error()
+    assert lib.phyai_fp8_weight_to_operand_order_inplace(at, 16, 128 * 129, None) == -2       # K beyond the kernel
+    assert lib.phyai_fp8_weight_to_operand_order_inplace(at + 8, 16, 128, None) == -1
+    assert lib.phyai_fp8_weight_to_operand_order_inplace(None, 0, 128, None) == 0
+
+
 def test_kernel_selection_for_the_benchmark_shapes(monkeypatch):
     """The dispatcher's choice, read back as text (host only).  The rules behind these cases were
     measured on the GPU: weight streaming up to 64 token rows; 256 x 256 tiles when they fill the
