@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PHYAI_FP8_ABI_VERSION 8
+#define PHYAI_FP8_ABI_VERSION 9
 
 enum {
     PHYAI_FP8_OK = 0,

@@ -19,7 +19,7 @@ STAMPS_LIB_PATH = os.path.join(_PKG, "lib", "libphyai_fp8_stamps.so")
 LIB_PATH = {"stamps": STAMPS_LIB_PATH, "ablate": os.path.join(_PKG, "lib", "libphyai_fp8_ablate.so")}.get(
     os.environ.get("PHYAI_FP8_LIBRARY", ""), os.path.join(_PKG, "lib", "libphyai_fp8.so"))
 CSRC_DIR = os.path.join(_PKG, "csrc")
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 # name -> (restype, argtypes); mirrors include/phyai_fp8.h one to one.
 _i64, _vp, _int, _sz = ctypes.c_int64, ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t

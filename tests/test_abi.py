@@ -37,6 +37,23 @@ def test_library_exports_every_declared_symbol():
     assert lib.phyai_fp8_abi_version() == _lib.ABI_VERSION
 
 
+# Entry points that each version added to the one before (8: those of the first versions together).  A client that asks
+# phyai_fp8_abi_version() learns from it what it may call, so a new entry point is a new version and a line here.
+ADDED = {
+    8: """abi_version last_error quant_rowwise quant_static weight_quant_rowwise weight_to_operand_order linear_workspace_bytes gemm
+          linear mlp_workspace_bytes mlp describe_mlp_plan linear_static gemm_addcmul linear_addcmul rmsnorm_quant adarmsnorm_quant
+          describe_plan describe_linear_plan debug_cast_e4m3 debug_stamps debug_mfma_rate""",
+    9: "weight_to_operand_order_inplace linear_per_tensor adarmsnorm_linear adarmsnorm_mlp",
+}
+
+
+def test_the_version_says_which_entry_points_there_are():
+    from phyai_amd import _lib
+
+    assert sorted("phyai_fp8_" + n for names in ADDED.values() for n in names.split()) == declared_functions()
+    assert _lib.load().phyai_fp8_abi_version() == max(ADDED)
+
+
 def test_workspace_query_and_argument_validation_without_gpu():
     """Size queries and argument checks run entirely on the host."""
     from phyai_amd import _lib
