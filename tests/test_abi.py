@@ -107,6 +107,78 @@ def test_in_place_relay_refuses_what_no_kernel_could_read():
     assert lib.phyai_fp8_weight_to_operand_order_inplace(None, 0, 128, None) == 0
 
 
+def _host_buffer(nbytes, align=256):
+    buf = ctypes.create_string_buffer(nbytes + align)
+    return buf, (ctypes.addressof(buf) + align - 1) // align * align
+
+
+def test_norm_linear_and_mlp_check_their_arguments_on_the_host():
+    from phyai_amd import _lib
+
+    lib = _lib.load()
+    keep, p = _host_buffer(4096)
+    M, N, K = 4, 64, 64
+    need, room = lib.phyai_fp8_linear_workspace_bytes(M, N, K, 0), 1 << 20
+    keep_ws, ws = _host_buffer(room)
+    base = dict(x=p, ldx=K, mod=p, ld_mod=3 * K, rows=1, eps=1e-6, w=p, ws=p, bias=None, out=p, ldo=N, M=M, N=N, K=K, epi=0, buf=ws, n=room, st=None)
+
+    def linear(**kw):
+        return lib.phyai_fp8_adarmsnorm_linear(*{**base, **kw}.values())
+
+    assert linear(M=0) == 0
+    for bad in (dict(M=-1), dict(N=0), dict(K=0), dict(mod=None), dict(mod=p + 8), dict(ld_mod=3 * K - 8), dict(ld_mod=3 * K + 4),
+                dict(rows=0), dict(rows=3), dict(rows=-1), dict(x=None), dict(x=p + 8), dict(ldx=K - 8), dict(w=None), dict(w=p + 8),
+                dict(ws=None), dict(out=None), dict(ldo=N - 16), dict(epi=9), dict(epi=0x800), dict(buf=ws + 16)):
+        assert linear(**bad) == -1, bad
+        assert lib.phyai_fp8_last_error(), bad
+    assert linear(K=60, ldx=64, ld_mod=192) == -2 and linear(K=72, ldx=72, ld_mod=216) == -2   # multiples of 8, of 16
+    assert linear(epi=0x200) == -2                                                              # operand order, K % 128
+    assert linear(N=48, epi=1, ldo=24) == -2                                                    # gated: N % 32
+    # (unlike phyai_fp8_linear there is no form without a workspace: the norm may run in front of the linear)
+    assert linear(buf=None, n=0) == -3 and linear(n=need - 1) == -3
+
+    H, I, O = 64, 64, 48
+    need = lib.phyai_fp8_mlp_workspace_bytes(M, H, I, O, 1)
+    base_mlp = dict(x=p, ldx=H, mod=p, ld_mod=3 * H, rows=2, eps=1e-6, w1=p, s1=p, b1=None, f1=0, w2=p, s2=p, b2=None, f2=0, res=None, ld_res=0,
+                    gate=None, ld_gate=0, gate_rows=0, out=p, ldo=O, M=M, H=H, I=I, O=O, epi=1, buf=ws, n=room, st=None)
+
+    def mlp(**kw):
+        return lib.phyai_fp8_adarmsnorm_mlp(*{**base_mlp, **kw}.values())
+
+    assert mlp(M=0) == 0
+    for bad in (dict(H=0), dict(O=-16), dict(mod=None), dict(mod=p + 2), dict(ld_mod=2 * H), dict(rows=0), dict(rows=3), dict(epi=0), dict(epi=7),
+                dict(epi=0x201), dict(f1=1), dict(f2=2), dict(res=p, ld_res=O), dict(gate=p, ld_gate=O, gate_rows=1), dict(x=None), dict(w1=None),
+                dict(s2=None), dict(out=None), dict(ldo=O - 16), dict(res=p, ld_res=O, gate=p + 8, ld_gate=O, gate_rows=1),
+                dict(res=p, ld_res=O - 8, gate=p, ld_gate=O, gate_rows=1), dict(res=p, ld_res=O, gate=p, ld_gate=O, gate_rows=3),
+                dict(f1=0x600, f2=0x600), dict(buf=ws + 64)):
+        assert mlp(**bad) in (-1, -2), bad
+        assert lib.phyai_fp8_last_error(), bad
+    assert mlp(H=72, ldx=72, ld_mod=216) == -2 and mlp(I=40) == -2 and mlp(O=40, ldo=40) == -2
+    assert mlp(buf=None) == -3 and mlp(n=need - 1) == -3
+
+
+def test_per_tensor_linear_checks_its_arguments_on_the_host():
+    from phyai_amd import _lib
+
+    lib = _lib.load()
+    keep, p = _host_buffer(4096)
+    M, N, K = 4, 64, 64
+    need, room = lib.phyai_fp8_linear_workspace_bytes(M, N, K, 0), 1 << 20
+    keep_ws, ws = _host_buffer(room)
+    base = dict(x=p, ldx=K, scale=p, w=p, ws=p, bias=None, res=None, ld_res=0, gate=None, ld_gate=0, gate_rows=0, out=p, ldo=N, M=M, N=N, K=K,
+                epi=0, buf=ws, n=room, st=None)
+
+    def call(**kw):
+        return lib.phyai_fp8_linear_per_tensor(*{**base, **kw}.values())
+
+    assert call(M=0) == 0
+    for bad in (dict(M=-1), dict(K=0), dict(scale=None), dict(x=None), dict(x=p + 2), dict(ldx=K + 4), dict(w=None), dict(out=None), dict(epi=6),
+                dict(res=p, ld_res=N), dict(res=p, ld_res=N, gate=p, ld_gate=N, gate_rows=3), dict(buf=ws + 16),
+                dict(epi=4, res=p, ld_res=N, gate=p, ld_gate=N, gate_rows=1)):
+        assert call(**bad) == -1, bad
+    assert call(K=72, ldx=72) == -2 and call(N=40) == -2 and call(buf=None) == -3 and call(n=need - 1) == -3
+
+
 def test_kernel_selection_for_the_benchmark_shapes(monkeypatch):
     """The dispatcher's choice, read back as text (host only).  The rules behind these cases were
     measured on the GPU: weight streaming up to 64 token rows; 256 x 256 tiles when they fill the
