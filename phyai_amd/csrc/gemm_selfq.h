@@ -37,6 +37,24 @@ constexpr int selfq_prev_steps(int steps) {
         if (s < steps) prev = s;
     return prev;
 }
+// Longest K that a workgroup of 4 rg rows and nt weight tiles is taken for: where this one launch stops being ahead of
+// quantizer + GEMM.  What decides is nt: the rows leave the fewer registers for weights in flight the longer K is
+// (selfq_window: nt = 4 holds 3 steps at K = 6016, nt = 1 all 6), and a row-major tile is pulled in 64-byte pieces.
+// Below, one launch / two launches in us, in a graph over 600 MB of weights and called eagerly (a launch costs the host
+// 3.3 us), accepted where the product of the two ratios is below one - measured at M = 1 ... 128, N = 256 ... 16384:
+//   operand order  nt = 1  15 x  1024 x 16384  10.3 / 14.3, 10.6 / 14.5     4 x 256 x 16384   7.2 /  9.4,  7.3 / 10.1
+//                  nt = 2  15 x  4096 x 12160  13.7 / 14.1, 13.6 / 14.0    15 x 4096 x 16384 18.2 / 17.5, 18.1 / 17.4
+//                  nt = 4  15 x  5552 x  4096 ratios 1.06, 0.91            15 x 5552 x  6016 12.9 / 11.6, 12.7 / 11.3
+//                  nt = 8  M x N x 2048 one scale 1.02, 0.76               M x N x 2176 1.23, 1.01
+//   row-major      nt = 1  15 x  1024 x  8192   8.8 /  9.1,  8.9 /  9.8    15 x 1024 x 10240 11.5 / 11.3, 11.6 / 11.4
+//                  nt = 2, 8 rows  M x N x 3088 ratios 1.02, 0.76          15 x 4096 x  4224 10.5 /  8.3, 10.7 / 10.0
+//                  nt = 4  M x N x 2032 ratios 0.86, 0.80                  15 x 5552 x  2064 10.1 /  7.8, 10.2 / 10.0
+//                  nt = 8  M x N x 1040 ratios 1.05, 0.72 (one scale: 1552 1.07, 0.80)   M x N x 1168 1.29, 0.89
+// With one scale 8 rows in operand order stop at 8192 (M x N x 10240 1.07, 1.01 with nt = 1): its quantizer is cheaper.
+constexpr int selfq_max_k(int rg, int nt, bool operand, bool one_scale) {
+    if (operand) return nt >= 8 ? 2048 : nt == 4 ? 4096 : rg == 1 ? 16384 : one_scale ? 8192 : nt == 2 ? 12288 : 16384;
+    return nt >= 8 ? (one_scale ? 1600 : 1088) : nt == 4 ? 2048 : nt == 2 && rg == 2 ? 4096 : 8192;
+}
 // steps of weights in flight: what a wavefront's 256 registers leave beside the rows, the sums and about 80 for the
 // conversions and addresses
 constexpr int selfq_window(int rg, int nt, int steps) {

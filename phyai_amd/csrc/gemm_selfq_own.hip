@@ -7,10 +7,10 @@ namespace phyai {
 
 static int sq_ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// Up to 48 token rows - 128 with one static scale, which spares the tables and their barriers - whose workgroups - 4 or 8 rows, as few weight tiles each as keeps the grid within the 256 CUs -
-// run in one round: with a second round the repeated conversions (rows x K elements, 5.5 / 64 cycles each) cost more
-// than the quantizer's launch.  Activation epilogues exist for row-major weights up to K = 2048 (gemm_skinny_fused.hip
-// serves the rest of what an MLP's first projection is).
+// Up to 48 token rows - 128 with one static scale, which spares the tables and their barriers - whose workgroups (4 or 8
+// rows, as few weight tiles each as keeps the grid within the 256 CUs) run in one round: with a second round the repeated
+// conversions (rows x K elements, 5.5 / 64 cycles each) cost more than the quantizer's launch.  Activation epilogues
+// exist for row-major weights up to K = 2048 (gemm_skinny_fused.hip serves the rest of what an MLP's first projection is).
 SelfqPlan selfq_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout, int source) {
     SelfqPlan pl = {0, 0, 0, 0, 0};
     if (const char* e = tuning_env("PHYAI_FP8_FUSED")) { if (atoi(e) == 0) return pl; }
@@ -27,11 +27,7 @@ SelfqPlan selfq_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_
     for (int nt = 1; nt <= (steps <= 4 ? 8 : 4); nt *= 2) {
         const int tiles = sq_ceil_div(cols, per_tile * nt);
         if ((int64_t)tiles * msplit > 256) continue;
-        // What a workgroup pulls through its CU (row-major weights at 62 of the 100 GB/s that rows and weights in
-        // operand order come at): beyond about 3.6 us of that, with the conversions beside it, the quantizer's launch is
-        // the smaller cost (one launch / two: 15 x 5552 x 6240 row-major 15.8 / 10.4 us, 20 x 2944 x 6016 14.0 / 10.1,
-        // 128 x 2048 x 4096 10.9 / 9.6, 128 x 256 x 16384 14.2 / 12.6; 100 x 2048 x 2048 6.6 / 9.6, 2 x 304 x 12160 6.5 / 10.4).
-        if ((double)K * (8 * rg + 16 * nt * (weight_layout == W_ROW_MAJOR ? 1.6 : 1.0)) > 360e3) break;
+        if (K > selfq_max_k(rg, nt, weight_layout != W_ROW_MAJOR, source == SELFQ_FROM_SCALAR)) break;
         pl.rg = rg; pl.nt = nt; pl.steps = steps; pl.tiles = tiles; pl.msplit = msplit;
         break;
     }

@@ -304,6 +304,23 @@ def test_whole_linear_selection_one_launch_or_two(monkeypatch):
     assert d(50, 1024, 4096) == "one launch: small-m rows=16 nt=1 kpw=4 grid=64x4"    # exists, forced for tests only
 
 
+def test_rows_in_registers_are_taken_where_they_were_measured_ahead(monkeypatch):
+    """The limits of csrc/gemm_selfq.h on both sides, as (rows, columns, K): one launch in which the rows stay in registers,
+    or the quantizer and a GEMM."""
+    from phyai_amd import ops
+
+    monkeypatch.delenv("PHYAI_FP8_FUSED", raising=False)
+    one = dict(operand=[(15, 1024, 16384), (48, 256, 16384), (4, 4096, 12160), (15, 4096, 12160), (4, 4112, 16384), (33, 3072, 4096)],
+               row_major=[(2, 304, 8192), (15, 2048, 8192), (2, 4112, 8192), (15, 4096, 3088), (15, 8192, 2032), (48, 5360, 1040)])
+    two = dict(operand=[(15, 4096, 16384), (15, 5552, 4224), (48, 5376, 2176), (49, 256, 8192)],
+               row_major=[(2, 304, 12160), (15, 1024, 10240), (15, 4096, 4224), (15, 5552, 2064), (3, 8208, 2176), (48, 5360, 1168)])
+    for shapes, start in ((one, "one launch: rows in registers"), (two, "quantizer + ")):
+        for layout, cases in shapes.items():
+            for m, n, k in cases:
+                plan = ops.describe_linear_plan(m, n, k, weight_layout=layout)
+                assert plan.startswith(start), (m, n, k, layout, plan)
+
+
 def test_tuning_variables_are_ignored_without_the_switch():
     """A stray PHYAI_FP8_* variable must not change the kernel selection of a process that did not
     set PHYAI_FP8_TUNING (fresh processes: the switch is read once)."""
