@@ -1,5 +1,5 @@
 // Small-M linear that quantizes its own rows, for what gemm_skinny_fused.hip does not take: K that is no multiple of
-// 128, K up to 16384, activations with one static scale.  One launch instead of quantizer + GEMM.
+// 128, K up to 16384, activations with one static scale.  One launch instead of quantizer + GEMM where selfq_max_k says.
 //
 // What bounds these calls is the host: a launch costs it 3.3 us (2.5 us of it inside the runtime), and for a few token
 // rows neither the quantizer nor the GEMM lasts as long.  So the quantizer's launch goes, at the price of every workgroup
@@ -8,7 +8,7 @@
 //  * a workgroup (8 wavefronts) owns 16 NT weight rows x 4 RG token rows over the whole K; wavefront w takes the
 //    128-byte K steps w, w + 8, ... as in the other weight-streaming kernels, so sums come out in the same order;
 //  * the bf16 rows stay in registers from their arrival until their conversion (the row maximum needs all of K first):
-//    128 registers per lane at K = 16384 with 8 rows, which leaves 64 for weights in flight;
+//    128 registers per lane at K = 16384 with 8 rows, which leaves room for five K steps of weights in flight (selfq_window);
 //  * weights go straight into registers in both layouts: operand order in 1 KB runs; row-major with 64 contiguous bytes
 //    per row, which a CU pulls at 62 GB/s against 110 - enough beside the conversions, and it needs no LDS staging;
 //  * WINDOW steps of weights are in flight ahead of the MFMAs, the first ones requested right behind the rows;
@@ -54,6 +54,15 @@ constexpr int selfq_prev_steps(int steps) {
 constexpr int selfq_max_k(int rg, int nt, bool operand, bool one_scale) {
     if (operand) return nt >= 8 ? 2048 : nt == 4 ? 4096 : rg == 1 ? 16384 : one_scale ? 8192 : nt == 2 ? 12288 : 16384;
     return nt >= 8 ? (one_scale ? 1600 : 1088) : nt == 4 ? 2048 : nt == 2 && rg == 2 ? 4096 : 8192;
+}
+// Shapes that exist as kernels: those that some K is taken for, less what gemm_skinny_fused.hip serves first - its own
+// maxima up to K = 4096 in operand order, where only grids of four tiles beyond K = 2048 are left to this kernel, and
+// handed-over maxima up to K = 1024 in operand order, where only grids of eight are.
+constexpr bool selfq_exists(int rg, int nt, int steps, bool operand, int scale) {
+    if (1024 * selfq_prev_steps(steps) >= selfq_max_k(rg, nt, operand, scale == SELFQ_STATIC)) return false;
+    if (operand && scale == SELFQ_OWN && steps <= 4) return steps == 4 && nt == 4;
+    if (operand && scale == SELFQ_HANDED && steps == 1) return nt == 8;
+    return true;
 }
 // steps of weights in flight: what a wavefront's 256 registers leave beside the rows, the sums and about 80 for the
 // conversions and addresses
@@ -373,19 +382,22 @@ __global__ __launch_bounds__(SQ_THREADS) void gemm_fp8_selfq_kernel(
     }
 }
 
+template <int RG, int NT, int STEPS, int EPI, bool OPERAND, int SCALE>
+static int selfq_launch_layout(const GemmProblem& g, const SelfqPlan& pl, const void* handed, hipStream_t st) {
+    if constexpr ((OPERAND && EPI != EPI_NONE) || !selfq_exists(RG, NT, STEPS, OPERAND, SCALE)) {
+        return -2;
+    } else {
+        hipLaunchKernelGGL((gemm_fp8_selfq_kernel<RG, NT, STEPS, EPI, OPERAND, SCALE>), dim3(pl.tiles, pl.msplit), dim3(SQ_THREADS), 0, st, g.w,
+                           reinterpret_cast<const uint8_t*>(g.x_bf16), g.K, g.N, g.M, (int)(g.ldx * 2), handed, g.amax_parts, g.w_scale, g.bias,
+                           g.out, g.ldo, residual_of(g), EPI != EPI_NONE ? g.amax_out : nullptr);
+        return 0;
+    }
+}
+
 template <int RG, int NT, int STEPS, int EPI, int SCALE>
 static int selfq_launch(const GemmProblem& g, const SelfqPlan& pl, const void* handed, hipStream_t st) {
-    const dim3 grid(pl.tiles, pl.msplit);
-#define PHYAI_SQ_ARGS g.w, reinterpret_cast<const uint8_t*>(g.x_bf16), g.K, g.N, g.M, (int)(g.ldx * 2), handed, g.amax_parts, g.w_scale, \
-                      g.bias, g.out, g.ldo, residual_of(g), EPI != EPI_NONE ? g.amax_out : nullptr
-    if (g.weight_layout == W_ROW_MAJOR)
-        hipLaunchKernelGGL((gemm_fp8_selfq_kernel<RG, NT, STEPS, EPI, false, SCALE>), grid, dim3(SQ_THREADS), 0, st, PHYAI_SQ_ARGS);
-    else if constexpr (EPI == EPI_NONE)
-        hipLaunchKernelGGL((gemm_fp8_selfq_kernel<RG, NT, STEPS, EPI, true, SCALE>), grid, dim3(SQ_THREADS), 0, st, PHYAI_SQ_ARGS);
-    else
-        return -2;
-#undef PHYAI_SQ_ARGS
-    return 0;
+    return g.weight_layout == W_ROW_MAJOR ? selfq_launch_layout<RG, NT, STEPS, EPI, false, SCALE>(g, pl, handed, st)
+                                          : selfq_launch_layout<RG, NT, STEPS, EPI, true, SCALE>(g, pl, handed, st);
 }
 
 template <int RG, int STEPS, int EPI, int SCALE>
@@ -394,7 +406,7 @@ static int selfq_launch_nt(const GemmProblem& g, const SelfqPlan& pl, const void
     case 1: return selfq_launch<RG, 1, STEPS, EPI, SCALE>(g, pl, handed, st);
     case 2: return selfq_launch<RG, 2, STEPS, EPI, SCALE>(g, pl, handed, st);
     case 4: return selfq_launch<RG, 4, STEPS, EPI, SCALE>(g, pl, handed, st);
-    case 8: if constexpr (STEPS <= 4) return selfq_launch<RG, 8, STEPS, EPI, SCALE>(g, pl, handed, st); else return -2;
+    case 8: return selfq_launch<RG, 8, STEPS, EPI, SCALE>(g, pl, handed, st);
     default: return -2;
     }
 }

@@ -24,10 +24,12 @@ SelfqPlan selfq_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_
     for (int s : kSelfqSteps)
         if (s >= per_wave) { steps = s; break; }
     const int rg = M <= 4 ? 1 : 2, msplit = sq_ceil_div(M, 4 * rg), per_tile = gated ? 8 : 16;
-    for (int nt = 1; nt <= (steps <= 4 ? 8 : 4); nt *= 2) {
+    for (int nt = 1; nt <= 8; nt *= 2) {
         const int tiles = sq_ceil_div(cols, per_tile * nt);
         if ((int64_t)tiles * msplit > 256) continue;
-        if (K > selfq_max_k(rg, nt, weight_layout != W_ROW_MAJOR, source == SELFQ_FROM_SCALAR)) break;
+        const bool operand = weight_layout != W_ROW_MAJOR;
+        if (K > selfq_max_k(rg, nt, operand, source == SELFQ_FROM_SCALAR)) break;
+        if (!selfq_exists(rg, nt, steps, operand, source)) continue;
         pl.rg = rg; pl.nt = nt; pl.steps = steps; pl.tiles = tiles; pl.msplit = msplit;
         break;
     }
