@@ -371,14 +371,17 @@ struct GemmChoice {
     bool takes_amax;   // FUSED, SELFQ: the plan is the one for handed-over row maxima
 };
 
-// Kernel choice (measured on the expert and prefill shapes, M = 50 .. 13056):
-//   M <= 64                      weight-streaming kernel, nothing else comes close;
-//   pipelined tile kernel        when big_plan finds a tile shape that fills the chip, or more
-//                                than 64 tiles of 128 x 128;
-//   64 < M <= 1024 otherwise     weight-streaming kernel again (few output columns: at
-//                                N = 1024 it wins up to M = 1000, at N = 2560 up to M = 300);
-//   32 .. 64 small tiles         pipelined tile kernel after all (M > 1024);
-//   the rest                     generic LDS tile kernel (any K, any alignment).
+// Kernel choice (measured over M = 136 .. 13056, N = 256 .. 32768, K = 1024 .. 16384, both weight layouts, graphs of
+// weight sets beyond the Infinity Cache; us: weight streaming / best tile shape):
+//   M <= 64                          weight-streaming kernel, nothing else comes close;
+//   up to 64 tiles of 128 x 128      weight streaming up to M = 4096 (few output columns: 300 x 2048 x 2048 7.1 / 8.3,
+//                                    1000 x 1024 x 4096 11.7 / 13.0, 1000 x 1024 x 8192 17.5 / 21.4, 400 x 2048 x 16384
+//                                    29.7 / 35.3, 2048 x 512 x 2048 8.1 / 8.7; from 65 tiles up the tile kernels are ahead:
+//                                    1100 x 1024 x 6144 21.6 / 18.1, 560 x 2048 x 16384 45.6 / 36.3) - except long K of
+//                                    many rows (below);
+//   pipelined tile kernel            where big_plan has a tile shape, except one round of 64-column workgroups (below);
+//   the rest                         weight streaming where it applies, else the generic LDS tile kernel (any K, any
+//                                    alignment).
 // vec_ok: scales, bias and output are aligned for the weight-streaming kernel's 128- and 64-bit
 // accesses; out16: the output is 16-byte addressable (pointer and row stride), which the pipelined
 // tile kernel's epilogue needs.
@@ -425,7 +428,12 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
     if (skinny_ok && M <= 64) return small();
     if (!tuning_env("PHYAI_FP8_TILE")) {
         const BigPlan bp = big_plan(M, N, K, epilogue, layout != W_ROW_MAJOR);
-        const bool few_small_tiles = bp.tile == 128 && bp.cols == 128 && bp.tiles <= 64 && !tuning_env("PHYAI_FP8_BIG");
+        // Beyond 1024 rows every weight tile is walked by 16 workgroups and more, whose codes no L2 holds once K is 8192: with
+        // 48 tiles of 128 x 128 and more (split in two along K) the tile kernel is ahead (2048 x 384 x 8192 23.5 / 22.9 us,
+        // 2500 x 384 x 8192 26.5 / 23.3, 1800 x 512 x 16384 38.8 / 34.9, 2048 x 512 x 16384 42.4 / 35.0; level at 1548 x 512 x
+        // 16384, 52 tiles; behind below: 1800 x 384 x 8192, 45 tiles, 19.3 / 22.6).
+        const bool long_k_of_many_rows = M > 1024 && K >= 8192 && bp.tiles >= 48;
+        const bool few_small_tiles = bp.tile == 128 && bp.cols == 128 && bp.tiles <= 64 && !long_k_of_many_rows && !tuning_env("PHYAI_FP8_BIG");
         // ... and its 128 x 64 tiles lose to one round of weight-streaming workgroups on long K (777 x 1168 x 4304: 17.4
         // against 15.0 us; level at K = 4096, 700 x 1408; 7.6 against 8.4 at K = 2048)
         bool one_round = false;

@@ -259,6 +259,18 @@ def test_kernel_selection_for_the_benchmark_shapes(monkeypatch):
         d(50, 1000, 1024)
 
 
+def test_weight_streaming_beyond_1024_rows(monkeypatch):
+    """Few columns and many rows: weight streaming up to 64 tiles of 128 x 128, except long K from 48 tiles up."""
+    from phyai_amd import ops
+
+    for var in ("PHYAI_FP8_BIG", "PHYAI_FP8_BIG_SPLITS", "PHYAI_FP8_TILE", "PHYAI_FP8_SKINNY_PLAN", "PHYAI_FP8_SKINNY_MAXM"):
+        monkeypatch.delenv(var, raising=False)
+    for m, n, k in ((2048, 512, 2048), (1800, 384, 8192), (1100, 512, 16384), (1000, 1024, 16384), (3500, 256, 6016)):
+        assert ops.describe_plan(m, n, k).startswith("small-m "), (m, n, k)
+    for m, n, k in ((2048, 384, 8192), (2500, 384, 8192), (1548, 512, 16384), (2048, 512, 16384)):
+        assert ops.describe_plan(m, n, k).startswith("tile 128x128 depth=4 splits=2 "), (m, n, k)
+
+
 def test_whole_linear_selection_one_launch_or_two(monkeypatch):
     """phyai_fp8_linear runs one kernel that quantizes its own token rows where that was measured
     faster (up to 128 rows, K <= 4096, a grid of at most 256 workgroups), and quantizer + GEMM
