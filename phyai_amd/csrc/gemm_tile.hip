@@ -434,12 +434,16 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
         // 16384, 52 tiles; behind below: 1800 x 384 x 8192, 45 tiles, 19.3 / 22.6).
         const bool long_k_of_many_rows = M > 1024 && K >= 8192 && bp.tiles >= 48;
         const bool few_small_tiles = bp.tile == 128 && bp.cols == 128 && bp.tiles <= 64 && !long_k_of_many_rows && !tuning_env("PHYAI_FP8_BIG");
-        // ... and its 128 x 64 tiles lose to one round of weight-streaming workgroups on long K (777 x 1168 x 4304: 17.4
-        // against 15.0 us; level at K = 4096, 700 x 1408; 7.6 against 8.4 at K = 2048)
+        // ... and its 128 x 64 tiles lose to one round of weight-streaming workgroups above K = 4096 where K is no multiple of a
+        // K step (777 x 1168 x 4304 17.8 / 16.3 us, 900 x 1040 x 4112 17.5 / 15.4) or the workgroups that share a weight tile
+        // meet on half of the XCDs, i.e. with an even number of 64-column tiles (22 tiles: 700 x 1408 x K 16.4 / 14.8 at K =
+        // 5120, 17.0 / 15.8 at 6016, 19.2 / 17.4 at 7168; 26 tiles: 560 x 1664 x 6144 17.3 / 15.9).  With an odd number every
+        // XCD fetches every weight tile, and the tile kernel is ahead: 1296 columns 13.4 / 14.9 at K = 4224, 17.1 / 19.8 at
+        // 6016; 420 x 2064 x 5120 15.1 / 18.5.  (Not asked up to K = 4096, though 400 x 2304 x 2048, 36 tiles, is 8.5 / 7.8.)
         bool one_round = false;
         if (bp.tile == 128 && bp.cols == 64 && K > 4096 && skinny_ok && !tuning_env("PHYAI_FP8_BIG")) {
             const SkinnyPlan sp = skinny_plan(M, N, K, epilogue);
-            one_round = sp.tiles * sp.msplit <= 256;
+            one_round = sp.tiles * sp.msplit <= 256 && (K % 128 != 0 || sp.tiles % 2 == 0);
         }
         if (bp.tile && out16 && !((few_small_tiles || one_round) && skinny_ok)) {
             c.kind = GemmChoice::BIG;

@@ -271,6 +271,18 @@ def test_weight_streaming_beyond_1024_rows(monkeypatch):
         assert ops.describe_plan(m, n, k).startswith("tile 128x128 depth=4 splits=2 "), (m, n, k)
 
 
+def test_one_round_of_weight_streaming_in_place_of_narrow_tiles(monkeypatch):
+    """65 tiles of 128 x 128 and more, K between 4096 and 8192: an even number of 64-column tiles, or a ragged K."""
+    from phyai_amd import ops
+
+    for var in ("PHYAI_FP8_BIG", "PHYAI_FP8_TILE", "PHYAI_FP8_SKINNY_PLAN", "PHYAI_FP8_SKINNY_MAXM"):
+        monkeypatch.delenv(var, raising=False)
+    for m, n, k in ((700, 1408, 5120), (560, 1664, 7168), (777, 1168, 4304), (900, 1040, 4112)):
+        assert ops.describe_plan(m, n, k).startswith("small-m "), (m, n, k)
+    for m, n, k in ((700, 1296, 6016), (777, 1168, 4224), (420, 2064, 5120), (1300, 656, 7936), (700, 1408, 4096), (816, 1408, 5120)):
+        assert ops.describe_plan(m, n, k).startswith("tile 128x64 "), (m, n, k)
+
+
 def test_whole_linear_selection_one_launch_or_two(monkeypatch):
     """phyai_fp8_linear runs one kernel that quantizes its own token rows where that was measured
     faster (up to 128 rows, K <= 4096, a grid of at most 256 workgroups), and quantizer + GEMM
