@@ -125,7 +125,7 @@ int phyai_fp8_weight_to_operand_order(const void *w, int64_t N, int64_t K, int g
                                       void *stream);
 
 /*
- * The plain (not gated) form in place.  K <= 16384.
+ * The plain (not gated) form in place: K <= 16384, and less than 2^31 elements as in the form above.
  */
 int phyai_fp8_weight_to_operand_order_inplace(void *w, int64_t N, int64_t K, void *stream);
 
@@ -159,12 +159,12 @@ int phyai_fp8_gemm(const void *xq, const float *x_scale, int x_scale_is_scalar,
  * GEMM above, as one call.  Replaces TorchKernel._fp8_per_channel
  * (layers/linear/backends/torch.py:155-176) end to end.
  *
- * Up to 128 token rows, K <= 4096 (a multiple of 128), with x and its row stride 16-byte
- * aligned and a workgroup shape whose grid fits the chip at once (beyond K = 2048: projections up to
- * about 2048 wide), this is ONE kernel: every workgroup
- * quantizes the token rows it multiplies (same codes, same scales, same output bits as
- * the two launches) and the workspace is not touched: such a call may pass workspace = NULL.
- * Otherwise the quantizer writes codes and scales into the workspace and a GEMM kernel follows
+ * With x and its row stride 16-byte aligned and a workgroup shape whose grid fits the chip at once, this is ONE kernel
+ * for few token rows: up to 128 rows at K <= 4096 (a multiple of 128; beyond K = 2048 projections up to about 2048 wide),
+ * up to 48 rows at any other K while that is ahead (the fewer rows and columns the longer: up to K = 16384 with weights
+ * in operand order, 8192 row-major).  Every workgroup quantizes the token rows it multiplies (same codes, same
+ * scales, same output bits as the two launches) and the workspace is not touched: such a call may pass
+ * workspace = NULL.  Otherwise the quantizer writes codes and scales into the workspace and a GEMM kernel follows
  * (PHYAI_FP8_EWORKSPACE without one).  phyai_fp8_describe_linear_plan tells which.
  */
 int phyai_fp8_linear(const void *x, int64_t ldx, const void *w, const float *w_scale,
@@ -206,11 +206,12 @@ int phyai_fp8_linear_addcmul(const void *x, int64_t ldx, const void *w, const fl
  * phyai_fp8_linear_addcmul.  Same bits as phyai_fp8_linear (epilogue) followed by
  * phyai_fp8_linear[_addcmul] on its output.
  *
- * What the one call buys: when both projections are served by the kernel that quantizes its own token
- * rows (M <= 128, H <= 2048, I <= 4096, see phyai_fp8_describe_mlp_plan), the first one also leaves the
- * |h| maximum of every token row per workgroup column in the workspace, and the second one starts its
- * conversions from those instead of first passing over its rows - which is what makes one launch pay
- * for a down projection with K = 4096.  Otherwise it is the two linears back to back.
+ * What the one call buys: when both projections are served by kernels that quantize their own token
+ * rows (M <= 128, H <= 2048, I <= 4096; up to 48 rows also longer and ragged I, see phyai_fp8_linear;
+ * phyai_fp8_describe_mlp_plan tells), the first one also leaves the |h| maximum of every token row per
+ * workgroup column in the workspace, and the second one starts its conversions from those instead of
+ * first passing over its rows - which is what makes one launch pay for a down projection with K = 4096.
+ * Otherwise it is the two linears back to back.
  * Workspace: phyai_fp8_mlp_workspace_bytes(), same rules as for phyai_fp8_linear.
  */
 size_t phyai_fp8_mlp_workspace_bytes(int64_t M, int64_t H, int64_t I, int64_t O, int epilogue);
@@ -223,7 +224,8 @@ int phyai_fp8_mlp(const void *x, int64_t ldx, const void *w1, const float *w1_sc
 /*
  * phyai_fp8_quant_static + phyai_fp8_gemm (x_scale_is_scalar = 1) as one call: a linear whose activations have one
  * static scale (layers/linear/backends/torch.py:123-153).  residual / gate as for phyai_fp8_linear_addcmul, or both
- * null.  Up to 128 token rows and K = 16384 it is one launch where the grid fits the chip.
+ * null.  One launch up to 128 token rows where the grid fits the chip and that is ahead (the fewer rows and columns the
+ * longer: up to K = 8192; 16384 with up to 4 rows and weights in operand order).  The workspace is needed in any case.
  */
 int phyai_fp8_linear_per_tensor(const void *x, int64_t ldx, const float *input_scale, const void *w, const float *w_scale,
                                 const void *bias, const void *residual, int64_t ld_res, const void *gate, int64_t ld_gate,
@@ -321,6 +323,7 @@ int phyai_fp8_describe_plan(int64_t M, int64_t N, int64_t K, int epilogue, char 
 /*
  * The same for phyai_fp8_linear (bf16 activations in, dense rows): either
  *   "one launch: small-m rows=8 nt=5 kpw=1 grid=32x7"      the kernel that quantizes its own token rows
+ *   "one launch: rows in registers, rows=8 nt=1 steps=6 grid=64x2"   the one for K that the first does not take
  * or "quantizer + " followed by what phyai_fp8_describe_plan reports.  Host only.  The layout flag of
  * the weight matrix (PHYAI_FP8_FLAG_W_OPERAND_ORDER / _GATED) may be or-ed into `epilogue` as in the
  * calls: a few shapes are one launch only with weights in operand order (registers instead of LDS).

@@ -1,7 +1,7 @@
 // What a call of some shape needs besides its pointers - kernel choice, workspace carve - computed once per thread and
 // shape: the rules behind them loop over tile shapes with divisions and were evaluated several times per call, 1.0 us of
-// the 4.4 us that a small linear spent below Python.  Direct-mapped; a tuning run, whose choices follow the environment,
-// never reads it.
+// the 4.4 us that a small linear spent below Python.  Direct-mapped by a hash with the multipliers of the splitmix64
+// generator's mixer; a tuning run, whose choices follow the environment, never reads it.
 #pragma once
 #include <stdint.h>
 

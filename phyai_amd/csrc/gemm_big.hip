@@ -1,40 +1,41 @@
 // MFMA-bound fp8 GEMM for large M (prefix prefill, batched serving).
-// Workgroup = 4 wavefronts (2 x 2); a wavefront owns TM x TN blocks of 32 x 32, so the
-// workgroup tile is 64*TM x 64*TN: 256 x 256 (TM = TN = 4, one workgroup per CU) for long K,
-// 192 x 128 (TM = 3, TN = 2, two workgroups per CU) when there are plenty of tiles and K is short,
-// 128 x 128 (TM = TN = 2; ring of four stages, or of two with two workgroups per CU) for
-// mid-sized problems, 128 x 64 (TM = 2, TN = 1) when even those leave half of the CUs idle.
+// Workgroup = 4 wavefronts, 2 x 2 or 1 x 4; a wavefront owns TM x TN blocks of 32 x 32 outputs: 256 x 256 (4 x 4
+// blocks, one workgroup per CU) and 224 x 256 (7 x 2, wavefronts 1 x 4) for long K or many tiles, 192 x 128 (3 x 2, two
+// workgroups per CU) when there are plenty of tiles and K is short, 128 x 128 (2 x 2, or 4 x 1 with wavefronts 1 x 4;
+// ring of four stages, or of two with two workgroups per CU) for mid-sized problems, 96 x 128 (3 x 1, wavefronts 1 x 4)
+// and 128 x 64 (2 x 1) when even those leave CUs idle.
 //
-// Why 4 x 4 blocks per wavefront for the large tile.  One v_mfma_f32_32x32x64_f8f6f4 takes 64
-// cycles and consumes two 2 KB operand blocks.  A wavefront with TM x TN blocks reads (TM + TN)
-// blocks from LDS per TM*TN MFMAs; LDS delivers 128 bytes per clock to the whole CU, so four
-// wavefronts with 4 x 4 blocks ask for 64 bytes per clock, 2 x 2 blocks for 128.  The same ratio
-// governs the bytes that must come from L2: (BM + BN) * K per tile, and L2 -> CU delivery
-// (measured: 10-13 TB/s over all CUs inside these kernels) bounds the small tiles.  4 x 4 blocks
-// of 16 accumulators are 256 registers: they live in AGPRs, one wavefront per SIMD, and latency
-// is hidden inside the wavefront:
+// A 32 x 32 block is four v_mfma_f32_16x16x128_f8f6f4, 32 cycles each.  The chip runs these kernels at its power limit
+// (13056 x 32768 x 2048 + GeGLU 581 us on zeros, 745 on real data; 816 x 32768 x 2048 49 / 58), and this MFMA takes less
+// energy per product than the 32 x 32 x 64 one at the same rate: held in registers, on random codes, 4.5 against 4.1
+// PFLOP/s (both 5.0 on zeros); 4800 x 6144 x 2048 60.0 -> 58.2 us, 3264 x 32768 x 2048 + GeGLU 203 -> 197.
+//
+// Why 4 x 4 blocks per wavefront for the large tile.  A wavefront with TM x TN blocks reads (TM + TN) operand blocks of
+// 4 KB (32 rows x 128 bytes of K) from LDS per 4 TM TN MFMAs; LDS delivers 128 bytes per clock to the whole CU, so four
+// wavefronts with 4 x 4 blocks ask for 64 bytes per clock, 2 x 2 blocks for 128.  The same ratio governs the bytes that
+// must come from L2: (BM + BN) * K per tile, and L2 -> CU delivery (measured: 10-13 TB/s over all CUs inside these
+// kernels) bounds the small tiles.  4 x 4 blocks of 16 accumulators are 256 registers: they live in AGPRs, one wavefront
+// per SIMD, and latency is hidden inside the wavefront:
 //
 //  * global -> LDS copies bypass the register file (global_load_lds_dwordx4): lane i of a
 //    wavefront fetches one 16-byte chunk and the hardware deposits chunk i at LDS base + 16*i.
 //    An LDS row is 128 bytes of K - one L2 line per row per request; the XOR swizzle that keeps
 //    the 128-bit operand reads conflict-free is therefore applied on the global side: lane i
 //    (row i/8 of an 8-row group, slot i%8 of the row) fetches chunk (i%8) ^ swizzle(row).
-//  * K is consumed in 128-byte stage-loads through a ring of DEPTH LDS stages: the copies of
-//    load d+DEPTH are requested while loads d and d+1 are being multiplied, one or two copy
-//    instructions per MFMA, so the wavefront never waits on the memory pipeline's issue queue
-//    with its MFMA pipe empty.  One barrier per stage-load, placed in its second K half: it
-//    publishes the next stage and tells everyone that the stage about to be refilled is no
-//    longer read.  All wavefronts reach it at about the same time, with MFMAs queued.
-//    Where the weights are in MFMA operand order and a wavefront owns its column blocks
-//    (wavefronts 1 x 4: the 224 x 256 tile, and 128 x 128 tiles as 4 x 1 blocks per wavefront)
-//    they do not go through LDS at all - each wavefront loads its own weight blocks straight into
-//    a ring of register sets - and the barrier gives way to a hand-over through one progress word
-//    per wavefront in LDS, which lets a wavefront run a stage or two ahead of the slowest
-//    (see `hand_over` in the kernel).
-//  * the operand blocks that open the next K half are read from LDS during the later row groups
-//    of the current one into a second register set, and inside a half the A blocks of the later
-//    row groups are read before the first group's MFMAs are issued, so ds_read latency overlaps
-//    MFMA time.
+//  * K is consumed in 128-byte stage-loads - one K step of the MFMA - through a ring of DEPTH LDS stages: the copies of
+//    load d + DEPTH are requested while loads d and d + 1 are being multiplied, one copy instruction per MFMA, so the
+//    wavefront never waits on the memory pipeline's issue queue with its MFMA pipe empty.
+//  * a stage-load is multiplied in two halves, each with one 16-row half of the activation blocks and all of the
+//    weights.  Staged weights are read once per stage-load, block by block into the registers that their predecessor's
+//    last MFMA has just left; the activation blocks of a half are read during the half before it, so ds_read latency
+//    overlaps MFMA time.  Sums stay in place through inline assembly (`multiply`).
+//  * one barrier per stage-load, in its second half behind the first group of MFMAs: it publishes the next stage and
+//    tells everyone that the stage about to be refilled is no longer read.  All wavefronts reach it at about the same
+//    time, with MFMAs queued.  Where the weights are in MFMA operand order and a wavefront owns its column blocks
+//    (wavefronts 1 x 4: the 224 x 256 tile, and 128 x 128 tiles as 4 x 1 blocks per wavefront) they do not go through
+//    LDS at all - each wavefront loads its own weight blocks straight into a ring of register sets - and the barrier
+//    gives way to a hand-over through one progress word per wavefront in LDS, which lets a wavefront run a stage or two
+//    ahead of the slowest (see `hand_over` in the kernel).
 //  * epilogue: the weight block is the MFMA's first operand, which gives a lane runs of four
 //    consecutive output columns of one token row; each wavefront stages its bf16 tile in its own
 //    slice of the (now idle) LDS and writes it out row-wise, 16 bytes per lane, whole row
@@ -50,7 +51,7 @@
 // instantiations, weights staged row-major): the last stage-load is partial, its missing chunks arrive as zeros
 // (copy16_to_lds_checked), one extra VALU instruction per copy and nothing in the MFMA loop.  Such widths used to go
 // to the generic tile kernel: the MLP 1168 -> 4304 -> 1168 at M = 777 took 43 + 37 us of GEMM there, 85 us in all;
-// 38 us in all here.
+// 34 us in all now (its second projection by the weight-streaming kernel).
 #include "fp8_device.h"
 #include "launch.h"
 #include "tuning.h"
@@ -416,8 +417,8 @@ void gemm_fp8_big_kernel(
     // complete in LDS (SLACK <= CLAIM - 1) and the stage that stage-load d + LEAD refills has been read by everyone
     // (it held stage-load d + LEAD - DEPTH <= d - SLACK).  A wavefront may so run up to SLACK stages ahead of the
     // slowest instead of waiting for it at every stage: each stalls now and then on its own memory requests, and a
-    // barrier per stage makes all four pay for every such stall (224 x 256 main loop at K = 2048: 40.2 k cycles with
-    // the barrier, 32.7 k with none at all and with this).  The slowest wavefront never waits, so the scheme cannot
+    // barrier per stage makes all four pay for every such stall (224 x 256 main loop at K = 2048, earlier MFMA: 40.2 k
+    // cycles with the barrier, 32.7 k with none at all and with this).  The slowest wavefront never waits, so the scheme cannot
     // lock up; the spin is bounded all the same (a wavefront that gave up would read a stage early: wrong numbers,
     // never a hang).
     // The words are read BEFORE the stage's last batch of operand reads and looked at behind the MFMAs that follow it
@@ -909,7 +910,7 @@ void gemm_fp8_big_kernel(
     // write the staged tile out: 1 KB (whole rows) per instruction.  The output is written once
     // and never read here: non-temporal stores keep it from evicting the operands that the
     // neighbouring tiles still want from L2 (4800 x 8192 x 2048 + GELU: 113 -> 95 us;
-    // 13056 x 2560 x 2048: 76.6 -> 70.1 us; same box, alternating builds).
+    // 13056 x 2560 x 2048: 76.6 -> 70.1 us; same box, alternating builds of the earlier main loop).
 #pragma unroll 4
     for (int qd = 0; qd < STG_BYTES / 1024; ++qd) {
         const int byte = qd * 1024 + lane * 16;
@@ -933,11 +934,6 @@ static int big_tiles(int M, int N, int epilogue, int bm, int bn) {
     return big_ceil_div(M, bm) * big_ceil_div(gated ? N / 2 : N, gated ? bn / 2 : bn);
 }
 
-// Tile edge (256 or 128, 0 = this kernel does not apply) and K splits.  256 x 256 tiles once
-// they fill the chip; 128 x 128 tiles for problems that are still MFMA-sized but have fewer
-// tiles, and those are split along K when even the small tiles leave CUs idle: a CU can pull
-// only about 45 GB/s from L2, so a mid-sized GEMM finishes sooner on more CUs even though the
-// partial sums then make a round trip through memory.
 static int big_tile_cols(int tile) { return (tile == 256 || tile == 224) ? 256 : 128; }
 
 // Fraction of the tile slots that hold a tile, over all rounds of `slots` concurrent tiles.
@@ -946,6 +942,10 @@ static double big_fill(int tiles, int slots) {
     return rounds > 0 ? (double)tiles / ((double)rounds * slots) : 1.0;
 }
 
+// Tile shape, K splits, ring depth.  All times in here: graphs of weight sets beyond the Infinity Cache, every tile shape
+// forced in turn at 988 shapes (M = 136 .. 13056, N = 1024 .. 32768, K = 1024 .. 16384, both layouts); over all of them the
+// choice is 1.6 % behind the best shape in the geometric mean.  The lines were drawn on an earlier main loop (32 x 32 x 64
+// MFMAs); where another shape is ahead by now, the comment says so.
 BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     BigPlan pl = {0, 0, 1, 0, 0, 0};
     if (K < 512) return pl;   // the stage-loads must fill the ring
@@ -960,48 +960,50 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     // 256 x 256 tiles need the fewest bytes from L2 per flop but run one workgroup per CU, so a
     // tile's prologue and epilogue leave the MFMA pipe idle; 192 x 128 tiles fit twice and overlap
     // them.  The small tile wins once there are enough of them and while K is short enough for
-    // prologue and epilogue to matter (measured: 4-18 % up to K = 8192), unless M pads worse or
-    // its last round of 512 tiles would be much emptier than the large tile's last round of 256
-    // (6528 x 2048 x 2048: 544 small tiles take 42 us, 208 large ones 37.5 us).
+    // prologue and epilogue to matter (192 / 256, us: 4800 x 8192 x 2048 + GELU 93 / 118, 1632 x 32768 x 2048 +
+    // GeGLU 108 / 122, 4800 x 2048 x 8192 76 / 89), unless M pads worse or its last round of 512 tiles would be much
+    // emptier than the large tile's last round of 256 (6528 x 2048 x 2048: 544 small tiles 36.3, 208 large
+    // ones 33.2).  Row-major weights from K = 4096 on: 224 x 256 tiles are now ahead of both (3264 x 8192 x 4096 192:
+    // 102, 224: 92; 13056 x 2048 x 8192 193 / 170) and are not asked.
     else if (K <= 8192 && big_tiles(M, N, epilogue, 192, 128) >= 400 &&
              big_ceil_div(M, 192) * 192 <= big_ceil_div(M, 256) * 256 &&
              big_fill(big_tiles(M, N, epilogue, 192, 128), 512) >= big_fill(big_tiles(M, N, epilogue, 256, 256), 256) - 0.15)
         pl.tile = 192;
     // ... and also when it fits one round of two workgroups per CU while 128 x 128 tiles would just
-    // spill into a second one (3264 x 2560 x 2048: 340 tiles of 192 x 128 take 27 us, 520 of
-    // 128 x 128 take 33 us; with 416 of those, 3264 x 2048 x 2048, the smaller tile wins 20.6 to 25.3)
+    // spill into a second one (3264 x 2560 x 2048: 340 tiles of 192 x 128 take 24.1 us, 520 of
+    // 128 x 128 29.6; with 416 of those, 3264 x 2048 x 2048, the smaller tile wins 18.5 to 23.0)
     else if (K <= 8192 && big_tiles(M, N, epilogue, 256, 256) < 200 && big_tiles(M, N, epilogue, 192, 128) > 256 &&
              big_tiles(M, N, epilogue, 192, 128) <= 512 && big_tiles(M, N, epilogue, 128, 128) > 512)
         pl.tile = 192;
     else if (big_tiles(M, N, epilogue, 256, 256) >= 200)
         // 224 x 256 tiles (every wavefront walks all 224 token rows) when they need no more tile
         // rows than 256 x 256: the same number of workgroups, fewer MFMAs on padding (816 rows:
-        // 896 instead of 1024, gate_up 2048 -> 32768 at M = 816 67.4 -> 64.2 us).  The gain is
-        // smaller than the saved MFMAs because each wavefront then reads all of the tile's
-        // activation rows from LDS, which is the next limit (113 of 128 bytes per clock).
+        // 896 instead of 1024, gate_up 2048 -> 32768 at M = 816 64.7 -> 59.2 us row-major).  More tile rows
+        // are not tried, though where they fit the same rounds they are 8 - 10 % ahead now (6528 x 2048 x 2048, 240
+        // tiles against 208: 30.3 / 33.2; 1632 x 8192 x 2048 37.9 / 41.2).
         pl.tile = big_ceil_div(M, 224) == big_ceil_div(M, 256) ? 224 : 256;
     else if (big_tiles(M, N, epilogue, 128, 128) >= 32) pl.tile = 128;   // fewer: the weight-streaming kernel wins
     else return pl;
     if (pl.cols == 0) pl.cols = big_tile_cols(pl.tile);
     int tiles = big_tiles(M, N, epilogue, pl.tile, pl.cols);
     // Few 128 x 128 tiles and a plain epilogue: 128 x 64 tiles (2 x 1 blocks per wavefront) put twice
-    // as many CUs to work.  The kernel is bound by LDS bytes, and the narrow tile reads half as many
-    // again per MFMA, so it pays only while the 128 x 128 grid leaves at least half of the CUs idle
-    // (weights from HBM, 18 weight sets): 816 x 2048 x 2048 (112 -> 224 tiles) 11.4 -> 8.9 us,
-    // 816 x 2048 x 4096 17.7 -> 13.8 us, 1100 x 1024 x 4096 16.6 -> 12.4 us; 816 x 2560 x 2048
-    // (140 -> 280 tiles, a second round) 12.8 -> 15.1 us and stays; from K = 8192 on the 128 x 128
-    // form with K split in two is level or ahead (27.9 against 28.7 us, K = 16384: 44 against 51).
+    // as many CUs to work; the narrow tile reads half as many bytes again per MFMA, so it pays only while the
+    // 128 x 128 grid leaves at least half of the CUs idle (us: 816 x 2048 x 2048, 112 -> 224 tiles, 11.6 -> 8.6;
+    // 816 x 2048 x 4096 18.1 -> 13.2; 1100 x 1024 x 4096 17.6 -> 13.1; 816 x 2560 x 2048, 140 -> 280 tiles, a second
+    // round, 11.8 -> 14.2 and stays).  From K = 8192 on the 128 x 128 form with K split in two is taken: ahead at
+    // K = 16384 (816 rows: 38.3 against 42.6), no longer at 8192 (24.0 against 22.2).
     if (forced < 0 && pl.tile == 128 && !epi_is_gated(epilogue) && tiles > 64 && tiles <= 128 && K < 8192) {
         pl.cols = 64;
         tiles = big_tiles(M, N, epilogue, 128, 64);
     }
     // Between 129 and 255 tiles of 128 x 128 (and a plain epilogue) 96 x 128 tiles - wavefronts 1 x 4, three row
     // blocks each - put up to 256 CUs to work in one round where the 128-row grid leaves a fifth to a half of them
-    // idle and 128 x 64 tiles would need a second round: 8 - 11 % faster on every shape measured (weights from HBM,
-    // 12 - 18 weight sets): 816 x 2560 x 2048 (140 -> 180 tiles) 11.2 -> 9.95 us, 816 x 3072 x 2048 11.2 -> 10.1,
-    // 700 x 4096 x 1024 8.4 -> 7.7, 1000 x 2304 x 2048 11.1 -> 10.1, 650 x 3584 x 4096 16.4 -> 14.9, 816 x 2560 x 4096
-    // 16.1 -> 14.9, 560 x 4096 x 2048 10.9 -> 9.9.  Where the 128-row grid already fills the chip, or 128 x 64 tiles
-    // fit one round, it loses (816 x 2048 x 2048: 9.6 against 8.2 us; 1632 x 2560 x 2048: 17.5 against 15.4).
+    // idle and 128 x 64 tiles would need a second round (128 x 128 / 96 x 128, us: 816 x 2560 x 2048, 140 -> 180 tiles,
+    // 11.8 / 10.2, 816 x 3072 x 2048 11.9 / 10.3, 1000 x 2304 x 2048 12.0 / 10.4, 816 x 2560 x 4096 + GELU 19.2 / 16.3,
+    // 560 x 4096 x 2048 12.0 / 10.4).  Where the 128-row grid already fills the chip, or 128 x 64 tiles fit one round,
+    // it loses (816 x 2048 x 2048: 10.2 against 8.6; 1632 x 2560 x 2048: 18.5 against 15.7).  From K = 8192 on the
+    // split form is taken, and there 96 x 128 tiles are far ahead now (1100 x 2048 x 8192 40.2 / 26.4, 2400 x 1024 x 16384
+    // 60.8 / 46.7): the line at K = 8192 is the old loop's.
     if (forced < 0 && pl.tile == 128 && pl.cols == 128 && !epi_is_gated(epilogue) && tiles > 128 && tiles < 256 && K < 8192) {
         const int t96 = big_tiles(M, N, epilogue, 96, 128);
         if (t96 > tiles && t96 <= 256) { pl.tile = 96; tiles = t96; }
@@ -1011,16 +1013,16 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     bool to_224 = false;
     if (operand_w && forced < 0 && pl.tile != 224 && K >= 4096 && K % 512 == 0) {
         // Weights in operand order: the 224 x 256 tile loads them straight into registers and hands its activation
-        // stages over without barriers - its main loop runs at 0.88 of the MFMA rate where the other shapes reach
-        // 0.7 - 0.85 - and from K = 4096 on the prologue and epilogue that nothing overlaps in it weigh less than
-        // that.  Taken when it has at least 160 tiles and fills its rounds of 256 workgroups with useful rows and
-        // columns at least 0.8 times as well as the shape chosen above fills its own (weights from HBM, 4 - 6 weight
-        // sets, us: 6528 x 2048 x 16384 185 -> 166, 13056 x 2048 x 16384 366 -> 317, 6528 x 2048 x 8192 96 -> 86,
-        // 1632 x 8192 x 8192 96 -> 88, 4800 x 2048 x 8192 81 -> 74, 6528 x 4096 x 4096 106 -> 96, 13056 x 2048 x 4096
-        // 107 -> 98, 3264 x 16384 x 4096 + GeGLU 202 -> 189; level: 4800 x 8192 x 4096, 3264 x 8192 x 4096; not taken,
-        // and slower when forced: 2048 x 8192 x 8192 (320 tiles, two rounds: 150 against 103), 8000 x 1024 x 8192 (144
-        // tiles: 74 against 69), 3264 x 2048 x 16384 (120 tiles: 129 against 125).  At K = 2048 the shapes that run
-        // two workgroups per CU keep their lead.
+        // stages over without barriers, and from K = 4096 on the prologue and epilogue that nothing overlaps in it weigh
+        // less than what its main loop gains.  Taken when it has at least 160 tiles and fills its rounds of 256
+        // workgroups with useful rows and columns at least 0.8 times as well as the shape chosen above fills its own
+        // (chosen above / this, us: 6528 x 2048 x 16384 173 / 154, 13056 x 2048 x 16384 340 / 300, 6528 x 2048 x 8192 93.9 /
+        // 81.8, 1632 x 8192 x 8192 93.4 / 85.0, 6528 x 4096 x 4096 104 / 96, 13056 x 2048 x 4096 101 / 91, 3264 x 16384 x 4096 +
+        // GeGLU 184 / 181, 4800 x 8192 x 4096 141 / 134, 3264 x 8192 x 4096 101 / 89; level: 4800 x 2048 x 8192 74.1 / 73.6; not
+        // taken, and slower when forced: 2048 x 8192 x 8192 (320 tiles, two rounds) 101 / 147, 8000 x 1024 x 8192 (144
+        // tiles) 57.3 / 70.3, 3264 x 2048 x 16384 (120 tiles) 106 / 125).  0.8 lets a second round in that is nearly empty:
+        // 6528 x 2560 x 4096 (300 tiles) 64.9 / 88.7, 4800 x 4096 x 4096 (352) 78.4 / 90.3.  At K = 2048 the shapes that run
+        // two workgroups per CU are level or ahead.
         const int t224 = big_tiles(M, N, epilogue, 224, 256);
         const int slots = big_two_per_cu(pl.tile == 192 ? 3 : pl.tile == 256 ? 4 : 2, 2, pl.depth, 0) ? 512 : 256;
         const double area_now = (double)big_ceil_div(tiles * pl.splits, slots) * slots * pl.tile * pl.cols;
@@ -1034,13 +1036,13 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     if ((pl.tile == 128 && pl.cols == 64) || pl.tile == 96) {
         // always one round of at most 256 workgroups here, or forced: deep ring, no split
     } else if (pl.tile == 128) {
-        // Measured at M = 816: splitting pays for K = 16384 (67 -> 49 us with two splits) and
-        // costs for K = 2048 (19 -> 25 us): the partial-sum round trip is worth about 6 us.
+        // K split in two: the partial sums' round trip is worth 4 - 8 us (816 rows: 56.1 -> 38.3 us at K = 16384, 29.4 ->
+        // 24.0 at 8192, but 18.1 -> 18.7 at 4096, 11.6 -> 16.8 at 2048).
         if (tiles < 200 && K >= 8192 && (K % 256 == 0 || ragged)) pl.splits = 2;
         // With more tiles than CUs a ring of two stages lets two workgroups share a CU instead of
-        // queueing behind each other (800 x 8192 x 1024, 448 tiles: 17.5 -> 14.4 us; 1632 x 2560 x 2048,
-        // 260 tiles: 23.3 -> 18.3 us); up to one tile per CU the deeper ring hides more latency
-        // (1632 x 2048 x 2048, 208 tiles: 14.2 against 17.3 us).
+        // queueing behind each other (1632 x 2560 x 2048, 260 tiles: 21.5 -> 15.7 us; 800 x 8192 x 1024 +
+        // GeGLU, 448 tiles: 14.4 -> 11.4); up to one tile per CU the
+        // deeper ring hides more latency (1632 x 2048 x 2048, 208 tiles: 12.0 against 14.3).
         else if (tiles > 256) pl.depth = 2;
     }
     if (const char* e = tuning_env("PHYAI_FP8_BIG_SPLITS")) {
@@ -1056,7 +1058,8 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     // of four.  128 x 128 tiles with a ring of four LDS stages and a plain epilogue: wavefronts 1 x 4 with one column
     // block each and a ring of eight.  (Not the 96 x 128 tile: its main loop gains what its longer prologue - six
     // stage-loads requested up front, at what the CU's vector-memory path passes - loses: 816 x 2560 x 2048 10.0 ->
-    // 10.1 us.)
+    // 10.1 us on the earlier loop.  Up to K = 2048 the ring of eight is level with staged weights, and the ring of four of
+    // two workgroups per CU up to 14 % ahead of it from 160 tiles up: 2048 x 2048 x 2048 15.5 / 13.6.)
     if (operand_w && !(tuning_env("PHYAI_FP8_BIG_DIRECT") && atoi(tuning_env("PHYAI_FP8_BIG_DIRECT")) == 0)) {
         if (pl.tile == 224 && pl.splits == 1 && K % 512 == 0) pl.regs = 4;
         else if (pl.tile == 128 && pl.cols == 128 && pl.depth == 4 && (K / pl.splits) % 1024 == 0 && !epi_is_gated(epilogue)) pl.regs = 8;
@@ -1084,7 +1087,7 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
     // With few tile columns and long rows of activations (816 x B tokens into a 16384 -> 2048
     // projection) that is eight copies of the larger operand; then the roles are exchanged.
     // Estimated bytes from HBM: the operand an XCD does not own is read once per XCD (up to 8
-    // times), the other once per band.
+    // times), the other once per band.  (6528 x 2048 x 16384: 187 us by tile columns, 168 by tile rows.)
     double chosen_bytes = 0.0;
     {
         const double a_bytes = (double)g.M * g.K, b_bytes = (double)g.N * g.K;
@@ -1094,7 +1097,7 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
         a.by_rows = by_rows < 0.8 * by_cols;
         // ... unless the busiest XCD then needs one more round of tiles than in the other order
         // (13056 x 2560 x 2048 in 256 x 256 tiles: 510 tiles are 64 per XCD by tile columns, two
-        // rounds on 32 CUs, but 65 on some XCDs by tile rows: 92 against 75.5 us)
+        // rounds on 32 CUs, but 65 on some XCDs by tile rows: 93 against 75 us)
         const int slots = 32 * (big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1);
         const int rounds_c = big_ceil_div(big_max_tiles_per_xcd(a.m_tiles, a.n_tiles, 4), slots);
         const int rounds_r = big_ceil_div(big_max_tiles_per_xcd(a.n_tiles, a.m_tiles, 4), slots);
@@ -1112,8 +1115,7 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
     // Split along K: an XCD per K range (see the kernel).  Every XCD then fetches 1 / splits of the
     // activation codes instead of all of them, and the weights of its tile columns once.  Taken when
     // that is the smaller estimate and the tile columns divide evenly among the 8 / splits groups
-    // (816 x 2048 x 16384, K split in two: 155 -> 87 MB fetched; the time is the same to within 1 %,
-    // the kernel being bound by its LDS traffic, so this saves HBM bandwidth, not microseconds).
+    // (816 x 2048 x 16384, K split in two: 155 -> 87 MB fetched, 36.8 -> 35.3 us row-major, 35.4 -> 34.2 in operand order).
     if (splits == 2 || splits == 4 || splits == 8) {
         const int groups = 8 / splits, cols = big_ceil_div(a.n_tiles, groups);
         const double by_k = (double)g.M * g.K * 8.0 / splits + (double)g.N * g.K;

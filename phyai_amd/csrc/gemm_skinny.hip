@@ -423,15 +423,16 @@ static int sk_ceil_div(int a, int b) { return (a + b - 1) / b; }
 // Largest M served here.  Every group of token rows re-reads the weight tiles from L2, so with
 // enough output tiles the LDS-staged tile kernels win; the dispatcher prefers those as soon as
 // their grid is large enough (see launch_gemm) and falls back to this kernel up to here
-// (N = 1024: ahead of the 128 x 128 tile kernel up to M = 1000, 11.0 against 17.5 us at 800 x 1024 x 4096; beyond
-// M = 1024 where the tile kernels have fewer than 64 tiles, i.e. few columns: 1548 x 256 x 6016 47.9 -> 21.4 us).
+// (N = 1024: ahead of every tile shape up to M = 1000, 10.6 against 12.3 us at 816 x 1024 x 4096; beyond M = 1024 with
+// fewer than 64 tiles of 128 x 128, i.e. few columns: 1548 x 256 x 6016 14.9 against 16.0, 2048 x 512 x 2048 8.1 / 8.7).
 static int skinny_max_m() {
     if (const char* e = tuning_env("PHYAI_FP8_SKINNY_MAXM")) return atoi(e);
     return 4096;
 }
 
-// K that is not a multiple of 128 (staged form only): from three K steps on (ten with
-// more than 64 rows and few columns), the generic kernel's K splits cost it a round trip through memory (184 x 896 x 2256: 31.3 -> 9.1 us, 353 x 384 x 3216: 35.9 -> 9.0 us).
+// K that is not a multiple of 128 (staged form only): from three K steps on (ten with more than 64 rows and few
+// columns), the generic kernel's K splits cost it a round trip through memory (184 x 896 x 2256: 31.3 -> 9.1 us, 353 x
+// 384 x 3216: 35.9 -> 9.0 us).
 static bool skinny_takes_ragged(int M, int N, int K) {
     static const bool staged = []() { const char* e = tuning_env("PHYAI_FP8_SKINNY_STAGED"); return !(e && atoi(e) == 0); }();
     if (!staged || (int64_t)K * (N > M ? N : M) >= ((int64_t)1 << 31) || K >= (1 << 24)) return false;
@@ -467,7 +468,7 @@ SkinnyPlan skinny_plan(int M, int N, int K, int epilogue) {
     // columns: 1x1 with four workgroups along M; gate_up: 2x4) as at M = 100 .. 1000
     // (800 x 1024 x 4096: 4x4 11.0 us, 2x4 13.6, 4x3 15.8, 2x3 16.4, 2x2 17.9 for products 8, 12,
     // 14, 15, 16), where the winner beats a fixed 1 x 4 by 10-50 % and, on the 1024-wide
-    // projections, the 128 x 128 tile kernel (17.5 us).
+    // projections, the tile kernel's best shape (12.3 us).
     {
         int best_cost = 1 << 30;
         pl.nt = 1; pl.mb = 1;

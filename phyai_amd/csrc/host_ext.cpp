@@ -60,8 +60,8 @@ struct PyModules {
 } pm = {};
 
 PyObject *s_dispatcher, *s_generation, *s_selected, *s_params_dtype, *s_skip_bias_add, *s_bias;
-PyObject *s_host, *s_call, *s_forward_fused, *s_forward_addcmul, *s_forward_fp8, *s_supports, *s_forward, *s_fuse_activation, *s_gated, *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate,
-    *s_compiled, *s_hooks[4];
+PyObject *s_host, *s_call, *s_forward, *s_forward_fused, *s_forward_addcmul, *s_forward_fp8, *s_supports, *s_fuse_activation, *s_gated,
+    *s_epilogue, *s_modules, *s_gate_up, *s_down, *s_fc1, *s_fc2, *s_residual, *s_gate, *s_compiled, *s_hooks[4];
 PyObject *s_parameters, *s_weight, *s_weight_scale, *s_input_scale, *s_stream_weights, *s_weight_layout,
     *s_spec, *s_granularity, *s_apply, *s_quantize;
 
@@ -893,8 +893,9 @@ PyMODINIT_FUNC PyInit__phyai_host() {
         {&s_stream_weights, "stream_weights"}, {&s_weight_layout, "weight_layout"}, {&s_spec, "spec"},
         {&s_granularity, "granularity"}, {&s_apply, "apply"}, {&s_quantize, "quantize_activation"},
         {&s_dispatcher, "_dispatcher"}, {&s_generation, "generation"}, {&s_selected, "_selected"},
-        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"}, {&s_call, "__call__"}, {&s_forward_fused, "forward_fused"}, {&s_forward_addcmul, "forward_addcmul"},
-        {&s_forward_fp8, "forward_fp8"}, {&s_supports, "supports_fused_epilogue"}, {&s_forward, "forward"},
+        {&s_params_dtype, "params_dtype"}, {&s_skip_bias_add, "skip_bias_add"}, {&s_bias, "bias"}, {&s_host, "_host"},
+        {&s_call, "__call__"}, {&s_forward, "forward"}, {&s_forward_fused, "forward_fused"}, {&s_forward_addcmul, "forward_addcmul"},
+        {&s_forward_fp8, "forward_fp8"}, {&s_supports, "supports_fused_epilogue"},
         {&s_fuse_activation, "fuse_activation"}, {&s_gated, "gated"}, {&s_epilogue, "_epilogue"}, {&s_modules, "_modules"},
         {&s_gate_up, "gate_up_proj"}, {&s_down, "down_proj"}, {&s_fc1, "fc1"}, {&s_fc2, "fc2"}, {&s_residual, "residual"}, {&s_gate, "gate"},
         {&s_compiled, "_compiled_call_impl"}, {&s_hooks[0], "_forward_hooks"}, {&s_hooks[1], "_forward_pre_hooks"},

@@ -120,7 +120,7 @@ bool gemm_takes_row_maxima(const GemmProblem& p);
 // Text form of the whole-linear choice for aligned operands and dense activations / output.
 int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0);
 
-// Weight-streaming kernel for M <= 64 (gemm_skinny.hip).  It needs no workspace.
+// Weight-streaming kernel (gemm_skinny.hip): M <= 64, and up to M = 4096 with few output columns.  It needs no workspace.
 struct SkinnyPlan {
     int tiles;   // workgroups (each owns 16*nt weight rows over the whole K)
     int msplit;  // workgroups along M
@@ -147,7 +147,8 @@ constexpr int kRowAmaxSlots = 256;  // slots per token row of a table of handed-
 constexpr int kFusedAmaxSlots = 64; // ... that the consumer of gemm_skinny_fused.hip reads (that of gemm_selfq.h: all)
 int launch_gemm_fused(const GemmProblem& p, const FusedPlan& pl, hipStream_t st);
 
-// Small-M linear that quantizes its own rows at any K up to 16384 (gemm_selfq.h).  rg == 0: does not apply.
+// Small-M linear that quantizes its own rows (gemm_selfq.h): what the one above does not take, up to the longest K per
+// shape of workgroup that selfq_max_k lists (1088 ... 16384).  rg == 0: does not apply.
 struct SelfqPlan {
     int rg;      // groups of four token rows per workgroup (1 or 2)
     int nt;      // 16-row weight tiles per workgroup
@@ -163,8 +164,8 @@ int launch_selfq_own_act(const GemmProblem& p, const SelfqPlan& pl, hipStream_t 
 int launch_selfq_handed(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
 int launch_selfq_static(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
 
-// Pipelined tile kernel for large M (gemm_big.hip), 256 x 256 or 128 x 128 tiles; the small
-// tiles may be split along K (partials in the workspace, as for the generic tile kernel).
+// Pipelined tile kernel for large M (gemm_big.hip); 128 x 128 tiles may be split along K (partials in the workspace,
+// as for the generic tile kernel).
 struct BigPlan {
     int tile;    // tile rows: 256 (x 256 columns), 224 (x 256), 192 (x 128), 128 (x 128 or x 64), 96 (x 128), or 0 if the kernel does not apply
     int cols;    // tile columns

@@ -22,7 +22,7 @@ Three forms of the layer run on the same weights:
              linear behind it), 8 beyond;
 ``unfused``  the reference's structure on this library's kernels: norm, quantized linear,
              attention, quantized linear, ``torch.addcmul``, norm, MLP, ``torch.addcmul``
-             (12 kernels per layer).  Bit-equal to ``fused``;
+             (8 kernels per layer up to 128 token rows, 12 beyond).  Bit-equal to ``fused``;
 ``torch``    the reference's own arithmetic as torch library calls (norm and quantizer
              expressions, ``torch._scaled_mm``, ``gelu * up``, ``addcmul``): the yardstick the
              other two are held to, layer by layer.

@@ -2,8 +2,9 @@
 models/pi05/model_runner_pi05.py:689-738 and modeling_pi05.py:801-835) at the real shapes:
 18 layers, hidden 1024, 8 x 256 query heads, one KV head, MLP 4096, 50 action tokens.
 
-* the fused layer (8 kernels) equals the unfused one (12 kernels) bit for bit over 18 chained
-  layers and 3 Euler steps - every intermediate hidden state, not only the result;
+* the fused layer (four kernels: the norms and quantizers run inside the linears) equals the unfused one
+  (norms, linears, MLP and addcmul one by one) bit for bit over 18 chained layers and 3 Euler steps -
+  every intermediate hidden state, not only the result;
 * a graph replay equals the eager loop bit for bit, for several inputs, with eager work between;
 * layer by layer, on the hidden state the library's loop actually produced, each form is within
   the stated tolerance (max-abs <= 1e-2 max|ref|, cosine >= 0.9999) of the same layer computed
