@@ -90,7 +90,13 @@ __device__ __forceinline__ void copy16_to_lds(const uint8_t* base, uint32_t lane
                  :: "v"(lane_offset), "s"(base), "s"(lds_wave_base) : "memory", "m0");
 }
 
-// The same copy for data that should not stay in the caches behind it (read once per pass over a
+// One 4-byte word per lane: lane i's lands at lds_wave_base + 4*i.
+__device__ __forceinline__ void copy4_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t lds_wave_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(lane_offset), "s"(base), "s"(lds_wave_base) : "memory", "m0");
+}
+
+// copy16_to_lds for data that should not stay in the caches behind it (read once per pass over a
 // working set that is larger than they are).
 __device__ __forceinline__ void copy16_to_lds_nt(const uint8_t* base, uint32_t lane_offset, uint32_t lds_wave_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
@@ -198,6 +204,12 @@ __device__ __forceinline__ void addcmul4(float* y, uint2 res, uint2 gate) {
                         bf16_bits_to_f32(gate.y & 0xFFFFu), __uint_as_float(gate.y & 0xFFFF0000u)};
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[e] = r[e] + round_bf16(y[e]) * g[e];
+}
+// The same on two columns packed in a word, y already rounded.
+__device__ __forceinline__ uint32_t addcmul2(uint32_t y, uint32_t res, uint32_t gate) {
+    const float lo = bf16_bits_to_f32(y & 0xFFFFu) * bf16_bits_to_f32(gate & 0xFFFFu);
+    const float hi = __uint_as_float(y & 0xFFFF0000u) * __uint_as_float(gate & 0xFFFF0000u);
+    return pack_bf16x2(bf16_bits_to_f32(res & 0xFFFFu) + lo, __uint_as_float(res & 0xFFFF0000u) + hi);
 }
 
 }  // namespace phyai

@@ -39,7 +39,12 @@
 //  * epilogue: the weight block is the MFMA's first operand, which gives a lane runs of four
 //    consecutive output columns of one token row; each wavefront stages its bf16 tile in its own
 //    slice of the (now idle) LDS and writes it out row-wise, 16 bytes per lane, whole row
-//    segments per instruction.
+//    segments per instruction.  It is straight-line arithmetic on LDS and registers: scales and bias are in LDS since
+//    the prologue, the gated residual is added where the tile leaves row by row, and the sums of the tiles up to 128 x 128
+//    are in VGPRs, which the arithmetic can read where they are.  A 128 x 64 tile's took 1.9 k cycles while each group of four columns
+//    looked for a residual, and waited for its constants from memory; 0.8 k now, and its main loop 8.9 k instead of 9.4 k
+//    (us: 816 x 2048 x 2048 7.7 -> 7.4, 816 x 2560 x 2048 9.9 -> 9.4, 777 x 4304 x 1168 + GELU 12.0 -> 11.1,
+//    400 x 8192 x 1024 + GeGLU 8.2 -> 8.0, 1632 x 2048 x 2048 11.1 -> 10.0, 4800 x 6144 x 2048 59.3 -> 57.9; 816 x 32768 x 2048 level).
 //
 // The smaller tiles (192 x 128, and 128 x 128 with a ring of two) keep within the register and
 // LDS budget of two workgroups per CU, so that one workgroup's prologue and epilogue run under
@@ -112,6 +117,10 @@ struct BigArgs {
 // cut into 8 runs of equal length (within one), one per XCD: still whole or half columns per
 // XCD, and every XCD gets the same number of tiles.  Ids past an XCD's run have no tile.
 struct BigTile { int m, n; };
+// Tile order, weight layout and kind of row scale in one argument.
+static int big_order(int band, int by_rows, int operand_w, int scale_is_scalar) {
+    return band | by_rows << 8 | operand_w << 10 | scale_is_scalar << 11;
+}
 __device__ __forceinline__ BigTile big_tile_of(int id, int m_tiles, int n_tiles, int band_rows) {
     const int full = n_tiles >> 3, rest = n_tiles & 7;   // whole groups of 8 tile columns; columns after them
     const int per_band = 8 * (band_rows * full + ((rest * band_rows + 7) >> 3));
@@ -183,6 +192,10 @@ __host__ __device__ constexpr bool big_two_per_cu(int tm, int tn, int depth, int
     return (depth == 2 && tm < 4) || (wmode == 2 && tm == 4 && tn == 1 && depth == 4);
 }
 
+// The epilogue's constants ride with the first stage-load, except in 192 x 128 tiles, two of which fill the LDS to the last
+// byte.  Asked for in the epilogue they were a trip to memory that nothing overlapped.
+__host__ __device__ constexpr bool big_constants_ride(int tm, int tn) { return !(tm == 3 && tn == 2); }
+
 // DEPTH: stages of the LDS ring, each holding BIG_BK bytes of K for the whole tile.
 // Variants whose ring leaves room for two workgroups per CU are held to the register budget of
 // two wavefronts per SIMD: while one workgroup is in its prologue or epilogue the other one
@@ -201,19 +214,23 @@ __host__ __device__ constexpr bool big_two_per_cu(int tm, int tn, int depth, int
 template <int TM, int TN, int DEPTH, int EPI, bool SPLIT, int WGM = 2, int WGN = 2, int WMODE = 0, bool RAGGED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1)))
 void gemm_fp8_big_kernel(
-    const uint8_t* __restrict__ a_a, const uint8_t* __restrict__ a_b, int a_K, int a_M, int a_N, int a_m_tiles,
-    int a_n_tiles, int a_band, int a_by_rows, int a_k_per_split, const float* __restrict__ a_a_scale,
-    const float* __restrict__ a_b_scale, const uint16_t* __restrict__ a_bias, uint16_t* __restrict__ a_out,
-    int64_t a_ldo, int a_a_scale_scalar, float* __restrict__ a_partials, int* __restrict__ a_counters,
-    const ResidualArgs a_res) {
-    // scalar arguments, what the prologue needs first (the first 16 dwords are preloaded into SGPRs)
+    const uint8_t* __restrict__ a_a, const uint8_t* __restrict__ a_b, int a_K, int a_M, int a_N, int a_m_tiles, int a_order,
+    int a_k_per_split, const float* __restrict__ a_a_scale, const float* __restrict__ a_b_scale,
+    const uint16_t* __restrict__ a_bias, uint16_t* __restrict__ a_out, int64_t a_ldo, float* __restrict__ a_partials,
+    int* __restrict__ a_counters, const ResidualArgs a_res) {
+    // scalar arguments, what the prologue needs first (the first 16 dwords, up to a_bias, are preloaded into SGPRs)
     BigArgs p;
     p.a = a_a; p.b = a_b; p.a_scale = a_a_scale; p.b_scale = a_b_scale; p.bias = a_bias; p.out = a_out;
-    p.ldo = a_ldo; p.M = a_M; p.N = a_N; p.K = a_K; p.a_scale_scalar = a_a_scale_scalar;
-    p.k_per_split = a_k_per_split; p.partials = a_partials; p.counters = a_counters;
-    // a_by_rows = tile order | weights in operand order << 4
-    p.m_tiles = a_m_tiles; p.n_tiles = a_n_tiles; p.band = a_band; p.by_rows = a_by_rows & 15; p.res = a_res;
-    p.operand_w = __builtin_amdgcn_readfirstlane(a_by_rows >> 4);
+    p.ldo = a_ldo; p.M = a_M; p.N = a_N; p.K = a_K;
+    p.k_per_split = a_k_per_split; p.partials = a_partials; p.counters = a_counters; p.m_tiles = a_m_tiles; p.res = a_res;
+    // a_order: see big_order
+    p.band = a_order & 255; p.by_rows = (a_order >> 8) & 3;
+    p.operand_w = __builtin_amdgcn_readfirstlane((a_order >> 10) & 1);
+    p.a_scale_scalar = (a_order >> 11) & 1;
+    {
+        constexpr int bn_eff = (epi_is_gated(EPI) ? 16 : 32) * TN * WGN;
+        p.n_tiles = ((epi_is_gated(EPI) ? p.N / 2 : p.N) + bn_eff - 1) / bn_eff;
+    }
     PHYAI_STAMP_BEGIN
     constexpr bool GATED = epi_is_gated(EPI);
     constexpr bool OPW = WMODE != 0, BDIRECT = WMODE == 2;
@@ -256,8 +273,14 @@ void gemm_fp8_big_kernel(
     // (the epilogue stages the bf16 tile in the same LDS; where the ring is smaller than that, the ring grows)
     constexpr int EPI_STAGING = 4 * WM * ((GATED ? TN / 2 : TN) * 64);
     constexpr int LDS_BYTES = DEPTH * STAGE_BYTES > EPI_STAGING ? DEPTH * STAGE_BYTES : EPI_STAGING;
+    // What the epilogue multiplies with - BM row scales, BN weight scales, BN bias values - rides along with the first
+    // stage-load into LDS of its own, a word per lane, in blocks of 64 words.
+    constexpr bool RIDE = big_constants_ride(TM, TN);
+    constexpr int XBLOCKS = (BM + 63) / 64, WBLOCKS = BN / 64, BBLOCKS = (BN + 127) / 128;
+    constexpr int CONSTS = RIDE ? (XBLOCKS + WBLOCKS + BBLOCKS + 3) / 4 : 0;   // copies of a wavefront
+    constexpr int CONST_AT = LDS_BYTES + (BDIRECT ? 16 : 0), CONST_BYTES = RIDE ? (XBLOCKS + WBLOCKS + BBLOCKS) * 256 : 0;
     // (weights in registers: 16 more bytes for the four wavefronts' progress words, see the main loop)
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_BYTES + (BDIRECT ? 16 : 0)];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[CONST_AT + CONST_BYTES];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WGN, wn = wave % WGN;
@@ -292,9 +315,9 @@ void gemm_fp8_big_kernel(
     for (int e = 0; e < TM * TN * 4; ++e) acc[e / (TN * 4)][e / 4 % TN][e / 2 % 2][e % 2] = v4f{0.f, 0.f, 0.f, 0.f};
     // The multiply in inline assembly, with the sum in place: left to the compiler, a sum may land in other registers than
     // it came from, and with 96 - 256 of them live that ends in copies and spills (3 x 2 blocks: 174 registers this way,
-    // 256 the other; 7 x 2 did not fit).  AGPRs where a wavefront has its SIMD to itself.  The s_nop covers a VALU write of
-    // an operand just before (the hazards inside an asm are not the compiler's).
-    constexpr bool ACC_IN_AGPR = !big_two_per_cu(TM, TN, DEPTH, WMODE);
+    // 256 the other; 7 x 2 did not fit).  AGPRs where the VGPRs do not hold them (the split kernels' epilogue wants those for the
+    // other half).  The s_nop covers a VALU write of an operand just before (the hazards inside an asm are not the compiler's).
+    constexpr bool ACC_IN_AGPR = TM * TN >= 14 || SPLIT;
     auto multiply = [&](v8i w, v8i x, v4f& c) {
         if constexpr (ACC_IN_AGPR) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
         else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+v"(c) : "v"(w), "v"(x));
@@ -371,6 +394,7 @@ void gemm_fp8_big_kernel(
             }
     }
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
+    const uint32_t const_base = __builtin_amdgcn_readfirstlane(lds_base + CONST_AT);
     const uint32_t wave_a = __builtin_amdgcn_readfirstlane(lds_base + wave * (CA * 1024));
     const uint32_t wave_b = __builtin_amdgcn_readfirstlane(lds_base + BM * BIG_BK + wave * (CB * 1024));
     // copy c (0 .. COPIES-1) of this wavefront's share of stage-load `d` (K bytes [128 d, 128 d + 128))
@@ -396,6 +420,56 @@ void gemm_fp8_big_kernel(
         }
     };
     using Slot0 = std::integral_constant<int, 0>;
+    const bool bias_rides = p.bias != nullptr && (reinterpret_cast<uintptr_t>(p.bias) & 3) == 0;
+    // Blocks of the constants: row scales of the tile, then the weight scales of its columns (gated: gate columns, then up
+    // columns), then their bias values, two to a word; past the matrix its last ones.  Every wavefront makes CONSTS copies (the
+    // waits count them): with fewer blocks than that one of them again.  No bias, or one that is not a row of words: its
+    // place is filled by hand.
+    const int M = p.M, N = p.N, one_scale = p.a_scale_scalar;
+    auto issue_constants = [&, M, N, one_scale](const void* x_scale, const void* w_scale, const void* bias) {
+#pragma unroll
+        for (int c = 0; c < CONSTS; ++c) {
+            constexpr int LAST = XBLOCKS + WBLOCKS + BBLOCKS - 1;
+            const int w = __builtin_amdgcn_readfirstlane(c * 4 + wave);
+            int blk = w < LAST ? w : LAST;
+            if (blk >= XBLOCKS + WBLOCKS && !bias_rides) blk = XBLOCKS;
+            const void* base;
+            uint32_t at;
+            if (blk < XBLOCKS) {
+                const int m = m0 + blk * 64 + lane;
+                base = x_scale;
+                at = one_scale ? 0u : (uint32_t)(m < M ? m : M - 1) * 4;
+            } else {
+                // column j of the tile; bias: the even one of the pair
+                const bool of_bias = blk >= XBLOCKS + WBLOCKS;
+                int j = of_bias ? (blk - XBLOCKS - WBLOCKS) * 128 + 2 * lane : (blk - XBLOCKS) * 64 + lane;
+                if (j >= BN) j = 0;
+                int n;
+                if constexpr (GATED) {
+                    const int up = j >= BN / 2 ? 1 : 0;
+                    n = n0 + j - up * (BN / 2);
+                    n = (n < half_n ? n : half_n - 2) + up * half_n;
+                } else {
+                    n = n0 + j;
+                    n = n < N ? n : N - 2;
+                }
+                base = of_bias ? bias : w_scale;
+                at = (uint32_t)n * (of_bias ? 2u : 4u);
+            }
+            const uint64_t b64 = reinterpret_cast<uint64_t>(base);   // (uniform, which the compiler does not see)
+            const uint64_t b_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b64);
+            const uint64_t b_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b64 >> 32));
+            copy4_to_lds(reinterpret_cast<const uint8_t*>(b_lo | b_hi << 32), at, __builtin_amdgcn_readfirstlane(const_base + blk * 256));
+        }
+        if (CONSTS > 0 && !bias_rides && tid < BN) {
+            uint16_t v = 0;
+            if (bias != nullptr) {
+                const int up = GATED && tid >= BN / 2 ? 1 : 0, n = n0 + tid - up * (BN / 2), lim = GATED ? half_n : N;
+                v = static_cast<const uint16_t*>(bias)[(n < lim ? n : lim - 1) + up * half_n];
+            }
+            reinterpret_cast<uint16_t*>(lds + CONST_AT + (XBLOCKS + WBLOCKS) * 256)[tid] = v;
+        }
+    };
 
     // stage-loads in all, >= DEPTH
     const int n_loads = RAGGED && SPLIT ? ((k_begin + p.k_per_split < p.K ? p.k_per_split : p.K - k_begin) + BIG_BK - 1) / BIG_BK
@@ -583,6 +657,7 @@ void gemm_fp8_big_kernel(
         part(S0{}, 0, CA);
         part(S1{}, 0, CA);
         if constexpr (CLAIM == 3) part(S2{}, 0, CA);
+        issue_constants(p.a_scale, p.b_scale, p.bias);
         part(S1{}, CA, IDX_END);
         if constexpr (CLAIM == 3) part(S2{}, CA, IDX_END);
         if constexpr (CLAIM == 2) part(S2{}, 0, IDX_END);
@@ -593,9 +668,11 @@ void gemm_fp8_big_kernel(
         }
     } else {
 #pragma unroll
-        for (int d = 0; d < DEPTH - 1; ++d)
+        for (int d = 0; d < DEPTH - 1; ++d) {
 #pragma unroll
             for (int c = 0; c < COPIES; ++c) issue(d, c, Slot0{});
+            if (d == 0) issue_constants(p.a_scale, p.b_scale, p.bias);
+        }
 #pragma unroll
         for (int c = 0; c < HEAD_IDX; ++c) issue(DEPTH - 1, c, Slot0{});
     }
@@ -607,10 +684,10 @@ void gemm_fp8_big_kernel(
     }
     if constexpr (BDIRECT) {
         // stage-load 0 and the activations up to stage-load CLAIM - 1 have landed (what progress word -1 stands for)
-        wait_copies<(LEAD - CLAIM) * COPIES + (CLAIM - 1) * (COPIES - CA)>();
+        wait_copies<(LEAD - CLAIM) * COPIES + (CLAIM - 1) * (COPIES - CA) + CONSTS>();
         if (lane == 0) progress[wave] = -1;
     } else {
-        wait_copies<COPIES * (LEAD - 2) + HEAD>();   // stage-load 0 has landed
+        wait_copies<COPIES * (LEAD - 2) + HEAD + CONSTS>();   // stage-load 0 has landed
     }
     __syncthreads();
     PHYAI_STAMP(1)
@@ -754,17 +831,26 @@ void gemm_fp8_big_kernel(
     static_assert(4 * STG_BYTES <= LDS_BYTES, "staging fits in the operand LDS");
     const int n_lim = GATED ? half_n : p.N;
     const int nbase = n0 + wn * (GATED ? WN / 2 : WN);
+    const float* const const_x = reinterpret_cast<const float*>(lds + CONST_AT);   // where RIDE
+    const float* const const_w = const_x + XBLOCKS * 64;
+    const uint16_t* const const_bias = reinterpret_cast<const uint16_t*>(const_w + BN);
     // column constants are read 4 at a time when the arrays allow it (N is a multiple of 16, so
     // a run of four columns is valid or invalid as a whole)
     const bool vec_cols = (reinterpret_cast<uintptr_t>(p.b_scale) & 15) == 0 &&
                           (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0;
-    auto load_cols = [&](int n, v4f& sc, v4f& bi) {
-        if (vec_cols) {
+    auto bias4 = [](uint2 b, v4f& bi) {
+        bi[0] = bf16_bits_to_f32(b.x & 0xFFFFu); bi[1] = __uint_as_float(b.x & 0xFFFF0000u);
+        bi[2] = bf16_bits_to_f32(b.y & 0xFFFFu); bi[3] = __uint_as_float(b.y & 0xFFFF0000u);
+    };
+    // four columns from n of the matrix, which are columns c .. of the constants that rode
+    auto load_cols = [&](int n, int c, v4f& sc, v4f& bi) {
+        if constexpr (RIDE) {
+            sc = *reinterpret_cast<const v4f*>(const_w + c);
+            bias4(*reinterpret_cast<const uint2*>(const_bias + c), bi);
+        } else if (vec_cols) {
             sc = *reinterpret_cast<const v4f*>(p.b_scale + n);
             if (p.bias) {
-                const uint2 b = *reinterpret_cast<const uint2*>(p.bias + n);
-                bi[0] = bf16_bits_to_f32(b.x & 0xFFFFu); bi[1] = __uint_as_float(b.x & 0xFFFF0000u);
-                bi[2] = bf16_bits_to_f32(b.y & 0xFFFFu); bi[3] = __uint_as_float(b.y & 0xFFFF0000u);
+                bias4(*reinterpret_cast<const uint2*>(p.bias + n), bi);
             } else {
                 bi[0] = bi[1] = bi[2] = bi[3] = 0.f;
             }
@@ -777,12 +863,18 @@ void gemm_fp8_big_kernel(
         }
     };
     float sa[TM][2];
+    if constexpr (!RIDE) {
 #pragma unroll
-    for (int e = 0; e < 2 * TM; ++e) {
-        const int m = m0 + wm * WM + e * 16 + l16;
-        sa[e >> 1][e & 1] = p.a_scale[p.a_scale_scalar ? 0 : (m < p.M ? m : p.M - 1)];
+        for (int e = 0; e < 2 * TM; ++e) {
+            const int m = m0 + wm * WM + e * 16 + l16;
+            sa[e >> 1][e & 1] = p.a_scale[p.a_scale_scalar ? 0 : (m < p.M ? m : p.M - 1)];
+        }
     }
-    __syncthreads();  // every wavefront is done reading operands from LDS
+    __syncthreads();  // every wavefront is done reading operands from LDS, and its share of the constants has landed
+    if constexpr (RIDE) {
+#pragma unroll
+        for (int e = 0; e < 2 * TM; ++e) sa[e >> 1][e & 1] = const_x[wm * WM + e * 16 + l16];
+    }
     uint8_t* stg = lds + wave * STG_BYTES;
     // the other workgroup's 16 partial sums of block (i, j) (element (i TN + j) 16 + r of its fragment, splitk.h)
     auto other_half = [&](int i, int j, float* po) {
@@ -806,10 +898,20 @@ void gemm_fp8_big_kernel(
                 const int n_safe = n < n_lim ? n : 0;
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    sgk[b][c] = p.b_scale[n_safe + c];
-                    suk[b][c] = p.b_scale[half_n + n_safe + c];
-                    bgk[b][c] = p.bias ? bf16_bits_to_f32(p.bias[n_safe + c]) : 0.f;
-                    buk[b][c] = p.bias ? bf16_bits_to_f32(p.bias[half_n + n_safe + c]) : 0.f;
+                    if constexpr (RIDE) {
+                        sgk[b][c] = const_w[n - n0 + c];
+                        suk[b][c] = const_w[BN / 2 + n - n0 + c];
+                    } else {
+                        sgk[b][c] = p.b_scale[n_safe + c];
+                        suk[b][c] = p.b_scale[half_n + n_safe + c];
+                    }
+                    if constexpr (RIDE) {
+                        bgk[b][c] = bf16_bits_to_f32(const_bias[n - n0 + c]);
+                        buk[b][c] = bf16_bits_to_f32(const_bias[BN / 2 + n - n0 + c]);
+                    } else {
+                        bgk[b][c] = p.bias ? bf16_bits_to_f32(p.bias[n_safe + c]) : 0.f;
+                        buk[b][c] = p.bias ? bf16_bits_to_f32(p.bias[half_n + n_safe + c]) : 0.f;
+                    }
                 }
             }
             float pn[16] = {};
@@ -846,8 +948,8 @@ void gemm_fp8_big_kernel(
         for (int b = 0; b < 2; ++b) {
             const int n = nbase + j * 32 + 16 * b + 4 * q;
             const int n_safe = n < n_lim ? n : 0;
-            load_cols(n_safe, sg[b], bg[b]);
-            if constexpr (GATED) load_cols(half_n + n_safe, su[b], bu[b]);
+            load_cols(n_safe, n - n0, sg[b], bg[b]);
+            if constexpr (GATED) load_cols(half_n + n_safe, BN / 2 + n - n0, su[b], bu[b]);
         }
         float pn[16] = {}, un[16] = {};
         other_half(0, j, pn);
@@ -886,17 +988,6 @@ void gemm_fp8_big_kernel(
                     o[1] = apply_act<EPI>(__uint_as_float(g01 & 0xFFFF0000u));
                     o[2] = apply_act<EPI>(__uint_as_float(g23 << 16));
                     o[3] = apply_act<EPI>(__uint_as_float(g23 & 0xFFFF0000u));
-                } else {
-                    if (p.res.residual != nullptr) {       // out = residual + bf16(linear) * gate
-                        const int m = m0 + wm * WM + row;
-                        const int n = nbase + j * 32 + 16 * b + 4 * q;
-                        if (m < p.M && n < n_lim) {
-                            const uint2 rs = *reinterpret_cast<const uint2*>(p.res.residual + (int64_t)m * p.res.ld_res + n);
-                            const uint2 gt = *reinterpret_cast<const uint2*>(
-                                p.res.gate + (int64_t)(m / p.res.gate_group) * p.res.ld_gate + n);
-                            addcmul4(o, rs, gt);
-                        }
-                    }
                 }
                 uint2 w;
                 w.x = pack_bf16x2(o[0], o[1]);
@@ -911,15 +1002,31 @@ void gemm_fp8_big_kernel(
     // and never read here: non-temporal stores keep it from evicting the operands that the
     // neighbouring tiles still want from L2 (4800 x 8192 x 2048 + GELU: 113 -> 95 us;
     // 13056 x 2560 x 2048: 76.6 -> 70.1 us; same box, alternating builds of the earlier main loop).
+    auto write_out = [&](auto residual) {
 #pragma unroll 4
-    for (int qd = 0; qd < STG_BYTES / 1024; ++qd) {
-        const int byte = qd * 1024 + lane * 16;
-        const int row = byte / ROWB, slot = (byte % ROWB) / 16;
-        const int sw = (row / ROWS_PER_PASS) & (SLOTS - 1);
-        const v4i v = *reinterpret_cast<const v4i*>(stg + row * ROWB + ((slot ^ sw) << 4));
-        const int m = m0 + wm * WM + row;
-        const int n = nbase + slot * 8;
-        if (m < p.M && n < n_lim) __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(p.out + (int64_t)m * p.ldo + n));
+        for (int qd = 0; qd < STG_BYTES / 1024; ++qd) {
+            const int byte = qd * 1024 + lane * 16;
+            const int row = byte / ROWB, slot = (byte % ROWB) / 16;
+            const int sw = (row / ROWS_PER_PASS) & (SLOTS - 1);
+            v4i v = *reinterpret_cast<const v4i*>(stg + row * ROWB + ((slot ^ sw) << 4));
+            const int m = m0 + wm * WM + row;
+            const int n = nbase + slot * 8;
+            if (m >= p.M || n >= n_lim) continue;
+            if constexpr (decltype(residual)::value) {   // out = residual + bf16(linear) * gate, row-wise like the output
+                const int grow = p.res.gate_group >= p.M ? 0 : m / p.res.gate_group;
+                const uint4 rs = *reinterpret_cast<const uint4*>(p.res.residual + (int64_t)m * p.res.ld_res + n);
+                const uint4 gt = *reinterpret_cast<const uint4*>(p.res.gate + (int64_t)grow * p.res.ld_gate + n);
+                v[0] = (int)addcmul2((uint32_t)v[0], rs.x, gt.x); v[1] = (int)addcmul2((uint32_t)v[1], rs.y, gt.y);
+                v[2] = (int)addcmul2((uint32_t)v[2], rs.z, gt.z); v[3] = (int)addcmul2((uint32_t)v[3], rs.w, gt.w);
+            }
+            __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(p.out + (int64_t)m * p.ldo + n));
+        }
+    };
+    if constexpr (EPI == EPI_NONE) {
+        if (p.res.residual != nullptr) write_out(std::true_type{});
+        else write_out(std::false_type{});
+    } else {
+        write_out(std::false_type{});
     }
     PHYAI_STAMP(5)
     PHYAI_STAMP_END(g_big_stamps, ((size_t)blockIdx.x + (size_t)gridDim.x * blockIdx.z) * 4 + wave, lane)
@@ -1127,8 +1234,8 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
             grid = dim3(8 * cols * a.m_tiles, 1, 1);
         }
     }
-#define PHYAI_BIG_ARGS a.a, a.b, a.K, a.M, a.N, a.m_tiles, a.n_tiles, a.band, a.by_rows | (a.operand_w << 4), a.k_per_split, a.a_scale, \
-                       a.b_scale, a.bias, a.out, a.ldo, a.a_scale_scalar, a.partials, a.counters, a.res
+#define PHYAI_BIG_ARGS a.a, a.b, a.K, a.M, a.N, a.m_tiles, big_order(a.band, a.by_rows, a.operand_w, a.a_scale_scalar), a.k_per_split, \
+                       a.a_scale, a.b_scale, a.bias, a.out, a.ldo, a.partials, a.counters, a.res
     if (splits > 1) {
         // (K splits: 128 x 128 tiles with a ring of four, staged or with weights in registers.  The 256 x 256 tile is
         // not built with them: its 256 accumulators leave the gather no registers, and a kernel that spills has
