@@ -49,6 +49,12 @@ int check_epilogue(int epilogue, int64_t N) {
     return 0;
 }
 
+// Bytes of a row of staged codes: padded where that changes something and the GEMMs' 32-bit offsets reach all of it.
+int64_t code_row_bytes(int64_t M, int64_t K) {
+    const int64_t padded = phyai::padded_row_bytes(K);
+    return K % 16 == 0 && M * padded < kMaxElems ? padded : K;
+}
+
 // Workspace layout of phyai_fp8_linear: [GEMM region][xq codes][x_scale].
 struct LinearCarve {
     size_t gemm_bytes, xq_off, xs_off, total;
@@ -63,7 +69,7 @@ LinearCarve make_carve(int64_t M, int64_t N, int64_t K, int epilogue) {
         c.gemm_bytes = align_up(a > b ? a : b, 256);
     }
     c.xq_off = c.gemm_bytes;
-    c.xs_off = c.xq_off + align_up((size_t)(M > 0 ? M : 0) * (size_t)(K > 0 ? K : 0), 256);
+    c.xs_off = c.xq_off + align_up((size_t)(M > 0 ? M : 0) * (size_t)(K > 0 ? code_row_bytes(M, K) : 0), 256);
     c.total = c.xs_off + align_up((size_t)(M > 0 ? M : 0) * sizeof(float), 256);
     return c;
 }
@@ -127,7 +133,7 @@ int phyai_fp8_quant_rowwise(const void* x, int64_t M, int64_t K, int64_t ldx, vo
     if (int rc = check_quant_args("phyai_fp8_quant_rowwise", x, M, K, ldx, xq)) return rc;
     if (M == 0) return PHYAI_FP8_OK;
     if (!x_scale) return fail(PHYAI_FP8_EINVAL, "phyai_fp8_quant_rowwise: null x_scale");
-    phyai::launch_quant_rowwise(x, M, K, ldx, xq, x_scale, static_cast<hipStream_t>(stream));
+    phyai::launch_quant_rowwise(x, M, K, ldx, xq, K, x_scale, static_cast<hipStream_t>(stream));
     return check_launch("phyai_fp8_quant_rowwise");
 }
 
@@ -136,7 +142,7 @@ int phyai_fp8_quant_static(const void* x, int64_t M, int64_t K, int64_t ldx,
     if (int rc = check_quant_args("phyai_fp8_quant_static", x, M, K, ldx, xq)) return rc;
     if (M == 0) return PHYAI_FP8_OK;
     if (!input_scale) return fail(PHYAI_FP8_EINVAL, "phyai_fp8_quant_static: null input_scale");
-    phyai::launch_quant_static(x, M, K, ldx, input_scale, xq, static_cast<hipStream_t>(stream));
+    phyai::launch_quant_static(x, M, K, ldx, input_scale, xq, K, static_cast<hipStream_t>(stream));
     return check_launch("phyai_fp8_quant_static");
 }
 
@@ -209,7 +215,7 @@ int check_residual(const char* fn, const ResidualSpec& r, int64_t M, int64_t N, 
 int prepare_gemm(const char* fn, const void* xq, const float* x_scale, int x_scale_is_scalar, const void* w,
                  const float* w_scale, const void* bias, const ResidualSpec& res, void* out, int64_t ldo, int64_t M,
                  int64_t N, int64_t K, int flagged_epilogue, void* workspace, size_t workspace_bytes,
-                 phyai::GemmProblem* problem, const void* x_bf16 = nullptr, int64_t ldx = 0) {
+                 phyai::GemmProblem* problem, const void* x_bf16 = nullptr, int64_t ldx = 0, int64_t ldq = 0) {
     if (M < 0 || N <= 0 || K <= 0)
         return fail(PHYAI_FP8_EINVAL, "%s: bad shape M=%lld N=%lld K=%lld", fn, (long long)M, (long long)N, (long long)K);
     const int flags = flagged_epilogue & ~PHYAI_FP8_EPILOGUE_MASK;
@@ -258,6 +264,7 @@ int prepare_gemm(const char* fn, const void* xq, const float* x_scale, int x_sca
     g.workspace = workspace;
     g.workspace_bytes = workspace_bytes;
     g.gate_group = 1;
+    g.xq_padded = ldq > K ? 1 : 0;   // (ldq: code_row_bytes, or 0 for dense rows)
     g.x_bf16 = static_cast<const uint16_t*>(x_bf16);
     g.ldx = ldx;
     if (res.residual) {
@@ -307,6 +314,7 @@ int check_norm_spec(const char* fn, const NormSpec& n, int64_t M, int64_t D) {
         return fail(PHYAI_FP8_EINVAL, "%s: M=%lld must be a non-zero multiple of the modulation rows (%lld)", fn, (long long)M, (long long)n.mod_rows);
     return 0;
 }
+int64_t code_stride(const phyai::GemmProblem& g) { return g.xq_padded ? phyai::padded_row_bytes(g.K) : g.K; }
 // What turns bf16 rows into the codes at g.xq / g.x_scale in front of the GEMM `g`, unless the kernel that serves g does
 // that itself: the quantizer, or the norm with the quantizer behind it (g.x_bf16 is then dropped: those rows are not
 // what the GEMM multiplies).
@@ -316,14 +324,14 @@ int launch_producer(const char* fn, const NormSpec* norm, phyai::GemmProblem* g,
     float* xs = const_cast<float*>(g->x_scale);
     if (norm == nullptr) {
         if (phyai::gemm_quantizes_itself(*g)) return 0;
-        phyai::launch_quant_rowwise(g->x_bf16, M, K, g->ldx, xq, xs, st);
+        phyai::launch_quant_rowwise(g->x_bf16, M, K, g->ldx, xq, code_stride(*g), xs, st);
         return check_launch(fn);
     }
     if (phyai::gemm_normalises_itself(*g)) return 0;
     phyai::NormQuantArgs a = {};
     a.x = g->x_bf16; a.ldx = g->ldx; a.D = (int)K; a.eps = norm->eps;
     a.mod = static_cast<const uint16_t*>(norm->modulation); a.ld_mod = norm->ld_mod; a.group = (int)(M / norm->mod_rows);
-    a.xq = xq; a.scale = xs;
+    a.xq = xq; a.ldq = code_stride(*g); a.scale = xs;
     g->x_bf16 = nullptr;
     g->norm_mod = nullptr;
     if (phyai::launch_norm_quant(a, M, true, st) != 0) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: no norm kernel for D=%lld", fn, (long long)K);
@@ -343,7 +351,7 @@ int run_linear_at(const char* fn, const void* x, int64_t ldx, const void* w, con
     if (int rc = check_quant_args(fn, x, M, K, ldx, xq)) return rc;
     phyai::GemmProblem g;
     if (int rc = prepare_gemm(fn, xq, xs, 0, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, gemm_ws,
-                              gemm_ws_bytes, &g, x, ldx))
+                              gemm_ws_bytes, &g, x, ldx, code_row_bytes(M, K)))
         return rc;
     // small token counts: one kernel quantizes its rows and multiplies them; otherwise two launches
     set_norm(norm, &g);
@@ -424,10 +432,10 @@ int phyai_fp8_linear_per_tensor(const void* x, int64_t ldx, const float* input_s
     if (int rc = check_quant_args(fn, x, M, K, ldx, xq)) return rc;
     const ResidualSpec res = {residual, ld_res, gate, ld_gate, gate_rows};
     phyai::GemmProblem g;
-    if (int rc = prepare_gemm(fn, xq, input_scale, 1, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, workspace, c.gemm_bytes, &g, x, ldx))
+    if (int rc = prepare_gemm(fn, xq, input_scale, 1, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, workspace, c.gemm_bytes, &g, x, ldx, code_row_bytes(M, K)))
         return rc;
     if (!phyai::gemm_quantizes_itself(g)) {
-        phyai::launch_quant_static(x, M, K, ldx, input_scale, xq, static_cast<hipStream_t>(stream));
+        phyai::launch_quant_static(x, M, K, ldx, input_scale, xq, code_stride(g), static_cast<hipStream_t>(stream));
         if (int rc = check_launch(fn)) return rc;
     }
     return launch_prepared(fn, g, stream);
@@ -496,10 +504,12 @@ int run_mlp(const char* fn, const NormSpec* norm, const void* x, int64_t ldx, co
     phyai::GemmProblem g1, g2;
     if (int rc = check_quant_args(fn, x, M, H, ldx, ws + c.first.xq_off)) return rc;
     if (int rc = prepare_gemm(fn, ws + c.first.xq_off, reinterpret_cast<float*>(ws + c.first.xs_off), 0, w1, w1_scale, bias1,
-                              ResidualSpec{}, h, I, M, n1, H, epilogue | flags1, workspace, c.first.gemm_bytes, &g1, x, ldx))
+                              ResidualSpec{}, h, I, M, n1, H, epilogue | flags1, workspace, c.first.gemm_bytes, &g1, x, ldx,
+                              code_row_bytes(M, H)))
         return rc;
     if (int rc = prepare_gemm(fn, ws + c.second.xq_off, reinterpret_cast<float*>(ws + c.second.xs_off), 0, w2, w2_scale, bias2,
-                              res, out, ldo, M, O, I, PHYAI_FP8_EPI_NONE | flags2, workspace, c.second.gemm_bytes, &g2, h, I))
+                              res, out, ldo, M, O, I, PHYAI_FP8_EPI_NONE | flags2, workspace, c.second.gemm_bytes, &g2, h, I,
+                              code_row_bytes(M, I)))
         return rc;
     set_norm(norm, &g1);
     if (norm && g1.norm_mod && !phyai::gemm_normalises_itself(g1)) g1.norm_mod = nullptr;
@@ -586,7 +596,7 @@ int phyai_fp8_linear_static(const void* x, int64_t ldx, const void* w, const flo
         if (int rc = check_launch(fn)) return rc;
     }
     if (!phyai::gemm_quantizes_itself(g)) {
-        phyai::launch_quant_rowwise(x, M, K, ldx, xq, xs, st);
+        phyai::launch_quant_rowwise(x, M, K, ldx, xq, K, xs, st);   // (dense: no shape may outgrow the array by padding)
         if (int rc = check_launch(fn)) return rc;
     }
     return launch_prepared(fn, g, stream);
@@ -622,7 +632,7 @@ int phyai_fp8_rmsnorm_quant(const void* x, int64_t ldx, const void* weight, int 
     a.weight = static_cast<const uint16_t*>(weight); a.gemma = gemma ? 1 : 0;
     a.group = 1;
     a.out = static_cast<uint16_t*>(out); a.ldo = ldo;
-    a.xq = static_cast<uint8_t*>(xq); a.scale = x_scale;
+    a.xq = static_cast<uint8_t*>(xq); a.ldq = D; a.scale = x_scale;
     if (phyai::launch_norm_quant(a, M, false, static_cast<hipStream_t>(stream)) != 0)
         return fail(PHYAI_FP8_EUNSUPPORTED, "phyai_fp8_rmsnorm_quant: no kernel for D=%lld", (long long)D);
     return check_launch("phyai_fp8_rmsnorm_quant");
@@ -645,7 +655,7 @@ int phyai_fp8_adarmsnorm_quant(const void* x, int64_t ldx, const void* modulatio
     a.mod = static_cast<const uint16_t*>(modulation); a.ld_mod = ld_mod; a.group = (int)(M / mod_rows);
     a.out = static_cast<uint16_t*>(out); a.ldo = ldo;
     a.gate = static_cast<uint16_t*>(gate_out); a.ld_gate = ld_gate;
-    a.xq = static_cast<uint8_t*>(xq); a.scale = x_scale;
+    a.xq = static_cast<uint8_t*>(xq); a.ldq = D; a.scale = x_scale;
     if (phyai::launch_norm_quant(a, M, true, static_cast<hipStream_t>(stream)) != 0)
         return fail(PHYAI_FP8_EUNSUPPORTED, "phyai_fp8_adarmsnorm_quant: no kernel for D=%lld", (long long)D);
     return check_launch("phyai_fp8_adarmsnorm_quant");

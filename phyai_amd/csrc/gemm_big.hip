@@ -117,9 +117,9 @@ struct BigArgs {
 // cut into 8 runs of equal length (within one), one per XCD: still whole or half columns per
 // XCD, and every XCD gets the same number of tiles.  Ids past an XCD's run have no tile.
 struct BigTile { int m, n; };
-// Tile order, weight layout and kind of row scale in one argument.
-static int big_order(int band, int by_rows, int operand_w, int scale_is_scalar) {
-    return band | by_rows << 8 | operand_w << 10 | scale_is_scalar << 11;
+// Tile order, weight layout, kind of row scale and of rows (GemmProblem::xq_padded) in one argument.
+static int big_order(int band, int by_rows, int operand_w, int scale_is_scalar, int padded) {
+    return band | by_rows << 8 | operand_w << 10 | scale_is_scalar << 11 | padded << 12;
 }
 __device__ __forceinline__ BigTile big_tile_of(int id, int m_tiles, int n_tiles, int band_rows) {
     const int full = n_tiles >> 3, rest = n_tiles & 7;   // whole groups of 8 tile columns; columns after them
@@ -326,13 +326,16 @@ void gemm_fp8_big_kernel(
 
     // ---- copy geometry: wavefront w moves 8-row groups w*CA .. of A and w*CB .. of B; lane i
     // fills slot i%8 of row i/8 of its group with the chunk that the swizzle assigns to it ------
+    // (padded rows of codes begin on a line and end in zeros: nothing to check in them)
+    const bool a_padded = RAGGED && ((a_order >> 12) & 1);
+    const uint32_t lda = a_padded ? ((uint32_t)p.K + 127u) & ~127u : (uint32_t)p.K;
     uint32_t aoff[CA], boff[CB > 0 ? CB : 1];
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
         const int rt = (wave * CA + i) * 8 + (lane >> 3);         // row of the tile
         int r = m0 + rt;
         r = r < p.M ? r : p.M - 1;
-        aoff[i] = (uint32_t)r * (uint32_t)p.K + (((lane & 7) ^ big_swizzle(rt)) << 4);
+        aoff[i] = (uint32_t)r * lda + (((lane & 7) ^ big_swizzle(rt)) << 4);
     }
     // first 16-row unit of the tile in an operand-order matrix (plain: 16 weight rows; gated: 8 gate
     // columns and the 8 up columns that pair with them), and the units the matrix has
@@ -372,10 +375,10 @@ void gemm_fp8_big_kernel(
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int ra = (wave * CA + e) * 8 + (lane >> 3), rb = (wave * CB + e) * 8 + (lane >> 3);
-            a_gone[e] = (((lane & 7) ^ big_swizzle(ra)) << 4) >= tail ? kCopyNothing : 0u;
+            a_gone[e] = !a_padded && (((lane & 7) ^ big_swizzle(ra)) << 4) >= tail ? kCopyNothing : 0u;
             b_gone[e] = (((lane & 7) ^ big_swizzle(rb)) << 4) >= tail ? kCopyNothing : 0u;
         }
-        a_source = copy_source(p.a, (uint32_t)p.M * (uint32_t)p.K);
+        a_source = copy_source(p.a, (uint32_t)p.M * lda);
         b_source = copy_source(p.b, (uint32_t)p.N * (uint32_t)p.K);
     }
     const int b_step_shift = (OPW || p.operand_w) ? 4 : 0;   // a K step of operand-order weights is 2 KB away, not 128 bytes
@@ -1234,7 +1237,7 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
             grid = dim3(8 * cols * a.m_tiles, 1, 1);
         }
     }
-#define PHYAI_BIG_ARGS a.a, a.b, a.K, a.M, a.N, a.m_tiles, big_order(a.band, a.by_rows, a.operand_w, a.a_scale_scalar), a.k_per_split, \
+#define PHYAI_BIG_ARGS a.a, a.b, a.K, a.M, a.N, a.m_tiles, big_order(a.band, a.by_rows, a.operand_w, a.a_scale_scalar, g.xq_padded), a.k_per_split, \
                        a.a_scale, a.b_scale, a.bias, a.out, a.ldo, a.partials, a.counters, a.res
     if (splits > 1) {
         // (K splits: 128 x 128 tiles with a ring of four, staged or with weights in registers.  The 256 x 256 tile is

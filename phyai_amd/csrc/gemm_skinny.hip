@@ -42,7 +42,7 @@
 namespace phyai {
 
 struct SkinnyArgs {
-    const uint8_t* __restrict__ xq;  // [M, K]
+    const uint8_t* __restrict__ xq;  // [M, K], rows possibly padded
     const uint8_t* __restrict__ w;   // [N, K]
     const float* __restrict__ x_scale;
     const float* __restrict__ w_scale;
@@ -54,6 +54,7 @@ struct SkinnyArgs {
     int rounds;  // K steps are consumed in rounds of SK_WAVES * KPW
     int stream_w;  // weights with non-temporal loads
     int operand_w; // weights in MFMA operand order (weight_layout.h; the gated form for gated epilogues)
+    int padded;    // GemmProblem::xq_padded
     ResidualArgs res;
 };
 
@@ -88,11 +89,11 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
     const float* __restrict__ a_w_scale, const uint16_t* __restrict__ a_bias, int a_K, int a_N, int a_m_flags,
     uint16_t* __restrict__ a_out, int64_t a_ldo, const ResidualArgs a_res) {
     // 13 preloaded dwords: everything the operand requests and the early epilogue loads need.
-    // a_m_flags = M | operand-order weights << 28 | stream_weights << 29 | x_scale_is_scalar << 30; the
-    // rounds follow from K.
+    // a_m_flags = M | padded rows of xq << 27 | operand-order weights << 28 | stream_weights << 29 | x_scale_is_scalar << 30;
+    // the rounds follow from K.
     SkinnyArgs p;
     p.xq = a_xq; p.w = a_w; p.x_scale = a_x_scale; p.w_scale = a_w_scale; p.bias = a_bias; p.out = a_out;
-    p.ldo = a_ldo; p.M = a_m_flags & 0x0FFFFFFF; p.N = a_N; p.K = a_K; p.x_scale_scalar = (a_m_flags >> 30) & 1;
+    p.ldo = a_ldo; p.M = a_m_flags & 0x07FFFFFF; p.N = a_N; p.K = a_K; p.x_scale_scalar = (a_m_flags >> 30) & 1;
     // weights read with non-temporal loads: a matrix that the caller does not want to displace
     // others from the Infinity Cache (STAGED form only; the hint is ignored otherwise)
     const bool stream_w = __builtin_amdgcn_readfirstlane((a_m_flags >> 29) & 1) != 0;
@@ -101,6 +102,9 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
     // gated epilogues the gated order is exactly the row order of a gated tile); a K step is 2 KB away
     // instead of 128 bytes, a 16-byte chunk 256 bytes instead of 16.
     const bool operand_w = __builtin_amdgcn_readfirstlane((a_m_flags >> 28) & 1) != 0;
+    // padded rows of xq begin on a 128-byte line and end in zeros
+    const bool padded = __builtin_amdgcn_readfirstlane((a_m_flags >> 27) & 1) != 0;
+    const uint32_t ldq = padded ? ((uint32_t)a_K + 127u) & ~127u : (uint32_t)a_K;
     const int w_step_shift = operand_w ? 11 : 7;
     const uint32_t w_units = (uint32_t)a_N >> 4;
     auto w_unit = [&](int nt) -> uint32_t {
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
         const int w_hi = operand_w ? 4 * (int)kOperandChunkBytes : 64;   // chunk 4 + q
         const uint8_t* xrow[MB];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) xrow[mb] = p.xq + (size_t)x_row(mb, l16) * p.K + q * 16;
+        for (int mb = 0; mb < MB; ++mb) xrow[mb] = p.xq + (size_t)x_row(mb, l16) * ldq + q * 16;
 
         for (int rnd = 0; rnd < p.rounds; ++rnd) {
             v4i wlo[KPW][NT], whi[KPW][NT], xlo[KPW][MB], xhi[KPW][MB];
@@ -280,7 +284,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
                 woff[nt][hf] = operand_w ? operand_row_offset(w_unit(nt), 0, p.K) + hf * 1024 + lane * 16
                                          : __umul24((uint32_t)w_row(nt, r16), (uint32_t)p.K) + chunk;
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) xoff[mb][hf] = __umul24((uint32_t)x_row(mb, r16), (uint32_t)p.K) + chunk;
+            for (int mb = 0; mb < MB; ++mb) xoff[mb][hf] = __umul24((uint32_t)x_row(mb, r16), ldq) + chunk;
         }
         // K not a multiple of 128: kCopyNothing for this lane's chunk in the last K step, see copy16_to_lds_checked
         const bool ragged = (p.K & 127) != 0;
@@ -304,7 +308,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
                 if (s < total_steps) {
                     const uint32_t dst = lds_wave + j * (BLOCKS * 2048);
                     if (ragged && s == total_steps - 1) {
-                        const v4i ws = copy_source(p.w, (uint32_t)p.N * (uint32_t)p.K), xs = copy_source(p.xq, (uint32_t)p.M * (uint32_t)p.K);
+                        const v4i ws = copy_source(p.w, (uint32_t)p.N * (uint32_t)p.K), xs = copy_source(p.xq, (uint32_t)p.M * ldq);
 #pragma unroll
                         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -314,7 +318,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
                         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                             for (int hf = 0; hf < 2; ++hf)
-                                copy16_to_lds_checked(xs, xoff[mb][hf] | gone[hf], (uint32_t)s << 7, dst + ((NT + mb) * 2 + hf) * 1024);
+                                copy16_to_lds_checked(xs, xoff[mb][hf] | (padded ? 0u : gone[hf]), (uint32_t)s << 7, dst + ((NT + mb) * 2 + hf) * 1024);
                         continue;
                     }
                     // one branch per K step: the weights of this call either pass the caches by or not
@@ -432,16 +436,18 @@ static int skinny_max_m() {
 
 // K that is not a multiple of 128 (staged form only): from three K steps on (ten with more than 64 rows and few
 // columns), the generic kernel's K splits cost it a round trip through memory (184 x 896 x 2256: 31.3 -> 9.1 us, 353 x
-// 384 x 3216: 35.9 -> 9.0 us).
-static bool skinny_takes_ragged(int M, int N, int K) {
+// 384 x 3216: 35.9 -> 9.0 us).  With padded codes from three K steps on throughout, quantizer included: 200 x 512 x 1040
+// 22.6 -> 5.6 us, 560 x 656 x 1168 29.4 -> 7.5, 500 x 640 x 784 + GeGLU 17.9 -> 6.4, 900 x 272 x 720 21.0 -> 6.6 (dense codes of
+// such shapes still go to the generic kernel).
+static bool skinny_takes_ragged(int M, int N, int K, bool padded) {
     static const bool staged = []() { const char* e = tuning_env("PHYAI_FP8_SKINNY_STAGED"); return !(e && atoi(e) == 0); }();
     if (!staged || (int64_t)K * (N > M ? N : M) >= ((int64_t)1 << 31) || K >= (1 << 24)) return false;
-    return K > 256 && (M <= 64 || N >= 1024 || K >= 1280);
+    return K > 256 && (padded || M <= 64 || N >= 1024 || K >= 1280);
 }
 
-bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo) {
+bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo, bool padded) {
     if (M > skinny_max_m() || ldo % 4 != 0) return false;
-    if (K % 128 != 0 && !skinny_takes_ragged(M, N, K)) return false;
+    if (K % 128 != 0 && !skinny_takes_ragged(M, N, K, padded)) return false;
     if (epi_is_gated(epilogue)) return (N / 2) % 8 == 0;
     return N % 8 == 0;
 }
@@ -506,13 +512,13 @@ static void sk_launch_one(const SkinnyArgs& a, const dim3& grid, hipStream_t st)
     if constexpr (fits) {
         if (want && a.K * (int64_t)(a.N > a.M ? a.N : a.M) < ((int64_t)1 << 32) && a.K < (1 << 24) && a.N < (1 << 24)) {
             hipLaunchKernelGGL((gemm_fp8_skinny_kernel<MB, NT, KPW, EPI, true>), grid, dim3(SK_THREADS), 0, st,
-                               a.w, a.xq, a.x_scale, a.w_scale, a.bias, a.K, a.N, a.M | (a.x_scale_scalar ? 1 << 30 : 0) | (a.stream_w ? 1 << 29 : 0) | (a.operand_w ? 1 << 28 : 0),
+                               a.w, a.xq, a.x_scale, a.w_scale, a.bias, a.K, a.N, a.M | (a.x_scale_scalar ? 1 << 30 : 0) | (a.stream_w ? 1 << 29 : 0) | (a.operand_w ? 1 << 28 : 0) | (a.padded ? 1 << 27 : 0),
                                a.out, a.ldo, a.res);
             return;
         }
     }
     hipLaunchKernelGGL((gemm_fp8_skinny_kernel<MB, NT, KPW, EPI, false>), grid, dim3(SK_THREADS), 0, st,
-                       a.w, a.xq, a.x_scale, a.w_scale, a.bias, a.K, a.N, a.M | (a.x_scale_scalar ? 1 << 30 : 0) | (a.stream_w ? 1 << 29 : 0) | (a.operand_w ? 1 << 28 : 0),
+                       a.w, a.xq, a.x_scale, a.w_scale, a.bias, a.K, a.N, a.M | (a.x_scale_scalar ? 1 << 30 : 0) | (a.stream_w ? 1 << 29 : 0) | (a.operand_w ? 1 << 28 : 0) | (a.padded ? 1 << 27 : 0),
                        a.out, a.ldo, a.res);
 }
 
@@ -557,6 +563,7 @@ int launch_gemm_skinny(const GemmProblem& g, const SkinnyPlan& pl, hipStream_t s
     a.rounds = pl.rounds;
     a.stream_w = g.stream_weights;
     a.operand_w = g.weight_layout != W_ROW_MAJOR;
+    a.padded = g.xq_padded;
     a.res = residual_of(g);
     switch (g.epilogue) {
     case EPI_NONE: return sk_launch_epi<EPI_NONE>(a, pl, st);

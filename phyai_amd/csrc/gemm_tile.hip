@@ -47,6 +47,7 @@ struct TileArgs {
     int* __restrict__ counters;
     int64_t ldo;
     int M, N, K;
+    int lda;                // bytes from one row of a to the next: K, or K padded
     int a_scale_scalar;
     int k_tiles_per_split;  // in BK slabs
     int operand_w;          // weights in MFMA operand order (weight_layout.h; needs K % 128 == 0)
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_tile_kernel(const TileArgs p) {
     for (int i = 0; i < PA; ++i) {
         int r = m0 + i * 32 + lrow;
         r = r < p.M ? r : p.M - 1;
-        a_off[i] = r * p.K;
+        a_off[i] = r * p.lda;
     }
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
@@ -387,9 +388,9 @@ struct GemmChoice {
 // tile kernel's epilogue needs.
 // have_x: the bf16 activations are at hand (whole-linear entry points), so a kernel that quantizes
 // its own rows may serve the call (one_scale: with one static scale for all of them; amax_parts > 0: with
-// row maxima in that many slots per row): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
+// row maxima in that many slots per row; padded: GemmProblem::xq_padded where the codes are staged): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
 static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
-                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false) {
+                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false, bool padded = false) {
     GemmChoice c = {};
     if (norm) {   // rows still to be normalised: one kernel does it or the caller launches the norm itself
         c.kind = GemmChoice::FUSED;
@@ -418,7 +419,7 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
             if (selfq(SELFQ_FROM_ROWS)) return c;
         }
     }
-    const bool skinny_ok = vec_ok && skinny_applicable(M, N, K, epilogue, ldo);
+    const bool skinny_ok = vec_ok && skinny_applicable(M, N, K, epilogue, ldo, padded);
     auto small = [&]() {
         c.kind = GemmChoice::SKINNY;
         c.sk = skinny_plan(M, N, K, epilogue);
@@ -472,10 +473,10 @@ static const GemmChoice& choose_gemm(const GemmProblem& g) {
     const int parts = maxima ? g.amax_parts : 0;
     const bool norm = g.norm_mod != nullptr, one_scale = g.x_scale_is_scalar != 0;
     const int64_t how = (int64_t)g.epilogue | (int64_t)vec_ok << 8 | (int64_t)out16 << 9 | (int64_t)have_x << 10 | (int64_t)norm << 11 |
-                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)parts << 16;
+                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)(g.xq_padded != 0) << 15 | (int64_t)parts << 16;
     static thread_local CallMemo<GemmChoice, 128> memo;
     return memo.get((int64_t)g.M | how << 32, g.N, g.K, g.ldo, [&]() {
-        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale);
+        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.xq_padded != 0);
     });
 }
 
@@ -506,10 +507,10 @@ size_t gemm_scratch_need(const GemmProblem& g) {
     return choose_gemm(g).need;
 }
 
-int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout) {
+int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout, bool padded) {
     // operands that satisfy every alignment requirement, dense output
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout);
+    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, padded);
     switch (c.kind) {
     case GemmChoice::SKINNY:
         return snprintf(buf, n, "small-m nt=%d mb=%d kpw=%d rounds=%d", c.sk.nt, c.sk.mb, c.sk.kpw, c.sk.rounds);
@@ -526,14 +527,15 @@ int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, i
 
 int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout) {
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout);
+    const bool padded = K % 128 != 0;   // (as the linears stage their codes)
+    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, padded);
     if (c.kind == GemmChoice::FUSED)
         return snprintf(buf, n, "one launch: small-m rows=%d nt=%d kpw=%d grid=%dx%d", c.fq.rows, c.fq.nt, c.fq.kpw, c.fq.tiles, c.fq.msplit);
     if (c.kind == GemmChoice::SELFQ)
         return snprintf(buf, n, "one launch: rows in registers, rows=%d nt=%d steps=%d grid=%dx%d", 4 * c.sq.rg, c.sq.nt, c.sq.steps, c.sq.tiles, c.sq.msplit);
     const int len = snprintf(buf, n, "quantizer + ");
     if (len < 0 || (size_t)len >= n) return len;
-    return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout);
+    return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout, padded);
 }
 
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order) {
@@ -585,6 +587,7 @@ int launch_gemm(const GemmProblem& g, hipStream_t st) {
     TileArgs a;
     a.a = g.xq; a.b = g.w; a.a_scale = g.x_scale; a.b_scale = g.w_scale; a.bias = g.bias;
     a.out = g.out; a.ldo = g.ldo; a.M = g.M; a.N = g.N; a.K = g.K;
+    a.lda = g.xq_padded ? (int)padded_row_bytes(g.K) : g.K;
     a.a_scale_scalar = g.x_scale_is_scalar;
     a.res = residual_of(g);
     a.operand_w = g.weight_layout != W_ROW_MAJOR;

@@ -7,12 +7,13 @@
 
 namespace phyai {
 
-int launch_quant_rowwise(const void* x, int64_t M, int64_t K, int64_t ldx, void* xq, float* xs,
+// The quantizers' codes have rows of ldq >= K bytes (a multiple of 8, at most K rounded up to 128); bytes K .. ldq are zeros.
+int launch_quant_rowwise(const void* x, int64_t M, int64_t K, int64_t ldx, void* xq, int64_t ldq, float* xs,
                          hipStream_t st);
 int launch_weight_quant(const void* w, int64_t N, int64_t K, int64_t ldw, void* wq, float* ws,
                         hipStream_t st);
 int launch_quant_static(const void* x, int64_t M, int64_t K, int64_t ldx, const float* input_scale,
-                        void* xq, hipStream_t st);
+                        void* xq, int64_t ldq, hipStream_t st);
 int launch_debug_cast(const float* v, int64_t n, void* codes, hipStream_t st);
 // Row-major fp8 weights -> MFMA operand order (weight_layout.hip); gated: the fused gate | up form.
 int launch_weight_to_operand_order(const void* w, int64_t N, int64_t K, int gated, void* out, hipStream_t st);
@@ -37,12 +38,19 @@ struct NormQuantArgs {
     uint16_t* gate;           // adaptive: [M / group, D] bf16 or null
     int64_t ld_gate;
     uint8_t* xq;              // [M, D] codes or null
+    int64_t ldq;              //        row stride in bytes, as above
     float* scale;             // [M]
 };
 int launch_norm_quant(const NormQuantArgs& a, int64_t M, bool adaptive, hipStream_t st);  // -2: D too large
 
+// Codes that a quantizer of this library hands to a GEMM of this library begin every row on a 128-byte line: a K that is no
+// multiple of 128 is rounded up and the rest of the row is zeros.  Dense rows of such a K straddle two lines per request
+// and their last K step has to be read chunk by chunk (us, dense / padded codes: 777 x 4304 x 1168 + GELU 11.7 / 11.0,
+// 3264 x 8192 x 1040 41.8 / 38.3, 6528 x 4096 x 4112 133 / 118).
+inline int64_t padded_row_bytes(int64_t K) { return (K + 127) & ~(int64_t)127; }
+
 struct GemmProblem {
-    const uint8_t* xq;      // [M, K]
+    const uint8_t* xq;      // [M, K], or [M, padded_row_bytes(K)] with zeros behind K (xq_padded)
     const float* x_scale;   // [M] or [1]
     int x_scale_is_scalar;
     const uint8_t* w;       // [N, K]
@@ -51,6 +59,7 @@ struct GemmProblem {
     uint16_t* out;          // [M, N_out] bf16
     int64_t ldo;
     int M, N, K;
+    int xq_padded;          // K is no multiple of 128 and xq's rows are padded
     int epilogue;
     void* workspace;        // header (counters) + split-K partials
     size_t workspace_bytes;
@@ -129,7 +138,7 @@ struct SkinnyPlan {
     int kpw;     // K steps per wavefront per round
     int rounds;
 };
-bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo);
+bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo, bool padded = false);
 SkinnyPlan skinny_plan(int M, int N, int K, int epilogue);
 int launch_gemm_skinny(const GemmProblem& p, const SkinnyPlan& pl, hipStream_t st);
 
@@ -186,6 +195,6 @@ int launch_set_stamp_sink_fused(unsigned long long* buf, unsigned int records);
 // Text form of what phyai_fp8_mlp launches for aligned, row-major operands.
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order = false);
 // Text form of launch_gemm's choice for aligned operands and a dense output; returns its length.
-int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0);
+int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0, bool padded = false);
 
 }  // namespace phyai

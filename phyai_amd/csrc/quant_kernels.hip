@@ -39,7 +39,7 @@ __device__ __forceinline__ uint4 nt_load16(const uint16_t* p) {
 
 template <int THREADS, int CHUNKS, int MODE, bool STREAM_IN>
 __global__ __launch_bounds__(THREADS) void quant_rows_reg_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, int K, uint8_t* __restrict__ xq,
+    const uint16_t* __restrict__ x, int64_t ldx, int K, int ldq, uint8_t* __restrict__ xq,
     float* __restrict__ scale) {
     __shared__ uint32_t smem[THREADS / kWave];
     const int64_t row = blockIdx.x;
@@ -57,11 +57,12 @@ __global__ __launch_bounds__(THREADS) void quant_rows_reg_kernel(
     const float s = scale_from_amax_bits<MODE>(m);
     if (threadIdx.x == 0) scale[row] = s;
     const RowDivisor d = make_divisor<MODE>(s);
-    uint8_t* qr = xq + row * (int64_t)K;
+    uint8_t* qr = xq + row * (int64_t)ldq;
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         const int k = (c * THREADS + threadIdx.x) * 8;
         if (k < K) *reinterpret_cast<uint2*>(qr + k) = encode8<MODE>(v[c], d);
+        else if (k < ldq) *reinterpret_cast<uint2*>(qr + k) = make_uint2(0, 0);
     }
 }
 
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(THREADS) void quant_rows_reg_kernel(
 // (the second one hits L2).
 template <int MODE>
 __global__ __launch_bounds__(256) void quant_rows_loop_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, int K, uint8_t* __restrict__ xq,
+    const uint16_t* __restrict__ x, int64_t ldx, int K, int ldq, uint8_t* __restrict__ xq,
     float* __restrict__ scale) {
     __shared__ uint32_t smem[256 / kWave];
     const int64_t row = blockIdx.x;
@@ -81,20 +82,20 @@ __global__ __launch_bounds__(256) void quant_rows_loop_kernel(
     const float s = scale_from_amax_bits<MODE>(m);
     if (threadIdx.x == 0) scale[row] = s;
     const RowDivisor d = make_divisor<MODE>(s);
-    uint8_t* qr = xq + row * (int64_t)K;
-    for (int k = threadIdx.x * 8; k < K; k += 256 * 8)
-        *reinterpret_cast<uint2*>(qr + k) = encode8<MODE>(*reinterpret_cast<const uint4*>(xr + k), d);
+    uint8_t* qr = xq + row * (int64_t)ldq;
+    for (int k = threadIdx.x * 8; k < ldq; k += 256 * 8)
+        *reinterpret_cast<uint2*>(qr + k) = k < K ? encode8<MODE>(*reinterpret_cast<const uint4*>(xr + k), d) : make_uint2(0, 0);
 }
 
 // Static per-tensor quantizer: clamp(fp32(x)/s, +-448) -> e4m3fn, NaN elements to NaN codes as torch.clamp lets them
 // through.  Bound by its bytes: a wavefront takes 2048 elements of one row, four loads in flight per lane and no index
 // division (one per 8 elements took as long as the bytes: the linear 10143 x 512 x 2944 41.7 -> 34.5 us with both).
 __global__ __launch_bounds__(256) void quant_static_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, int M, int K, const float* __restrict__ input_scale, uint8_t* __restrict__ xq) {
+    const uint16_t* __restrict__ x, int64_t ldx, int M, int K, int ldq, const float* __restrict__ input_scale, uint8_t* __restrict__ xq) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= M) return;
     const uint16_t* xr = x + row * ldx;
-    uint8_t* qr = xq + row * (int64_t)K;
+    uint8_t* qr = xq + row * (int64_t)ldq;
     const StaticDivisor d = make_static_divisor(*input_scale);
     uint4 v[4];
 #pragma unroll
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(256) void quant_static_kernel(
         if (k < K)
             *reinterpret_cast<uint2*>(qr + k) =
                 __builtin_expect(!d.fast || any_nan_or_inf(v[c]), 0) ? encode8_static_exact(v[c], d.s) : encode8_static_fast(v[c], d);
+        else if (k < ldq) *reinterpret_cast<uint2*>(qr + k) = make_uint2(0, 0);
     }
 }
 
@@ -118,7 +120,7 @@ __global__ __launch_bounds__(256) void debug_cast_kernel(const float* __restrict
 }
 
 template <int MODE>
-static int launch_quant_rows(const void* x, int64_t M, int64_t K, int64_t ld, void* xq,
+static int launch_quant_rows(const void* x, int64_t M, int64_t K, int64_t ld, void* xq, int64_t ldq,
                              float* scale, hipStream_t st) {
     if (M == 0) return 0;
     const uint16_t* xp = static_cast<const uint16_t*>(x);
@@ -129,9 +131,9 @@ static int launch_quant_rows(const void* x, int64_t M, int64_t K, int64_t ld, vo
 #define PHYAI_QL(T, C)                                                                                             \
     do {                                                                                                           \
         if (C >= 4 && stream_in)                                                                                   \
-            hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, (C >= 4)>), grid, dim3(T), 0, st, xp, ld, k, qp, scale); \
+            hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, (C >= 4)>), grid, dim3(T), 0, st, xp, ld, k, (int)ldq, qp, scale); \
         else                                                                                                       \
-            hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, false>), grid, dim3(T), 0, st, xp, ld, k, qp, scale);   \
+            hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, false>), grid, dim3(T), 0, st, xp, ld, k, (int)ldq, qp, scale);   \
     } while (0)
     if (K <= 512) PHYAI_QL(64, 1);
     else if (K <= 1024) PHYAI_QL(128, 1);
@@ -140,18 +142,18 @@ static int launch_quant_rows(const void* x, int64_t M, int64_t K, int64_t ld, vo
     else if (K <= 8192) PHYAI_QL(256, 4);
     else if (K <= 16384) PHYAI_QL(256, 8);
     else if (K <= 32768) PHYAI_QL(256, 16);
-    else hipLaunchKernelGGL((quant_rows_loop_kernel<MODE>), grid, dim3(256), 0, st, xp, ld, k, qp, scale);
+    else hipLaunchKernelGGL((quant_rows_loop_kernel<MODE>), grid, dim3(256), 0, st, xp, ld, k, (int)ldq, qp, scale);
 #undef PHYAI_QL
     return 0;
 }
 
-int launch_quant_rowwise(const void* x, int64_t M, int64_t K, int64_t ldx, void* xq, float* xs,
+int launch_quant_rowwise(const void* x, int64_t M, int64_t K, int64_t ldx, void* xq, int64_t ldq, float* xs,
                          hipStream_t st) {
-    return launch_quant_rows<QUANT_ACT_DYNAMIC>(x, M, K, ldx, xq, xs, st);
+    return launch_quant_rows<QUANT_ACT_DYNAMIC>(x, M, K, ldx, xq, ldq, xs, st);
 }
 int launch_weight_quant(const void* w, int64_t N, int64_t K, int64_t ldw, void* wq, float* ws,
                         hipStream_t st) {
-    return launch_quant_rows<QUANT_WEIGHT>(w, N, K, ldw, wq, ws, st);
+    return launch_quant_rows<QUANT_WEIGHT>(w, N, K, ldw, wq, K, ws, st);
 }
 // ---- RMSNorm / adaptive RMSNorm + quantizer ----------------------------------------------
 template <int THREADS>
@@ -187,12 +189,12 @@ __global__ __launch_bounds__(THREADS) void norm_quant_kernel(
     const uint16_t* __restrict__ a_x, int64_t a_ldx, int a_D, int a_group, const uint16_t* __restrict__ a_mod,
     int64_t a_ld_mod, const uint16_t* __restrict__ a_weight, float a_eps, int a_gemma, uint8_t* __restrict__ a_xq,
     float* __restrict__ a_scale, uint16_t* __restrict__ a_out, int64_t a_ldo, uint16_t* __restrict__ a_gate,
-    int64_t a_ld_gate) {
+    int64_t a_ld_gate, int64_t a_ldq) {
     // scalar arguments in the order the kernel needs them (the first 16 dwords are preloaded)
     NormQuantArgs p;
     p.x = a_x; p.ldx = a_ldx; p.D = a_D; p.eps = a_eps; p.weight = a_weight; p.gemma = a_gemma; p.mod = a_mod;
     p.ld_mod = a_ld_mod; p.group = a_group; p.out = a_out; p.ldo = a_ldo; p.gate = a_gate; p.ld_gate = a_ld_gate;
-    p.xq = a_xq; p.scale = a_scale;
+    p.xq = a_xq; p.ldq = a_ldq; p.scale = a_scale;
     __shared__ float ssum[THREADS / kWave];
     __shared__ uint32_t smax[THREADS / kWave];
     const int64_t row = blockIdx.x;
@@ -249,11 +251,12 @@ __global__ __launch_bounds__(THREADS) void norm_quant_kernel(
     const float s = scale_from_amax_bits<QUANT_ACT_DYNAMIC>(m);
     if (threadIdx.x == 0) p.scale[row] = s;
     const RowDivisor d = make_divisor<QUANT_ACT_DYNAMIC>(s);
-    uint8_t* qr = p.xq + row * (int64_t)p.D;
+    uint8_t* qr = p.xq + row * p.ldq;
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         const int k = (c * THREADS + threadIdx.x) * 8;
         if (k < p.D) *reinterpret_cast<uint2*>(qr + k) = encode8<QUANT_ACT_DYNAMIC>(ob[c], d);
+        else if (k < p.ldq) *reinterpret_cast<uint2*>(qr + k) = make_uint2(0, 0);
     }
 }
 
@@ -264,12 +267,12 @@ __global__ __launch_bounds__(256) void norm_quant_loop_kernel(
     const uint16_t* __restrict__ a_x, int64_t a_ldx, int a_D, int a_group, const uint16_t* __restrict__ a_mod,
     int64_t a_ld_mod, const uint16_t* __restrict__ a_weight, float a_eps, int a_gemma, uint8_t* __restrict__ a_xq,
     float* __restrict__ a_scale, uint16_t* __restrict__ a_out, int64_t a_ldo, uint16_t* __restrict__ a_gate,
-    int64_t a_ld_gate) {
+    int64_t a_ld_gate, int64_t a_ldq) {
     // scalar arguments in the order the kernel needs them (the first 16 dwords are preloaded)
     NormQuantArgs p;
     p.x = a_x; p.ldx = a_ldx; p.D = a_D; p.eps = a_eps; p.weight = a_weight; p.gemma = a_gemma; p.mod = a_mod;
     p.ld_mod = a_ld_mod; p.group = a_group; p.out = a_out; p.ldo = a_ldo; p.gate = a_gate; p.ld_gate = a_ld_gate;
-    p.xq = a_xq; p.scale = a_scale;
+    p.xq = a_xq; p.ldq = a_ldq; p.scale = a_scale;
     __shared__ float ssum[256 / kWave];
     __shared__ uint32_t smax[256 / kWave];
     const int64_t row = blockIdx.x;
@@ -322,15 +325,15 @@ __global__ __launch_bounds__(256) void norm_quant_loop_kernel(
     const float s = scale_from_amax_bits<QUANT_ACT_DYNAMIC>(m);
     if (threadIdx.x == 0) p.scale[row] = s;
     const RowDivisor d = make_divisor<QUANT_ACT_DYNAMIC>(s);
-    uint8_t* qr = p.xq + row * (int64_t)p.D;
-    for (int k = threadIdx.x * 8; k < p.D; k += 256 * 8)
-        *reinterpret_cast<uint2*>(qr + k) = encode8<QUANT_ACT_DYNAMIC>(result8(k), d);
+    uint8_t* qr = p.xq + row * p.ldq;
+    for (int k = threadIdx.x * 8; k < p.ldq; k += 256 * 8)
+        *reinterpret_cast<uint2*>(qr + k) = k < p.D ? encode8<QUANT_ACT_DYNAMIC>(result8(k), d) : make_uint2(0, 0);
 }
 
 template <bool ADAPTIVE>
 static int launch_norm_quant_t(const NormQuantArgs& a, int64_t M, hipStream_t st) {
     const dim3 grid((unsigned)M);
-#define PHYAI_NQ_ARGS a.x, a.ldx, a.D, a.group, a.mod, a.ld_mod, a.weight, a.eps, a.gemma, a.xq, a.scale, a.out, a.ldo, a.gate, a.ld_gate
+#define PHYAI_NQ_ARGS a.x, a.ldx, a.D, a.group, a.mod, a.ld_mod, a.weight, a.eps, a.gemma, a.xq, a.scale, a.out, a.ldo, a.gate, a.ld_gate, a.ldq
 #define PHYAI_NQ(T, C) hipLaunchKernelGGL((norm_quant_kernel<T, C, ADAPTIVE>), grid, dim3(T), 0, st, PHYAI_NQ_ARGS)
     if (a.D <= 512) PHYAI_NQ(64, 1);
     else if (a.D <= 1024) PHYAI_NQ(128, 1);
@@ -349,11 +352,11 @@ int launch_norm_quant(const NormQuantArgs& a, int64_t M, bool adaptive, hipStrea
 }
 
 int launch_quant_static(const void* x, int64_t M, int64_t K, int64_t ldx, const float* input_scale,
-                        void* xq, hipStream_t st) {
+                        void* xq, int64_t ldq, hipStream_t st) {
     if (M == 0) return 0;
     // (M < 2^31; the grid's x covers the rows)
     hipLaunchKernelGGL(quant_static_kernel, dim3((unsigned)((M + 3) / 4), (unsigned)((K + 2047) / 2048)), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(x), ldx, (int)M, (int)K, input_scale, static_cast<uint8_t*>(xq));
+                       static_cast<const uint16_t*>(x), ldx, (int)M, (int)K, (int)ldq, input_scale, static_cast<uint8_t*>(xq));
     return 0;
 }
 int launch_debug_cast(const float* v, int64_t n, void* codes, hipStream_t st) {
