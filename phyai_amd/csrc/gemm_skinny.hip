@@ -19,7 +19,10 @@
 //    together with the scales and bias the epilogue will want - and only then starts to
 //    compute.  The operands go global -> LDS (the wavefront's own slice, see STAGED below) ->
 //    VGPRs in MFMA operand layout; nobody else reads that slice, so there is no barrier
-//    between the loads and the math.
+//    between the loads and the math.  K beyond what the slices hold comes in rounds; the next round is asked for
+//    when a round's operands are in registers, before they are multiplied (1 - 4 % of a GEMM on ready codes in two rounds
+//    and more, us: 800 x 1024 x 4096 9.2 -> 8.9, 300 x 2048 x 2048 6.0 -> 5.8, 777 x 1168 x 4304 15.4 -> 15.0; behind a quantizer,
+//    whose codes come from other XCDs, level to 2 %).
 //  * v_mfma_f32_16x16x128_f8f6f4: lane l supplies operand row (l % 16) and 32 of
 //    the 128 K bytes of a step.  Which 32 is free as long as both operands agree;
 //    lane group q = l / 16 takes bytes [16q, 16q+16) and [64+16q, 64+16q+16), so
@@ -299,9 +302,8 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
         // a staged unit in operand order: chunk q of row l16 at (16 q + l16) * 16 = 16 * lane, chunk 4 + q 1 KB on
         const int wrd_lo = operand_w ? lane * 16 : rd_lo, wrd_hi = operand_w ? 1024 + lane * 16 : rd_hi;
 
-        for (int rnd = 0; rnd < p.rounds; ++rnd) {
-            if (rnd > 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // last round's reads have landed
-            // ---- 1. request every byte of this round ------------------------------------
+        // every byte of round rnd
+        auto request = [&](int rnd) {
 #pragma unroll
             for (int j = 0; j < KPW; ++j) {
                 const int s = __builtin_amdgcn_readfirstlane((rnd * KPW + j) * SK_WAVES + wave);
@@ -342,28 +344,39 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_fp8_skinny_kernel(
                             copy16_to_lds(p.xq + ((size_t)s << 7), xoff[mb][hf], dst + ((NT + mb) * 2 + hf) * 1024);
                 }
             }
-            if (rnd == 0) request_residual();
+        };
+        request(0);
+        request_residual();
+        for (int rnd = 0; rnd < p.rounds; ++rnd) {
+            if (__builtin_amdgcn_readfirstlane(rnd * KPW * SK_WAVES + wave) >= total_steps) break;   // no step left for this wavefront
             wait_copies<0>();   // everything this wavefront asked for (epilogue operands included)
-            // ---- 2. MFMA ---------------------------------------------------------------------
+            // The round's operands into registers; then the slots are free, and the next round is asked for before this one
+            // is multiplied: its trip to memory runs under the MFMAs instead of behind them.
+            v8i xb[KPW][MB], wb[KPW][NT];
+#pragma unroll
+            for (int j = 0; j < KPW; ++j) {
+                const uint8_t* blk = my_stage + j * (BLOCKS * 2048);
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    xb[j][mb] = join(*reinterpret_cast<const v4i*>(blk + (NT + mb) * 2048 + rd_lo),
+                                     *reinterpret_cast<const v4i*>(blk + (NT + mb) * 2048 + rd_hi));
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    wb[j][nt] = join(*reinterpret_cast<const v4i*>(blk + nt * 2048 + wrd_lo),
+                                     *reinterpret_cast<const v4i*>(blk + nt * 2048 + wrd_hi));
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (rnd + 1 < p.rounds) request(rnd + 1);
 #pragma unroll
             for (int j = 0; j < KPW; ++j) {
                 const int s = __builtin_amdgcn_readfirstlane((rnd * KPW + j) * SK_WAVES + wave);
                 if (s < total_steps) {
-                    const uint8_t* blk = my_stage + j * (BLOCKS * 2048);
-                    v8i xb[MB];
 #pragma unroll
-                    for (int mb = 0; mb < MB; ++mb)
-                        xb[mb] = join(*reinterpret_cast<const v4i*>(blk + (NT + mb) * 2048 + rd_lo),
-                                      *reinterpret_cast<const v4i*>(blk + (NT + mb) * 2048 + rd_hi));
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-                        const v8i a = join(*reinterpret_cast<const v4i*>(blk + nt * 2048 + wrd_lo),
-                                           *reinterpret_cast<const v4i*>(blk + nt * 2048 + wrd_hi));
+                    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                         for (int mb = 0; mb < MB; ++mb)
                             acc[nt][mb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                                a, xb[mb], acc[nt][mb], 0, 0, 0, 0, 0, 0);
-                    }
+                                wb[j][nt], xb[j][mb], acc[nt][mb], 0, 0, 0, 0, 0, 0);
                 }
             }
         }
