@@ -62,7 +62,7 @@ __global__ __launch_bounds__(THREADS) void quant_rows_reg_kernel(
     for (int c = 0; c < CHUNKS; ++c) {
         const int k = (c * THREADS + threadIdx.x) * 8;
         if (k < K) *reinterpret_cast<uint2*>(qr + k) = encode8<MODE>(v[c], d);
-        else if (k < ldq) *reinterpret_cast<uint2*>(qr + k) = make_uint2(0, 0);
+        else if (MODE != QUANT_WEIGHT && k < ldq) *reinterpret_cast<uint2*>(qr + k) = make_uint2(0, 0);   // (weights have no padding)
     }
 }
 
