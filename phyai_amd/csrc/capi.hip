@@ -265,6 +265,7 @@ int prepare_gemm(const char* fn, const void* xq, const float* x_scale, int x_sca
     g.workspace_bytes = workspace_bytes;
     g.gate_group = 1;
     g.xq_padded = ldq > K ? 1 : 0;   // (ldq: code_row_bytes, or 0 for dense rows)
+    g.staged = x_bf16 != nullptr ? 1 : 0;
     g.x_bf16 = static_cast<const uint16_t*>(x_bf16);
     g.ldx = ldx;
     if (res.residual) {
@@ -566,20 +567,32 @@ int phyai_fp8_linear_static(const void* x, int64_t ldx, const void* w, const flo
     // The GEMM gets whatever the staging at the tail leaves; its need depends on the kernel that
     // serves exactly this call and is checked before anything is launched.
     if (M >= kMaxElems || K >= kMaxElems) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: tensor too large", fn);
-    const size_t xs_bytes = align_up((size_t)M * sizeof(float), 256), xq_bytes = align_up((size_t)M * (size_t)K, 256);
+    const size_t xs_bytes = align_up((size_t)M * sizeof(float), 256), dense_bytes = align_up((size_t)M * (size_t)K, 256);
+    // (padded rows like phyai_fp8_linear's, unless the array is too small for those; below)
+    int64_t ldq = code_row_bytes(M, K);
+    size_t xq_bytes = align_up((size_t)M * (size_t)ldq, 256);
+    if (xs_bytes + xq_bytes + PHYAI_FP8_WORKSPACE_HEADER_BYTES > kScratch) { ldq = K; xq_bytes = dense_bytes; }
     if (xs_bytes + xq_bytes + PHYAI_FP8_WORKSPACE_HEADER_BYTES > kScratch)
         return fail(PHYAI_FP8_EWORKSPACE, "%s: the activation codes of this shape need %zu bytes, the static array holds %zu; "
                     "use phyai_fp8_linear with a caller-owned workspace", fn, xs_bytes + xq_bytes, kScratch);
     void* base = nullptr;
     if (int rc = static_scratch_of(&base)) return rc;
     uint8_t* ws = static_cast<uint8_t*>(base);
-    const size_t xq_off = kScratch - xs_bytes - xq_bytes, gemm_bytes = xq_off;
-    void* xq = ws + xq_off;
-    float* xs = reinterpret_cast<float*>(ws + xq_off + xq_bytes);
-    if (int rc = check_quant_args(fn, x, M, K, ldx, xq)) return rc;
+    void* xq = nullptr;
+    float* xs = nullptr;
     phyai::GemmProblem g;
-    if (int rc = prepare_gemm(fn, xq, xs, 0, w, w_scale, bias, ResidualSpec{}, out, ldo, M, N, K, epilogue, ws,
-                              gemm_bytes, &g, x, ldx)) {
+    for (;;) {
+        const size_t xq_off = kScratch - xs_bytes - xq_bytes;
+        xq = ws + xq_off;
+        xs = reinterpret_cast<float*>(ws + xq_off + xq_bytes);
+        if (int rc = check_quant_args(fn, x, M, K, ldx, xq)) return rc;
+        const int rc = prepare_gemm(fn, xq, xs, 0, w, w_scale, bias, ResidualSpec{}, out, ldo, M, N, K, epilogue, ws, xq_off, &g, x, ldx, ldq);
+        if (rc == 0) break;
+        if (rc == PHYAI_FP8_EWORKSPACE && ldq > K) {
+            ldq = K;
+            xq_bytes = dense_bytes;
+            continue;
+        }
         if (rc == PHYAI_FP8_EWORKSPACE)
             return fail(rc, "%s: this shape needs more scratch than the static array holds (%zu bytes, %zu of them for "
                         "activation codes); use phyai_fp8_linear with a caller-owned workspace", fn, kScratch, xs_bytes + xq_bytes);
@@ -596,7 +609,7 @@ int phyai_fp8_linear_static(const void* x, int64_t ldx, const void* w, const flo
         if (int rc = check_launch(fn)) return rc;
     }
     if (!phyai::gemm_quantizes_itself(g)) {
-        phyai::launch_quant_rowwise(x, M, K, ldx, xq, K, xs, st);   // (dense: no shape may outgrow the array by padding)
+        phyai::launch_quant_rowwise(x, M, K, ldx, xq, ldq, xs, st);
         if (int rc = check_launch(fn)) return rc;
     }
     return launch_prepared(fn, g, stream);

@@ -1052,6 +1052,41 @@ static double big_fill(int tiles, int slots) {
     return rounds > 0 ? (double)tiles / ((double)rounds * slots) : 1.0;
 }
 
+// Whether an XCD takes tile rows instead of tile columns, and the bytes from HBM that this was chosen by.
+// By default an XCD takes tile columns: its L2 then holds the weight rows of those columns once, but every XCD streams all
+// activation rows it meets.  With few tile columns and long rows of activations (816 x B tokens into a 16384 -> 2048
+// projection) that is eight copies of the larger operand; then the roles are exchanged.  Estimated bytes: the operand an XCD
+// does not own is read once per XCD (up to 8 times), the other once per band.  (6528 x 2048 x 16384: 187 us by tile columns,
+// 168 by tile rows.)
+// ... unless the busiest XCD then needs one more round of tiles than in the other order (13056 x 2560 x 2048 in 256 x 256
+// tiles: 510 tiles are 64 per XCD by tile columns, two rounds on 32 CUs, but 65 on some XCDs by tile rows: 93 against 75 us).
+static bool big_takes_rows(int M, int N, int K, int m_tiles, int n_tiles, int slots, double* bytes) {
+    const double a_bytes = (double)M * K, b_bytes = (double)N * K;
+    const int band_c = 4, band_r = 4;
+    const double by_cols = a_bytes * (n_tiles < 8 ? n_tiles : 8) + b_bytes * big_ceil_div(m_tiles, band_c);
+    const double by_rows = b_bytes * (m_tiles < 8 ? m_tiles : 8) + a_bytes * big_ceil_div(n_tiles, band_r);
+    bool rows = by_rows < 0.8 * by_cols;
+    const int rounds_c = big_ceil_div(big_max_tiles_per_xcd(m_tiles, n_tiles, 4), slots);
+    const int rounds_r = big_ceil_div(big_max_tiles_per_xcd(n_tiles, m_tiles, 4), slots);
+    if (rounds_c != rounds_r) rows = rounds_r < rounds_c;
+    *bytes = rows ? by_rows : by_cols;
+    return rows;
+}
+
+// The ring of register sets that a shape's weights in operand order go through (0: staged in LDS).
+static int big_register_ring(const BigPlan& pl, int K, int epilogue) {
+    if (const char* e = tuning_env("PHYAI_FP8_BIG_DIRECT")) { if (atoi(e) == 0) return 0; }
+    if (K % 128 != 0) return 0;
+    if (pl.tile == 224 && pl.splits == 1 && K % 512 == 0) return 4;
+    if (pl.tile == 128 && pl.cols == 128 && pl.depth == 4 && (K / pl.splits) % 1024 == 0 && !epi_is_gated(epilogue)) return 8;
+    // (more tiles than CUs: two workgroups per CU, each with a ring of four)
+    if (pl.tile == 128 && pl.cols == 128 && pl.depth == 2 && pl.splits == 1 && K % 512 == 0 && !epi_is_gated(epilogue)) return 4;
+    return 0;
+}
+
+// Shapes that share a CU in pairs.
+static bool big_two_of(const BigPlan& pl) { return pl.depth == 2 && (pl.tile == 192 || pl.tile == 128); }
+
 // Tile shape, K splits, ring depth.  All times in here: graphs of weight sets beyond the Infinity Cache, every tile shape
 // forced in turn at 988 shapes (M = 136 .. 13056, N = 1024 .. 32768, K = 1024 .. 16384, both layouts); over all of them the
 // choice is 1.6 % behind the best shape in the geometric mean.  The lines were drawn on an earlier main loop (32 x 32 x 64
@@ -1170,13 +1205,70 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     // stage-loads requested up front, at what the CU's vector-memory path passes - loses: 816 x 2560 x 2048 10.0 ->
     // 10.1 us on the earlier loop.  Up to K = 2048 the ring of eight is level with staged weights, and the ring of four of
     // two workgroups per CU up to 14 % ahead of it from 160 tiles up: 2048 x 2048 x 2048 15.5 / 13.6.)
-    if (operand_w && !(tuning_env("PHYAI_FP8_BIG_DIRECT") && atoi(tuning_env("PHYAI_FP8_BIG_DIRECT")) == 0)) {
-        if (pl.tile == 224 && pl.splits == 1 && K % 512 == 0) pl.regs = 4;
-        else if (pl.tile == 128 && pl.cols == 128 && pl.depth == 4 && (K / pl.splits) % 1024 == 0 && !epi_is_gated(epilogue)) pl.regs = 8;
-        // (more tiles than CUs: two workgroups per CU, each with a ring of four)
-        else if (pl.tile == 128 && pl.cols == 128 && pl.depth == 2 && pl.splits == 1 && K % 512 == 0 && !epi_is_gated(epilogue)) pl.regs = 4;
-    }
+    pl.regs = operand_w ? big_register_ring(pl, K, epilogue) : 0;
     return pl;
+}
+
+// ---- what a tile shape costs ----------------------------------------------------------------------------------------------
+// Microseconds beyond what every linear pays (launches, quantizer), from the workgroups that the busiest XCD runs on its 32
+// CUs: R rounds of them, x of a round each round's worth (R >= x > R - 1), S stages of 128 bytes of K.  A workgroup's life
+// is prologue and epilogue plus S stages, and both depend on how many CUs are at work beside it:
+//     one workgroup per CU    R round + x part + S (R round_step + x part_step)
+//     two                     the same beyond one round of single workgroups; within it alone + x alone_part + S (alone_step + x alone_part_step)
+// plus x S ragged where K is no multiple of 128, and the activation's arithmetic.  Least squares over 9800 linears drawn
+// over M = 130 .. 13056, N = 256 .. 32768, K = 512 .. 16384 (every shape forced in turn, weight sets beyond the Infinity
+// Cache): 3 - 7 % off a single time.
+struct BigCost {
+    double round, part, round_step, part_step, ragged, act, gated;
+    double alone, alone_part, alone_step, alone_part_step;   // two per CU
+};
+static BigCost big_cost_of(const BigPlan& pl) {
+    const bool regs = pl.regs != 0;
+    switch (pl.tile) {
+    case 256: return {4.59, 2.45, 1.240, 0.153, 0.258, 4.33, 1.07, 0, 0, 0, 0};
+    case 224: return regs ? BigCost{4.63, 2.12, 0.894, 0.275, 0, 3.84, 1.09, 0, 0, 0, 0} : BigCost{3.30, 2.15, 1.161, 0.137, 0.264, 3.77, 1.25, 0, 0, 0, 0};
+    case 192: return {2.30, 0.93, 0.616, 0.652, 0.102, 1.84, 0.37, 0.84, 1.06, 0.737, 0.472};
+    case 96: return {-0.12, 1.56, 0.364, 0.049, 0.108, 0.79, 0, 0, 0, 0, 0};
+    default: break;
+    }
+    if (pl.cols == 64) return {-0.52, 1.71, 0.288, 0.026, 0.062, 0.50, 0, 0, 0, 0, 0};
+    if (pl.depth == 2)
+        return regs ? BigCost{0.80, 1.24, 0.433, 0.440, 0, 1.28, 0, 0.08, 1.10, 0.464, 0.274} : BigCost{0.31, 1.56, 0.702, 0.211, 0.114, 1.29, 0.40, -0.34, 0.50, 0.647, 0.404};
+    // (K split in two: the halves' round trip through memory)
+    const double split = pl.splits > 1 ? 5.0 : 0.0;
+    return regs ? BigCost{1.02 + split, 1.06, 0.356, 0.112, 0, 1.09, 0, 0, 0, 0, 0} : BigCost{0.63 + split, 1.23, 0.393, 0.095, 0.109, 1.06, 0.33, 0, 0, 0, 0};
+}
+double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue) {
+    const BigCost c = big_cost_of(pl);
+    const bool gated = epi_is_gated(epilogue), two = big_two_of(pl);
+    const int bn = gated ? pl.cols / 2 : pl.cols;
+    const int m_tiles = big_ceil_div(M, pl.tile), n_tiles = big_ceil_div(gated ? N / 2 : N, bn), slots = two ? 64 : 32;
+    double bytes;
+    const bool by_rows = big_takes_rows(M, N, K, m_tiles, n_tiles, slots, &bytes);
+    const int busiest = pl.splits * (by_rows ? big_max_tiles_per_xcd(n_tiles, m_tiles, 4) : big_max_tiles_per_xcd(m_tiles, n_tiles, 4));
+    const double S = (double)big_ceil_div(K, 128 * pl.splits), R = big_ceil_div(busiest, slots), x = (double)busiest / slots;
+    const double ragged = K % 128 != 0 ? c.ragged : 0.0, epi = gated ? c.gated : epilogue != EPI_NONE ? c.act : 0.0;
+    if (!two) return R * (c.round + epi) + x * c.part + S * (R * c.round_step + x * (c.part_step + ragged));
+    const double t = busiest <= 32 ? c.alone + x * c.alone_part + S * (c.alone_step + x * c.alone_part_step)
+                                   : R * c.round + x * c.part + S * (R * c.round_step + x * c.part_step);
+    return t + (x > 1.0 ? x : 1.0) * (S * ragged + epi);
+}
+
+// The cheapest unsplit tile shape by that account, `rule` (big_plan's choice, or no tile at all) where nothing is 8 % ahead
+// of it, `shared` being what all of them pay.  All unsplit shapes add in the same order of K.
+BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared) {
+    static const BigPlan shapes[] = {{256, 256, 1, 0, 2, 0}, {224, 256, 1, 0, 2, 0}, {192, 128, 1, 0, 2, 0}, {128, 128, 1, 0, 4, 0},
+                                     {128, 128, 1, 0, 2, 0}, {128, 64, 1, 0, 4, 0}, {96, 128, 1, 0, 4, 0}};
+    BigPlan best = rule;
+    double lowest = rule.tile ? 0.92 * (big_cost(rule, M, N, K, epilogue) + shared) : 1e30;
+    for (BigPlan pl : shapes) {
+        if (epi_is_gated(epilogue) && (pl.cols == 64 || pl.tile == 96)) continue;
+        pl.regs = operand_w ? big_register_ring(pl, K, epilogue) : 0;
+        const double t = big_cost(pl, M, N, K, epilogue) + shared;
+        if (t < lowest) { lowest = t; best = pl; }
+    }
+    best.tiles = big_tiles(M, N, epilogue, best.tile, best.cols);
+    return best;
 }
 
 size_t big_partial_bytes(int M, int N, int epilogue, const BigPlan& pl) {
@@ -1192,29 +1284,10 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
     const int bn_eff = gated ? BN / 2 : BN;
     a.n_tiles = big_ceil_div(gated ? g.N / 2 : g.N, bn_eff);
     a.m_tiles = big_ceil_div(g.M, BM);
-    // Which operand the XCDs share.  By default an XCD takes tile columns: its L2 then holds the
-    // weight rows of those columns once, but every XCD streams all activation rows it meets.
-    // With few tile columns and long rows of activations (816 x B tokens into a 16384 -> 2048
-    // projection) that is eight copies of the larger operand; then the roles are exchanged.
-    // Estimated bytes from HBM: the operand an XCD does not own is read once per XCD (up to 8
-    // times), the other once per band.  (6528 x 2048 x 16384: 187 us by tile columns, 168 by tile rows.)
-    double chosen_bytes = 0.0;
-    {
-        const double a_bytes = (double)g.M * g.K, b_bytes = (double)g.N * g.K;
-        const int band_c = 4, band_r = 4;
-        const double by_cols = a_bytes * (a.n_tiles < 8 ? a.n_tiles : 8) + b_bytes * big_ceil_div(a.m_tiles, band_c);
-        const double by_rows = b_bytes * (a.m_tiles < 8 ? a.m_tiles : 8) + a_bytes * big_ceil_div(a.n_tiles, band_r);
-        a.by_rows = by_rows < 0.8 * by_cols;
-        // ... unless the busiest XCD then needs one more round of tiles than in the other order
-        // (13056 x 2560 x 2048 in 256 x 256 tiles: 510 tiles are 64 per XCD by tile columns, two
-        // rounds on 32 CUs, but 65 on some XCDs by tile rows: 93 against 75 us)
-        const int slots = 32 * (big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1);
-        const int rounds_c = big_ceil_div(big_max_tiles_per_xcd(a.m_tiles, a.n_tiles, 4), slots);
-        const int rounds_r = big_ceil_div(big_max_tiles_per_xcd(a.n_tiles, a.m_tiles, 4), slots);
-        if (rounds_c != rounds_r) a.by_rows = rounds_r < rounds_c;
-        if (const char* e = tuning_env("PHYAI_FP8_BY_ROWS")) a.by_rows = atoi(e) != 0;
-        chosen_bytes = a.by_rows ? by_rows : by_cols;
-    }
+    // which operand the XCDs share
+    double chosen_bytes;
+    a.by_rows = big_takes_rows(g.M, g.N, g.K, a.m_tiles, a.n_tiles, 32 * (big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1), &chosen_bytes);
+    if (const char* e = tuning_env("PHYAI_FP8_BY_ROWS")) a.by_rows = atoi(e) != 0;
     // bands of 4 tile rows; a grid of up to 8 tile rows whose activation rows still fit an XCD's
     // L2 beside the weight stream is one band, so that the weights come from HBM once
     a.band = 4;

@@ -517,6 +517,13 @@ SkinnyPlan skinny_plan(int M, int N, int K, int epilogue) {
     return pl;
 }
 
+// Microseconds on the scale of big_cost (gemm_big.hip), fitted with it: rounds of workgroups, the operand blocks that one pulls
+// per K step of a wavefront, its sums' trip through LDS.  10 % off a single time.
+double skinny_cost(const SkinnyPlan& pl, int K) {
+    const double R = sk_ceil_div(pl.tiles * pl.msplit, 256), steps = sk_ceil_div(K, 128) / (double)SK_WAVES;
+    return R * (-0.89 + (0.250 + (K % 128 != 0 ? 0.025 : 0.0)) * steps * (pl.nt + pl.mb) + 0.181 * pl.nt * pl.mb);
+}
+
 // The staged form wherever its LDS fits (8 wavefronts x KPW steps x (NT + MB) blocks of 2 KB).
 template <int MB, int NT, int KPW, int EPI>
 static void sk_launch_one(const SkinnyArgs& a, const dim3& grid, hipStream_t st) {

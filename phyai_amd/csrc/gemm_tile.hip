@@ -390,7 +390,7 @@ struct GemmChoice {
 // its own rows may serve the call (one_scale: with one static scale for all of them; amax_parts > 0: with
 // row maxima in that many slots per row; padded: GemmProblem::xq_padded where the codes are staged): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
 static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
-                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false, bool padded = false) {
+                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false, bool padded = false, bool staged = false) {
     GemmChoice c = {};
     if (norm) {   // rows still to be normalised: one kernel does it or the caller launches the norm itself
         c.kind = GemmChoice::FUSED;
@@ -427,6 +427,16 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
         return c;
     };
     if (skinny_ok && M <= 64) return small();
+    // Codes that a linear stages for itself: what the rules below say, corrected by the fitted costs of gemm_big.hip where these
+    // see something 8 % ahead.  The rules' lines were drawn one by one; over 3400 linears that neither saw, their choice is
+    // 2.7 % behind the best in the geometric mean, the corrected one 0.8 %.  What changes, one in nine, gains 13 % in the mean (us, quantizer
+    // included: 3972 x 2208 x 10592 128 x 128 181 -> 192 x 128 121, 2032 x 9216 x 640 + GELU 256 x 256 42.0 -> 28.4, 4310 x 3648 x
+    // 1920 256 x 256 60.7 -> 128 x 128 42.7, 497 x 2432 x 11648 128 x 128 56.8 -> 128 x 64 41.3, 2489 x 384 x 1792 weight streaming
+    // 15.6 -> 128 x 64 11.6, 2553 x 864 x 13184 128 x 128 74.3 -> 96 x 128 63.2, 1665 x 7680 x 2560 256 x 256 43.6 -> 224 x 256 40.2).  Weight streaming or tiles is
+    // decided without a look at the weights' layout: the two add in different orders, and a layout changes no bit.
+    // Nothing becomes split along K that the rules leave whole.
+    const bool by_cost = staged && M >= 129 && K >= 512 && out16 && !tuning_env("PHYAI_FP8_BIG") && !tuning_env("PHYAI_FP8_TILE") &&
+                         !tuning_env("PHYAI_FP8_BIG_DEPTH") && !tuning_env("PHYAI_FP8_BIG_SPLITS") && !tuning_env("PHYAI_FP8_RULES");
     if (!tuning_env("PHYAI_FP8_TILE")) {
         const BigPlan bp = big_plan(M, N, K, epilogue, layout != W_ROW_MAJOR);
         // Beyond 1024 rows every weight tile is walked by 16 workgroups and more, whose codes no L2 holds once K is 8192: with
@@ -446,10 +456,27 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
             const SkinnyPlan sp = skinny_plan(M, N, K, epilogue);
             one_round = sp.tiles * sp.msplit <= 256 && (K % 128 != 0 || sp.tiles % 2 == 0);
         }
-        if (bp.tile && out16 && !((few_small_tiles || one_round) && skinny_ok)) {
+        bool tiles = bp.tile && out16 && !((few_small_tiles || one_round) && skinny_ok);
+        BigPlan chosen = bp;
+        if (by_cost && (tiles || skinny_ok)) {
+            const double shared = 5.2;   // launches and quantizer of a linear, us
+            const BigPlan rule = big_plan(M, N, K, epilogue, false), none = {0, 0, 1, 0, 0, 0};
+            if (skinny_ok && !(tiles && bp.splits > 1)) {   // (its estimate is poor at the long K that is split)
+                const double streaming = skinny_cost(skinny_plan(M, N, K, epilogue), K) + shared;
+                const double tiled = big_cost(big_plan_by_cost(M, N, K, epilogue, false, tiles ? rule : none, shared), M, N, K, epilogue) + shared;
+                if (tiles ? streaming < 0.92 * tiled : tiled < 0.92 * streaming) {
+                    tiles = !tiles;
+                    chosen = none;
+                }
+            }
+            // (split along K or not is another order too)
+            if (tiles && chosen.splits > 1 && big_plan_by_cost(M, N, K, epilogue, false, rule, shared).splits == 1) chosen = none;
+            if (tiles && chosen.splits == 1) chosen = big_plan_by_cost(M, N, K, epilogue, layout != W_ROW_MAJOR, chosen, shared);
+        }
+        if (tiles) {
             c.kind = GemmChoice::BIG;
-            c.big = bp;
-            c.need = bp.splits > 1 ? kHeaderBytes + big_partial_bytes(M, N, epilogue, bp) : 0;
+            c.big = chosen;
+            c.need = chosen.splits > 1 ? kHeaderBytes + big_partial_bytes(M, N, epilogue, chosen) : 0;
             return c;
         }
         if (skinny_ok) return small();
@@ -473,10 +500,10 @@ static const GemmChoice& choose_gemm(const GemmProblem& g) {
     const int parts = maxima ? g.amax_parts : 0;
     const bool norm = g.norm_mod != nullptr, one_scale = g.x_scale_is_scalar != 0;
     const int64_t how = (int64_t)g.epilogue | (int64_t)vec_ok << 8 | (int64_t)out16 << 9 | (int64_t)have_x << 10 | (int64_t)norm << 11 |
-                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)(g.xq_padded != 0) << 15 | (int64_t)parts << 16;
+                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)(g.xq_padded != 0) << 15 | (int64_t)parts << 16 | (int64_t)(g.staged != 0) << 26;
     static thread_local CallMemo<GemmChoice, 128> memo;
     return memo.get((int64_t)g.M | how << 32, g.N, g.K, g.ldo, [&]() {
-        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.xq_padded != 0);
+        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.xq_padded != 0, g.staged != 0);
     });
 }
 
@@ -507,10 +534,10 @@ size_t gemm_scratch_need(const GemmProblem& g) {
     return choose_gemm(g).need;
 }
 
-int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout, bool padded) {
+int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout, bool padded, bool staged) {
     // operands that satisfy every alignment requirement, dense output
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, padded);
+    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, padded, staged);
     switch (c.kind) {
     case GemmChoice::SKINNY:
         return snprintf(buf, n, "small-m nt=%d mb=%d kpw=%d rounds=%d", c.sk.nt, c.sk.mb, c.sk.kpw, c.sk.rounds);
@@ -528,14 +555,14 @@ int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, i
 int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout) {
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
     const bool padded = K % 128 != 0;   // (as the linears stage their codes)
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, padded);
+    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, padded, true);
     if (c.kind == GemmChoice::FUSED)
         return snprintf(buf, n, "one launch: small-m rows=%d nt=%d kpw=%d grid=%dx%d", c.fq.rows, c.fq.nt, c.fq.kpw, c.fq.tiles, c.fq.msplit);
     if (c.kind == GemmChoice::SELFQ)
         return snprintf(buf, n, "one launch: rows in registers, rows=%d nt=%d steps=%d grid=%dx%d", 4 * c.sq.rg, c.sq.nt, c.sq.steps, c.sq.tiles, c.sq.msplit);
     const int len = snprintf(buf, n, "quantizer + ");
     if (len < 0 || (size_t)len >= n) return len;
-    return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout, padded);
+    return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout, padded, true);
 }
 
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order) {

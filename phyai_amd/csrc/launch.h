@@ -60,6 +60,7 @@ struct GemmProblem {
     int64_t ldo;
     int M, N, K;
     int xq_padded;          // K is no multiple of 128 and xq's rows are padded
+    int staged;             // xq is this library's own scratch (the linear forms), not a caller's
     int epilogue;
     void* workspace;        // header (counters) + split-K partials
     size_t workspace_bytes;
@@ -140,6 +141,7 @@ struct SkinnyPlan {
 };
 bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo, bool padded = false);
 SkinnyPlan skinny_plan(int M, int N, int K, int epilogue);
+double skinny_cost(const SkinnyPlan& pl, int K);   // on the scale of big_cost
 int launch_gemm_skinny(const GemmProblem& p, const SkinnyPlan& pl, hipStream_t st);
 
 // Small-M GEMM that quantizes its own activation rows (gemm_skinny_fused.hip): the whole linear in
@@ -185,6 +187,10 @@ struct BigPlan {
                  // wavefront that owns the columns, the activation stages handed over without barriers; 0: staged through LDS
 };
 BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w = false);
+// The same choice from measured costs, for codes that this library staged itself (rule: what big_plan says, tile 0 if nothing;
+// shared: microseconds that every choice pays); what a shape costs beyond those, us.
+BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared);
+double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue);
 size_t big_partial_bytes(int M, int N, int epilogue, const BigPlan& pl);
 int launch_gemm_big(const GemmProblem& p, const BigPlan& pl, hipStream_t st);
 
@@ -195,6 +201,6 @@ int launch_set_stamp_sink_fused(unsigned long long* buf, unsigned int records);
 // Text form of what phyai_fp8_mlp launches for aligned, row-major operands.
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order = false);
 // Text form of launch_gemm's choice for aligned operands and a dense output; returns its length.
-int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0, bool padded = false);
+int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0, bool padded = false, bool staged = false);
 
 }  // namespace phyai

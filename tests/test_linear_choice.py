@@ -1,0 +1,79 @@
+"""The kernel that a linear's staged codes go to (choose_gemm with the fitted costs of csrc/gemm_big.hip)."""
+
+from __future__ import annotations
+
+import random
+
+import pytest
+import torch
+
+from conftest import seeded
+
+GATED = "geglu_tanh"
+
+
+def _shapes(n):
+    rng = random.Random(1)
+    for _ in range(n):
+        m, k = rng.randint(129, 9000), 128 * rng.randint(4, 128)
+        yield m, 32 * rng.randint(8, 512), k, rng.choice([None, "gelu", GATED])
+
+
+def _kind(plan):
+    """What decides the order of the sums: weight streaming, tiles, tiles split along K."""
+    plan = plan.removeprefix("quantizer + ")
+    return plan.split()[0] + (plan.split("splits=")[1].split()[0] if "splits=" in plan else "")
+
+
+def test_layout_does_not_change_the_order_of_the_sums(monkeypatch):
+    from phyai_amd import ops
+
+    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "TILE", "FUSED", "RULES"):
+        monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    changed = 0
+    for m, n, k, epi in _shapes(1500):
+        if epi == GATED and n % 32 or m * k >= 1 << 31:
+            continue
+        lay = "operand_gated" if epi == GATED else "operand"
+        row, op = ops.describe_linear_plan(m, n, k, epi), ops.describe_linear_plan(m, n, k, epi, weight_layout=lay)
+        assert _kind(row) == _kind(op), (m, n, k, epi, row, op)
+        rule = ops.describe_plan(m, n, k, epi)
+        assert _kind(row) in (_kind(rule), "tile1", "small-m"), (m, n, k, epi, rule, row)   # nothing is newly split
+        changed += row.removeprefix("quantizer + ") != rule
+    assert changed > 50
+
+
+def test_rules_alone(monkeypatch):
+    from phyai_amd import ops
+
+    monkeypatch.setenv("PHYAI_FP8_RULES", "1")
+    for m, n, k, epi in _shapes(200):
+        assert ops.describe_linear_plan(m, n, k, epi).removeprefix("quantizer + ") == ops.describe_plan(m, n, k, epi)
+
+
+# (rows, columns, K, epilogue): rule's shape -> chosen shape, one per pair that occurs
+CHANGED = [(3000, 2208, 1536, None), (2032, 9216, 640, "gelu"), (4310, 3648, 640, None), (497, 2432, 8320, None), (2489, 384, 1792, None),
+           (2553, 864, 8320, None), (1665, 7680, 2560, None), (1301, 768, 8448, None), (1047, 896, 9216, None), (400, 6144, 8192, None)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,epi", CHANGED)
+def test_chosen_kernel_in_both_layouts_and_without_a_workspace_of_its_own(dev, M, N, K, epi):
+    """Operand order changes no bit, the static-scratch form gives the same where its array holds the codes, and the result is
+    the rules' kernel's up to the order of fp32 sums (2^-7 of the largest output covers one bf16 step on either side)."""
+    from phyai_amd import _lib, ops
+
+    x = seeded((M, K), M + K).to(dev)
+    wq, ws = ops.fp8_weight_quant(seeded((N, K), K, 0.02).to(dev))
+    got = ops.fp8_linear(x, wq, ws, epilogue=epi)
+    relaid = ops.fp8_linear(x, ops.fp8_weight_to_operand_order(wq), ws, epilogue=epi, weight_layout="operand")
+    assert torch.equal(got.view(torch.int16), relaid.view(torch.int16))
+    xq, xs = ops.fp8_quant_rowwise(x)
+    want = ops.fp8_gemm(xq, xs, wq, ws, epilogue=epi).float()
+    assert (got.float() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
+    out = torch.empty_like(got)
+    rc = _lib.load().phyai_fp8_linear_static(x.data_ptr(), K, wq.data_ptr(), ws.data_ptr(), None, out.data_ptr(), N, M, N, K,
+                                             {"gelu": 5}.get(epi, 0), torch.cuda.current_stream().cuda_stream)
+    if M * K < 24 << 20:
+        _lib.check(rc, "static")
+        assert torch.equal(got.view(torch.int16), out.view(torch.int16))
