@@ -165,7 +165,9 @@ int phyai_fp8_gemm(const void *xq, const float *x_scale, int x_scale_is_scalar,
  * in operand order, 8192 row-major).  Every workgroup quantizes the token rows it multiplies (same codes, same
  * scales, same output bits as the two launches) and the workspace is not touched: such a call may pass
  * workspace = NULL.  Otherwise the quantizer writes codes and scales into the workspace and a GEMM kernel follows
- * (PHYAI_FP8_EWORKSPACE without one).  phyai_fp8_describe_linear_plan tells which.
+ * (PHYAI_FP8_EWORKSPACE without one).  What else has more than 48 rows, up to K = 1024 (row-major below 768) and about 500 tiles of 16 rows
+ * x 64 or 128 columns, one launch serves the call too, unless out lies inside x's rows; a workspace is asked for all the same.
+ * phyai_fp8_describe_linear_plan tells which.
  */
 int phyai_fp8_linear(const void *x, int64_t ldx, const void *w, const float *w_scale,
                      const void *bias, void *out, int64_t ldo, int64_t M, int64_t N,

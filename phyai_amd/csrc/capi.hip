@@ -372,12 +372,13 @@ int run_linear(const char* fn, const void* x, int64_t ldx, const void* w, const 
     if (!workspace || workspace_bytes < c.total) {
         // The kernel that quantizes its own rows touches neither staged codes nor GEMM scratch: a call
         // that it serves needs no workspace at all (x stands in for the code and scale pointers, which
-        // are never dereferenced then).
+        // are never dereferenced then).  (gemm_panel.hip asks
+        // for one as the two launches do in whose place it came.)
         phyai::GemmProblem g;
         if (!norm && x && check_quant_args(fn, x, M, K, ldx, x) == 0 &&
             prepare_gemm(fn, x, static_cast<const float*>(x), 0, w, w_scale, bias, res, out, ldo, M, N, K, epilogue, nullptr,
                          0, &g, x, ldx) == 0 &&
-            phyai::gemm_quantizes_itself(g))
+            phyai::gemm_quantizes_itself(g, true))
             return launch_prepared(fn, g, stream);
         return fail(PHYAI_FP8_EWORKSPACE, "%s: workspace of %zu bytes is too small, need %zu", fn,
                     workspace ? workspace_bytes : (size_t)0, c.total);

@@ -361,10 +361,12 @@ static int launch_epi(const TileArgs& a, const TileConfig& c, dim3 grid, hipStre
 
 // launch_gemm's choice of kernel for one problem, and the scratch that choice needs.
 struct GemmChoice {
-    enum Kind { SKINNY, BIG, GENERIC, FUSED, SELFQ } kind;
+    enum Kind { SKINNY, BIG, GENERIC, FUSED, SELFQ, PANEL } kind;
     FusedPlan fq;
     SelfqPlan sq;
     int sq_source;
+    PanelPlan pn;
+    bool panel_by_waves;
     SkinnyPlan sk;
     BigPlan big;
     TileConfig tc;
@@ -389,7 +391,7 @@ struct GemmChoice {
 // have_x: the bf16 activations are at hand (whole-linear entry points), so a kernel that quantizes
 // its own rows may serve the call (one_scale: with one static scale for all of them; amax_parts > 0: with
 // row maxima in that many slots per row; padded: GemmProblem::xq_padded where the codes are staged): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
-static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
+static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
                               int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false, bool padded = false, bool staged = false) {
     GemmChoice c = {};
     if (norm) {   // rows still to be normalised: one kernel does it or the caller launches the norm itself
@@ -487,6 +489,22 @@ static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bo
     return c;
 }
 
+// What serves a call; `panel`: one launch may take the place of the quantizer and the kernel of the shape, whose order of
+// sums it then keeps (it needs the rows as bf16, and an output that lies apart from them: its workgroups read rows while
+// others store).
+static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x, int layout, int amax_parts,
+                              bool norm, bool one_scale, bool padded, bool staged, bool panel) {
+    GemmChoice c = choose_kernel(M, N, K, epilogue, ldo, vec_ok, out16, have_x, layout, amax_parts, norm, one_scale, padded, staged);
+    if (panel && have_x && vec_ok && !norm && (c.kind == GemmChoice::SKINNY || (c.kind == GemmChoice::BIG && c.big.splits == 1))) {
+        c.pn = panel_plan(M, N, K, epilogue, ldo, layout);
+        if (c.pn.nt) {
+            c.panel_by_waves = c.kind == GemmChoice::SKINNY;
+            c.kind = GemmChoice::PANEL;
+        }
+    }
+    return c;
+}
+
 static const GemmChoice& choose_gemm(const GemmProblem& g) {
     const bool vec_ok = (reinterpret_cast<uintptr_t>(g.w_scale) % 16 == 0) &&
                         (reinterpret_cast<uintptr_t>(g.bias) % 8 == 0) &&
@@ -498,12 +516,14 @@ static const GemmChoice& choose_gemm(const GemmProblem& g) {
     const bool maxima = g.amax_in != nullptr && g.amax_parts >= 1 && g.amax_parts <= kRowAmaxSlots &&
                         (reinterpret_cast<uintptr_t>(g.amax_in) & 15) == 0;
     const int parts = maxima ? g.amax_parts : 0;
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(g.x_bf16), o0 = reinterpret_cast<uintptr_t>(g.out);
+    const bool apart = have_x && ((x0 + 2 * ((uint64_t)(g.M - 1) * g.ldx + g.K) <= o0) || (o0 + 2 * ((uint64_t)(g.M - 1) * g.ldo + g.N) <= x0));
     const bool norm = g.norm_mod != nullptr, one_scale = g.x_scale_is_scalar != 0;
     const int64_t how = (int64_t)g.epilogue | (int64_t)vec_ok << 8 | (int64_t)out16 << 9 | (int64_t)have_x << 10 | (int64_t)norm << 11 |
-                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)(g.xq_padded != 0) << 15 | (int64_t)parts << 16 | (int64_t)(g.staged != 0) << 26;
+                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)(g.xq_padded != 0) << 15 | (int64_t)parts << 16 | (int64_t)(g.staged != 0) << 26 | (int64_t)apart << 27;
     static thread_local CallMemo<GemmChoice, 128> memo;
     return memo.get((int64_t)g.M | how << 32, g.N, g.K, g.ldo, [&]() {
-        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.xq_padded != 0, g.staged != 0);
+        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.xq_padded != 0, g.staged != 0, apart);
     });
 }
 
@@ -523,10 +543,10 @@ bool gemm_takes_row_maxima(const GemmProblem& g) {
     return choose_gemm(g).takes_amax;
 }
 
-bool gemm_quantizes_itself(const GemmProblem& g) {
+bool gemm_quantizes_itself(const GemmProblem& g, bool without_workspace) {
     if (g.M == 0 || g.N == 0) return false;
     const GemmChoice& c = choose_gemm(g);
-    return c.kind == GemmChoice::FUSED || c.kind == GemmChoice::SELFQ;
+    return c.kind == GemmChoice::FUSED || c.kind == GemmChoice::SELFQ || (c.kind == GemmChoice::PANEL && !without_workspace);
 }
 
 size_t gemm_scratch_need(const GemmProblem& g) {
@@ -537,7 +557,7 @@ size_t gemm_scratch_need(const GemmProblem& g) {
 int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout, bool padded, bool staged) {
     // operands that satisfy every alignment requirement, dense output
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, padded, staged);
+    const GemmChoice c = choose_kernel(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, padded, staged);
     switch (c.kind) {
     case GemmChoice::SKINNY:
         return snprintf(buf, n, "small-m nt=%d mb=%d kpw=%d rounds=%d", c.sk.nt, c.sk.mb, c.sk.kpw, c.sk.rounds);
@@ -555,11 +575,13 @@ int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, i
 int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout) {
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
     const bool padded = K % 128 != 0;   // (as the linears stage their codes)
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, padded, true);
+    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, padded, true, true);
     if (c.kind == GemmChoice::FUSED)
         return snprintf(buf, n, "one launch: small-m rows=%d nt=%d kpw=%d grid=%dx%d", c.fq.rows, c.fq.nt, c.fq.kpw, c.fq.tiles, c.fq.msplit);
     if (c.kind == GemmChoice::SELFQ)
         return snprintf(buf, n, "one launch: rows in registers, rows=%d nt=%d steps=%d grid=%dx%d", 4 * c.sq.rg, c.sq.nt, c.sq.steps, c.sq.tiles, c.sq.msplit);
+    if (c.kind == GemmChoice::PANEL)
+        return snprintf(buf, n, "one launch: panel of 16 rows, nt=%d grid=%dx%d", c.pn.nt, c.pn.n_tiles, c.pn.m_tiles);
     const int len = snprintf(buf, n, "quantizer + ");
     if (len < 0 || (size_t)len >= n) return len;
     return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout, padded, true);
@@ -569,10 +591,10 @@ int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_
     const int n1 = epi_is_gated(epilogue) ? 2 * I : I;
     const int lay1 = !operand_order ? W_ROW_MAJOR : (epi_is_gated(epilogue) ? W_OPERAND_GATED : W_OPERAND_PLAIN);
     const int lay2 = operand_order ? W_OPERAND_PLAIN : W_ROW_MAJOR;
-    const GemmChoice a = choose_gemm(M, n1, H, epilogue, I, true, I % 8 == 0, true, lay1);
+    const GemmChoice a = choose_kernel(M, n1, H, epilogue, I, true, I % 8 == 0, true, lay1);
     const int parts = a.kind == GemmChoice::FUSED ? a.fq.tiles : a.kind == GemmChoice::SELFQ ? a.sq.tiles : 0;
     const bool some = parts > 0 && parts <= kRowAmaxSlots;
-    const GemmChoice b = choose_gemm(M, O, I, EPI_NONE, O, true, O % 8 == 0, true, lay2, some ? parts : 0);
+    const GemmChoice b = choose_kernel(M, O, I, EPI_NONE, O, true, O % 8 == 0, true, lay2, some ? parts : 0);
     const bool handed = some && b.takes_amax;
     int len = handed ? snprintf(buf, n, "row maxima handed over: ") : 0;
     if (len < 0 || (size_t)len >= n) return len;
@@ -595,6 +617,7 @@ int launch_gemm(const GemmProblem& g, hipStream_t st) {
     const GemmChoice& ch = choose_gemm(g);
     if (ch.need > 0 && (g.workspace == nullptr || g.workspace_bytes < ch.need)) return -3;
     if (ch.kind == GemmChoice::SELFQ) return launch_gemm_selfq(g, ch.sq, ch.sq_source, st);
+    if (ch.kind == GemmChoice::PANEL) return launch_gemm_panel(g, ch.pn, ch.panel_by_waves, st);
     if (ch.kind == GemmChoice::FUSED) {
         if (ch.fq.rows == 0) return -2;
         if (g.amax_in != nullptr && !ch.takes_amax) {   // the plan finds the row maxima itself

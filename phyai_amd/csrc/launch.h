@@ -117,8 +117,8 @@ size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int epilogue, int64
 size_t gemm_scratch_need(const GemmProblem& p);
 int launch_gemm(const GemmProblem& p, hipStream_t st);
 // True when launch_gemm would serve this problem (x_bf16 set) with the kernel that quantizes its own
-// rows: the caller then skips the quantizer launch.
-bool gemm_quantizes_itself(const GemmProblem& p);
+// rows: the caller then skips the quantizer launch.  without_workspace: only where such a call may come without one.
+bool gemm_quantizes_itself(const GemmProblem& p, bool without_workspace = false);
 // True when launch_gemm would serve this problem (x_bf16 and norm_mod set) with the kernel that normalises its rows too.
 bool gemm_normalises_itself(const GemmProblem& p);
 // Row maxima handed from one linear to the next (GemmProblem::amax_out / amax_in).  Slots per token row
@@ -174,6 +174,15 @@ int launch_selfq_own(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
 int launch_selfq_own_act(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
 int launch_selfq_handed(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
 int launch_selfq_static(const GemmProblem& p, const SelfqPlan& pl, hipStream_t st);
+
+// Linear of more than 48 rows and up to 1024 of K in one launch (gemm_panel.hip), where the two above do not apply.  nt == 0:
+// does not apply either.
+struct PanelPlan {
+    int nt;                 // 16-row weight tiles per wavefront
+    int n_tiles, m_tiles;   // workgroups along N and M
+};
+PanelPlan panel_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout);
+int launch_gemm_panel(const GemmProblem& p, const PanelPlan& pl, bool by_waves, hipStream_t st);
 
 // Pipelined tile kernel for large M (gemm_big.hip); 128 x 128 tiles may be split along K (partials in the workspace,
 // as for the generic tile kernel).

@@ -92,14 +92,17 @@ __device__ __forceinline__ uint2 encode8_static_exact(uint4 q, float s) {
     return make_uint2(c[0] | (c[1] << 16), c[2] | (c[3] << 16));
 }
 // clamp(x / s) -> codes of 8 elements that are no NaNs, scale in the fast range.  (The first clamp keeps the correction
-// of a product that is out of range anyway from overflowing into a NaN.)
-__device__ __forceinline__ uint2 encode8_static_fast(uint4 q, const StaticDivisor& d) {
+// of a product that is out of range anyway from overflowing into a NaN; below 2^64 in magnitude - kStaticPlainBf16 as bits -
+// no product with a reciprocal in the fast range overflows: encode8_static_plain.)
+constexpr uint32_t kStaticPlainBf16 = 0x5F80u;
+template <bool PLAIN>
+__device__ __forceinline__ uint2 encode8_static_in_range(uint4 q, const StaticDivisor& d) {
     const uint32_t w[4] = {q.x, q.y, q.z, q.w};
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const float x = __uint_as_float((i & 1) ? w[i >> 1] & 0xFFFF0000u : w[i >> 1] << 16);
-        const float a = __builtin_amdgcn_fmed3f(x * d.r, -512.0f, 512.0f);
+        const float a = PLAIN ? x * d.r : __builtin_amdgcn_fmed3f(x * d.r, -512.0f, 512.0f);
         v[i] = __builtin_amdgcn_fmed3f(quotient(x, a, d.s, d.r), -kFp8Max, kFp8Max);
     }
     int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false), hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
@@ -107,6 +110,8 @@ __device__ __forceinline__ uint2 encode8_static_fast(uint4 q, const StaticDiviso
     hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
     return make_uint2((uint32_t)lo, (uint32_t)hi);
 }
+__device__ __forceinline__ uint2 encode8_static_fast(uint4 q, const StaticDivisor& d) { return encode8_static_in_range<false>(q, d); }
+__device__ __forceinline__ uint2 encode8_static_plain(uint4 q, const StaticDivisor& d) { return encode8_static_in_range<true>(q, d); }
 __device__ __forceinline__ bool any_nan_or_inf(uint4 q) { return absmax_finish(absmax8_pk(q, 0u)) >= 0x7F80u; }
 
 template <int MODE>
