@@ -56,7 +56,7 @@
 // instantiations, weights staged row-major): the last stage-load is partial, its missing chunks arrive as zeros
 // (copy16_to_lds_checked), one extra VALU instruction per copy and nothing in the MFMA loop.  Such widths used to go
 // to the generic tile kernel: the MLP 1168 -> 4304 -> 1168 at M = 777 took 43 + 37 us of GEMM there, 85 us in all;
-// 34 us in all now (its second projection by the weight-streaming kernel).
+// 31 us in all now (its second projection by the weight-streaming kernel, both on codes in padded rows).
 #include "fp8_device.h"
 #include "launch.h"
 #include "tuning.h"
