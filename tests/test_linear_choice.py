@@ -1,4 +1,4 @@
-"""The kernel that a linear's staged codes go to (choose_gemm with the fitted costs of csrc/gemm_big.hip)."""
+"""The kernel that a linear's staged codes go to (choose_gemm with the fitted costs of csrc/gemm_big.hip), or that takes its rows."""
 
 from __future__ import annotations
 
@@ -28,8 +28,9 @@ def _kind(plan):
 def test_layout_does_not_change_the_order_of_the_sums(monkeypatch):
     from phyai_amd import ops
 
-    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "TILE", "FUSED", "RULES"):
+    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "TILE", "RULES"):
         monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    monkeypatch.setenv("PHYAI_FP8_FUSED", "0")   # (one launch in their place keeps their order: tests/test_gpu_panel.py)
     changed = 0
     for m, n, k, epi in _shapes(1500):
         if epi == GATED and n % 32 or m * k >= 1 << 31:
@@ -47,8 +48,32 @@ def test_rules_alone(monkeypatch):
     from phyai_amd import ops
 
     monkeypatch.setenv("PHYAI_FP8_RULES", "1")
+    monkeypatch.setenv("PHYAI_FP8_FUSED", "0")
     for m, n, k, epi in _shapes(200):
         assert ops.describe_linear_plan(m, n, k, epi).removeprefix("quantizer + ") == ops.describe_plan(m, n, k, epi)
+
+
+def test_where_one_launch_takes_more_rows(monkeypatch):
+    """csrc/gemm_panel.hip: only in the place of weight streaming or an unsplit tile, within the K and grid that were measured."""
+    from phyai_amd import ops
+
+    for var in ("BIG", "TILE", "SKINNY_PLAN", "FUSED", "RULES"):
+        monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    rng, seen = random.Random(2), 0
+    for _ in range(3000):
+        m, n, k = rng.randint(1, 2000), 16 * rng.randint(1, 300), rng.choice([16 * rng.randint(1, 80), 128 * rng.randint(1, 10)])
+        lay = rng.choice([None, "operand"]) if k % 128 == 0 else None
+        epi = rng.choice([None, None, None, "gelu"])
+        plan = ops.describe_linear_plan(m, n, k, epi, weight_layout=lay)
+        if not plan.startswith("one launch: panel"):
+            continue
+        seen += 1
+        grid = [int(v) for v in plan.split("grid=")[1].split("x")]
+        assert epi is None and m > 48 and k <= 1024 and (lay or k < 768) and grid[0] * grid[1] <= (512 if lay else 768), (m, n, k, lay, plan)
+        with monkeypatch.context() as two:
+            two.setenv("PHYAI_FP8_FUSED", "0")
+            assert _kind(ops.describe_linear_plan(m, n, k, epi, weight_layout=lay)) in ("small-m", "tile1"), (m, n, k, lay)
+    assert seen > 100
 
 
 # (rows, columns, K, epilogue): rule's shape -> chosen shape, one per pair that occurs
