@@ -198,8 +198,10 @@ void gemm_fp8_panel_kernel(const uint8_t* __restrict__ a_w, const uint8_t* __res
 
 // Where one launch is ahead: workgroups of 64 columns up to 512 of them (two per CU at once), of 128 columns up to 512 again.
 // A third round eats it: 513 - 768 workgroups of 128 columns 0.98 (K = 512) to 0.83 (K = 1024) of the speed of two launches.
-// Row-major weights arrive in 64-byte pieces, and rows a multiple of 256 bytes apart meet in the memory channels: K = 768 0.75 -
-// 1.22, 896 0.68 - 0.92, so K < 768 there, with 64 columns up to 768 workgroups.  Over 520 linears drawn from what the rule
+// Row-major weights cost more the longer K is: K = 768 0.75 - 1.22 of the speed of two launches, 896 0.68 - 0.92 (why is not
+// known: eight lanes to a row with the halves exchanged between lanes, i.e. 128-byte pieces, is level, and K steps in another
+// order per wavefront 5 - 10 % worse), so K < 768 there, with 64 columns up to 768 workgroups.
+// Over 520 linears drawn from what the rule
 // takes (M = 49 - 11000, N = 16 - 23000), two launches took 1.4 to 1.5 times as long in the geometric mean, 1.01 at the least
 // (89 x 6016 x 640 row-major).
 PanelPlan panel_plan(int M, int N, int K, int epilogue, int64_t ldo, int weight_layout) {
