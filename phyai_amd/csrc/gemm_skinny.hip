@@ -447,20 +447,19 @@ static int skinny_max_m() {
     return 4096;
 }
 
-// K that is not a multiple of 128 (staged form only): from three K steps on (ten with more than 64 rows and few
-// columns), the generic kernel's K splits cost it a round trip through memory (184 x 896 x 2256: 31.3 -> 9.1 us, 353 x
-// 384 x 3216: 35.9 -> 9.0 us).  With padded codes from three K steps on throughout, quantizer included: 200 x 512 x 1040
-// 22.6 -> 5.6 us, 560 x 656 x 1168 29.4 -> 7.5, 500 x 640 x 784 + GeGLU 17.9 -> 6.4, 900 x 272 x 720 21.0 -> 6.6 (dense codes of
-// such shapes still go to the generic kernel).
-static bool skinny_takes_ragged(int M, int N, int K, bool padded) {
+// K that is not a multiple of 128 (staged form only): from three K steps on, where the generic kernel's K splits cost it a
+// round trip through memory (184 x 896 x 2256: 31.3 -> 9.1 us, 353 x 384 x 3216: 35.9 -> 9.0 us; quantizer included, on padded
+// codes: 200 x 512 x 1040 22.6 -> 5.6 us, 560 x 656 x 1168 29.4 -> 7.5, 500 x 640 x 784 + GeGLU 17.9 -> 6.4, 900 x 272 x 720
+// 21.0 -> 6.6).  Dense rows or padded ones, the line is the same: the two kernels add in different orders.
+static bool skinny_takes_ragged(int M, int N, int K) {
     static const bool staged = []() { const char* e = tuning_env("PHYAI_FP8_SKINNY_STAGED"); return !(e && atoi(e) == 0); }();
     if (!staged || (int64_t)K * (N > M ? N : M) >= ((int64_t)1 << 31) || K >= (1 << 24)) return false;
-    return K > 256 && (padded || M <= 64 || N >= 1024 || K >= 1280);
+    return K > 256;
 }
 
-bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo, bool padded) {
+bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo) {
     if (M > skinny_max_m() || ldo % 4 != 0) return false;
-    if (K % 128 != 0 && !skinny_takes_ragged(M, N, K, padded)) return false;
+    if (K % 128 != 0 && !skinny_takes_ragged(M, N, K)) return false;
     if (epi_is_gated(epilogue)) return (N / 2) % 8 == 0;
     return N % 8 == 0;
 }

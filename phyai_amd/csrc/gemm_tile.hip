@@ -390,9 +390,10 @@ struct GemmChoice {
 // tile kernel's epilogue needs.
 // have_x: the bf16 activations are at hand (whole-linear entry points), so a kernel that quantizes
 // its own rows may serve the call (one_scale: with one static scale for all of them; amax_parts > 0: with
-// row maxima in that many slots per row; padded: GemmProblem::xq_padded where the codes are staged): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
+// row maxima in that many slots per row): gemm_skinny_fused.hip first, gemm_selfq.h for what that does not take.
+// staged: GemmProblem::staged.
 static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x,
-                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false, bool padded = false, bool staged = false) {
+                              int layout = W_ROW_MAJOR, int amax_parts = 0, bool norm = false, bool one_scale = false, bool staged = false) {
     GemmChoice c = {};
     if (norm) {   // rows still to be normalised: one kernel does it or the caller launches the norm itself
         c.kind = GemmChoice::FUSED;
@@ -421,7 +422,7 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
             if (selfq(SELFQ_FROM_ROWS)) return c;
         }
     }
-    const bool skinny_ok = vec_ok && skinny_applicable(M, N, K, epilogue, ldo, padded);
+    const bool skinny_ok = vec_ok && skinny_applicable(M, N, K, epilogue, ldo);
     auto small = [&]() {
         c.kind = GemmChoice::SKINNY;
         c.sk = skinny_plan(M, N, K, epilogue);
@@ -429,24 +430,27 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
         return c;
     };
     if (skinny_ok && M <= 64) return small();
-    // Codes that a linear stages for itself: what the rules below say, corrected by the fitted costs of gemm_big.hip where these
-    // see something 8 % ahead.  The rules' lines were drawn one by one; over 3400 linears that neither saw, their choice is
-    // 2.7 % behind the best in the geometric mean, the corrected one 0.8 %.  What changes, one in nine, gains 13 % in the mean (us, quantizer
+    // What the rules below say, corrected by the fitted costs of gemm_big.hip where these see something 8 % ahead.  The rules'
+    // lines were drawn one by one; over 3400 linears that neither saw, their choice is 2.7 % behind the best in the geometric
+    // mean, the corrected one 0.8 %.  What changes, one in nine, gains 13 % in the mean (us, quantizer
     // included: 3972 x 2208 x 10592 128 x 128 181 -> 192 x 128 121, 2032 x 9216 x 640 + GELU 256 x 256 42.0 -> 28.4, 4310 x 3648 x
     // 1920 256 x 256 60.7 -> 128 x 128 42.7, 497 x 2432 x 11648 128 x 128 56.8 -> 128 x 64 41.3, 2489 x 384 x 1792 weight streaming
-    // 15.6 -> 128 x 64 11.6, 2553 x 864 x 13184 128 x 128 74.3 -> 96 x 128 63.2, 1665 x 7680 x 2560 256 x 256 43.6 -> 224 x 256 40.2).  Weight streaming or tiles is
-    // decided without a look at the weights' layout: the two add in different orders, and a layout changes no bit.
+    // 15.6 -> 128 x 64 11.6, 2553 x 864 x 13184 128 x 128 74.3 -> 96 x 128 63.2, 1665 x 7680 x 2560 256 x 256 43.6 -> 224 x 256 40.2).
+    // Weight streaming, tiles and tiles split along K add in different orders, so which of them it is depends on the shape alone:
+    // not on the weights' layout, nor on whether the linear staged the codes itself or a caller had them ready (a norm's
+    // forward_fp8 and the linear behind it stand for the norm and the linear, bit for bit).  Among tile shapes, which add alike,
+    // the costs choose for staged codes; ready ones keep the rules' shape where it adds in that order.
     // Nothing becomes split along K that the rules leave whole.
-    const bool by_cost = staged && M >= 129 && K >= 512 && out16 && !tuning_env("PHYAI_FP8_BIG") && !tuning_env("PHYAI_FP8_TILE") &&
+    const bool by_cost = M >= 129 && K >= 512 && out16 && !tuning_env("PHYAI_FP8_BIG") && !tuning_env("PHYAI_FP8_TILE") &&
                          !tuning_env("PHYAI_FP8_BIG_DEPTH") && !tuning_env("PHYAI_FP8_BIG_SPLITS") && !tuning_env("PHYAI_FP8_RULES");
     if (!tuning_env("PHYAI_FP8_TILE")) {
-        const BigPlan bp = big_plan(M, N, K, epilogue, layout != W_ROW_MAJOR);
+        const BigPlan none = {0, 0, 1, 0, 0, 0}, rule = big_plan(M, N, K, epilogue, false);
         // Beyond 1024 rows every weight tile is walked by 16 workgroups and more, whose codes no L2 holds once K is 8192: with
         // 48 tiles of 128 x 128 and more (split in two along K) the tile kernel is ahead (2048 x 384 x 8192 23.5 / 22.9 us,
         // 2500 x 384 x 8192 26.5 / 23.3, 1800 x 512 x 16384 38.8 / 34.9, 2048 x 512 x 16384 42.4 / 35.0; level at 1548 x 512 x
         // 16384, 52 tiles; behind below: 1800 x 384 x 8192, 45 tiles, 19.3 / 22.6).
-        const bool long_k_of_many_rows = M > 1024 && K >= 8192 && bp.tiles >= 48;
-        const bool few_small_tiles = bp.tile == 128 && bp.cols == 128 && bp.tiles <= 64 && !long_k_of_many_rows && !tuning_env("PHYAI_FP8_BIG");
+        const bool long_k_of_many_rows = M > 1024 && K >= 8192 && rule.tiles >= 48;
+        const bool few_small_tiles = rule.tile == 128 && rule.cols == 128 && rule.tiles <= 64 && !long_k_of_many_rows && !tuning_env("PHYAI_FP8_BIG");
         // ... and its 128 x 64 tiles lose to one round of weight-streaming workgroups above K = 4096 where K is no multiple of a
         // K step (777 x 1168 x 4304 17.8 / 16.3 us, 900 x 1040 x 4112 17.5 / 15.4) or the workgroups that share a weight tile
         // meet on half of the XCDs, i.e. with an even number of 64-column tiles (22 tiles: 700 x 1408 x K 16.4 / 14.8 at K =
@@ -454,31 +458,31 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
         // XCD fetches every weight tile, and the tile kernel is ahead: 1296 columns 13.4 / 14.9 at K = 4224, 17.1 / 19.8 at
         // 6016; 420 x 2064 x 5120 15.1 / 18.5.  (Not asked up to K = 4096, though 400 x 2304 x 2048, 36 tiles, is 8.5 / 7.8.)
         bool one_round = false;
-        if (bp.tile == 128 && bp.cols == 64 && K > 4096 && skinny_ok && !tuning_env("PHYAI_FP8_BIG")) {
+        if (rule.tile == 128 && rule.cols == 64 && K > 4096 && skinny_ok && !tuning_env("PHYAI_FP8_BIG")) {
             const SkinnyPlan sp = skinny_plan(M, N, K, epilogue);
             one_round = sp.tiles * sp.msplit <= 256 && (K % 128 != 0 || sp.tiles % 2 == 0);
         }
-        bool tiles = bp.tile && out16 && !((few_small_tiles || one_round) && skinny_ok);
-        BigPlan chosen = bp;
+        bool tiles = rule.tile && out16 && !((few_small_tiles || one_round) && skinny_ok);
+        bool as_ruled = true;   // the rules' tile shape adds in the order decided on
+        const double shared = 5.2;   // launches and quantizer of a linear, us
         if (by_cost && (tiles || skinny_ok)) {
-            const double shared = 5.2;   // launches and quantizer of a linear, us
-            const BigPlan rule = big_plan(M, N, K, epilogue, false), none = {0, 0, 1, 0, 0, 0};
-            if (skinny_ok && !(tiles && bp.splits > 1)) {   // (its estimate is poor at the long K that is split)
+            const BigPlan best = big_plan_by_cost(M, N, K, epilogue, false, tiles ? rule : none, shared);
+            if (skinny_ok && !(tiles && rule.splits > 1)) {   // (its estimate is poor at the long K that is split)
                 const double streaming = skinny_cost(skinny_plan(M, N, K, epilogue), K) + shared;
-                const double tiled = big_cost(big_plan_by_cost(M, N, K, epilogue, false, tiles ? rule : none, shared), M, N, K, epilogue) + shared;
+                const double tiled = big_cost(best, M, N, K, epilogue) + shared;
                 if (tiles ? streaming < 0.92 * tiled : tiled < 0.92 * streaming) {
                     tiles = !tiles;
-                    chosen = none;
+                    as_ruled = false;
                 }
             }
-            // (split along K or not is another order too)
-            if (tiles && chosen.splits > 1 && big_plan_by_cost(M, N, K, epilogue, false, rule, shared).splits == 1) chosen = none;
-            if (tiles && chosen.splits == 1) chosen = big_plan_by_cost(M, N, K, epilogue, layout != W_ROW_MAJOR, chosen, shared);
+            if (tiles && as_ruled && rule.splits > 1 && best.splits == 1) as_ruled = false;
         }
         if (tiles) {
             c.kind = GemmChoice::BIG;
-            c.big = chosen;
-            c.need = chosen.splits > 1 ? kHeaderBytes + big_partial_bytes(M, N, epilogue, chosen) : 0;
+            c.big = layout == W_ROW_MAJOR ? rule : big_plan(M, N, K, epilogue, true);
+            if (!as_ruled || (by_cost && staged && c.big.splits == 1))
+                c.big = big_plan_by_cost(M, N, K, epilogue, layout != W_ROW_MAJOR, as_ruled ? c.big : none, shared);
+            c.need = c.big.splits > 1 ? kHeaderBytes + big_partial_bytes(M, N, epilogue, c.big) : 0;
             return c;
         }
         if (skinny_ok) return small();
@@ -493,8 +497,8 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
 // sums it then keeps (it needs the rows as bf16, and an output that lies apart from them: its workgroups read rows while
 // others store).
 static GemmChoice choose_gemm(int M, int N, int K, int epilogue, int64_t ldo, bool vec_ok, bool out16, bool have_x, int layout, int amax_parts,
-                              bool norm, bool one_scale, bool padded, bool staged, bool panel) {
-    GemmChoice c = choose_kernel(M, N, K, epilogue, ldo, vec_ok, out16, have_x, layout, amax_parts, norm, one_scale, padded, staged);
+                              bool norm, bool one_scale, bool staged, bool panel) {
+    GemmChoice c = choose_kernel(M, N, K, epilogue, ldo, vec_ok, out16, have_x, layout, amax_parts, norm, one_scale, staged);
     if (panel && have_x && vec_ok && !norm && (c.kind == GemmChoice::SKINNY || (c.kind == GemmChoice::BIG && c.big.splits == 1))) {
         c.pn = panel_plan(M, N, K, epilogue, ldo, layout);
         if (c.pn.nt) {
@@ -520,10 +524,10 @@ static const GemmChoice& choose_gemm(const GemmProblem& g) {
     const bool apart = have_x && ((x0 + 2 * ((uint64_t)(g.M - 1) * g.ldx + g.K) <= o0) || (o0 + 2 * ((uint64_t)(g.M - 1) * g.ldo + g.N) <= x0));
     const bool norm = g.norm_mod != nullptr, one_scale = g.x_scale_is_scalar != 0;
     const int64_t how = (int64_t)g.epilogue | (int64_t)vec_ok << 8 | (int64_t)out16 << 9 | (int64_t)have_x << 10 | (int64_t)norm << 11 |
-                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)(g.xq_padded != 0) << 15 | (int64_t)parts << 16 | (int64_t)(g.staged != 0) << 26 | (int64_t)apart << 27;
+                        (int64_t)one_scale << 12 | (int64_t)g.weight_layout << 13 | (int64_t)parts << 16 | (int64_t)(g.staged != 0) << 26 | (int64_t)apart << 27;
     static thread_local CallMemo<GemmChoice, 128> memo;
     return memo.get((int64_t)g.M | how << 32, g.N, g.K, g.ldo, [&]() {
-        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.xq_padded != 0, g.staged != 0, apart);
+        return choose_gemm(g.M, g.N, g.K, g.epilogue, g.ldo, vec_ok, out16, have_x, g.weight_layout, parts, norm, one_scale, g.staged != 0, apart);
     });
 }
 
@@ -554,10 +558,10 @@ size_t gemm_scratch_need(const GemmProblem& g) {
     return choose_gemm(g).need;
 }
 
-int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout, bool padded, bool staged) {
+int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout, bool staged) {
     // operands that satisfy every alignment requirement, dense output
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
-    const GemmChoice c = choose_kernel(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, padded, staged);
+    const GemmChoice c = choose_kernel(M, N, K, epilogue, ldo, true, ldo % 8 == 0, false, weight_layout, 0, false, false, staged);
     switch (c.kind) {
     case GemmChoice::SKINNY:
         return snprintf(buf, n, "small-m nt=%d mb=%d kpw=%d rounds=%d", c.sk.nt, c.sk.mb, c.sk.kpw, c.sk.rounds);
@@ -574,8 +578,7 @@ int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, i
 
 int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout) {
     const int64_t ldo = epi_is_gated(epilogue) ? N / 2 : N;
-    const bool padded = K % 128 != 0;   // (as the linears stage their codes)
-    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, padded, true, true);
+    const GemmChoice c = choose_gemm(M, N, K, epilogue, ldo, true, ldo % 8 == 0, true, weight_layout, 0, false, false, true, true);
     if (c.kind == GemmChoice::FUSED)
         return snprintf(buf, n, "one launch: small-m rows=%d nt=%d kpw=%d grid=%dx%d", c.fq.rows, c.fq.nt, c.fq.kpw, c.fq.tiles, c.fq.msplit);
     if (c.kind == GemmChoice::SELFQ)
@@ -584,7 +587,7 @@ int describe_linear_plan(int M, int N, int K, int epilogue, char* buf, size_t n,
         return snprintf(buf, n, "one launch: panel of 16 rows, nt=%d grid=%dx%d", c.pn.nt, c.pn.n_tiles, c.pn.m_tiles);
     const int len = snprintf(buf, n, "quantizer + ");
     if (len < 0 || (size_t)len >= n) return len;
-    return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout, padded, true);
+    return len + describe_gemm_plan(M, N, K, epilogue, buf + len, n - len, weight_layout, true);
 }
 
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order) {

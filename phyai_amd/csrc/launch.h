@@ -139,7 +139,7 @@ struct SkinnyPlan {
     int kpw;     // K steps per wavefront per round
     int rounds;
 };
-bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo, bool padded = false);
+bool skinny_applicable(int M, int N, int K, int epilogue, int64_t ldo);
 SkinnyPlan skinny_plan(int M, int N, int K, int epilogue);
 double skinny_cost(const SkinnyPlan& pl, int K);   // on the scale of big_cost
 int launch_gemm_skinny(const GemmProblem& p, const SkinnyPlan& pl, hipStream_t st);
@@ -196,7 +196,7 @@ struct BigPlan {
                  // wavefront that owns the columns, the activation stages handed over without barriers; 0: staged through LDS
 };
 BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w = false);
-// The same choice from measured costs, for codes that this library staged itself (rule: what big_plan says, tile 0 if nothing;
+// The same choice from measured costs (rule: what big_plan says, tile 0 if nothing;
 // shared: microseconds that every choice pays); what a shape costs beyond those, us.
 BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared);
 double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue);
@@ -210,6 +210,6 @@ int launch_set_stamp_sink_fused(unsigned long long* buf, unsigned int records);
 // Text form of what phyai_fp8_mlp launches for aligned, row-major operands.
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order = false);
 // Text form of launch_gemm's choice for aligned operands and a dense output; returns its length.
-int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0, bool padded = false, bool staged = false);
+int describe_gemm_plan(int M, int N, int K, int epilogue, char* buf, size_t n, int weight_layout = 0, bool staged = false);
 
 }  // namespace phyai

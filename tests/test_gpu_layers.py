@@ -273,7 +273,7 @@ def test_graph_replays_of_the_split_k_tile_kernel(L, dev):
 
 
 
-def test_a_graph_keeps_its_workspace_when_other_work_outgrows_it(L, dev):
+def test_a_graph_keeps_its_workspace_when_other_work_outgrows_it(L, dev, monkeypatch):
     """A recorded graph holds the addresses of its scratch (activation codes, split-K counters and
     partial sums).  Larger problems that later run eagerly - on the pooled stream the graph was
     recorded on as well as on the current one - must neither free nor share that scratch: the
@@ -281,7 +281,8 @@ def test_a_graph_keeps_its_workspace_when_other_work_outgrows_it(L, dev):
     from phyai_amd import ops
     from phyai_amd.runtime import HipGraph
 
-    x = seeded((200, 1040), 60).to(dev)                      # generic kernel, K split: counters + partial sums
+    monkeypatch.setenv("PHYAI_FP8_TILE", "128,128,3")        # the generic kernel, K split: counters + partial sums
+    x = seeded((200, 1040), 60).to(dev)
     wq, ws = ops.fp8_weight_quant(seeded((512, 1040), 61, 0.02).to(dev))
     assert ops.describe_plan(200, 512, 1040).startswith("generic 128x128 splits=")
     eager = ops.fp8_linear(x, wq, ws)

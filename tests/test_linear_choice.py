@@ -11,6 +11,10 @@ from conftest import seeded
 
 GATED = "geglu_tanh"
 
+# where the rules' lines alone or the width of a row of dense codes would have ready codes add in another order than staged ones
+APART = [(947, 768, 768), (1435, 640, 512), (738, 768, 1040), (1847, 1152, 8192), (643, 1280, 1024), (964, 768, 1040), (300, 384, 272),
+         (200, 512, 1040), (1894, 256, 736), (248, 2384, 704), (412, 2176, 15488), (178, 3584, 512)]
+
 
 def _shapes(n):
     rng = random.Random(1)
@@ -42,6 +46,26 @@ def test_layout_does_not_change_the_order_of_the_sums(monkeypatch):
         assert _kind(row) in (_kind(rule), "tile1", "small-m"), (m, n, k, epi, rule, row)   # nothing is newly split
         changed += row.removeprefix("quantizer + ") != rule
     assert changed > 50
+
+
+def test_ready_codes_add_in_the_order_of_staged_ones(monkeypatch):
+    """A norm's forward_fp8 and the linear behind it stand for the norm and the linear: a GEMM on ready codes adds in the order
+    of the linear that stages its own, at every size (one launch in the place of the two keeps that order, on the GPU)."""
+    from phyai_amd import ops
+
+    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "TILE", "RULES", "SKINNY_PLAN", "SKINNY_MAXM"):
+        monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    monkeypatch.setenv("PHYAI_FP8_FUSED", "0")
+    rng, shapes = random.Random(3), [(m, n, k, None) for m, n, k in APART]
+    for _ in range(4000):
+        m, n = round(2 ** rng.uniform(0, 13.7)), rng.choice([32 * rng.randint(1, 64), 128 * rng.randint(1, 100)])
+        k = rng.choice([16 * rng.randint(1, 128), 16 * rng.randint(1, 1024), 128 * rng.randint(1, 128)])
+        if m * k < 1 << 31:
+            shapes.append((m, n, k, rng.choice([None, None, "gelu", GATED])))
+    for m, n, k, epi in shapes:
+        for lay in [None, "operand_gated" if epi == GATED else "operand"][:2 if k % 128 == 0 else 1]:
+            ready, staged = ops.describe_plan(m, n, k, epi, weight_layout=lay), ops.describe_linear_plan(m, n, k, epi, weight_layout=lay)
+            assert _kind(ready) == _kind(staged), (m, n, k, epi, lay, ready, staged)
 
 
 def test_rules_alone(monkeypatch):
@@ -102,3 +126,32 @@ def test_chosen_kernel_in_both_layouts_and_without_a_workspace_of_its_own(dev, M
     if M * K < 24 << 20:
         _lib.check(rc, "static")
         assert torch.equal(got.view(torch.int16), out.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", APART)
+def test_ready_codes_give_the_bits_of_the_linear(dev, M, N, K):
+    """Per token, one static scale, and the adaptive norm in front: separate calls and the one that stands for them."""
+    from test_gpu_norm_linear import _norm_linear
+
+    from phyai_amd import _lib, ops
+
+    lib = _lib.load()
+    x, bias, mod = seeded((M, K), M + K).to(dev), seeded((N,), 4).to(dev), seeded((1, 3 * K), 6, 0.2).to(dev)
+    w, ws = ops.fp8_weight_quant(seeded((N, K), K, 0.02).to(dev))
+    one = torch.full((1,), 0.02, device=dev)
+    for layout in (None, "operand")[:2 if K % 128 == 0 else 1]:
+        wq = ops.fp8_weight_to_operand_order(w) if layout else w
+        how = dict(weight_layout=layout)
+        same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))
+        assert same(ops.fp8_linear(x, wq, ws, bias, **how), ops.fp8_gemm(*ops.fp8_quant_rowwise(x), wq, ws, bias, **how))
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        scratch = torch.zeros(lib.phyai_fp8_linear_workspace_bytes(M, N, K, 0), dtype=torch.uint8, device=dev)
+        _lib.check(lib.phyai_fp8_linear_per_tensor(
+            x.data_ptr(), K, one.data_ptr(), wq.data_ptr(), ws.data_ptr(), bias.data_ptr(), None, 0, None, 0, 0, out.data_ptr(), N, M, N, K,
+            ops.WEIGHT_LAYOUTS[layout], scratch.data_ptr(), scratch.numel(), torch.cuda.current_stream().cuda_stream), "per tensor")
+        assert same(out, ops.fp8_gemm(ops.fp8_quant_static(x, one), one, wq, ws, bias, **how))
+        xq, xs, _ = ops.adarmsnorm_fp8(x, mod, 1e-6)
+        ready = ops.fp8_gemm(xq, xs, wq, ws, bias, **how)
+        assert same(ops.fp8_linear(ops.adarmsnorm(x, mod, 1e-6)[0], wq, ws, bias, **how), ready)
+        assert same(_norm_linear(x, mod, wq, ws, bias, None, layout)[0], ready)
