@@ -975,8 +975,7 @@ def main() -> int:
     OPTS["operand"] = not args.row_major
     OPTS["mlp"] = not args.separate_linears
     if args.stamps:
-        if os.environ.get("PHYAI_FP8_LIBRARY") != "ablate":   # (`make ablate ABLATE=n`: the same table with parts of a main loop left out)
-            os.environ["PHYAI_FP8_LIBRARY"] = "stamps"        # before the library is opened
+        os.environ["PHYAI_FP8_LIBRARY"] = "stamps"            # before the library is opened
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py: this path is built and measured on ONE GPU (TP=1, no collectives); "
               "run with --gpus 1", file=sys.stderr)

@@ -69,17 +69,6 @@
 namespace phyai {
 
 constexpr int BIG_BK = 128;   // bytes of K per LDS row: one L2 cache line
-// Measurement only (make stamps ABLATE=n builds the time-stamp library with it; results are WRONG by design): parts
-// of the main loop left out, to see from the time stamps what each costs.  Bit 1: no copies / weight loads inside
-// the loop (the operands of the prologue are multiplied over and over); bit 2: the activation blocks of a K half
-// are not re-read from LDS; bit 4: no barrier / no hand-over between the wavefronts in the loop; bit 8 (weights in
-// registers): only the weight loads of the loop are left out; bit 16 (either variant): only the activation copies.
-#ifndef PHYAI_FP8_ABLATE
-#define PHYAI_FP8_ABLATE 0
-#endif
-#if PHYAI_FP8_ABLATE && !defined(PHYAI_FP8_STAMPS)
-#error "PHYAI_FP8_ABLATE is for the time-stamp build only"
-#endif
 // (debug build only: where the kernels below leave their time stamps - 1 first stage published, 2 main loop done,
 // 3 split-K sums gathered, 4 epilogue arithmetic done and tile staged, 5 stores issued)
 PHYAI_STAMP_SINK(g_big_stamps)
@@ -412,10 +401,9 @@ void gemm_fp8_big_kernel(
             return;
         }
         if (c < CA) {
-            if (!(PHYAI_FP8_ABLATE & 16) || d < LEAD) copy16_to_lds(p.a + k, aoff[c], wave_a + stage_off + c * 1024);
+            copy16_to_lds(p.a + k, aoff[c], wave_a + stage_off + c * 1024);
         } else if constexpr (BDIRECT) {
             constexpr int S = decltype(slot)::value;
-            if ((PHYAI_FP8_ABLATE & 8) && d >= LEAD) return;
             const int e = c - CA, j = e >> 2, b = (e >> 1) & 1, pr = e & 1;   // half pr of unit b of block j
             bring[S][j][b][pr] = *reinterpret_cast<const v4i*>(bsrc[j][b] + ((size_t)d << 11) + pr * 1024 + lane16);
         } else {
@@ -549,7 +537,7 @@ void gemm_fp8_big_kernel(
     {                                                                                                          \
         multiply(FB, FA, ACC);                                                                                 \
         _Pragma("unroll") for (int c_ = 0; c_ < CPS; ++c_)                                                     \
-            if (req_ && (SLOT_) * CPS + c_ < IDX_END && !(PHYAI_FP8_ABLATE & 1)) {                             \
+            if (req_ && (SLOT_) * CPS + c_ < IDX_END) {                                                        \
                 /* (register set of the load: its number modulo DEPTH) */                                      \
                 if (after_) issue(load_, (SLOT_) * CPS + c_, std::integral_constant<int, (stage_slot_ + LEAD) % DEPTH>{});     \
                 else issue(load_, (SLOT_) * CPS + c_, std::integral_constant<int, (stage_slot_ + LEAD - 1) % DEPTH>{}); \
@@ -565,7 +553,7 @@ void gemm_fp8_big_kernel(
         const uint8_t* nbuf_ = (P) == 0 ? stage_ptr(d_) : stage_ptr(d_ + 1);                                   \
         if ((P) == 0) {                                                                                        \
             _Pragma("unroll") for (int a_ = 0; a_ < AHEAD_BLOCKS; ++a_)                                        \
-                fa[1][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[0][a_] : big_frag(nbuf_, arow + a_ * 32 + 16, q);      \
+                fa[1][a_] = big_frag(nbuf_, arow + a_ * 32 + 16, q);                                           \
         }                                                                                                      \
         _Pragma("unroll") for (int jj_ = 0; jj_ < 2 * TN; ++jj_) {                                             \
             const bool after_ = (P) == 1 && jj_ >= 1;   /* past this stage-load's barrier */                   \
@@ -575,18 +563,18 @@ void gemm_fp8_big_kernel(
             _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) {                                                \
                 PHYAI_MFMA_SLOT(fb[jj_], fa[P][i_], acc[i_][jj_ >> 1][P][jj_ & 1], slot0_ + i_)                \
                 if (i_ >= AHEAD_BLOCKS && jj_ == 2 * TN - 1 && ((P) == 0 || (NEXT)))                           \
-                    fa[1 - (P)][i_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][i_] : big_frag(nbuf_, arow + i_ * 32 + 16 * (1 - (P)), q); \
+                    fa[1 - (P)][i_] = big_frag(nbuf_, arow + i_ * 32 + 16 * (1 - (P)), q);                     \
             }                                                                                                  \
             if ((P) == 1 && (NEXT)) {                                                                          \
                 if (jj_ == 0) {                                                                                \
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* my reads of stage-load D have landed */ \
                     wait_copies<COPIES * (AHEAD)>();               /* ... my copies of D+1 too ... */          \
-                    if (!(PHYAI_FP8_ABLATE & 4)) __syncthreads();  /* ... and so have everybody's */           \
+                    __syncthreads();  /* ... and so have everybody's */                                        \
                 }                                                                                              \
                 fb[jj_] = read_b(nbuf_, jj_);                                                                  \
                 /* the activation blocks of the next half 0: one or two behind each of the first groups */     \
                 _Pragma("unroll") for (int a_ = 0; a_ < AHEAD_BLOCKS; ++a_)                                    \
-                    if (a_ * TN / TM == jj_) fa[0][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[1][a_] : big_frag(nbuf_, arow + a_ * 32, q); \
+                    if (a_ * TN / TM == jj_) fa[0][a_] = big_frag(nbuf_, arow + a_ * 32, q);                   \
             }                                                                                                  \
         }                                                                                                      \
     }
@@ -596,7 +584,7 @@ void gemm_fp8_big_kernel(
 #define PHYAI_HAND_OVER(D_, AHEAD)                                                                             \
     {                                                                                                          \
         wait_copies<(AHEAD) == 0 ? 0 : ((AHEAD) - 1) * COPIES + (COPIES - CA)>();                              \
-        if (!(PHYAI_FP8_ABLATE & 4)) hand_over(D_, seen_);                                                     \
+        hand_over(D_, seen_);                                                                                  \
         asm volatile("" ::: "memory");                                                                         \
     }
 // Half P of stage-load D with weights in registers: row block after row block.  Four row blocks: all of a half's blocks are
@@ -613,11 +601,11 @@ void gemm_fp8_big_kernel(
         _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) {                                                    \
             if (i_ == 0 && !A_ALL_AHEAD) {                                                                     \
                 _Pragma("unroll") for (int a_ = 1; a_ < TM; ++a_)                                              \
-                    fa[P][a_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][0] : big_frag(abuf_, arow + a_ * 32 + 16 * (P), q); \
+                    fa[P][a_] = big_frag(abuf_, arow + a_ * 32 + 16 * (P), q);                                 \
             }                                                                                                  \
             if (A_ALL_AHEAD && (P) == 0 && i_ == TM - 1) seen_ = progress_words();                             \
             if (A_ALL_AHEAD && (NEXT))                                                                         \
-                fa[1 - (P)][i_] = (PHYAI_FP8_ABLATE & 2) ? fa[P][i_] : big_frag(nbuf_, arow + i_ * 32 + 16 * (1 - (P)), q); \
+                fa[1 - (P)][i_] = big_frag(nbuf_, arow + i_ * 32 + 16 * (1 - (P)), q);                         \
             if (i_ == 1 + (TM - 1) / (TN + 1) && !A_ALL_AHEAD && (NEXT)) fa[1 - (P)][0] = big_frag(nbuf_, arow + 16 * (1 - (P)), q); \
             const bool after_ = (P) == 1 && (i_ >= 1 || A_ALL_AHEAD);   /* past this stage-load's hand-over */ \
             const bool req_ = after_ ? (ISSUE) : (ISSUE_P);                                                    \
