@@ -128,16 +128,16 @@ __device__ __forceinline__ BigTile big_tile_of(int id, int m_tiles, int n_tiles,
     }
     return t;
 }
-// Tiles of the busiest XCD under that order (host side; the same arithmetic, band by band).
+// Tiles of the busiest XCD under that order (host side; the same arithmetic: whole bands and the last one).
 static int big_max_tiles_per_xcd(int m_tiles, int n_tiles, int band_rows) {
-    const int full = n_tiles >> 3, rest = n_tiles & 7;
-    int per_xcd[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int m = 0; m < m_tiles; m += band_rows) {
-        const int bm = m_tiles - m < band_rows ? m_tiles - m : band_rows;
-        for (int x = 0; x < 8; ++x) per_xcd[x] += bm * full + ((((x + 1) * rest * bm) >> 3) - ((x * rest * bm) >> 3));
-    }
+    const int full = n_tiles >> 3, rest = n_tiles & 7, bands = m_tiles / band_rows, last = m_tiles % band_rows;
     int mx = 0;
-    for (int x = 0; x < 8; ++x) mx = per_xcd[x] > mx ? per_xcd[x] : mx;
+    for (int x = 0; x < 8; ++x) {
+        const int of_band = (((x + 1) * rest * band_rows) >> 3) - ((x * rest * band_rows) >> 3);
+        const int of_last = (((x + 1) * rest * last) >> 3) - ((x * rest * last) >> 3);
+        const int n = m_tiles * full + bands * of_band + of_last;
+        mx = n > mx ? n : mx;
+    }
     return mx;
 }
 // Ids that order needs (host side).
@@ -1040,7 +1040,8 @@ static double big_fill(int tiles, int slots) {
     return rounds > 0 ? (double)tiles / ((double)rounds * slots) : 1.0;
 }
 
-// Whether an XCD takes tile rows instead of tile columns, and the bytes from HBM that this was chosen by.
+// Whether an XCD takes tile rows instead of tile columns, the bytes from HBM that this was chosen by, and the tiles that the
+// busiest XCD then has.
 // By default an XCD takes tile columns: its L2 then holds the weight rows of those columns once, but every XCD streams all
 // activation rows it meets.  With few tile columns and long rows of activations (816 x B tokens into a 16384 -> 2048
 // projection) that is eight copies of the larger operand; then the roles are exchanged.  Estimated bytes: the operand an XCD
@@ -1048,16 +1049,17 @@ static double big_fill(int tiles, int slots) {
 // 168 by tile rows.)
 // ... unless the busiest XCD then needs one more round of tiles than in the other order (13056 x 2560 x 2048 in 256 x 256
 // tiles: 510 tiles are 64 per XCD by tile columns, two rounds on 32 CUs, but 65 on some XCDs by tile rows: 93 against 75 us).
-static bool big_takes_rows(int M, int N, int K, int m_tiles, int n_tiles, int slots, double* bytes) {
+static bool big_takes_rows(int M, int N, int K, int m_tiles, int n_tiles, int slots, double* bytes, int* busiest) {
     const double a_bytes = (double)M * K, b_bytes = (double)N * K;
     const int band_c = 4, band_r = 4;
     const double by_cols = a_bytes * (n_tiles < 8 ? n_tiles : 8) + b_bytes * big_ceil_div(m_tiles, band_c);
     const double by_rows = b_bytes * (m_tiles < 8 ? m_tiles : 8) + a_bytes * big_ceil_div(n_tiles, band_r);
     bool rows = by_rows < 0.8 * by_cols;
-    const int rounds_c = big_ceil_div(big_max_tiles_per_xcd(m_tiles, n_tiles, 4), slots);
-    const int rounds_r = big_ceil_div(big_max_tiles_per_xcd(n_tiles, m_tiles, 4), slots);
+    const int most_c = big_max_tiles_per_xcd(m_tiles, n_tiles, 4), most_r = big_max_tiles_per_xcd(n_tiles, m_tiles, 4);
+    const int rounds_c = big_ceil_div(most_c, slots), rounds_r = big_ceil_div(most_r, slots);
     if (rounds_c != rounds_r) rows = rounds_r < rounds_c;
     *bytes = rows ? by_rows : by_cols;
+    *busiest = rows ? most_r : most_c;
     return rows;
 }
 
@@ -1232,8 +1234,9 @@ double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue) {
     const int bn = gated ? pl.cols / 2 : pl.cols;
     const int m_tiles = big_ceil_div(M, pl.tile), n_tiles = big_ceil_div(gated ? N / 2 : N, bn), slots = two ? 64 : 32;
     double bytes;
-    const bool by_rows = big_takes_rows(M, N, K, m_tiles, n_tiles, slots, &bytes);
-    const int busiest = pl.splits * (by_rows ? big_max_tiles_per_xcd(n_tiles, m_tiles, 4) : big_max_tiles_per_xcd(m_tiles, n_tiles, 4));
+    int busiest;
+    big_takes_rows(M, N, K, m_tiles, n_tiles, slots, &bytes, &busiest);
+    busiest *= pl.splits;
     const double S = (double)big_ceil_div(K, 128 * pl.splits), R = big_ceil_div(busiest, slots), x = (double)busiest / slots;
     const double ragged = K % 128 != 0 ? c.ragged : 0.0, epi = gated ? c.gated : epilogue != EPI_NONE ? c.act : 0.0;
     if (!two) return R * (c.round + epi) + x * c.part + S * (R * c.round_step + x * (c.part_step + ragged));
@@ -1244,16 +1247,18 @@ double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue) {
 
 // The cheapest unsplit tile shape by that account, `rule` (big_plan's choice, or no tile at all) where nothing is 8 % ahead
 // of it, `shared` being what all of them pay.  All unsplit shapes add in the same order of K.
-BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared) {
+BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared, double* cost) {
     static const BigPlan shapes[] = {{256, 256, 1, 0, 2, 0}, {224, 256, 1, 0, 2, 0}, {192, 128, 1, 0, 2, 0}, {128, 128, 1, 0, 4, 0},
                                      {128, 128, 1, 0, 2, 0}, {128, 64, 1, 0, 4, 0}, {96, 128, 1, 0, 4, 0}};
     BigPlan best = rule;
-    double lowest = rule.tile ? 0.92 * (big_cost(rule, M, N, K, epilogue) + shared) : 1e30;
+    const double of_rule = rule.tile ? big_cost(rule, M, N, K, epilogue) + shared : 1e30;
+    double lowest = 0.92 * of_rule;
+    *cost = of_rule;
     for (BigPlan pl : shapes) {
         if (epi_is_gated(epilogue) && (pl.cols == 64 || pl.tile == 96)) continue;
         pl.regs = operand_w ? big_register_ring(pl, K, epilogue) : 0;
         const double t = big_cost(pl, M, N, K, epilogue) + shared;
-        if (t < lowest) { lowest = t; best = pl; }
+        if (t < lowest) { *cost = lowest = t; best = pl; }
     }
     best.tiles = big_tiles(M, N, epilogue, best.tile, best.cols);
     return best;
@@ -1274,7 +1279,8 @@ static void big_launch(BigArgs a, const GemmProblem& g, int splits, hipStream_t 
     a.m_tiles = big_ceil_div(g.M, BM);
     // which operand the XCDs share
     double chosen_bytes;
-    a.by_rows = big_takes_rows(g.M, g.N, g.K, a.m_tiles, a.n_tiles, 32 * (big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1), &chosen_bytes);
+    int busiest;
+    a.by_rows = big_takes_rows(g.M, g.N, g.K, a.m_tiles, a.n_tiles, 32 * (big_two_per_cu(TM, TN, DEPTH, WMODE) ? 2 : 1), &chosen_bytes, &busiest);
     if (const char* e = tuning_env("PHYAI_FP8_BY_ROWS")) a.by_rows = atoi(e) != 0;
     // bands of 4 tile rows; a grid of up to 8 tile rows whose activation rows still fit an XCD's
     // L2 beside the weight stream is one band, so that the weights come from HBM once

@@ -465,11 +465,12 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
         bool tiles = rule.tile && out16 && !((few_small_tiles || one_round) && skinny_ok);
         bool as_ruled = true;   // the rules' tile shape adds in the order decided on
         const double shared = 5.2;   // launches and quantizer of a linear, us
+        BigPlan best = rule;
+        double tiled;
         if (by_cost && (tiles || skinny_ok)) {
-            const BigPlan best = big_plan_by_cost(M, N, K, epilogue, false, tiles ? rule : none, shared);
+            best = big_plan_by_cost(M, N, K, epilogue, false, tiles ? rule : none, shared, &tiled);
             if (skinny_ok && !(tiles && rule.splits > 1)) {   // (its estimate is poor at the long K that is split)
                 const double streaming = skinny_cost(skinny_plan(M, N, K, epilogue), K) + shared;
-                const double tiled = big_cost(best, M, N, K, epilogue) + shared;
                 if (tiles ? streaming < 0.92 * tiled : tiled < 0.92 * streaming) {
                     tiles = !tiles;
                     as_ruled = false;
@@ -479,9 +480,13 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
         }
         if (tiles) {
             c.kind = GemmChoice::BIG;
-            c.big = layout == W_ROW_MAJOR ? rule : big_plan(M, N, K, epilogue, true);
-            if (!as_ruled || (by_cost && staged && c.big.splits == 1))
-                c.big = big_plan_by_cost(M, N, K, epilogue, layout != W_ROW_MAJOR, as_ruled ? c.big : none, shared);
+            const bool priced = !as_ruled || (by_cost && staged && rule.splits == 1);
+            if (layout == W_ROW_MAJOR) {
+                c.big = priced ? best : rule;
+            } else {
+                c.big = as_ruled ? big_plan(M, N, K, epilogue, true) : none;
+                if (priced) c.big = big_plan_by_cost(M, N, K, epilogue, true, c.big, shared, &tiled);
+            }
             c.need = c.big.splits > 1 ? kHeaderBytes + big_partial_bytes(M, N, epilogue, c.big) : 0;
             return c;
         }

@@ -197,8 +197,8 @@ struct BigPlan {
 };
 BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w = false);
 // The same choice from measured costs (rule: what big_plan says, tile 0 if nothing;
-// shared: microseconds that every choice pays); what a shape costs beyond those, us.
-BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared);
+// shared: microseconds that every choice pays), with what it costs, those included; what a shape costs beyond those, us.
+BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, const BigPlan& rule, double shared, double* cost);
 double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue);
 size_t big_partial_bytes(int M, int N, int epilogue, const BigPlan& pl);
 int launch_gemm_big(const GemmProblem& p, const BigPlan& pl, hipStream_t st);
