@@ -12,10 +12,14 @@ from oracle import ref
 pytestmark = pytest.mark.gpu
 
 TILES = ["256", "224", "192", "128", "128/2", "96", "12864"]
+SPLIT = "128x2"   # 128 x 128 tiles, K split in two
 
 
 def _force(monkeypatch, tile):
     t, _, depth = tile.partition("/")
+    if tile == SPLIT:
+        t = "128"
+        monkeypatch.setenv("PHYAI_FP8_BIG_SPLITS", "2")
     monkeypatch.setenv("PHYAI_FP8_BIG", t)
     if depth:
         monkeypatch.setenv("PHYAI_FP8_BIG_DEPTH", depth)
@@ -28,8 +32,9 @@ def _codes(dev, m, k, seed):
 
 
 @pytest.mark.parametrize("layout", [None, "operand"])
-@pytest.mark.parametrize("tile", TILES)
-@pytest.mark.parametrize("M,N,K,epi", [(97, 144, 512, None), (225, 272, 640, "gelu"), (257, 528, 1024, "geglu_tanh"), (130, 96, 1040, "swiglu")])
+@pytest.mark.parametrize("tile", TILES + [SPLIT])
+@pytest.mark.parametrize("M,N,K,epi", [(97, 144, 512, None), (225, 272, 640, "gelu"), (257, 544, 1024, "geglu_tanh"), (130, 160, 1040, "swiglu"),
+                                       (257, 528, 1024, None)])
 def test_constants_from_any_address(dev, monkeypatch, tile, layout, M, N, K, epi):
     """Bias in whole words, at an odd 16-bit address (filled in by hand) and absent; tiles that end past M and N; one scale
     for all rows.  Every form against the values it stands for: the address changes no bit, no bias is a bias of zeros, one
@@ -37,19 +42,21 @@ def test_constants_from_any_address(dev, monkeypatch, tile, layout, M, N, K, epi
     from phyai_amd import ops
 
     gated = epi in ("geglu_tanh", "swiglu")
-    if tile in ("96", "12864") and gated or layout and K % 128:
+    if tile in ("96", "12864") and gated or layout and K % 128 or tile == SPLIT and K != 1024:
         pytest.skip("no such kernel")
+    assert not gated or N % 32 == 0 and N // 2 > 64     # more than one tile column of gate | up pairs
     _force(monkeypatch, tile)
     lay = None if layout is None else ("operand_gated" if gated else "operand")
-    if N % 32 and gated:
-        pytest.skip("gated widths are multiples of 32")
     xq, xs = _codes(dev, M, K, M + N)
     wq, ws = ops.fp8_weight_quant(seeded((N, K), M + K, 0.02).to(dev))
     if layout:
         wq = ops.fp8_weight_to_operand_order(wq, gated=gated)
     room = seeded((N + 8,), 7, 0.5).to(dev)
     run = lambda bias, scale=xs: ops.fp8_gemm(xq, scale, wq, ws, bias, epilogue=epi, weight_layout=lay).view(torch.int16)
-    assert ops.describe_plan(M, N, K, epi, weight_layout=lay).startswith("tile ")
+    plan = ops.describe_plan(M, N, K, epi, weight_layout=lay)
+    assert plan.startswith("tile ") and ("splits=2" in plan) == (tile == SPLIT)
+    if layout and not gated and K == 1024 and tile in ("128", SPLIT):   # (K / 2 is no trip round the ring of eight)
+        assert plan.endswith("ring of 8") == (tile == "128")
     odd = room[1:N + 1]
     assert odd.data_ptr() % 4 == 2
     assert torch.equal(run(odd), run(odd.clone()))
