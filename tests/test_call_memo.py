@@ -69,6 +69,11 @@ rnd = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(torch.bflo
 st = torch.cuda.current_stream().cuda_stream
 ws = torch.zeros(64 << 20, dtype=torch.uint8, device=dev)
 N, K = 1056, 1024
+# a linear that one launch takes (csrc/gemm_panel.hip) unless its output lies inside its rows; K that is padded where it is staged
+rows = rnd(400, 512)
+square, s_sq = ops.fp8_weight_quant(rnd(512, 512, scale=0.02))
+square = ops.fp8_weight_to_operand_order(square)
+ragged = [(rnd(m, k), *ops.fp8_weight_quant(rnd(n, k, scale=0.02))) for m, n, k in ((300, 1056, 656), (900, 272, 720), (70, 512, 1040))]
 xs = {m: rnd(m, K) for m in (1, 40, 100, 130, 300)}
 mod, gate = rnd(1, 3 * K, scale=0.2), rnd(1, N)
 w, s = ops.fp8_weight_quant(rnd(N, K, scale=0.02))
@@ -100,6 +105,21 @@ def calls():
             yield ("mlp", m, epi), out, lambda: lib.phyai_fp8_mlp(x.data_ptr(), K, w.data_ptr(), s.data_ptr(), None, 0, w2.data_ptr(), s2.data_ptr(), None, 0,
                 None, 0, None, 0, 0, out.data_ptr(), K, m, K, N // 2, K, epi, ws.data_ptr(), ws.numel(), st)
 
+    apart, inside = torch.zeros_like(rows), torch.zeros_like(rows)
+    square_call = lambda x, out: lib.phyai_fp8_linear(x.data_ptr(), 512, square.data_ptr(), s_sq.data_ptr(), None, out.data_ptr(), 512, 400, 512, 512,
+                                                      FLAG["op"], ws.data_ptr(), ws.numel(), st)
+    yield ("apart",), apart, lambda: square_call(rows, apart)
+    yield ("inside",), inside, lambda: square_call(inside.copy_(rows), inside)
+    for x, W, sc in ragged:
+        (m, k), n = x.shape, W.shape[0]
+        xq, xsc = ops.fp8_quant_rowwise(x)
+        out = torch.zeros(m, n, dtype=torch.bfloat16, device=dev)
+        tail = (out.data_ptr(), n, m, n, k, 0, ws.data_ptr(), ws.numel(), st)
+        yield ("ragged linear", m), out, lambda: lib.phyai_fp8_linear(x.data_ptr(), k, W.data_ptr(), sc.data_ptr(), None, *tail)
+        yield ("ragged static", m), out, lambda: lib.phyai_fp8_linear_per_tensor(x.data_ptr(), k, scalar.data_ptr(), W.data_ptr(), sc.data_ptr(), None,
+                                                                                 None, 0, None, 0, 0, *tail)
+        yield ("ragged gemm", m), out, lambda: lib.phyai_fp8_gemm(xq.data_ptr(), xsc.data_ptr(), 0, W.data_ptr(), sc.data_ptr(), None, *tail)
+
 results = {}
 for sweep in range(2):
     for name, out, call in calls():
@@ -109,6 +129,8 @@ for sweep in range(2):
         if sweep and not torch.equal(got.view(torch.int16), results[name].view(torch.int16)):
             sys.exit(f"second sweep differs: {name}")
         results[name] = got
+same = lambda a, b: torch.equal(results[a].view(torch.int16), results[b].view(torch.int16))
+assert same(("apart",), ("inside",)) and all(same(("ragged linear", x.shape[0]), ("ragged gemm", x.shape[0])) for x, _, _ in ragged)
 torch.save(results, sys.argv[1])
 print(len(results), "calls")
 """
