@@ -72,18 +72,22 @@ def test_weight_streaming_takes_every_padded_width(dev, monkeypatch, M, N, K, ep
     assert (got - want).norm() <= 2.0 ** -9 * want.norm()
 
 
-@pytest.mark.parametrize("M,D", [(1, 528), (150, 1040), (140, 8200), (3, 33808)])
-def test_quantizers_fill_the_rest_of_a_row_with_zeros(dev, M, D):
-    """Through the linears, whose scratch starts out full of NaN codes: per-token, static, and the adaptive norm's."""
+@pytest.mark.parametrize("M,K", [(140, 272), (1, 528), (150, 1040), (140, 2064), (139, 4112), (140, 8208), (70, 16400), (3, 33808)])
+def test_quantizers_fill_the_rest_of_a_row_with_zeros(dev, monkeypatch, M, K):
+    """Through the linears, whose scratch starts out full of NaN codes: per-token, static, and the adaptive norm's.  One K that
+    is padded in each of the launch forms of the quantizers (64, 128 and 256 threads, 1 - 16 chunks each, the loop)."""
     from phyai_amd import _lib, ops
 
-    lib, N = _lib.load(), 64
-    K = D // 16 * 16
-    x = _rows(max(M, 3), K, K)[:M].nan_to_num(0.0, 1.0, -1.0).to(dev)
+    monkeypatch.setenv("PHYAI_FP8_FUSED", "0")       # codes staged at every size
+    assert K % 128 != 0
+    lib, N, ldq = _lib.load(), 64, (K + 127) // 128 * 128
+    x = _rows(max(M, 3), K, K)[-M:].nan_to_num(0.0, 1.0, -1.0).to(dev)
     wq, ws = ops.fp8_weight_quant(seeded((N, K), K, 0.02).to(dev))
     scale, mod = torch.full((1,), 0.02, device=dev), seeded((1, 3 * K), 3, 0.1).to(dev)
     st = torch.cuda.current_stream().cuda_stream
     need = lib.phyai_fp8_linear_workspace_bytes(M, N, K, 0)
+    up = lambda n: (n + 255) // 256 * 256
+    codes_at = need - up(4 * M) - up(M * ldq)        # (the scratch ends in the codes and a scale per row)
     ref = {}
     for fill in (0, 0x7F):
         for name in ("token", "static", "norm"):
@@ -102,4 +106,6 @@ def test_quantizers_fill_the_rest_of_a_row_with_zeros(dev, M, D):
             _lib.check(rc, name)
             torch.cuda.synchronize()
             assert not bool(out.isnan().any())
+            codes = wsp[codes_at:codes_at + M * ldq].view(M, ldq)
+            assert not bool(codes[:, K:].any()) and bool(codes[:, :K].any())
             assert torch.equal(ref.setdefault(name, out), out)
