@@ -1,4 +1,4 @@
-"""Linears of more than 128 rows in one launch (csrc/gemm_panel.hip) against quantizer + GEMM, bit for bit: the edges of its
+"""Linears of more than 48 rows in one launch (csrc/gemm_panel.hip) against quantizer + GEMM, bit for bit: the edges of its
 tiles and of its K, both orders of sums, both kinds of scale, rows that are not finite, scales at the ends of the range,
 strided rows and outputs, a gated residual; and what it does not take over: an output inside its own rows, a call without a
 workspace."""

@@ -101,13 +101,24 @@ def test_where_one_launch_takes_more_rows(monkeypatch):
 
 
 # (rows, columns, K, epilogue): rule's shape -> chosen shape, one per pair that occurs
-CHANGED = [(3000, 2208, 1536, None), (2032, 9216, 640, "gelu"), (4310, 3648, 640, None), (497, 2432, 8320, None), (2489, 384, 1792, None),
-           (2553, 864, 8320, None), (1665, 7680, 2560, None), (1301, 768, 8448, None), (1047, 896, 9216, None), (400, 6144, 8192, None)]
+CHANGED = [(2032, 9216, 640, "gelu"), (4310, 3648, 640, None), (497, 2432, 8320, None), (2489, 384, 1792, None), (2553, 864, 8320, None),
+           (400, 6144, 8192, None), (3548, 3392, 5120, None), (3531, 8160, 640, None), (2740, 1056, 8448, None), (278, 3072, 9600, None)]
+
+
+@pytest.mark.parametrize("M,N,K,epi", CHANGED)
+def test_costs_choose_another_shape_than_the_rules(monkeypatch, M, N, K, epi):
+    from phyai_amd import ops
+
+    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "TILE", "RULES", "FUSED"):
+        monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    chosen = ops.describe_linear_plan(M, N, K, epi)
+    monkeypatch.setenv("PHYAI_FP8_RULES", "1")
+    assert chosen.startswith("quantizer + ") and ops.describe_linear_plan(M, N, K, epi) != chosen
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,epi", CHANGED)
-def test_chosen_kernel_in_both_layouts_and_without_a_workspace_of_its_own(dev, M, N, K, epi):
+def test_chosen_kernel_in_both_layouts_and_without_a_workspace_of_its_own(dev, monkeypatch, M, N, K, epi):
     """Operand order changes no bit, the static-scratch form gives the same where its array holds the codes, and the result is
     the rules' kernel's up to the order of fp32 sums (2^-7 of the largest output covers one bf16 step on either side)."""
     from phyai_amd import _lib, ops
@@ -118,7 +129,11 @@ def test_chosen_kernel_in_both_layouts_and_without_a_workspace_of_its_own(dev, M
     relaid = ops.fp8_linear(x, ops.fp8_weight_to_operand_order(wq), ws, epilogue=epi, weight_layout="operand")
     assert torch.equal(got.view(torch.int16), relaid.view(torch.int16))
     xq, xs = ops.fp8_quant_rowwise(x)
-    want = ops.fp8_gemm(xq, xs, wq, ws, epilogue=epi).float()
+    ready = ops.fp8_gemm(xq, xs, wq, ws, epilogue=epi)
+    assert torch.equal(got.view(torch.int16), ready.view(torch.int16))
+    with monkeypatch.context() as rules:
+        rules.setenv("PHYAI_FP8_RULES", "1")
+        want = ops.fp8_linear(x, wq, ws, epilogue=epi).float()
     assert (got.float() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
     out = torch.empty_like(got)
     rc = _lib.load().phyai_fp8_linear_static(x.data_ptr(), K, wq.data_ptr(), ws.data_ptr(), None, out.data_ptr(), N, M, N, K,
