@@ -148,6 +148,8 @@ size_t phyai_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int epi
  * Per-tensor layers (torch.py:123-153) pass x_scale_is_scalar = 1 and a pointer
  * to the single input scale.  Requires K % 16 == 0 and N % 16 == 0
  * (the same gate as TorchKernel.can_handle, torch.py:91).
+ * Products are summed in the order of the linear of the same shape: a quantizer of this library
+ * followed by this call gives the bits of phyai_fp8_linear / _linear_per_tensor (same alignment of out).
  */
 int phyai_fp8_gemm(const void *xq, const float *x_scale, int x_scale_is_scalar,
                    const void *w, const float *w_scale, const void *bias,
@@ -326,7 +328,9 @@ int phyai_fp8_describe_plan(int64_t M, int64_t N, int64_t K, int epilogue, char 
  * The same for phyai_fp8_linear (bf16 activations in, dense rows): either
  *   "one launch: small-m rows=8 nt=5 kpw=1 grid=32x7"      the kernel that quantizes its own token rows
  *   "one launch: rows in registers, rows=8 nt=1 steps=6 grid=64x2"   the one for K that the first does not take
- * or "quantizer + " followed by what phyai_fp8_describe_plan reports.  Host only.  The layout flag of
+ *   "one launch: panel of 16 rows, nt=2 grid=20x25"        the one for more rows and K up to 1024
+ * or "quantizer + " followed by a GEMM in the words of phyai_fp8_describe_plan (the same order of sums as on ready codes,
+ * maybe another tile).  Host only.  The layout flag of
  * the weight matrix (PHYAI_FP8_FLAG_W_OPERAND_ORDER / _GATED) may be or-ed into `epilogue` as in the
  * calls: a few shapes are one launch only with weights in operand order (registers instead of LDS).
  */

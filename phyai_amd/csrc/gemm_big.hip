@@ -1078,9 +1078,10 @@ static int big_register_ring(const BigPlan& pl, int K, int epilogue) {
 static bool big_two_of(const BigPlan& pl) { return pl.depth == 2 && (pl.tile == 192 || pl.tile == 128); }
 
 // Tile shape, K splits, ring depth.  All times in here: graphs of weight sets beyond the Infinity Cache, every tile shape
-// forced in turn at 988 shapes (M = 136 .. 13056, N = 1024 .. 32768, K = 1024 .. 16384, both layouts); over all of them the
-// choice is 1.6 % behind the best shape in the geometric mean.  The lines were drawn on an earlier main loop (32 x 32 x 64
-// MFMAs); where another shape is ahead by now, the comment says so.
+// forced in turn at 988 shapes (M = 136 .. 13056, N = 1024 .. 32768, K = 1024 .. 16384, both layouts).  The lines were drawn on
+// an earlier main loop (32 x 32 x 64 MFMAs) and epilogue, whose times these are; where another shape is ahead by now, the comment
+// says so.  With the fitted costs below (launch_gemm's choice: the order of sums for every GEMM, the tile shape for codes that a
+// linear stages) ready codes are 1.0 % behind the best of all shapes in the geometric mean, linears 0.6 %.
 BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     BigPlan pl = {0, 0, 1, 0, 0, 0};
     if (K < 512) return pl;   // the stage-loads must fill the ring

@@ -4,7 +4,8 @@
 // What bounds these calls is not bytes or operations (400 x 2560 x 1024: 1.1 us of either) but the two kernels' dependent
 // trips to memory and the quantizer's own node and launch: 7.6 us in a graph (now 6.7), and called eagerly two launches, which
 // cost the host 6 us (the call takes 1.27 - 1.45 times as long as one launch's: 400 x 2560 x 1024, 1000 x 1024 x 512,
-// 100 x 1536 x 656).  Here everything a workgroup needs is asked for at once and nothing is waited for twice:
+// 100 x 1536 x 656).  Here a workgroup asks for rows, weights, scales and bias
+// at once and waits for them once (for a gated residual and its gate once more, behind the MFMAs):
 //
 //  * four wavefronts own 64 NT weight rows x 16 token rows over the whole K; wavefront w converts four of the rows for all
 //    of them (one barrier) and multiplies 16 NT weight rows, whose whole K is in flight in registers from the first
