@@ -55,7 +55,7 @@ def test_linear_equals_gemm_on_dense_codes(dev, monkeypatch, kernel, M, N, K, ep
 @pytest.mark.parametrize("K", [272, 400, 1040, 1264, 16368])
 @pytest.mark.parametrize("M,N,epi", [(65, 512, None), (200, 640, "gelu"), (130, 544, "swiglu"), (1100, 272, None)])
 def test_weight_streaming_takes_every_padded_width(dev, monkeypatch, M, N, K, epi):
-    """... also where dense codes of that K go to the generic kernel: against that one, whose sums come in another order
+    """Against the generic kernel, whose sums come in another order
     (fp32 sums of up to K products: a relative 2^-9 of the largest output covers the bf16 rounding on both sides)."""
     from phyai_amd import ops
 
