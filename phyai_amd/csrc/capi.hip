@@ -744,10 +744,11 @@ int phyai_fp8_debug_stamps(uint64_t* records, int64_t n_records) {
         return fail(PHYAI_FP8_EINVAL, "phyai_fp8_debug_stamps: bad arguments");
     const int a = phyai::launch_set_stamp_sink_big(reinterpret_cast<unsigned long long*>(records), (unsigned int)n_records);
     const int b = phyai::launch_set_stamp_sink_fused(reinterpret_cast<unsigned long long*>(records), (unsigned int)n_records);
-    if (a == -2 || b == -2)
+    const int c = phyai::launch_set_stamp_sink_tall(reinterpret_cast<unsigned long long*>(records), (unsigned int)n_records);
+    if (a == -2 || b == -2 || c == -2)
         return fail(PHYAI_FP8_EUNSUPPORTED, "phyai_fp8_debug_stamps: this library was built without time stamps "
                     "(make stamps builds lib/libphyai_fp8_stamps.so)");
-    if (a != 0 || b != 0) return fail(PHYAI_FP8_ELAUNCH, "phyai_fp8_debug_stamps: hipMemcpyToSymbol failed");
+    if (a != 0 || b != 0 || c != 0) return fail(PHYAI_FP8_ELAUNCH, "phyai_fp8_debug_stamps: hipMemcpyToSymbol failed");
     return PHYAI_FP8_OK;
 }
 

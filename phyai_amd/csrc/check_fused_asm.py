@@ -17,7 +17,7 @@ returns a list of violations over every instantiation of the kernel:
   wait's ``N``;
 * the kernel uses scratch memory (a spilled register in that stretch could be one of the loads').
 
-``check_tile_usage`` is the guard of gemm_big.hip, whose global -> LDS copies are inline assembly too and whose
+``check_tile_usage`` is the guard of gemm_big.hip and gemm_tall.hip, whose global -> LDS copies are inline assembly too and whose
 ``s_waitcnt vmcnt(N)`` count, by hand, the vector-memory instructions of a wavefront in issue order: a kernel of that
 file that spills has scratch loads and stores of the compiler's among them, and a wait would then let a stage be
 read before it has landed.  It reads the compiler's resource-usage remarks that the Makefile keeps beside every
@@ -162,12 +162,32 @@ def usage_problems(text: str, kernel: str = "gemm_fp8_big_kernel", min_kernels: 
     return bad
 
 
+def tall_usage_problems(text: str, min_kernels: int = 50) -> list[str]:
+    """gemm_tall.hip: no scratch either, and no accumulation registers beyond the 16 per row block that hold the sums.  Its
+    MFMAs are inline assembly: were sums moved between registers, or others kept in these, the compiler would place such
+    moves without the wait states that an MFMA's result needs."""
+    bad, name = usage_problems(text, "gemm_fp8_tall_kernel", min_kernels), None
+    for line in text.split("\n"):
+        m = re.search(r"remark: Function Name: (\S+)", line)
+        if m:
+            name = re.search(r"gemm_fp8_tall_kernelILi(\d+)E", m.group(1))
+            continue
+        m = re.search(r"remark:\s+AGPRs: (\d+)", line)
+        if m and name is not None and int(m.group(1)) != 16 * int(name.group(1)):
+            bad.append(f"{name.group(0)}: {m.group(1)} accumulation registers for {name.group(1)} row blocks")
+    return bad
+
+
 def check_tile_usage(stamps: bool = False) -> list[str]:
     """The pipelined tile kernels of the built library (or of the time-stamp build) use no scratch memory."""
-    path = os.path.join(CSRC, "_obj", ("stamps_" if stamps else "") + "gemm_big.o.usage")
-    if not os.path.exists(path):
-        return [f"{path} is missing (make -C {CSRC} all stamps writes it)"]
-    return usage_problems(open(path, encoding="utf-8", errors="replace").read())
+    bad = []
+    for source, problems in (("gemm_big", usage_problems), ("gemm_tall", tall_usage_problems)):
+        path = os.path.join(CSRC, "_obj", ("stamps_" if stamps else "") + source + ".o.usage")
+        if not os.path.exists(path):
+            bad.append(f"{path} is missing (make -C {CSRC} all stamps writes it)")
+        else:
+            bad += problems(open(path, encoding="utf-8", errors="replace").read())
+    return bad
 
 
 if __name__ == "__main__":

@@ -442,7 +442,7 @@ static GemmChoice choose_kernel(int M, int N, int K, int epilogue, int64_t ldo, 
     // the costs choose for staged codes; ready ones keep the rules' shape where it adds in that order.
     // Nothing becomes split along K that the rules leave whole.
     const bool by_cost = M >= 129 && K >= 512 && out16 && !tuning_env("PHYAI_FP8_BIG") && !tuning_env("PHYAI_FP8_TILE") &&
-                         !tuning_env("PHYAI_FP8_BIG_DEPTH") && !tuning_env("PHYAI_FP8_BIG_SPLITS") && !tuning_env("PHYAI_FP8_RULES");
+                         !tuning_env("PHYAI_FP8_BIG_DEPTH") && !tuning_env("PHYAI_FP8_BIG_SPLITS") && !tuning_env("PHYAI_FP8_TALL") && !tuning_env("PHYAI_FP8_RULES");
     if (!tuning_env("PHYAI_FP8_TILE")) {
         const BigPlan none = {0, 0, 1, 0, 0, 0}, rule = big_plan(M, N, K, epilogue, false);
         // Beyond 1024 rows every weight tile is walked by 16 workgroups and more, whose codes no L2 holds once K is 8192: with

@@ -187,7 +187,8 @@ int launch_gemm_panel(const GemmProblem& p, const PanelPlan& pl, bool by_waves, 
 // Pipelined tile kernel for large M (gemm_big.hip); 128 x 128 tiles may be split along K (partials in the workspace,
 // as for the generic tile kernel).
 struct BigPlan {
-    int tile;    // tile rows: 256 (x 256 columns), 224 (x 256), 192 (x 128), 128 (x 128 or x 64), 96 (x 128), or 0 if the kernel does not apply
+    int tile;    // tile rows: 256 (x 256 columns), 224 (x 256), 192 (x 128), 128 (x 128 or x 64), 96 (x 128), or 0 if the kernel does not apply;
+                 // 144 .. 256 in steps of 16 (x 256) with regs = 4: gemm_tall.hip
     int cols;    // tile columns
     int splits;
     int tiles;   // output tiles of that size
@@ -202,10 +203,14 @@ BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, cons
 double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue);
 size_t big_partial_bytes(int M, int N, int epilogue, const BigPlan& pl);
 int launch_gemm_big(const GemmProblem& p, const BigPlan& pl, hipStream_t st);
+// Tiles of `rows` (144 .. 256, a multiple of 16) x 256 for weights in operand order, K a multiple of 512 (gemm_tall.hip).
+int launch_gemm_tall(const GemmProblem& p, int rows, hipStream_t st);
+bool tall_reaches(const GemmProblem& p);   // whether rows of output, residual and gate lie close enough for it
 
 // Debug build (-DPHYAI_FP8_STAMPS) only: where the kernels of gemm_big.hip / gemm_skinny_fused.hip write their time
 // stamps (stamps.h); -2 in the normal build.
 int launch_set_stamp_sink_big(unsigned long long* buf, unsigned int records);
+int launch_set_stamp_sink_tall(unsigned long long* buf, unsigned int records);
 int launch_set_stamp_sink_fused(unsigned long long* buf, unsigned int records);
 // Text form of what phyai_fp8_mlp launches for aligned, row-major operands.
 int describe_mlp_plan(int M, int H, int I, int O, int epilogue, char* buf, size_t n, bool operand_order = false);
