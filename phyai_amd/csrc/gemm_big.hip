@@ -971,7 +971,7 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     const bool ragged = K % 128 != 0;
     if (const char* e = tuning_env("PHYAI_FP8_TALL")) {   // rows of a tile of gemm_tall.hip, where it takes the problem
         const int rows = atoi(e);
-        if (operand_w && K % 512 == 0 && rows >= 144 && rows <= 256 && rows % 16 == 0) return {rows, 256, 1, big_tiles(M, N, epilogue, rows, 256), 2, 4};
+        if (operand_w && K % 128 == 0 && rows >= 144 && rows <= 256 && rows % 16 == 0) return {rows, 256, 1, big_tiles(M, N, epilogue, rows, 256), 2, 4};
     }
     int forced = -1;
     if (const char* e = tuning_env("PHYAI_FP8_BIG")) forced = atoi(e);   // "0": never; "256"/"192"/"128": force
@@ -1172,7 +1172,7 @@ BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, cons
     // Tall tiles where they are ahead of that (by 4 % below 60 us, where the costs are less sure): in half of 1800 linears that
     // tiles serve, 7.3 % less time in the geometric mean over all of them, quantizer included (0.9 % behind the best shape), and
     // more than 2 % slower in 9.
-    if (operand_w && K % 512 == 0) {
+    if (operand_w && K % 128 == 0) {
         lowest = (big_tall(best) || *cost - shared >= 60.0 ? 1.0 : 0.96) * *cost;
         for (int rows = 144; rows <= 256; rows += 16) {
             const BigPlan pl = {rows, 256, 1, 0, 2, 4};

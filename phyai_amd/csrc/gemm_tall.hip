@@ -61,7 +61,6 @@ void gemm_fp8_tall_kernel(
     constexpr int STAGE_BYTES = CA * 32 * BIG_BK;
     constexpr int DEPTH = 4, LEAD = 3, CLAIM = 2, SLACK = 1;   // (see hand_over)
     constexpr int SLOTS_AFTER = 4 * (H1 - 1);        // MFMAs of a stage-load behind its hand-over
-    constexpr int CPS = (COPIES + SLOTS_AFTER - 1) / SLOTS_AFTER;   // requests behind each of them
     static_assert(R >= 9 && R <= 16, "144 to 256 rows");
     // a staged row block of the epilogue; two per wavefront
     constexpr int TNO = GATED ? 1 : 2;               // output column blocks of 32 per wavefront
@@ -125,15 +124,14 @@ void gemm_fp8_tall_kernel(
     };
 
     // ---- requests ----------------------------------------------------------------------------------
-    v4i bring[DEPTH][4][2];                          // [stage-load % DEPTH][block][chunk pair]
-    // request c of stage-load d: the wavefront's activation copies, then its weights
-    auto issue = [&](int d, int c, auto slot) __attribute__((always_inline)) {
-        if (c < CA) {
-            copy16_to_lds(a_a + d * BIG_BK, aoff[c], wave_a + decltype(slot)::value * STAGE_BYTES + c * 1024);
-        } else {
-            const int e = c - CA, jj = e >> 1, pr = e & 1;
-            bring[decltype(slot)::value][jj][pr] = *reinterpret_cast<const v4i*>(bsrc[jj] + ((size_t)d << 11) + pr * 1024 + lane16);
-        }
+    v4i bring[DEPTH][4][2];                          // [set][block][chunk pair]
+    // Stage-load d of a tile lies in stage (ring + d) % 4 of LDS: the ring goes on from tile to tile, whatever K leaves over
+    // beyond a multiple of four.  Register sets have to be named at compile time: see `turn`.
+    int ring = 0;
+    auto stage_at = [&](int base, int d) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_readfirstlane(((base + d) & 3) * STAGE_BYTES); };
+    auto copy = [&](int d, int c, uint32_t at) __attribute__((always_inline)) { copy16_to_lds(a_a + d * BIG_BK, aoff[c], wave_a + at + c * 1024); };
+    auto load = [&](int d, int e, auto set) __attribute__((always_inline)) {
+        bring[decltype(set)::value][e >> 1][e & 1] = *reinterpret_cast<const v4i*>(bsrc[e >> 1] + ((size_t)d << 11) + (e & 1) * 1024 + lane16);
     };
     const bool bias_rides = a_bias != nullptr && (reinterpret_cast<uintptr_t>(a_bias) & 3) == 0;
     // Blocks of the constants: row scales of the tile, the weight scales of its columns (gated: gate columns, then up
@@ -187,13 +185,13 @@ void gemm_fp8_tall_kernel(
     // Request n of a tile's opening, stage-loads 0 and 1: first what stage 0 waits for - its weights come from HBM - and the
     // activations that progress word -1 vouches for (0 .. CLAIM - 1), then the constants and the weights of stage-load 1.
     constexpr int OPENING = 2 * COPIES + CONSTS;
-    auto opening = [&](auto n_, int const_at) __attribute__((always_inline)) {
+    auto opening = [&](auto n_, int const_at, int base) __attribute__((always_inline)) {
         constexpr int n = decltype(n_)::value;
-        if constexpr (n < BL) issue(0, CA + n, S0{});
-        else if constexpr (n < BL + CA) issue(0, n - BL, S0{});
-        else if constexpr (n < BL + 2 * CA) issue(1, n - BL - CA, S1{});
+        if constexpr (n < BL) load(0, n, S0{});
+        else if constexpr (n < BL + CA) copy(0, n - BL, stage_at(base, 0));
+        else if constexpr (n < BL + 2 * CA) copy(1, n - BL - CA, stage_at(base, 1));
         else if constexpr (n < BL + 2 * CA + CONSTS) constants(n - BL - 2 * CA, const_at);
-        else issue(1, n - COPIES - CONSTS, S1{});
+        else load(1, n - BL - 2 * CA - CONSTS, S1{});
     };
 
     // ---- hand-over ---------------------------------------------------------------------------------
@@ -234,87 +232,88 @@ void gemm_fp8_tall_kernel(
     using No = std::integral_constant<int, 0>; using Yes = std::integral_constant<int, 1>;
     v8i fa[2][H0];
     constexpr int AHEAD = 2;   // blocks of a half that are read during the half before it
-    // Lane (l16, q) of row block b reads chunks q and 4 + q of its row.  Two base addresses per chunk, for stages 0, 1 and 2, 3 of
-    // the ring: the rest of an address fits the instruction's 16-bit offset.
-    uint32_t frag_at[2][2];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        frag_at[e >> 1][e & 1] = lds_base + (e >> 1) * (2 * STAGE_BYTES) + l16 * BIG_BK + (((q + 4 * (e & 1)) ^ big_swizzle(l16)) << 4);
-        asm volatile("" : "+v"(frag_at[e >> 1][e & 1]));
-    }
-    auto frag = [&](auto slot, int b) __attribute__((always_inline)) {
-        constexpr int S = decltype(slot)::value;
-        const int at = (S & 1) * STAGE_BYTES + b * (16 * BIG_BK);
-        return big_join(*(const lds_v4i_t*)(frag_at[S >> 1][0] + at), *(const lds_v4i_t*)(frag_at[S >> 1][1] + at));
+    // Lane (l16, q) of row block b reads chunks q and 4 + q of its row: frag_lo and frag_hi beyond the stage's place and the block.
+    uint32_t frag_lo = lds_base + l16 * BIG_BK + ((q ^ big_swizzle(l16)) << 4), frag_hi = lds_base + l16 * BIG_BK + (((q + 4) ^ big_swizzle(l16)) << 4);
+    asm volatile("" : "+v"(frag_lo), "+v"(frag_hi));
+    auto frag = [&](uint32_t lo, uint32_t hi, int b) __attribute__((always_inline)) {
+        return big_join(*(const lds_v4i_t*)(lo + b * (16 * BIG_BK)), *(const lds_v4i_t*)(hi + b * (16 * BIG_BK)));
     };
-    // Half P of stage-load d: row blocks P * H0 .. of it against all four weight blocks.  The blocks that open a half are read
-    // during the half before it, the others behind the first MFMAs' issue; the hand-over comes behind the first row block of
-    // half 1.  Requests go out between the MFMAs, spread over both halves - four wavefronts that send theirs in one half keep
-    // each other waiting for the CU's address unit: the weights of stage-load d + 2 in half 0, behind the hand-over of half 1 the
-    // activation copies of stage-load d + LEAD.
-    // next: stage-load d + 1 follows; in_flight: stage-loads from d + CLAIM on that have been requested; ask: 1 as said, 2 copies
-    // and weights both (half 0 of a tile's first stage-load, half 1 of the last but three), 0 nothing;
-    // first: the tile's first stage-load; beside(n): other work behind MFMA n.
-    auto half = [&](int d, auto slot, auto p_, auto next, auto in_flight, auto ask, auto first, auto beside) __attribute__((always_inline)) {
-        constexpr int S = decltype(slot)::value, P = decltype(p_)::value, HP = P ? H1 : H0;
+    // Half P of stage-load d (register set S): row blocks P * H0 .. of it against all four weight blocks.  The blocks that open a
+    // half are read during the half before it, the others behind the first MFMAs' issue; the hand-over comes behind the first
+    // row block of half 1.  Requests go out between the MFMAs, spread over both halves - four wavefronts that send theirs in one
+    // half keep each other waiting for the CU's address unit: the weights of stage-load d + 2 in half 0, behind the hand-over of
+    // half 1 the activation copies of stage-load d + LEAD.
+    // next: stage-load d + 1 follows in the main loop; ask: 1 as said, 2 (half 0 of a tile's first stage-load) copies and weights
+    // both, 0 nothing; first: that stage-load; beside(n): other work behind MFMA n.
+    auto half = [&](int d, auto set, auto p_, auto next, auto ask, auto first, auto beside) __attribute__((always_inline)) {
+        constexpr int S = decltype(set)::value, P = decltype(p_)::value, HP = P ? H1 : H0, ASK = decltype(ask)::value;
         constexpr bool NEXT = decltype(next)::value;
-        constexpr int ASK = decltype(ask)::value;
-        constexpr int F = decltype(in_flight)::value, OPEN_NEXT = HP - AHEAD < 3 ? HP - AHEAD : 3;
-        constexpr std::integral_constant<int, P ? (S + 1) % DEPTH : S> opens;   // the stage whose block opens the next half
+        constexpr int OPEN_NEXT = HP - AHEAD < 3 ? HP - AHEAD : 3;
+        const uint32_t here_at = stage_at(ring, d), next_at = P ? stage_at(ring, d + 1) : here_at;   // ... whose block opens the next half
+        const uint32_t lo = frag_lo + here_at, hi = frag_hi + here_at, next_lo = P ? frag_lo + next_at : lo, next_hi = P ? frag_hi + next_at : hi;
+        const uint32_t copies_at = stage_at(ring, d + 2 + P);
         v4i seen = {0, 0, 0, 0};
         if constexpr (P == 1 && NEXT) seen = progress_words();
 #pragma unroll
         for (int i = 0; i < HP; ++i) {
             if (i == 0) {
 #pragma unroll
-                for (int b = AHEAD; b < HP; ++b) fa[P][b] = frag(slot, P * H0 + b);
+                for (int b = AHEAD; b < HP; ++b) fa[P][b] = frag(lo, hi, P * H0 + b);
             }
-            if (i >= OPEN_NEXT && i < OPEN_NEXT + AHEAD && (P == 0 || NEXT)) fa[1 - P][i - OPEN_NEXT] = frag(opens, (1 - P) * H0 + i - OPEN_NEXT);
+            if (i >= OPEN_NEXT && i < OPEN_NEXT + AHEAD && (P == 0 || NEXT)) fa[1 - P][i - OPEN_NEXT] = frag(next_lo, next_hi, (1 - P) * H0 + i - OPEN_NEXT);
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
                 multiply(big_join(bring[S][jj][0], bring[S][jj][1]), fa[P][i], acc[P * H0 + i][jj], first);
                 const int slot_n = P ? (i - 1) * 4 + jj : i * 4 + jj;
                 if constexpr (ASK == 2) {
-#pragma unroll
-                    for (int c = 0; c < (P ? CPS : 1); ++c) {
-                        const int n = slot_n * (P ? CPS : 1) + c;
-                        if (slot_n >= 0 && n < COPIES) issue(d + 2 + P, n, std::integral_constant<int, (S + 2 + P) % DEPTH>{});
-                    }
+                    if (slot_n < CA) copy(d + 2, slot_n, copies_at);
+                    else if (slot_n < COPIES) load(d + 2, slot_n - CA, std::integral_constant<int, (S + 2) % DEPTH>{});
                 } else if constexpr (ASK == 1) {
                     constexpr int REQUESTS = P ? CA : BL, MFMAS = P ? SLOTS_AFTER : 4 * H0;
                     const int n = slot_n * REQUESTS / MFMAS;
-                    if (slot_n == 0 || (slot_n > 0 && n != (slot_n - 1) * REQUESTS / MFMAS))
-                        issue(d + 2 + P, P ? n : CA + n, std::integral_constant<int, (S + 2 + P) % DEPTH>{});
+                    if (slot_n == 0 || (slot_n > 0 && n != (slot_n - 1) * REQUESTS / MFMAS)) {
+                        if constexpr (P == 0) load(d + 2, n, std::integral_constant<int, (S + 2) % DEPTH>{});
+                        else copy(d + LEAD, n, copies_at);
+                    }
                 }
                 beside(i * 4 + jj);
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (P == 1 && i == 0 && NEXT) {
-                // my activation copies of d + CLAIM have landed; its weights and everything later may be in flight
-                wait_copies<F == 0 ? 0 : (F - 1) * COPIES + BL>();
+                wait_copies<BL>();   // my activation copies of d + CLAIM have landed; its weights may be in flight
                 hand_over(d, seen);
                 asm volatile("" ::: "memory");
             }
         }
     };
     static_assert(COPIES <= 4 * H0, "the first stage-load's first half asks for stage-load 2");
-    auto nothing = [](int) __attribute__((always_inline)) {};
+    static_assert(CA <= SLOTS_AFTER && BL <= 4 * H0, "one request behind an MFMA");
     using Two = std::integral_constant<int, 2>;
-    auto stage = [&](int d, auto slot, auto next, auto in_flight, auto ask0, auto ask1) __attribute__((always_inline)) {
-        half(d, slot, No{}, Yes{}, No{}, ask0, No{}, nothing);
-        half(d, slot, Yes{}, next, in_flight, ask1, No{}, nothing);
+    auto nothing = [](int) __attribute__((always_inline)) {};
+    auto stage = [&](int d, auto set) __attribute__((always_inline)) {
+        half(d, set, No{}, Yes{}, Yes{}, No{}, nothing);
+        half(d, set, Yes{}, Yes{}, Yes{}, No{}, nothing);
+    };
+    // The loop over stage-loads names sets 0 .. 3 in turn and ends with sets 2 and 3.  Up to three stage-loads beyond a multiple of
+    // four come before it, each in set 1, the two behind it moving up.
+    auto turn = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            bring[1][e >> 1][e & 1] = bring[2][e >> 1][e & 1];
+            bring[2][e >> 1][e & 1] = bring[3][e >> 1][e & 1];
+        }
     };
 
     // ---- the last two stage-loads and the epilogue -------------------------------------------------
     // Row block by row block: the eight MFMAs that end block r's sums between the pieces of block r - 1's epilogue, which is
-    // several times as much VALU work.  (One wavefront per SIMD: nothing else would multiply meanwhile.)  Stages 0 and 1 of the
-    // ring and their register sets are free by now: the next tile's opening goes out in between, a request behind each piece
+    // several times as much VALU work.  (One wavefront per SIMD: nothing else would multiply meanwhile.)  Two stages of the ring and
+    // two register sets are free by now: the next tile's opening goes out in between, a request behind each piece
     // (asked for all at once, by all CUs, it would hold up the wavefront for 6 k cycles).
     // The weight block is the MFMA's first operand: register e of lane (l16, q) of block (r, jj) is token row 16 r + l16, column
     // 16 jj + 4 q + e of the wavefront (gated operand order: registers 0, 1 are gate and 2, 3 up of output columns 8 jj + 2 q,
     // + 1).  A finished row block passes through the wavefront's own two slots of LDS (16-byte slots XOR-swizzled with the row)
     // and leaves row-wise, 16 bytes per lane, two blocks later.  Output is written once and never read here: non-temporal.
-    auto tail = [&](const int em0, const int en0, const int const_at, const int next_const_at, const bool more) __attribute__((always_inline)) {
+    auto tail = [&](const int em0, const int en0, const int const_at, const int next_const_at, const int next_ring, const bool more) __attribute__((always_inline)) {
         const int lane = here(threadIdx.x & 63), l16 = lane & 15, q = lane >> 4;
         const float* const const_x = reinterpret_cast<const float*>(lds + const_at);
         const float* const const_w = const_x + XBLOCKS * 64;
@@ -340,7 +339,9 @@ void gemm_fp8_tall_kernel(
                 }
             }
         const int sw = (l16 / ROWS_PER_PASS) & (SLOTS - 1);
-        v8i f0 = frag(S2{}, 0), f1 = frag(S3{}, 0);
+        const uint32_t at0 = stage_at(ring, n_loads - 2), at1 = stage_at(ring, n_loads - 1);
+        const uint32_t lo0 = frag_lo + at0, hi0 = frag_hi + at0, lo1 = frag_lo + at1, hi1 = frag_hi + at1;
+        v8i f0 = frag(lo0, hi0, 0), f1 = frag(lo1, hi1, 0);
         float s_next = const_x[l16];
         // Where lane's 16 bytes of a row block go.  Through a buffer resource that ends with the matrix's last row, so that rows
         // past it are not written (nor the residual's read); lanes of columns past the matrix stay beyond the resource.  (A
@@ -366,8 +367,8 @@ void gemm_fp8_tall_kernel(
                 if constexpr (e == 0 && r >= 1 && r <= R) s = s_next;
                 if constexpr (r < R) {
                     multiply(big_join(bring[2 + (e >> 2)][e & 3][0], bring[2 + (e >> 2)][e & 3][1]), e < 4 ? f0 : f1, acc[r][e & 3], No{});
-                    if constexpr (e == 3 && r + 1 < R) f0 = frag(S2{}, r + 1);
-                    if constexpr (e == 7 && r + 1 < R) f1 = frag(S3{}, r + 1);
+                    if constexpr (e == 3 && r + 1 < R) f0 = frag(lo0, hi0, r + 1);
+                    if constexpr (e == 7 && r + 1 < R) f1 = frag(lo1, hi1, r + 1);
                 }
                 if constexpr (e == 0 && r >= 3) {   // block r - 3 leaves
 #pragma unroll
@@ -444,7 +445,7 @@ void gemm_fp8_tall_kernel(
                 }
                 constexpr int n = piece * OPENING / (8 * R);   // (evenly over the pieces beside MFMAs)
                 if constexpr (r < R && (piece == 0 || n != (piece - 1) * OPENING / (8 * R))) {
-                    if (more) opening(std::integral_constant<int, n>{}, next_const_at);
+                    if (more) opening(std::integral_constant<int, n>{}, next_const_at, next_ring);
                 }
                 __builtin_amdgcn_sched_barrier(0);
         });
@@ -454,10 +455,12 @@ void gemm_fp8_tall_kernel(
 #pragma unroll
     for (int step = 0; step <= CA; ++step) take_tile(step);
     int parity = 0;
-    tall_each<OPENING>([&](auto n) __attribute__((always_inline)) { opening(n, CONST_AT); });
+    tall_each<OPENING>([&](auto n) __attribute__((always_inline)) { opening(n, CONST_AT, 0); });
     fill_bias(CONST_AT);
 #pragma unroll
-    for (int c = 0; c < COPIES; ++c) issue(2, c, S2{});
+    for (int c = 0; c < CA; ++c) copy(2, c, stage_at(0, 2));
+#pragma unroll
+    for (int e = 0; e < BL; ++e) load(2, e, S2{});
     for (bool first = true;; first = false) {
         // Stage-load 0 and the activations up to stage-load CLAIM - 1 have landed (what progress word -1 stands for; the
         // stores of the tile before, younger than all of these, only make the wait stricter).  The first tile's stage-load 2
@@ -468,39 +471,40 @@ void gemm_fp8_tall_kernel(
         __syncthreads();
         PHYAI_STAMP(1)
 #pragma unroll
-        for (int b = 0; b < AHEAD; ++b) fa[0][b] = frag(S0{}, b);
-        if (first) half(0, S0{}, No{}, Yes{}, No{}, No{}, Yes{}, nothing);
-        else half(0, S0{}, No{}, Yes{}, No{}, Two{}, Yes{}, nothing);
+        for (int b = 0; b < AHEAD; ++b) fa[0][b] = frag(frag_lo + stage_at(ring, 0), frag_hi + stage_at(ring, 0), b);
+        if (first) half(0, S0{}, No{}, Yes{}, No{}, Yes{}, nothing);
+        else half(0, S0{}, No{}, Yes{}, Two{}, Yes{}, nothing);
         const bool more = next_tile();   // (behind MFMAs that are still to run)
-        half(0, S0{}, Yes{}, Yes{}, Yes{}, Yes{}, Yes{}, nothing);
-        // DEPTH stage-loads per trip: the register sets are named at compile time (the launcher sees to it that K holds a
-        // whole number of trips).
+        half(0, S0{}, Yes{}, Yes{}, Yes{}, Yes{}, nothing);
         int d = 0;
-        if (n_loads > DEPTH) {
-            stage(1, S1{}, Yes{}, Yes{}, Yes{}, Yes{});
-            stage(2, S2{}, Yes{}, Yes{}, Yes{}, Yes{});
-            stage(3, S3{}, Yes{}, Yes{}, Yes{}, Yes{});
-            for (d = DEPTH; d < n_loads - DEPTH; d += DEPTH) {
-                stage(d, S0{}, Yes{}, Yes{}, Yes{}, Yes{});
-                stage(d + 1, S1{}, Yes{}, Yes{}, Yes{}, Yes{});
-                stage(d + 2, S2{}, Yes{}, Yes{}, Yes{}, Yes{});
-                stage(d + 3, S3{}, Yes{}, Yes{}, Yes{}, Yes{});
-            }
-            stage(d, S0{}, Yes{}, Yes{}, Yes{}, Two{});   // stage n - 4 asks for all of the last stage-load
-        } else {
-#pragma unroll
-            for (int c = CA; c < COPIES; ++c) issue(LEAD, c, S3{});
+        for (; d < (n_loads & (DEPTH - 1)); ++d) {
+            stage(d + 1, S1{});
+            turn();
         }
+        if (d < n_loads - DEPTH) {
+            stage(d + 1, S1{});
+            stage(d + 2, S2{});
+            stage(d + 3, S3{});
+            for (d += DEPTH; d < n_loads - DEPTH; d += DEPTH) {
+                stage(d, S0{});
+                stage(d + 1, S1{});
+                stage(d + 2, S2{});
+                stage(d + 3, S3{});
+            }
+            stage(d, S0{});
+        }
+        half(d + 1, S1{}, No{}, Yes{}, Yes{}, No{}, nothing);
         const int em0 = m0, en0 = n0, const_at = CONST_AT + parity * CONST_BYTES;
-        half(d + 1, S1{}, No{}, Yes{}, No{}, No{}, No{}, take_tile);   // (nothing asks for this tile's rows any more)
-        half(d + 1, S1{}, Yes{}, No{}, No{}, No{}, No{}, nothing);
+        half(d + 1, S1{}, Yes{}, No{}, No{}, No{}, take_tile);   // (nothing asks for this tile's places any more)
         PHYAI_STAMP(2)
-        wait_copies<0>();
-        __syncthreads();   // the last two stage-loads and all constants have landed, everyone is done with those before
+        wait_copies<BL>();
+        __syncthreads();   // the activations of the last two stage-loads and all constants have landed, everyone is done with those before
         parity ^= 1;
         const int next_const_at = CONST_AT + parity * CONST_BYTES;
         PHYAI_STAMP(3)
-        tail(em0, en0, const_at, next_const_at, more);
+        const int next_ring = (ring + n_loads) & 3;
+        tail(em0, en0, const_at, next_const_at, next_ring, more);
+        ring = next_ring;
         PHYAI_STAMP(4)
         if (!more) break;
         fill_bias(next_const_at);
@@ -548,7 +552,7 @@ bool tall_reaches(const GemmProblem& g) {
 }
 
 int launch_gemm_tall(const GemmProblem& g, int rows, hipStream_t st) {
-    if (g.weight_layout == W_ROW_MAJOR || g.K % (4 * BIG_BK) != 0 || g.K < 4 * BIG_BK) return -2;
+    if (g.weight_layout == W_ROW_MAJOR || g.K % BIG_BK != 0 || g.K < 4 * BIG_BK) return -2;
     if (g.ldo % 8 != 0 || (reinterpret_cast<uintptr_t>(g.out) & 15) != 0 || !tall_reaches(g)) return -2;   // (16 bytes per lane leave)
     switch (rows) {
     case 144: return tall_launch_epi<9>(g, st);

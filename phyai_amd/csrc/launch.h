@@ -203,7 +203,7 @@ BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, cons
 double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue);
 size_t big_partial_bytes(int M, int N, int epilogue, const BigPlan& pl);
 int launch_gemm_big(const GemmProblem& p, const BigPlan& pl, hipStream_t st);
-// Tiles of `rows` (144 .. 256, a multiple of 16) x 256 for weights in operand order, K a multiple of 512 (gemm_tall.hip).
+// Tiles of `rows` (144 .. 256, a multiple of 16) x 256 for weights in operand order, K a multiple of 128 from 512 on (gemm_tall.hip).
 int launch_gemm_tall(const GemmProblem& p, int rows, hipStream_t st);
 bool tall_reaches(const GemmProblem& p);   // whether rows of output, residual and gate lie close enough for it
 

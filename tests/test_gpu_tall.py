@@ -40,7 +40,7 @@ def _both(monkeypatch, rows, call, M, N, K, epi=None):
     return got, want
 
 
-# one trip round the ring of stages (K = 512) and several; one row, a row short of a tile, a row over, many; columns that end in
+# one trip round the ring of stages (K = 512) and several, one to three stages of 128 beyond; one row, a row short of a tile, a row over, many; columns that end in
 # the first, second and last 16 of a tile; gated: half of them, in steps of 16
 @pytest.mark.parametrize("rows", ROWS)
 @pytest.mark.parametrize("epi", [None, "gelu", "gelu_tanh", "geglu_tanh", "geglu_erf", "swiglu"])
@@ -48,7 +48,8 @@ def test_edges_of_tiles(dev, monkeypatch, rows, epi):
     from phyai_amd import ops
 
     gated = bool(epi) and epi.startswith(("geglu", "swiglu"))
-    for M, N, K in ((rows - 1, 272, 512), (rows + 1, 1056, 1024), (129, 2048, 1536), (2 * rows + 17, 288, 2048), (3 * rows, 512, 512)):
+    for M, N, K in ((rows - 1, 272, 512), (rows + 1, 1056, 1024), (129, 2048, 1536), (2 * rows + 17, 288, 2048), (3 * rows, 512, 512),
+                    (rows + 33, 288, 640), (rows, 544, 768), (rows + 1, 288, 896), (2 * rows, 288, 1152), (rows - 7, 288, 1664), (rows + 2, 288, 1408)):
         N = (N + 31) // 32 * 32 if gated else N
         xq, xs, wq, ws, wo = _operands(dev, M, N, K, gated)
         bias = seeded((N + 1,), N, 0.1).to(dev)
@@ -61,10 +62,11 @@ def test_edges_of_tiles(dev, monkeypatch, rows, epi):
 @pytest.mark.parametrize("epi", [None, "geglu_tanh"])
 def test_several_tiles_per_workgroup(dev, monkeypatch, rows, epi):
     """More tiles than workgroups (256): openings under epilogues, both halves of the constants' place, the order of the tiles
-    with and without columns beyond the last eight; every pass gives the same."""
+    with and without columns beyond the last eight, tiles that open on every stage of the ring; every pass gives the same."""
     from phyai_amd import ops
 
-    for M, N, K in ((5 * rows + 40, 16384 + 32, 512), (40 * rows - 5, 2048, 1024), (17 * rows, 5 * 1024, 512)):
+    for M, N, K in ((5 * rows + 40, 16384 + 32, 512), (40 * rows - 5, 2048, 1024), (17 * rows, 5 * 1024, 512),
+                    (41 * rows + 1, 4096, 640), (40 * rows - 5, 4096 + 32, 768), (36 * rows, 4096, 896), (35 * rows, 2048, 1664)):
         xq, xs, wq, ws, wo = _operands(dev, M, N, K, epi is not None)
         for _ in range(2):
             got, want = _both(monkeypatch, rows, lambda lay: ops.fp8_gemm(xq, xs, wo, ws, epilogue=epi, weight_layout=lay), M, N, K, epi)
@@ -135,4 +137,5 @@ def test_planner_takes_tall_tiles_of_the_height_that_fills_the_rounds():
         plan = d(m, n, k, epi, weight_layout="operand_gated" if epi else "operand")
         assert plan.startswith(f"quantizer + tile {rows}x256 ") and plan.endswith(R4), plan
     assert "x256" not in d(816, 2048, 2048, weight_layout="operand")                 # 32 tiles
-    assert R4 not in d(4800, 2048, 8192) and R4 not in d(4800, 2048, 8192 + 128, weight_layout="operand")
+    assert R4 not in d(4800, 2048, 8192) and R4 not in d(4800, 2048, 8192 + 32, weight_layout="operand")
+    assert d(5000, 1280, 5120, weight_layout="operand").endswith(R4) and d(4800, 2048, 8192 + 128, weight_layout="operand").endswith(R4)
