@@ -140,27 +140,30 @@ __device__ __forceinline__ float gelu_tanh_f(float v) {
     const float e = __builtin_amdgcn_exp2f(v * __builtin_fmaf(b, v * v, a));
     return __builtin_fmaf(-v, __builtin_amdgcn_rcpf(e + 1.0f), v);
 }
-// gelu(v) = 0.5 v (1 + erf(v / sqrt 2)) without branches.  For x >= 0, erfc(x) = t P(t) exp(-x^2)
-// with t = 1 / (1 + 0.4 x) and P a degree-8 polynomial fitted to erfc(x) exp(x^2) with relative
-// error 1.2e-7 on [0, 30] (the form of Abramowitz & Stegun 7.1.26, more terms).  1 + erf(v / sqrt 2)
-// is erfc(|x|) for v < 0 - no cancellation in the negative tail - and 2 - erfc(x) otherwise.
-// Relative error of the result below 1e-5, so it rounds to the same bf16 as the exact value
-// except for about one input in 10^4.
+// gelu(v) = 0.5 v (1 + erf(v / sqrt 2)) = max(v, 0) - 0.5 |v| erfc(x), x = |v| / sqrt 2, without branches.
+// erfc(x) = t P(t) exp(-x^2) with t = 1 / (1 + 0.42 x) and P a degree-7 polynomial (the form of Abramowitz & Stegun
+// 7.1.26, more terms), fitted to erfc(x) exp(x^2) / t on [0, 9.4] - beyond, exp(-x^2) underflows - with relative error below
+// 2.6e-8 (1 + 0.3 x^2): it may grow as the exponential's own does.  The coefficients hold the 0.5.  No cancellation in the
+// negative tail.  Over all bf16 inputs with a result: relative error of at most 3.5e-6 below -8, 1.3e-6 to -4, 5e-7 elsewhere (rms
+// 1e-7), and each rounds to the bf16 of the exact value.  17 instructions, 2 of them at quarter rate; the epilogue of a large
+// tile is made of little else, and nothing else runs beside it (with a polynomial of degree 8 and the sign chosen by compare and
+// select it was 20, with the same error: 4800 x 8192 x 2048 + GELU in 208-row tiles 91.0 -> 86.6 us, 9600 x 4096 x 2048 99.8 -> 95.2,
+// 2400 x 16384 x 2048 + GeGLU 83.3 -> 80.6).  min keeps +inf * 0 out; -inf gives NaN, as 0.5 v (1 + erf) does.  (In assembly: the
+// compiler's min and max quiet their operand first, an instruction more.)
 __device__ __forceinline__ float gelu_erf_f(float v) {
-    const float av = __builtin_fabsf(v);
-    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.4f * 0.70710678118654752f, av, 1.0f));
-    float q = __builtin_fmaf(t, 0.04973088949918747f, -0.18051011860370636f);
-    q = __builtin_fmaf(t, q, 0.16458380222320557f);
-    q = __builtin_fmaf(t, q, -0.0010123166721314192f);
-    q = __builtin_fmaf(t, q, 0.13867421448230743f);
-    q = __builtin_fmaf(t, q, 0.169526606798172f);
-    q = __builtin_fmaf(t, q, 0.20764122903347015f);
-    q = __builtin_fmaf(t, q, 0.2256908118724823f);
-    q = __builtin_fmaf(t, q, 0.22567500174045563f);
+    float finite, positive;
+    asm("v_min_f32 %0, %1, %2" : "=v"(finite) : "s"(3.4028234663852886e38f), "v"(v));
+    asm("v_max_f32 %0, %1, %2" : "=v"(positive) : "s"(-0.0f), "v"(v));   // (-0: gelu(-0) is -0)
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.42f * 0.70710678118654752f, __builtin_fabsf(v), 1.0f));
+    float q = __builtin_fmaf(t, 0.03729753941297531f, -0.16925470530986786f);
+    q = __builtin_fmaf(t, q, 0.2361270934343338f);
+    q = __builtin_fmaf(t, q, -0.07985885441303253f);
+    q = __builtin_fmaf(t, q, 0.1421242356300354f);
+    q = __builtin_fmaf(t, q, 0.09500597417354584f);
+    q = __builtin_fmaf(t, q, 0.12017125636339188f);
+    q = __builtin_fmaf(t, q, 0.11838746070861816f);
     const float e = __builtin_amdgcn_exp2f((v * v) * (-0.5f * 1.4426950408889634f));
-    const float erfc_abs = (q * t) * e;
-    const float one_plus_erf = v < 0.0f ? erfc_abs : 2.0f - erfc_abs;
-    return (0.5f * v) * one_plus_erf;
+    return __builtin_fmaf(-__builtin_fabsf(q * (t * finite)), e, positive);
 }
 __device__ __forceinline__ float silu_f(float v) { return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v)); }
 

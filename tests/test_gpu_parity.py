@@ -8,6 +8,8 @@ sums are exact in fp32 must be bit-exact.
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -315,6 +317,28 @@ def test_epilogue_activation_values(dev, monkeypatch, epi_name, epi, M, force_bi
     clean = y[:, :K] > -2.0
     agree = float((got == want)[clean].float().mean())
     assert agree > 0.995, f"{epi_name}: only {agree:.4f} of the rounded results agree"
+
+
+@pytest.mark.parametrize("M", [16, 256])
+def test_gelu_of_every_bf16(dev, M):
+    """Zero weights hand the bias to the activation: all 65536 bf16 values of it.  gelu is computed to a relative 3.5e-6, so a
+    result is within that and half a bf16 step (2^-8 of the power of two below it) of the exact value; results
+    below 2^-126 may be flushed.  NaN and -inf give NaN (0.5 v (1 + erf v) does), +inf itself, zeros zeros."""
+    ops = _ops()
+    N, K = 65536, 128
+    bias = torch.arange(N, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    xq = torch.zeros(M, K, dtype=torch.float8_e4m3fn, device=dev)
+    wq = torch.zeros(N, K, dtype=torch.float8_e4m3fn, device=dev)
+    got = ops.fp8_gemm(xq, torch.ones(M, 1, device=dev), wq, torch.ones(N, device=dev), bias.to(dev), epilogue="gelu").cpu()
+    assert bool((got.view(torch.int16) == got[:1].view(torch.int16)).all())
+    got, v = got[0].double(), bias.double()
+    nan = torch.isnan(v) | (v == -math.inf)
+    assert torch.equal(torch.isnan(got), nan) and bool((got[v == math.inf] == math.inf).all())
+    assert bool((got[v == 0] == 0).all())
+    ok = ~nan & torch.isfinite(v)
+    exact = (0.5 * v * torch.special.erfc(-v / math.sqrt(2.0)))[ok]
+    half_step = 2.0 ** (torch.floor(torch.log2(exact.abs().clamp_min(2.0 ** -126))) - 8)
+    assert bool(((got[ok] - exact).abs() <= half_step + 3.5e-6 * exact.abs() + 2.0 ** -126).all())
 
 
 def test_linear_no_bias_and_batched(dev):
