@@ -41,6 +41,7 @@ struct Lib {
     decltype(&phyai_fp8_weight_quant_rowwise) weight_quant;
     decltype(&phyai_fp8_weight_to_operand_order) relay;
     decltype(&phyai_fp8_weight_to_operand_order_inplace) relay_inplace;
+    int (*relay_gated)(void*, int64_t, int64_t, void*, void*);   // phyai_host_relay_gated (weight_layout.hip)
     decltype(&phyai_fp8_linear_per_tensor) per_tensor;
     decltype(&phyai_fp8_rmsnorm_quant) rmsnorm;
     decltype(&phyai_fp8_adarmsnorm_quant) adarmsnorm;
@@ -575,6 +576,11 @@ PyObject* py_relay_weight(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* p = w->mutable_data_ptr();
     if (!gated && lib.relay_inplace(p, N, K, at_.stream) == 0) Py_RETURN_TRUE;
     at::Tensor t = at::Tensor(at::detail::empty_cuda(w->sizes(), w->scalar_type(), at_.dev, std::nullopt));
+    if (gated) {
+        const int rc = lib.relay_gated(p, N, K, t.mutable_data_ptr(), at_.stream);
+        if (rc == 0) Py_RETURN_TRUE;
+        TORCH_CHECK(rc == -2, "relay_weight: a launch failed");   // (some units may be re-laid already)
+    }
     // (a plain copy first and the re-lay back: the allocator's stream order covers the temporary)
     if (hipMemcpyAsync(t.mutable_data_ptr(), p, (size_t)(N * K), hipMemcpyDeviceToDevice, at_.stream) != hipSuccess) return declined();
     if (lib.relay(t.const_data_ptr(), N, K, gated, p, at_.stream) != 0) return declined();
@@ -814,6 +820,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     get(l.weight_quant, "phyai_fp8_weight_quant_rowwise");
     get(l.relay, "phyai_fp8_weight_to_operand_order");
     get(l.relay_inplace, "phyai_fp8_weight_to_operand_order_inplace");
+    get(l.relay_gated, "phyai_host_relay_gated");
     get(l.per_tensor, "phyai_fp8_linear_per_tensor");
     get(l.rmsnorm, "phyai_fp8_rmsnorm_quant");
     get(l.adarmsnorm, "phyai_fp8_adarmsnorm_quant");

@@ -1,11 +1,12 @@
 // Re-lays a row-major fp8 weight matrix into MFMA operand order (weight_layout.h), once per layer
-// after loading.  One thread moves one 16-byte chunk; consecutive threads write consecutive chunks
+// after loading.  One thread moves four 16-byte chunks; consecutive threads write consecutive chunks
 // of the destination, so the writes are contiguous and the reads are 16-byte pieces of 16
-// neighbouring rows.
+// neighbouring rows.  Bound by bytes (6.8 TB/s); four requests in flight per thread instead of one keep it there.
 //
 // A plain matrix is re-laid in place: unit u (16 rows x K) holds the same bytes in both orders, so a workgroup takes them
 // into its registers, waits for everyone and writes them back - half the bytes of re-laying into a second matrix and
-// copying that back.  A gated unit takes rows from both halves of the matrix, so that form stays out of place.
+// copying that back.  A gated unit takes rows from both halves of the matrix and goes through a second one, three quarters of
+// it where the matrix is large (phyai_host_relay_gated).
 #include <hip/hip_runtime.h>
 
 #include "fp8_device.h"
@@ -14,18 +15,34 @@
 
 namespace phyai {
 
-__global__ __launch_bounds__(256) void weight_to_operand_order_kernel(const uint4* __restrict__ w, uint4* __restrict__ out,
-                                                                      uint32_t N, uint32_t K, int gated, uint64_t chunks) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;   // destination chunk
-    if (i >= chunks) return;
+// Chunks [first * K, first * K + chunks) of the destination, i.e. units from `first` on (a unit is K chunks).  Gated: gate rows
+// from `gate`, up rows from `up`, both counted from column 0; plain: rows of the matrix at `gate`.
+__global__ __launch_bounds__(256) void weight_to_operand_order_kernel(const v4i* gate, const v4i* up, v4i* out,
+                                                                      uint32_t first, uint32_t K, int gated, uint32_t chunks) {
     const uint32_t steps = K >> 7;
-    const uint32_t r = (uint32_t)(i & 15), c = (uint32_t)((i >> 4) & 7);
-    const uint64_t us = i >> 7;                                     // u * steps + s
-    const uint32_t u = (uint32_t)(us / steps), s = (uint32_t)(us % steps);
-    uint32_t row;
-    if (gated) row = ((r >> 1) & 1) * (N >> 1) + 8 * u + 2 * (r >> 2) + (r & 1);
-    else row = 16 * u + r;
-    out[i] = w[((uint64_t)row * K + ((uint64_t)s << 7) + (c << 4)) >> 4];
+    v4i v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t t = blockIdx.x * 1024 + j * 256 + threadIdx.x, i = t < chunks ? t : chunks - 1;
+        const uint32_t r = i & 15, c = (i >> 4) & 7, us = i >> 7;   // us = u * steps + s
+        const uint32_t u = first + us / steps, s = us % steps;
+        const uint32_t row = gated ? 8 * u + 2 * (r >> 2) + (r & 1) : 16 * u + r;
+        v[j] = (gated && (r & 2) ? up : gate)[(size_t)row * (K >> 4) + s * 8 + c];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t i = blockIdx.x * 1024 + j * 256 + threadIdx.x;
+        if (i < chunks) out[(size_t)first * K + i] = v[j];
+    }
+}
+
+// The up half of a gated matrix, `half` chunks from chunk `half` on, and its first `kept` chunks behind it.
+__global__ __launch_bounds__(256) void weight_save_kernel(const v4i* __restrict__ w, v4i* __restrict__ saved, uint32_t half, uint32_t kept) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t i = blockIdx.x * 1024 + j * 256 + threadIdx.x;
+        if (i < half + kept) saved[i] = w[i < half ? half + i : i - half];
+    }
 }
 
 // CHUNKS 16-byte chunks per thread: K <= 1024 * CHUNKS.
@@ -61,13 +78,39 @@ int launch_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, hipStr
     return 0;
 }
 
+static void launch_units(const v4i* gate, const v4i* up, v4i* out, uint32_t first, uint32_t end, uint32_t K, int gated, hipStream_t st) {
+    const uint32_t chunks = (end - first) * K;
+    hipLaunchKernelGGL(weight_to_operand_order_kernel, dim3((chunks + 1023) / 1024), dim3(256), 0, st, gate, up, out, first, K, gated, chunks);
+}
+
 int launch_weight_to_operand_order(const void* w, int64_t N, int64_t K, int gated, void* out, hipStream_t st) {
-    const uint64_t chunks = (uint64_t)N * (uint64_t)K / 16;
-    const uint64_t blocks = (chunks + 255) / 256;
-    if (blocks > 0x7FFFFFFFull) return -2;
-    hipLaunchKernelGGL(weight_to_operand_order_kernel, dim3((unsigned)blocks), dim3(256), 0, st,
-                       static_cast<const uint4*>(w), static_cast<uint4*>(out), (uint32_t)N, (uint32_t)K, gated, chunks);
+    if (N * K > 0x7FFFFFFFll) return -2;
+    const v4i* rows = static_cast<const v4i*>(w);
+    launch_units(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st);
     return 0;
 }
 
 }  // namespace phyai
+
+// The gated form in place, for the host extension beside this library (no part of the C interface): w as
+// phyai_fp8_weight_to_operand_order() takes it, scratch of 3/4 N * K bytes.  -2: not for this form, nothing done.
+//
+// Saving the whole matrix and re-laying from there moves every byte four times.  The upper half of the units needs less: it
+// overwrites the up half of the matrix and reads the upper gate rows, which are still in place.  So the up half and the
+// lower gate rows are saved, the upper units go first and the lower ones, all of whose rows are saved, after them: 3.5 times,
+// for one more launch.  us, event-timed in a stream, whole copy / this: 32768 x 2048 43.8 / 39.4, 4096 x 16384 43.3 / 39.6, 32768 x 1024
+// 26.5 / 23.6, 16384 x 2048 25.4 / 23.3; at 10 and 17 MB between 4 % ahead and 2 % behind, so from 32 MB on.  (Going on by
+// halves saves bytes and loses more in launches: 42.6 with one more, 44.9 with two.)
+extern "C" int phyai_host_relay_gated(void* w, int64_t N, int64_t K, void* scratch, void* stream) {
+    using namespace phyai;
+    if (N <= 0 || K <= 0 || N % 32 != 0 || K % 128 != 0 || N > 0x7FFFFFFFll || K > 0x7FFFFFFFll) return -2;
+    if (N * K < (1ll << 25) || N * K > 0x7FFFFFFFll || ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(scratch)) & 15) != 0) return -2;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    v4i *m = static_cast<v4i*>(w), *up = static_cast<v4i*>(scratch);
+    const uint32_t k = (uint32_t)K, units = (uint32_t)(N / 16), half = (uint32_t)(N / 2 * K / 16);
+    const uint32_t middle = units / 2, kept = middle * 8 * (k / 16);   // (N % 32 == 0: units is even)
+    hipLaunchKernelGGL(weight_save_kernel, dim3((half + kept + 1023) / 1024), dim3(256), 0, st, m, up, half, kept);
+    launch_units(m, up, m, middle, units, k, 1, st);
+    launch_units(up + half, up, m, 0, middle, k, 1, st);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}

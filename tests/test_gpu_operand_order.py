@@ -57,6 +57,22 @@ def test_relay_matches_index_arithmetic(dev, N, K, gated):
     assert torch.equal(got.view(torch.uint8).cpu(), _operand_order_on_cpu(w, gated))
 
 
+@pytest.mark.parametrize("N,K", [(32768, 1024),     # 2^25 bytes: the first that is re-laid in two halves
+                                 (32736, 1024),     # just below
+                                 (16416, 2048),     # an odd number of units in each half
+                                 (2048, 16512)])    # more K than the plain in-place form takes; the last workgroups not full
+def test_gated_relay_in_its_own_storage(dev, N, K):
+    """A layer's gated matrix keeps its storage, and nothing beside it is written."""
+    ops = _ops()
+    w = torch.randint(0, 256, (N, K), generator=torch.Generator().manual_seed(N + K), dtype=torch.uint8)
+    around = torch.full((N * K + 2048,), 0x5A, dtype=torch.uint8, device=dev)
+    mine = around[1024:1024 + N * K].view(N, K)
+    mine.copy_(w)
+    assert ops._native().relay_weight(mine.view(torch.float8_e4m3fn), True) is True
+    assert torch.equal(mine.cpu(), _operand_order_on_cpu(w, True))
+    assert (around[:1024] == 0x5A).all() and (around[1024 + N * K:] == 0x5A).all()
+
+
 def test_relay_refuses_what_it_cannot_do(dev):
     ops = _ops()
     from phyai_amd import _lib
