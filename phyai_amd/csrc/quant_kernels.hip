@@ -130,17 +130,23 @@ static int launch_quant_rows(const void* x, int64_t M, int64_t K, int64_t ld, vo
     const bool stream_in = M * K * 2 >= ((int64_t)100 << 20);   // only long rows get that large in practice
 #define PHYAI_QL(T, C)                                                                                             \
     do {                                                                                                           \
-        if (C >= 4 && stream_in)                                                                                   \
-            hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, (C >= 4)>), grid, dim3(T), 0, st, xp, ld, k, (int)ldq, qp, scale); \
+        if (T * C >= 1024 && stream_in)                                                                            \
+            hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, (T * C >= 1024)>), grid, dim3(T), 0, st, xp, ld, k, (int)ldq, qp, scale); \
         else                                                                                                       \
             hipLaunchKernelGGL((quant_rows_reg_kernel<T, C, MODE, false>), grid, dim3(T), 0, st, xp, ld, k, (int)ldq, qp, scale);   \
     } while (0)
+    // One load per thread where there are few rows: a row is then one trip to memory and a reduction.  Many rows fill the chip
+    // either way, and two wavefronts wait for each other less than four (us, 256 threads / 128: 816 x 2048 3.25 / 3.28, 3264 x 2048
+    // 6.2 / 5.9, 13056 x 2048 13.9 / 13.4).  Long rows: 512 threads instead of 256 (50 x 16384 3.9 / 3.5, 816 x 16384
+    // 9.5 / 9.3, 3264 x 16384 25.7 - 27.4 / 24.3 - 27.0, 13056 x 16384 95.0 / 94.1, 50 x 8192 3.1 / 2.9, 13056 x 8192 49.0 / 48.7); 1024 are
+    // slower again with many of them (58.4).
     if (K <= 512) PHYAI_QL(64, 1);
     else if (K <= 1024) PHYAI_QL(128, 1);
+    else if (K <= 2048 && M >= 2048) PHYAI_QL(128, 2);
     else if (K <= 2048) PHYAI_QL(256, 1);
     else if (K <= 4096) PHYAI_QL(256, 2);
-    else if (K <= 8192) PHYAI_QL(256, 4);
-    else if (K <= 16384) PHYAI_QL(256, 8);
+    else if (K <= 8192) PHYAI_QL(512, 2);
+    else if (K <= 16384) PHYAI_QL(512, 4);
     else if (K <= 32768) PHYAI_QL(256, 16);
     else hipLaunchKernelGGL((quant_rows_loop_kernel<MODE>), grid, dim3(256), 0, st, xp, ld, k, (int)ldq, qp, scale);
 #undef PHYAI_QL
@@ -181,9 +187,25 @@ __device__ __forceinline__ void unpack8(uint4 q, float* f) {
     }
 }
 
+// Eight values rounded to bf16: four hardware converts instead of some fifty instructions.  They differ from
+// f32_to_bf16_bits in the bits of a NaN only, so where a NaN may be among them that form is taken.
+__device__ __forceinline__ uint4 round8_bf16(const float* o) {
+    uint4 b = make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7]));
+    if (__builtin_expect(any_nan_or_inf(b), 0)) {
+        b.x = f32_to_bf16_bits(o[0]) | (f32_to_bf16_bits(o[1]) << 16);
+        b.y = f32_to_bf16_bits(o[2]) | (f32_to_bf16_bits(o[3]) << 16);
+        b.z = f32_to_bf16_bits(o[4]) | (f32_to_bf16_bits(o[5]) << 16);
+        b.w = f32_to_bf16_bits(o[6]) | (f32_to_bf16_bits(o[7]) << 16);
+    }
+    return b;
+}
+
 // One workgroup per row, the row in registers: sum of squares (fp32), normalise, affine, round to
 // bf16 - the tensor the reference's norm kernel would have written - and, on those bf16 values,
-// the per-token quantizer (row absmax, scale, codes) of quant_rows_reg_kernel.
+// the per-token quantizer (row absmax, scale, codes) of quant_rows_reg_kernel.  Its arithmetic takes as long as its bytes: the
+// affine part is asked for together with the row, the rows per modulation row are divided by in 32 bits, and values are rounded by
+// the hardware (us, before / with all three, plain and adaptive: 3264 x 2048 8.9 / 8.1 and 9.8 / 8.8, 13056 x 2048 21.5 / 18.8 and 23.5 /
+// 21.2, 4800 x 4096 16.3 / 13.4 and 16.9 / 14.6, 816 x 2048 4.4 / 4.2 and 4.7 / 4.4).
 template <int THREADS, int CHUNKS, bool ADAPTIVE>
 __global__ __launch_bounds__(THREADS) void norm_quant_kernel(
     const uint16_t* __restrict__ a_x, int64_t a_ldx, int a_D, int a_group, const uint16_t* __restrict__ a_mod,
@@ -199,13 +221,20 @@ __global__ __launch_bounds__(THREADS) void norm_quant_kernel(
     __shared__ uint32_t smax[THREADS / kWave];
     const int64_t row = blockIdx.x;
     const uint16_t* xr = p.x + row * p.ldx;
+    const int64_t mrow = ADAPTIVE ? (int64_t)((uint32_t)row / (uint32_t)p.group) : 0;   // (M < 2^31)
+    const uint16_t* mr = ADAPTIVE ? p.mod + mrow * p.ld_mod : nullptr;
     float xf[CHUNKS][8];
+    uint4 affine[CHUNKS][ADAPTIVE ? 2 : 1];   // weight, or scale and shift: asked for with the row, not after its sum is there
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         const int k = (c * THREADS + threadIdx.x) * 8;
         uint4 v = make_uint4(0, 0, 0, 0);
-        if (k < p.D) v = *reinterpret_cast<const uint4*>(xr + k);
+        if (k < p.D) {
+            v = *reinterpret_cast<const uint4*>(xr + k);
+            affine[c][0] = *reinterpret_cast<const uint4*>((ADAPTIVE ? mr : p.weight) + k);
+            if constexpr (ADAPTIVE) affine[c][1] = *reinterpret_cast<const uint4*>(mr + p.D + k);
+        }
         unpack8(v, xf[c]);
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += xf[c][e] * xf[c][e];
@@ -213,8 +242,6 @@ __global__ __launch_bounds__(THREADS) void norm_quant_kernel(
     ss = block_sum_f32<THREADS>(ss, ssum);
     const float rstd = 1.0f / sqrtf(ss / (float)p.D + p.eps);
 
-    const int64_t mrow = ADAPTIVE ? row / p.group : 0;
-    const uint16_t* mr = ADAPTIVE ? p.mod + mrow * p.ld_mod : nullptr;
     uint4 ob[CHUNKS];
     uint32_t m = 0;
 #pragma unroll
@@ -225,23 +252,20 @@ __global__ __launch_bounds__(THREADS) void norm_quant_kernel(
             float o[8];
             if constexpr (ADAPTIVE) {
                 float sc[8], sh[8];
-                unpack8(*reinterpret_cast<const uint4*>(mr + k), sc);
-                unpack8(*reinterpret_cast<const uint4*>(mr + p.D + k), sh);
+                unpack8(affine[c][0], sc);
+                unpack8(affine[c][1], sh);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[e] = (xf[c][e] * rstd) * (1.0f + sc[e]) + sh[e];
-                if (p.gate != nullptr && row % p.group == 0)
+                if (p.gate != nullptr && (uint32_t)row == (uint32_t)mrow * (uint32_t)p.group)
                     *reinterpret_cast<uint4*>(p.gate + mrow * p.ld_gate + k) =
                         *reinterpret_cast<const uint4*>(mr + 2 * p.D + k);
             } else {
                 float w[8];
-                unpack8(*reinterpret_cast<const uint4*>(p.weight + k), w);
+                unpack8(affine[c][0], w);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[e] = (xf[c][e] * rstd) * (p.gemma ? w[e] + 1.0f : w[e]);
             }
-            ob[c].x = f32_to_bf16_bits(o[0]) | (f32_to_bf16_bits(o[1]) << 16);
-            ob[c].y = f32_to_bf16_bits(o[2]) | (f32_to_bf16_bits(o[3]) << 16);
-            ob[c].z = f32_to_bf16_bits(o[4]) | (f32_to_bf16_bits(o[5]) << 16);
-            ob[c].w = f32_to_bf16_bits(o[6]) | (f32_to_bf16_bits(o[7]) << 16);
+            ob[c] = round8_bf16(o);
             if (p.out != nullptr) *reinterpret_cast<uint4*>(p.out + row * p.ldo + k) = ob[c];
         }
         m = absmax8(ob[c], m);
@@ -303,12 +327,7 @@ __global__ __launch_bounds__(256) void norm_quant_loop_kernel(
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = (f[e] * rstd) * (p.gemma ? w[e] + 1.0f : w[e]);
         }
-        uint4 b;
-        b.x = f32_to_bf16_bits(o[0]) | (f32_to_bf16_bits(o[1]) << 16);
-        b.y = f32_to_bf16_bits(o[2]) | (f32_to_bf16_bits(o[3]) << 16);
-        b.z = f32_to_bf16_bits(o[4]) | (f32_to_bf16_bits(o[5]) << 16);
-        b.w = f32_to_bf16_bits(o[6]) | (f32_to_bf16_bits(o[7]) << 16);
-        return b;
+        return round8_bf16(o);
     };
     uint32_t m = 0;
     for (int k = threadIdx.x * 8; k < p.D; k += 256 * 8) {

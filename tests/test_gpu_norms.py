@@ -175,3 +175,38 @@ def _norm_modules_body(dev, GemmaRMSNorm, AdaRMSNorm, ColumnParallelLinear, Dens
     for lin, shape in ((mlp.gate_up_proj, (8192, D)), (mlp.down_proj, (D, 4096))):
         lin.spec.quantize_weight_(lin, (torch.randn(*shape) * 0.02).to(torch.bfloat16).to(dev))
     assert torch.equal(mlp(v2), mlp(n2))
+
+
+@pytest.mark.parametrize("hidden", [256, 2048, 4096, 12288])
+@pytest.mark.parametrize("adaptive", [False, True])
+def test_nonfinite_affine_parts_give_the_canonical_nan(dev, hidden, adaptive):
+    """NaN results are 0x7FC0 whatever sign and payload the factor had, infinities stay, and the columns beside them
+    are what they are without."""
+    ops = _ops()
+    x = seeded((9, hidden), seed=hidden, scale=0.5).to(dev)
+    x[2, 9] = 0.0
+    w = seeded((3 * hidden if adaptive else hidden,), seed=5, scale=0.3).to(dev)
+
+    def run(w):
+        if adaptive:
+            return ops.adarmsnorm(x, w[None], 1e-6)[0]
+        return ops.rmsnorm(x, w, 1e-6)
+
+    plain = run(w).view(torch.int16)
+    bits = w.clone().view(torch.int16)
+    bits[5], bits[hidden - 1], bits[9] = 0xFFA1 - 0x10000, 0x7FFF, 0x7F80
+    got = run(bits.view(torch.bfloat16)).view(torch.int16)
+    assert (got[:, 5] == 0x7FC0).all() and (got[:, hidden - 1] == 0x7FC0).all()
+    assert got[2, 9] == 0x7FC0 and ((got[:, 9] & 0x7FFF) == 0x7F80).sum() == 8
+    keep = torch.ones(hidden, dtype=torch.bool, device=dev)
+    keep[[5, 9, hidden - 1]] = False
+    assert torch.equal(got[:, keep], plain[:, keep])
+
+
+@pytest.mark.parametrize("M,K", [(2047, 2048), (2048, 2048), (2048, 1040), (2050, 1168), (3, 4112), (3, 8192), (5, 8208), (2, 16384), (3300, 16000)])
+def test_quantizer_at_the_edges_of_its_workgroup_shapes(dev, M, K):
+    x = seeded((M, K), seed=M + K, scale=2.0)
+    x[M - 1, K - 1] = 77.0
+    xq, xs = _ops().fp8_quant_rowwise(x.to(dev))
+    q, s = ref.quant_rowwise(x)
+    assert torch.equal(xs.cpu(), s) and torch.equal(xq.cpu().view(torch.uint8), q.view(torch.uint8))
