@@ -22,6 +22,12 @@ returns a list of violations over every instantiation of the kernel:
 file that spills has scratch loads and stores of the compiler's among them, and a wait would then let a stage be
 read before it has landed.  It reads the compiler's resource-usage remarks that the Makefile keeps beside every
 object (``_obj/gemm_big.o.usage``) and reports every instantiation with a scratch size other than zero.
+
+``check_library`` is the guard of every kernel against a hazard that the hardware does not check: a vector-memory
+instruction may read an SGPR only five wait states after a VALU instruction wrote it.  The compiler keeps to that
+for its own instructions but does not look inside the inline assembly of the global -> LDS copies, in front of which
+it may put a ``v_readlane`` (a spilled SGPR read back) or ``v_readfirstlane`` of their base pointer.  It disassembles
+the code objects of the built library and follows every path through every kernel.
 """
 
 from __future__ import annotations
@@ -29,6 +35,7 @@ from __future__ import annotations
 import os
 import re
 import subprocess
+import tempfile
 
 CSRC = os.path.dirname(os.path.abspath(__file__))
 ASM = os.path.join(CSRC, "_obj", "gemm_skinny_fused.s")
@@ -190,10 +197,118 @@ def check_tile_usage(stamps: bool = False) -> list[str]:
     return bad
 
 
+LIB = os.path.join(os.path.dirname(CSRC), "lib")
+OBJDUMP = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+SETTLES = 5   # wait states from a VALU write of an SGPR to a vector-memory instruction that reads it
+_SGPR = re.compile(r"(?<![\w.])(?:s(?:\[(\d+):(\d+)\]|(\d+)\b)|(vcc)(_lo|_hi)?\b)")
+_TWO_RESULTS = re.compile(r"v_(?:add_co|sub_co|subrev_co|addc_co|subb_co|subbrev_co|div_scale|mad_u64_u32|mad_i64_i32)")
+_VCC = 1000   # a number beside the SGPRs'
+
+
+def _sgprs(text: str) -> set[int]:
+    out: set[int] = set()
+    for first, last, single, vcc, half in _SGPR.findall(text):
+        if vcc:
+            out |= {_VCC} if half == "_lo" else {_VCC + 1} if half == "_hi" else {_VCC, _VCC + 1}
+        elif single:
+            out.add(int(single))
+        else:
+            out |= set(range(int(first), int(last) + 1))
+    return out
+
+
+def functions_of(disassembly: str) -> list[str]:
+    return re.split(r"^(?=<(?!L\d+>)[^>]+>:$)", disassembly, flags=re.M)[1:]
+
+
+def sgpr_problems(function: str) -> tuple[list[str], int]:
+    """Vector-memory instructions of one disassembled function that may read an SGPR too soon, and how many there are of
+    them in all.  For each place: the wait states since each SGPR's last VALU write, the fewest over all ways there."""
+    lines = [line.split("//")[0].strip() for line in function.split("\n")]
+    name = lines[0].rstrip(":")
+    code = [t for t in lines[1:] if t]
+    label = {t[1:-2]: i for i, t in enumerate(code) if t.startswith("<") and t.endswith(">:")}
+    since: list[dict[int, int] | None] = [None] * (len(code) + 1)
+    bad: dict[int, int] = {}
+    todo = [0, *label.values()]   # (the second entry of a kernel with preloaded arguments is a label too)
+    for i in todo:
+        since[i] = {}
+
+    def reach(i: int, state: dict[int, int]) -> None:
+        if since[i] is None:
+            since[i] = dict(state)
+            todo.append(i)
+            return
+        sooner = {r: n for r, n in state.items() if n < since[i].get(r, SETTLES)}
+        if sooner:
+            since[i].update(sooner)
+            todo.append(i)
+
+    while todo:
+        i = todo.pop()
+        if i >= len(code):
+            continue
+        t, state = code[i], since[i]
+        if t.startswith("<"):
+            reach(i + 1, state)
+            continue
+        op, _, operands = t.partition(" ")
+        if op.startswith(_VMEM):
+            for r in _sgprs(operands) & state.keys():
+                bad[i] = min(state[r], bad.get(i, SETTLES))
+        states = int(operands, 0) + 1 if op == "s_nop" else 1
+        after = {r: n + states for r, n in state.items() if n + states < SETTLES}
+        if op.startswith("v_"):
+            first, _, rest = operands.partition(",")
+            written = _sgprs(first) | (_sgprs(rest.split(",")[0]) if _TWO_RESULTS.match(op) else set())
+            after.update(dict.fromkeys(written, 0))
+        if op.startswith(("s_setpc", "s_swappc", "s_call")):
+            bad[i] = -1   # (nothing here is called: a way that cannot be followed)
+        if op.startswith("s_cbranch") or op == "s_branch":
+            reach(label[operands.strip()], after)
+        if op not in ("s_branch", "s_endpgm"):
+            reach(i + 1, after)
+    memory = sum(t.startswith(_VMEM) for t in code)
+    return [f"{name}: `{code[i]}` " + ("cannot be followed" if n < 0 else f"reads an SGPR {n} wait states after a VALU write of it, not {SETTLES}")
+            for i, n in sorted(bad.items())], memory
+
+
+def check_disassembly(text: str) -> tuple[list[str], int, int]:
+    """Problems, functions, vector-memory instructions."""
+    functions = functions_of(text)
+    results = [sgpr_problems(f) for f in functions]
+    return [p for bad, _ in results for p in bad], len(functions), sum(n for _, n in results)
+
+
+def disassemble(library: str) -> list[str]:
+    """One text per code object of a built library."""
+    with tempfile.TemporaryDirectory() as d:
+        link = os.path.join(d, "lib.so")
+        os.symlink(os.path.abspath(library), link)
+        subprocess.run([OBJDUMP, "--offloading", link], check=True, capture_output=True, cwd=d)
+        objects = sorted(f for f in os.listdir(d) if f.endswith("gfx950"))
+        return [subprocess.run([OBJDUMP, "-d", "--symbolize-operands", "--no-show-raw-insn", "--no-leading-addr", os.path.join(d, f)],
+                               check=True, capture_output=True, text=True).stdout for f in objects]
+
+
+def check_library(stamps: bool = False, min_kernels: int = 1000) -> list[str]:
+    """The built library (or the time-stamp build), every kernel of it."""
+    path = os.path.join(LIB, "libphyai_fp8_stamps.so" if stamps else "libphyai_fp8.so")
+    if not os.path.exists(path):
+        return [f"{path} is missing"]
+    bad, functions, memory = [], 0, 0
+    for text in disassemble(path):
+        b, f, m = check_disassembly(text)
+        bad, functions, memory = bad + b, functions + f, memory + m
+    if functions < min_kernels or memory < 10 * functions:
+        bad.append(f"only {functions} functions with {memory} vector-memory instructions found in {path}")
+    return bad
+
+
 if __name__ == "__main__":
     import sys
 
-    problems = check_file(stamps="--stamps" in sys.argv) + check_tile_usage(stamps="--stamps" in sys.argv)
+    problems = check_file(stamps="--stamps" in sys.argv) + check_tile_usage(stamps="--stamps" in sys.argv) + check_library(stamps="--stamps" in sys.argv)
     for p in problems[:50]:
         print(p)
     print(f"{len(problems)} problem(s)")

@@ -85,15 +85,22 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 // One 16-byte chunk per lane from global memory straight into LDS: lane i's chunk lands at
 // lds_wave_base + 16*i.  Issued as inline assembly so that the compiler does not order its own
 // LDS reads behind copies that are still in flight; the waits are placed by hand below.
+// A vector-memory instruction may read an SGPR five wait states after a VALU instruction wrote it (v_readfirstlane, or the
+// v_readlane of a spilled one), which the hardware does not check and the compiler does not see in here.  s_mov and s_nop are
+// NOPS + 2 of them; with kBaseSettles the base may come from anywhere, otherwise no such write may stand close in front of a
+// copy (check_fused_asm.py looks through every kernel of the built library).
+constexpr int kBaseSettles = 3;
+template <int NOPS = 0>
 __device__ __forceinline__ void copy16_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :: "v"(lane_offset), "s"(base), "s"(lds_wave_base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop %3\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(lane_offset), "s"(base), "s"(lds_wave_base), "n"(NOPS) : "memory", "m0");
 }
 
 // One 4-byte word per lane: lane i's lands at lds_wave_base + 4*i.
+template <int NOPS = 0>
 __device__ __forceinline__ void copy4_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                 :: "v"(lane_offset), "s"(base), "s"(lds_wave_base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop %3\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(lane_offset), "s"(base), "s"(lds_wave_base), "n"(NOPS) : "memory", "m0");
 }
 
 // copy16_to_lds for data that should not stay in the caches behind it (read once per pass over a

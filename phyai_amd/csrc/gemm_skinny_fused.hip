@@ -42,10 +42,17 @@ constexpr int FQ_THREADS = FQ_WAVES * kWave;
 PHYAI_STAMP_SINK(g_fq_stamps)
 
 // A 16-byte load whose arrival the compiler does not track: the value may be used only after
-// landed() has waited for it.
+// landed() has waited for it.  (The five wait states that its base needs behind a VALU write of these SGPRs - see
+// copy16_to_lds - stand in the code around it wherever there is such a write, which check_fused_asm.py sees to; in the debug build,
+// where they do not, it brings them along.)
+#ifdef PHYAI_FP8_STAMPS
+#define PHYAI_FQ_SETTLE "s_nop 4\n\t"
+#else
+#define PHYAI_FQ_SETTLE ""
+#endif
 __device__ __forceinline__ v4i fq_load16_async(const uint8_t* base, uint32_t lane_offset) {
     v4i v;
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(v) : "v"(lane_offset), "s"(base) : "memory");
+    asm volatile(PHYAI_FQ_SETTLE "global_load_dwordx4 %0, %1, %2" : "=v"(v) : "v"(lane_offset), "s"(base) : "memory");
     return v;
 }
 // At most YOUNGER memory instructions of this wavefront issued after the load are still in flight;

@@ -129,7 +129,9 @@ void gemm_fp8_tall_kernel(
     // beyond a multiple of four.  Register sets have to be named at compile time: see `turn`.
     int ring = 0;
     auto stage_at = [&](int base, int d) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_readfirstlane(((base + d) & 3) * STAGE_BYTES); };
-    auto copy = [&](int d, int c, uint32_t at) __attribute__((always_inline)) { copy16_to_lds(a_a + d * BIG_BK, aoff[c], wave_a + at + c * 1024); };
+    // (SGPRs are short here: the compiler keeps some in VGPR lanes, the base pointers of copies among them, and reads them back right
+    // in front of a copy.  Hence kBaseSettles, and multiply_copy where copies are many.)
+    auto copy = [&](int d, int c, uint32_t at) __attribute__((always_inline)) { copy16_to_lds<kBaseSettles>(a_a + d * BIG_BK, aoff[c], wave_a + at + c * 1024); };
     auto load = [&](int d, int e, auto set) __attribute__((always_inline)) {
         bring[decltype(set)::value][e >> 1][e & 1] = *reinterpret_cast<const v4i*>(bsrc[e >> 1] + ((size_t)d << 11) + (e & 1) * 1024 + lane16);
     };
@@ -168,7 +170,7 @@ void gemm_fp8_tall_kernel(
         const uint64_t b64 = reinterpret_cast<uint64_t>(base);   // (uniform, which the compiler does not see)
         const uint64_t b_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b64);
         const uint64_t b_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b64 >> 32));
-        copy4_to_lds(reinterpret_cast<const uint8_t*>(b_lo | b_hi << 32), at, __builtin_amdgcn_readfirstlane(lds_base + at_byte + blk * 256));
+        copy4_to_lds<kBaseSettles>(reinterpret_cast<const uint8_t*>(b_lo | b_hi << 32), at, __builtin_amdgcn_readfirstlane(lds_base + at_byte + blk * 256));
     };
     auto fill_bias = [&](int at_byte) __attribute__((always_inline)) {
         if (bias_rides) return;
@@ -230,6 +232,18 @@ void gemm_fp8_tall_kernel(
         else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
     };
     using No = std::integral_constant<int, 0>; using Yes = std::integral_constant<int, 1>;
+    // The same with copy(d, k, at) behind it: the MFMA and its s_nop are among the wait states between what wrote the copy's base and
+    // the copy, at no cost in time (with kBaseSettles behind the MFMA instead 2441 x 13312 x 2048 + GeGLU took 65.8 us for 63.9).
+    auto multiply_copy = [&](v8i w, v8i x, v4f& c, auto first, int d, int k, uint32_t at) __attribute__((always_inline)) {
+        const uint8_t* const base = a_a + d * BIG_BK;
+        const uint32_t from = aoff[k], to = wave_a + at + k * 1024;
+        if constexpr (decltype(first)::value)
+            asm volatile("s_mov_b32 m0, %5\n\ts_nop 2\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0\n\tglobal_load_lds_dwordx4 %3, %4"
+                         : "=a"(c) : "v"(w), "v"(x), "v"(from), "s"(base), "s"(to) : "memory", "m0");
+        else
+            asm volatile("s_mov_b32 m0, %5\n\ts_nop 2\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
+                         : "+a"(c) : "v"(w), "v"(x), "v"(from), "s"(base), "s"(to) : "memory", "m0");
+    };
     v8i fa[2][H0];
     constexpr int AHEAD = 2;   // blocks of a half that are read during the half before it
     // Lane (l16, q) of row block b reads chunks q and 4 + q of its row: frag_lo and frag_hi beyond the stage's place and the block.
@@ -263,19 +277,15 @@ void gemm_fp8_tall_kernel(
             if (i >= OPEN_NEXT && i < OPEN_NEXT + AHEAD && (P == 0 || NEXT)) fa[1 - P][i - OPEN_NEXT] = frag(next_lo, next_hi, (1 - P) * H0 + i - OPEN_NEXT);
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
-                multiply(big_join(bring[S][jj][0], bring[S][jj][1]), fa[P][i], acc[P * H0 + i][jj], first);
                 const int slot_n = P ? (i - 1) * 4 + jj : i * 4 + jj;
-                if constexpr (ASK == 2) {
-                    if (slot_n < CA) copy(d + 2, slot_n, copies_at);
-                    else if (slot_n < COPIES) load(d + 2, slot_n - CA, std::integral_constant<int, (S + 2) % DEPTH>{});
-                } else if constexpr (ASK == 1) {
-                    constexpr int REQUESTS = P ? CA : BL, MFMAS = P ? SLOTS_AFTER : 4 * H0;
-                    const int n = slot_n * REQUESTS / MFMAS;
-                    if (slot_n == 0 || (slot_n > 0 && n != (slot_n - 1) * REQUESTS / MFMAS)) {
-                        if constexpr (P == 0) load(d + 2, n, std::integral_constant<int, (S + 2) % DEPTH>{});
-                        else copy(d + LEAD, n, copies_at);
-                    }
-                }
+                constexpr int REQUESTS = P ? CA : BL, MFMAS = P ? SLOTS_AFTER : 4 * H0;
+                const int n = ASK == 2 ? slot_n : slot_n * REQUESTS / MFMAS;   // the request behind this MFMA, if there is one
+                const bool asks = ASK == 2 ? n < COPIES : ASK == 1 && (slot_n == 0 || (slot_n > 0 && n != (slot_n - 1) * REQUESTS / MFMAS));
+                const bool copies = asks && (ASK == 2 ? n < CA : P == 1);
+                const v8i weights = big_join(bring[S][jj][0], bring[S][jj][1]);
+                if (copies) multiply_copy(weights, fa[P][i], acc[P * H0 + i][jj], first, ASK == 2 ? d + 2 : d + LEAD, n, copies_at);
+                else multiply(weights, fa[P][i], acc[P * H0 + i][jj], first);
+                if (asks && !copies) load(d + 2, ASK == 2 ? n - CA : n, std::integral_constant<int, (S + 2) % DEPTH>{});
                 beside(i * 4 + jj);
                 __builtin_amdgcn_sched_barrier(0);
             }

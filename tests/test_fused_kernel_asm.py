@@ -79,3 +79,47 @@ def test_tile_kernels_use_no_scratch(guard):
     bad = guard.usage_problems(planted, min_kernels=1)
     assert len(bad) == 1 and "268 bytes" in bad[0]
     assert any("only 1" in p for p in guard.usage_problems(planted, min_kernels=2))
+
+
+def test_copies_keep_their_distance_from_writes_of_their_base(guard):
+    """Five wait states between a VALU write of an SGPR and a vector-memory instruction that reads it, in every kernel of
+    the built library; the compiler does not see to that in front of inline assembly (the library's build runs the same
+    check, of the time-stamp build too)."""
+    if not os.path.exists(os.path.join(guard.LIB, "libphyai_fp8.so")) or not os.path.exists(guard.OBJDUMP):
+        pytest.skip("no built library or no disassembler here")
+    bad = guard.check_library()
+    assert not bad, "\n".join(bad[:20])
+
+
+HEAD = "<_Zkernel>:\n\ts_load_dwordx2 s[4:5], s[0:1], 0x0   // 000000001900: C0060080\n"
+
+
+@pytest.mark.parametrize("code,found", [
+    # in front of a copy: its own two states, four, five; a pointer in the middle of a longer run of SGPRs
+    ("v_readlane_b32 s4, v1, 3|s_mov_b32 m0, s6|s_nop 0|global_load_lds_dwordx4 v2, s[4:5]", 2),
+    ("v_readlane_b32 s4, v1, 3|v_readlane_b32 s5, v1, 4|v_add_u32_e32 v3, v3, v4|s_mov_b32 m0, s6|s_nop 0|global_load_lds_dword v2, s[4:5]", 3),
+    ("v_readfirstlane_b32 s5, v1|s_mov_b32 m0, s6|s_nop 3|global_load_lds_dwordx4 v2, s[4:5]", None),
+    ("v_readfirstlane_b32 s6, v1|s_nop 3|buffer_load_dwordx4 v2, s[4:7], s9 offen lds", 4),
+    ("v_readfirstlane_b32 s9, v1|s_nop 3|buffer_load_dwordx4 v2, s[4:7], s9 offen lds", 4),
+    ("v_readfirstlane_b32 s8, v1|buffer_load_dwordx4 v2, s[4:7], s9 offen lds", None),
+    # not a VALU write, or of another register
+    ("s_mov_b32 s4, s8|global_load_lds_dwordx4 v2, s[4:5]", None),
+    ("v_readlane_b32 s14, v1, 3|global_load_dword v9, v2, s[4:5]", None),
+    # a compare, a carry, a second result
+    ("v_cmp_lt_u32_e64 s[4:5], v1, v2|global_store_dword v2, v3, s[4:5]", 0),
+    ("v_cmp_lt_u32_e32 vcc, v1, v2|s_nop 1|global_store_dword v2, v3, vcc", 2),
+    ("v_add_co_u32_e64 v1, s[4:5], v2, v3|global_load_dword v9, v2, s[4:5]", 0),
+    # by way of a branch, round a loop, and only on the other arm
+    ("v_readlane_b32 s4, v1, 3|s_cbranch_scc0 L0|s_nop 7|<L0>:|global_load_lds_dwordx4 v2, s[4:5]", 1),
+    ("<L0>:|global_load_lds_dwordx4 v2, s[4:5]|v_readlane_b32 s5, v1, 3|s_cbranch_vccnz L0", 1),
+    ("v_readlane_b32 s4, v1, 3|s_branch L1|<L0>:|global_load_lds_dwordx4 v2, s[4:5]|s_endpgm|<L1>:|s_nop 2|s_cbranch_scc0 L0", None),
+    ("v_readlane_b32 s4, v1, 3|s_branch L1|<L0>:|global_load_lds_dwordx4 v2, s[4:5]|s_endpgm|<L1>:|s_nop 1|s_cbranch_scc0 L0", 4),
+])
+def test_planted_copies_too_close_are_caught(guard, code, found):
+    text = HEAD + "".join((t if t.startswith("<") else "\t" + t + "      // 00000000: 0") + "\n" for t in code.split("|")) + "\ts_endpgm   // 0\n"
+    bad, functions, _ = guard.check_disassembly(text)
+    assert functions == 1
+    if found is None:
+        assert not bad, bad
+    else:
+        assert len(bad) == 1 and f"reads an SGPR {found} wait states after" in bad[0], bad
