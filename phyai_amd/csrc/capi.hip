@@ -35,6 +35,13 @@ int check_launch(const char* what) {
     return PHYAI_FP8_OK;
 }
 
+// Of a re-lay: its own launch's status, whatever older error the thread has (weight_layout.hip).
+int relay_status(const char* what, int rc) {
+    if (rc == 0) return PHYAI_FP8_OK;
+    if (rc == -3) return fail(PHYAI_FP8_ELAUNCH, "%s: %s", what, hipGetErrorString(hipGetLastError()));
+    return fail(PHYAI_FP8_EUNSUPPORTED, "%s: no kernel", what);
+}
+
 bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -167,9 +174,7 @@ int phyai_fp8_weight_to_operand_order(const void* w, int64_t N, int64_t K, int g
     if (N * K >= kMaxElems) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: matrix larger than 2^31 elements", fn);
     const uintptr_t a = reinterpret_cast<uintptr_t>(w), b = reinterpret_cast<uintptr_t>(out), n = (uintptr_t)(N * K);
     if (a < b + n && b < a + n) return fail(PHYAI_FP8_EINVAL, "%s: out overlaps w (the re-lay is not in place)", fn);
-    if (phyai::launch_weight_to_operand_order(w, N, K, gated ? 1 : 0, out, static_cast<hipStream_t>(stream)) != 0)
-        return fail(PHYAI_FP8_EUNSUPPORTED, "%s: matrix too large", fn);
-    return check_launch(fn);
+    return relay_status(fn, phyai::launch_weight_to_operand_order(w, N, K, gated ? 1 : 0, out, static_cast<hipStream_t>(stream)));
 }
 
 int phyai_fp8_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, void* stream) {
@@ -180,9 +185,7 @@ int phyai_fp8_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, voi
     if (K % 128 != 0 || N % 16 != 0 || K > 16384)
         return fail(PHYAI_FP8_EUNSUPPORTED, "%s: needs K %% 128 == 0, K <= 16384 and N %% 16 == 0, got N=%lld K=%lld", fn, (long long)N, (long long)K);
     if (N >= kMaxElems || N * K >= kMaxElems) return fail(PHYAI_FP8_EUNSUPPORTED, "%s: matrix larger than 2^31 elements", fn);
-    if (phyai::launch_weight_to_operand_order_inplace(w, N, K, static_cast<hipStream_t>(stream)) != 0)
-        return fail(PHYAI_FP8_EUNSUPPORTED, "%s: no kernel", fn);
-    return check_launch(fn);
+    return relay_status(fn, phyai::launch_weight_to_operand_order_inplace(w, N, K, static_cast<hipStream_t>(stream)));
 }
 
 size_t phyai_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int epilogue) {

@@ -23,6 +23,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/phyai_fp8.h"
+#include "host_entry.h"
 
 namespace {
 
@@ -41,7 +42,7 @@ struct Lib {
     decltype(&phyai_fp8_weight_quant_rowwise) weight_quant;
     decltype(&phyai_fp8_weight_to_operand_order) relay;
     decltype(&phyai_fp8_weight_to_operand_order_inplace) relay_inplace;
-    int (*relay_gated)(void*, int64_t, int64_t, void*, void*);   // phyai_host_relay_gated (weight_layout.hip)
+    decltype(&phyai_host_relay_gated) relay_gated;
     decltype(&phyai_fp8_linear_per_tensor) per_tensor;
     decltype(&phyai_fp8_rmsnorm_quant) rmsnorm;
     decltype(&phyai_fp8_adarmsnorm_quant) adarmsnorm;
@@ -579,7 +580,7 @@ PyObject* py_relay_weight(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (gated) {
         const int rc = lib.relay_gated(p, N, K, t.mutable_data_ptr(), at_.stream);
         if (rc == 0) Py_RETURN_TRUE;
-        TORCH_CHECK(rc == -2, "relay_weight: a launch failed");   // (some units may be re-laid already)
+        TORCH_CHECK(rc == -2, "relay_weight: a launch failed");   // (half of the matrix is re-laid)
     }
     // (a plain copy first and the re-lay back: the allocator's stream order covers the temporary)
     if (hipMemcpyAsync(t.mutable_data_ptr(), p, (size_t)(N * K), hipMemcpyDeviceToDevice, at_.stream) != hipSuccess) return declined();

@@ -10,10 +10,20 @@
 #include <hip/hip_runtime.h>
 
 #include "fp8_device.h"
+#include "host_entry.h"
 #include "launch.h"
 #include "weight_layout.h"
 
 namespace phyai {
+
+// The launch's own status.  hipGetLastError() may return an older error of the thread, and a caller that went another way for
+// it would re-lay the matrix a second time.
+template <class T> struct AsIs { typedef T type; };
+template <class... P>
+static bool launched(void (*kernel)(P...), unsigned blocks, unsigned threads, hipStream_t st, typename AsIs<P>::type... a) {
+    void* args[] = {&a...};
+    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(blocks), dim3(threads), args, 0, st) == hipSuccess;
+}
 
 // Chunks [first * K, first * K + chunks) of the destination, i.e. units from `first` on (a unit is K chunks).  Gated: gate rows
 // from `gate`, up rows from `up`, both counted from column 0; plain: rows of the matrix at `gate`.
@@ -66,34 +76,35 @@ __global__ __launch_bounds__(1024) void weight_to_operand_order_inplace_kernel(v
 }
 
 int launch_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, hipStream_t st) {
-    const dim3 grid((unsigned)(N / 16));
+    const unsigned units = (unsigned)(N / 16);
     v4i* p = static_cast<v4i*>(w);
     const uint32_t k = (uint32_t)K;
-    if (K <= 1024) hipLaunchKernelGGL((weight_to_operand_order_inplace_kernel<1>), grid, dim3(1024), 0, st, p, k);
-    else if (K <= 2048) hipLaunchKernelGGL((weight_to_operand_order_inplace_kernel<2>), grid, dim3(1024), 0, st, p, k);
-    else if (K <= 4096) hipLaunchKernelGGL((weight_to_operand_order_inplace_kernel<4>), grid, dim3(1024), 0, st, p, k);
-    else if (K <= 8192) hipLaunchKernelGGL((weight_to_operand_order_inplace_kernel<8>), grid, dim3(1024), 0, st, p, k);
-    else if (K <= 16384) hipLaunchKernelGGL((weight_to_operand_order_inplace_kernel<16>), grid, dim3(1024), 0, st, p, k);
+    bool ok;
+    if (K <= 1024) ok = launched(weight_to_operand_order_inplace_kernel<1>, units, 1024, st, p, k);
+    else if (K <= 2048) ok = launched(weight_to_operand_order_inplace_kernel<2>, units, 1024, st, p, k);
+    else if (K <= 4096) ok = launched(weight_to_operand_order_inplace_kernel<4>, units, 1024, st, p, k);
+    else if (K <= 8192) ok = launched(weight_to_operand_order_inplace_kernel<8>, units, 1024, st, p, k);
+    else if (K <= 16384) ok = launched(weight_to_operand_order_inplace_kernel<16>, units, 1024, st, p, k);
     else return -2;
-    return 0;
+    return ok ? 0 : -3;
 }
 
-static void launch_units(const v4i* gate, const v4i* up, v4i* out, uint32_t first, uint32_t end, uint32_t K, int gated, hipStream_t st) {
+static bool launch_units(const v4i* gate, const v4i* up, v4i* out, uint32_t first, uint32_t end, uint32_t K, int gated, hipStream_t st) {
     const uint32_t chunks = (end - first) * K;
-    hipLaunchKernelGGL(weight_to_operand_order_kernel, dim3((chunks + 1023) / 1024), dim3(256), 0, st, gate, up, out, first, K, gated, chunks);
+    return launched(weight_to_operand_order_kernel, (chunks + 1023) / 1024, 256, st, gate, up, out, first, K, gated, chunks);
 }
 
 int launch_weight_to_operand_order(const void* w, int64_t N, int64_t K, int gated, void* out, hipStream_t st) {
     if (N * K > 0x7FFFFFFFll) return -2;
     const v4i* rows = static_cast<const v4i*>(w);
-    launch_units(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st);
-    return 0;
+    return launch_units(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st) ? 0 : -3;
 }
 
 }  // namespace phyai
 
 // The gated form in place, for the host extension beside this library (no part of the C interface): w as
-// phyai_fp8_weight_to_operand_order() takes it, scratch of 3/4 N * K bytes.  -2: not for this form, nothing done.
+// phyai_fp8_weight_to_operand_order() takes it, scratch of 3/4 N * K bytes.  -2: not for this form or not launched, the matrix is
+// as it was; -3: half of it is re-laid.
 //
 // Saving the whole matrix and re-laying from there moves every byte four times.  The upper half of the units needs less: it
 // overwrites the up half of the matrix and reads the upper gate rows, which are still in place.  So the up half and the
@@ -109,8 +120,7 @@ extern "C" int phyai_host_relay_gated(void* w, int64_t N, int64_t K, void* scrat
     v4i *m = static_cast<v4i*>(w), *up = static_cast<v4i*>(scratch);
     const uint32_t k = (uint32_t)K, units = (uint32_t)(N / 16), half = (uint32_t)(N / 2 * K / 16);
     const uint32_t middle = units / 2, kept = middle * 8 * (k / 16);   // (N % 32 == 0: units is even)
-    hipLaunchKernelGGL(weight_save_kernel, dim3((half + kept + 1023) / 1024), dim3(256), 0, st, m, up, half, kept);
-    launch_units(m, up, m, middle, units, k, 1, st);
-    launch_units(up + half, up, m, 0, middle, k, 1, st);
-    return hipGetLastError() == hipSuccess ? 0 : -3;
+    if (!launched(weight_save_kernel, (half + kept + 1023) / 1024, 256, st, m, up, half, kept)) return -2;
+    if (!launch_units(m, up, m, middle, units, k, 1, st)) return -2;
+    return launch_units(up + half, up, m, 0, middle, k, 1, st) ? 0 : -3;
 }

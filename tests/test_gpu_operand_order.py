@@ -73,6 +73,29 @@ def test_gated_relay_in_its_own_storage(dev, N, K):
     assert (around[:1024] == 0x5A).all() and (around[1024 + N * K:] == 0x5A).all()
 
 
+@pytest.mark.parametrize("N,K,gated", [(64, 256, False), (64, 256, True), (32768, 1024, True)])
+def test_relay_beside_an_older_error_of_the_thread(dev, N, K, gated):
+    """An error that another HIP call left pending is not this one's: the matrix is re-laid, once, and the error is still there."""
+    import ctypes
+
+    ops = _ops()
+    w = torch.randint(0, 256, (N, K), generator=torch.Generator().manual_seed(7), dtype=torch.uint8)
+    mine = w.to(dev).view(torch.float8_e4m3fn)
+    torch.cuda.synchronize()
+    runtime = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(runtime)
+    ops._native().relay_weight(w[:1], False)   # (bound and ready)
+    try:
+        refused = hip.hipSetDevice(4096)
+        assert refused != 0 and hip.hipPeekAtLastError() == refused
+        done = ops._native().relay_weight(mine, gated)
+        still = hip.hipPeekAtLastError()
+    finally:
+        hip.hipGetLastError()
+    assert done is True and still == refused
+    assert torch.equal(mine.view(torch.uint8).cpu(), _operand_order_on_cpu(w, gated))
+
+
 def test_relay_refuses_what_it_cannot_do(dev):
     ops = _ops()
     from phyai_amd import _lib
