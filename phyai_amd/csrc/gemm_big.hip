@@ -944,9 +944,14 @@ static double big_fill(int tiles, int slots) {
     return rounds > 0 ? (double)tiles / ((double)rounds * slots) : 1.0;
 }
 
+// (PHYAI_FP8_BIG_DIRECT=0: weights in operand order go through LDS in every tile shape)
+static bool big_registers_allowed() {
+    const char* e = tuning_env("PHYAI_FP8_BIG_DIRECT");
+    return e == nullptr || atoi(e) != 0;
+}
 // The ring of register sets that a shape's weights in operand order go through (0: staged in LDS).
 static int big_register_ring(const BigPlan& pl, int K, int epilogue) {
-    if (const char* e = tuning_env("PHYAI_FP8_BIG_DIRECT")) { if (atoi(e) == 0) return 0; }
+    if (!big_registers_allowed()) return 0;
     if (K % 128 != 0) return 0;
     if (pl.tile == 224 && pl.splits == 1 && K % 512 == 0) return 4;
     if (pl.tile == 128 && pl.cols == 128 && pl.depth == 4 && (K / pl.splits) % 1024 == 0 && !epi_is_gated(epilogue)) return 8;
@@ -1172,7 +1177,7 @@ BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, cons
     // Tall tiles where they are ahead of that (by 4 % below 60 us, where the costs are less sure): in half of 1800 linears that
     // tiles serve, 7.3 % less time in the geometric mean over all of them, quantizer included (0.9 % behind the best shape), and
     // more than 2 % slower in 9.
-    if (operand_w && K % 128 == 0) {
+    if (operand_w && K % 128 == 0 && big_registers_allowed()) {
         lowest = (big_tall(best) || *cost - shared >= 60.0 ? 1.0 : 0.96) * *cost;
         for (int rows = 144; rows <= 256; rows += 16) {
             const BigPlan pl = {rows, 256, 1, 0, 2, 4};

@@ -100,6 +100,21 @@ def test_where_one_launch_takes_more_rows(monkeypatch):
     assert seen > 100
 
 
+def test_weights_stay_out_of_registers_where_that_is_asked_for(monkeypatch):
+    """PHYAI_FP8_BIG_DIRECT=0: no tile shape, chosen by rule or by cost, takes weights in operand order straight into registers."""
+    from phyai_amd import ops
+
+    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "TALL", "TILE", "RULES"):
+        monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    monkeypatch.setenv("PHYAI_FP8_FUSED", "0")
+    shapes = [(*s, "operand_gated" if s[3] == GATED else "operand") for s in _shapes(300) if s[0] * s[2] < 1 << 31]
+    plans = lambda: [f(m, n, k, epi, weight_layout=lay) for m, n, k, epi, lay in shapes for f in (ops.describe_linear_plan, ops.describe_plan)]
+    assert sum("in registers" in p and "x256" in p for p in plans()) > 50
+    monkeypatch.setenv("PHYAI_FP8_BIG_DIRECT", "0")
+    staged = plans()
+    assert not [p for p in staged if "tile" in p and "in registers" in p]
+
+
 # (rows, columns, K, epilogue): rule's shape -> chosen shape, one per pair that occurs
 CHANGED = [(2032, 9216, 640, "gelu"), (4310, 3648, 640, None), (497, 2432, 8320, None), (2489, 384, 1792, None), (2553, 864, 8320, None),
            (400, 6144, 8192, None), (3548, 3392, 5120, None), (3531, 8160, 640, None), (2740, 1056, 8448, None), (278, 3072, 9600, None)]
