@@ -61,6 +61,7 @@
 #include "splitk.h"
 #include "stamps.h"
 #include "weight_layout.h"
+#include <math.h>
 #include <stdlib.h>
 #include <type_traits>
 
@@ -1121,15 +1122,19 @@ static BigCost big_cost_of(const BigPlan& pl) {
     const double split = pl.splits > 1 ? 5.0 : 0.0;
     return regs ? BigCost{1.02 + split, 1.06, 0.356, 0.112, 0, 1.09, 0, 0, 0, 0, 0} : BigCost{0.63 + split, 1.23, 0.393, 0.095, 0.109, 1.06, 0.33, 0, 0, 0, 0};
 }
+// Rounds of `slots` workgroups that the busiest XCD runs of a shape, in fractions.
+static double big_rounds(const BigPlan& pl, int M, int N, int K, int epilogue, int slots) {
+    const bool gated = epi_is_gated(epilogue);
+    double bytes;
+    int busiest;
+    big_takes_rows(M, N, K, big_ceil_div(M, pl.tile), big_ceil_div(gated ? N / 2 : N, gated ? pl.cols / 2 : pl.cols), slots, &bytes, &busiest);
+    return (double)(busiest * pl.splits) / slots;
+}
 // The same for a tall tile of h x 256 rows: a round is its opening and its epilogue plus S stages, all of them longer with the
 // rows.  Fitted to 2200 linears with weights in operand order (eight heights each, 2.4 % off a single time in the median); the
 // height that it chooses is 0.2 % behind the best of the eight in the geometric mean.
 static double tall_cost(const BigPlan& pl, int M, int N, int K, int epilogue) {
-    const bool gated = epi_is_gated(epilogue);
-    double bytes;
-    int busiest;
-    big_takes_rows(M, N, K, big_ceil_div(M, pl.tile), big_ceil_div(gated ? N / 2 : N, gated ? 128 : 256), 32, &bytes, &busiest);
-    const double S = K / 128, R = big_ceil_div(busiest, 32), x = busiest / 32.0, h = pl.tile / 256.0;
+    const double S = K / 128, x = big_rounds(pl, M, N, K, epilogue, 32), R = ceil(x), h = pl.tile / 256.0;
     double act = 0;
     switch (epilogue) {
     case EPI_GEGLU_TANH: act = 2.68; break;
@@ -1145,18 +1150,29 @@ double big_cost(const BigPlan& pl, int M, int N, int K, int epilogue) {
     if (big_tall(pl)) return tall_cost(pl, M, N, K, epilogue);
     const BigCost c = big_cost_of(pl);
     const bool gated = epi_is_gated(epilogue), two = big_two_of(pl);
-    const int bn = gated ? pl.cols / 2 : pl.cols;
-    const int m_tiles = big_ceil_div(M, pl.tile), n_tiles = big_ceil_div(gated ? N / 2 : N, bn), slots = two ? 64 : 32;
-    double bytes;
-    int busiest;
-    big_takes_rows(M, N, K, m_tiles, n_tiles, slots, &bytes, &busiest);
-    busiest *= pl.splits;
-    const double S = (double)big_ceil_div(K, 128 * pl.splits), R = big_ceil_div(busiest, slots), x = (double)busiest / slots;
+    const double S = (double)big_ceil_div(K, 128 * pl.splits), x = big_rounds(pl, M, N, K, epilogue, two ? 64 : 32), R = ceil(x);
     const double ragged = K % 128 != 0 ? c.ragged : 0.0, epi = gated ? c.gated : epilogue != EPI_NONE ? c.act : 0.0;
     if (!two) return R * (c.round + epi) + x * c.part + S * (R * c.round_step + x * (c.part_step + ragged));
-    const double t = busiest <= 32 ? c.alone + x * c.alone_part + S * (c.alone_step + x * c.alone_part_step)
-                                   : R * c.round + x * c.part + S * (R * c.round_step + x * c.part_step);
+    const double t = x <= 0.5 ? c.alone + x * c.alone_part + S * (c.alone_step + x * c.alone_part_step)
+                            : R * c.round + x * c.part + S * (R * c.round_step + x * c.part_step);
     return t + (x > 1.0 ? x : 1.0) * (S * ragged + epi);
+}
+
+// The same for 192 x 128 tiles as far as the choice between them and tall ones goes, weights in operand order: activations told
+// apart, and a shorter stage beside a longer start than the account over both layouts gives them.  Fitted to the difference of
+// the two in 663 linears: 4.8 % off (9.1 % by the costs).
+static double beside_tall_192(const BigPlan& pl, int M, int N, int K, int epilogue) {
+    const double x = big_rounds(pl, M, N, K, epilogue, 64), rounds = x > 1.0 ? x : 1.0;
+    double act = 0;
+    switch (epilogue) {
+    case EPI_GEGLU_TANH: act = -0.42; break;
+    case EPI_GEGLU_ERF: act = 1.29; break;
+    case EPI_SWIGLU: act = -0.22; break;
+    case EPI_GELU_TANH: act = 1.54; break;
+    case EPI_GELU_ERF: act = 5.86; break;
+    default: break;
+    }
+    return big_cost(pl, M, N, K, EPI_NONE) + 1.62 + rounds * (act - 0.158 * (K / 128));
 }
 
 // The cheapest unsplit tile shape by that account, `rule` (big_plan's choice, or no tile at all) where nothing is 8 % ahead
@@ -1174,11 +1190,20 @@ BigPlan big_plan_by_cost(int M, int N, int K, int epilogue, bool operand_w, cons
         const double t = big_cost(pl, M, N, K, epilogue) + shared;
         if (t < lowest) { *cost = lowest = t; best = pl; }
     }
-    // Tall tiles where they are ahead of that (by 4 % below 60 us, where the costs are less sure): in half of 1800 linears that
-    // tiles serve, 7.3 % less time in the geometric mean over all of them, quantizer included (0.9 % behind the best shape), and
-    // more than 2 % slower in 9.
+    // Tall tiles where they are ahead of that (by 4 % below 60 us, where the costs are less sure) - against 192 x 128 tiles also of
+    // `beside_tall_192`, with 2 % in their favour.  1300 drawn linears that the costs alone gave to tall tiles, timed in these and in the
+    // staged shape: 10.6 % less in the geometric mean, but 68 of them 3 % slower and more, 40 of these against 192 x 128 (short K, an
+    // activation in tanh form: 5719 x 14080 x 1152 + SwiGLU 98.9 / 110.7 us, 5398 x 17856 x 768 + GeGLU 93.1 / 103.8).  By the second
+    // account 45 go back, 31 of the 40 among them; 2 of the 45 gained more than 2 %.  In 900 others it is 19 of 24 among 25, and 3.
+    // (The rest, 128 x 128 tiles two to a CU against a tall grid of less than a round, is a toss-up: asked to be 7 % ahead, in
+    // the 900 as much is lost as won.)
     if (operand_w && K % 128 == 0 && big_registers_allowed()) {
+        const bool against_192 = best.tile == 192 && best.cols == 128;
         lowest = (big_tall(best) || *cost - shared >= 60.0 ? 1.0 : 0.96) * *cost;
+        if (against_192) {
+            const double limit = 1.02 * (beside_tall_192(best, M, N, K, epilogue) + shared);
+            lowest = limit < lowest ? limit : lowest;
+        }
         for (int rows = 144; rows <= 256; rows += 16) {
             const BigPlan pl = {rows, 256, 1, 0, 2, 4};
             const double t = big_cost(pl, M, N, K, epilogue) + shared;

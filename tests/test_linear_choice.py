@@ -115,6 +115,23 @@ def test_weights_stay_out_of_registers_where_that_is_asked_for(monkeypatch):
     assert not [p for p in staged if "tile" in p and "in registers" in p]
 
 
+@pytest.mark.parametrize("M,N,K,epi,tile", [
+    # 10 - 16 % slower in tall tiles
+    (5719, 14080, 1152, "swiglu", "192x128"), (5398, 17856, 768, GATED, "192x128"),
+    (8689, 11840, 896, "gelu_tanh", "192x128"), (5360, 32512, 512, "swiglu", "192x128"), (3694, 26880, 1408, "geglu_erf", "192x128"),
+    # 14 - 23 % faster in them
+    (816, 32768, 2048, GATED, "208x256"), (4800, 8192, 2048, "gelu", "208x256"), (4800, 6144, 2048, None, "240x256"),
+    (5000, 5120, 1280, None, "x256"), (3264, 2560, 2048, None, "144x256")])
+def test_tall_tiles_beside_staged_ones(monkeypatch, M, N, K, epi, tile):
+    from phyai_amd import ops
+
+    for var in ("BIG", "BIG_DEPTH", "BIG_SPLITS", "BIG_DIRECT", "TALL", "TILE", "RULES"):
+        monkeypatch.delenv("PHYAI_FP8_" + var, raising=False)
+    gated = epi is not None and not epi.startswith("gelu")
+    plan = ops.describe_linear_plan(M, N, K, epi, weight_layout="operand_gated" if gated else "operand")
+    assert tile in plan and ("in registers" in plan) == (tile != "192x128"), plan
+
+
 # (rows, columns, K, epilogue): rule's shape -> chosen shape, one per pair that occurs
 CHANGED = [(2032, 9216, 640, "gelu"), (4310, 3648, 640, None), (497, 2432, 8320, None), (2489, 384, 1792, None), (2553, 864, 8320, None),
            (400, 6144, 8192, None), (3548, 3392, 5120, None), (3531, 8160, 640, None), (2740, 1056, 8448, None), (278, 3072, 9600, None)]
