@@ -151,8 +151,8 @@ __device__ __forceinline__ float gelu_tanh_f(float v) {
 // erfc(x) = t P(t) exp(-x^2) with t = 1 / (1 + 0.42 x) and P a degree-7 polynomial (the form of Abramowitz & Stegun
 // 7.1.26, more terms), fitted to erfc(x) exp(x^2) / t on [0, 9.4] - beyond, exp(-x^2) underflows - with relative error below
 // 2.6e-8 (1 + 0.3 x^2): it may grow as the exponential's own does.  The coefficients hold the 0.5.  No cancellation in the
-// negative tail.  Over all bf16 inputs with a result: relative error of at most 3.5e-6 below -8, 1.3e-6 to -4, 5e-7 elsewhere (rms
-// 1e-7), and each rounds to the bf16 of the exact value.  17 instructions, 2 of them at quarter rate; the epilogue of a large
+// negative tail.  Over all bf16 inputs with a result: relative error of at most 4e-6 below -8, 1.7e-6 to -4, 8e-7 elsewhere, with a reciprocal
+// and an exponential within one ulp (rms 1e-7), and each rounds to the bf16 of the exact value.  17 instructions, 2 of them at quarter rate; the epilogue of a large
 // tile is made of little else, and nothing else runs beside it (with a polynomial of degree 8 and the sign chosen by compare and
 // select it was 20, with the same error: 4800 x 8192 x 2048 + GELU in 208-row tiles 91.0 -> 86.6 us, 9600 x 4096 x 2048 99.8 -> 95.2,
 // 2400 x 16384 x 2048 + GeGLU 83.3 -> 80.6).  min keeps +inf * 0 out; -inf gives NaN, as 0.5 v (1 + erf) does.  (In assembly: the

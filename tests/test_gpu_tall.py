@@ -73,6 +73,92 @@ def test_several_tiles_per_workgroup(dev, monkeypatch, rows, epi):
             assert torch.equal(_bits(got), _bits(want)), (M, N, K)
 
 
+# 257 to 600 tiles: a workgroup takes two or three, the constants of the second ride along under the epilogue of the first
+MANY = [(144, 40, 2048, 512), (208, 17, 4096 + 32, 768), (256, 35, 2048, 640)]
+
+
+@pytest.mark.parametrize("rows,blocks,N,K", MANY)
+@pytest.mark.parametrize("epi", [None, "gelu", "gelu_tanh", "geglu_tanh", "geglu_erf", "swiglu"])
+@pytest.mark.parametrize("one_scale", [False, True])
+def test_bias_and_scales_of_several_tiles(dev, monkeypatch, rows, blocks, N, K, epi, one_scale):
+    """Bias as words and value by value (an odd offset), row scales or one for all rows, every activation, over several tiles a
+    workgroup."""
+    from phyai_amd import ops
+
+    M, gated = blocks * rows - 7, bool(epi) and epi.startswith(("geglu", "swiglu"))
+    N = 2 * N if gated else N
+    xq, xs, wq, ws, wo = _operands(dev, M, N, K, gated)
+    xs = xs.flatten()[:1].contiguous() if one_scale else xs
+    bias = seeded((N + 1,), N, 0.1).to(dev)
+    for b in (bias[:N], bias[1:]):
+        got, want = _both(monkeypatch, rows, lambda lay: ops.fp8_gemm(xq, xs, wo, ws, b, epilogue=epi, weight_layout=lay), M, N, K, epi)
+        assert torch.equal(_bits(got), _bits(want))
+
+
+@pytest.mark.parametrize("rows,blocks,N,K", MANY)
+@pytest.mark.parametrize("gates", [1, 3, 0])
+def test_gated_residual_of_several_tiles(dev, monkeypatch, rows, blocks, N, K, gates):
+    """... with one gate row, with groups of token rows that end inside tiles, with a gate row each; into its own place too, and
+    out of rows that lie further apart than the output's."""
+    from phyai_amd import _lib, ops
+
+    M = 3 * ((blocks * rows - 7) // 3)
+    xq, xs, wq, ws, wo = _operands(dev, M, N, K, False)
+    bias = seeded((N + 1,), N, 0.1).to(dev)
+    gate = seeded((gates or M, N), 4, 0.3).to(dev)
+    wide = seeded((M, N + 40), 3).to(dev)
+    res = wide[:, 8:8 + N].contiguous()
+    scratch = torch.empty(1 << 20, dtype=torch.uint8, device=dev)
+    for b in (bias[:N], bias[1:]):
+        def spread(lay):
+            out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+            _lib.check(_lib.load().phyai_fp8_gemm_addcmul(
+                xq.data_ptr(), xs.data_ptr(), 0, wo.data_ptr(), ws.data_ptr(), b.data_ptr(), wide[:, 8:].data_ptr(), N + 40, gate.data_ptr(), N,
+                gate.shape[0], out.data_ptr(), N, M, N, K, 0x200, scratch.data_ptr(), scratch.numel(), torch.cuda.current_stream().cuda_stream), "addcmul")
+            return out
+
+        def in_place(lay):
+            out = res.clone()
+            return ops.fp8_gemm(xq, xs, wo, ws, b, residual=out, gate=gate, out=out, weight_layout=lay)
+
+        plain = lambda lay: ops.fp8_gemm(xq, xs, wo, ws, b, residual=res, gate=gate, weight_layout=lay)
+        got, want = _both(monkeypatch, rows, plain, M, N, K)
+        assert torch.equal(_bits(got), _bits(want))
+        for other in (in_place, spread):
+            again, _ = _both(monkeypatch, rows, other, M, N, K)
+            assert torch.equal(_bits(again), _bits(want)), other.__name__
+
+
+@pytest.mark.parametrize("epi", [None, "gelu", "geglu_tanh"])
+def test_operands_that_are_not_finite(dev, monkeypatch, epi):
+    """A NaN code or scale reaches its own rows and columns, an infinite scale or bias too, and nothing else changes."""
+    from phyai_amd import ops
+
+    rows, gated = 144, epi == "geglu_tanh"
+    M, N, K = 40 * rows - 5, 4096 if gated else 2048, 512
+    xq, xs, wq, ws, _ = _operands(dev, M, N, K, gated)
+    half = N // 2 if gated else N
+    bias = seeded((N,), N, 0.1).to(dev)
+    xs = xs.abs() + 0.01
+    call = lambda lay: ops.fp8_gemm(xq, xs, wo, ws, bias, epilogue=epi, weight_layout=lay)
+    wo = ops.fp8_weight_to_operand_order(wq, gated=gated)
+    clean = call("operand_gated" if gated else "operand")
+    x8, w8 = xq.view(torch.uint8), wq.view(torch.uint8)
+    x8[7, 3], x8[M - 1, K - 1], w8[33, 5] = 0x7F, 0xFF, 0x7F
+    xs.view(-1)[200] = float("inf")
+    xs.view(-1)[3 * rows] = float("nan")
+    ws[half - 1], bias[300] = float("nan"), float("inf")
+    wo = ops.fp8_weight_to_operand_order(wq, gated=gated)
+    got, want = _both(monkeypatch, rows, call, M, N, K, epi)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(got), nan) and torch.equal(_bits(got)[~nan], _bits(want)[~nan])
+    assert bool(nan[[7, M - 1, 3 * rows]].all()) and bool(nan[:, [33, half - 1]].all())
+    keep_r, keep_c = torch.ones(M, dtype=torch.bool, device=dev), torch.ones(half, dtype=torch.bool, device=dev)
+    keep_r[[7, 200, 3 * rows, M - 1]] = False
+    keep_c[[33, 300, half - 1]] = False
+    assert torch.equal(_bits(got[keep_r][:, keep_c]), _bits(clean[keep_r][:, keep_c]))
+
+
 @pytest.mark.parametrize("rows", ROWS)
 @pytest.mark.parametrize("gates", [1, 4, 0])
 def test_gated_residual(dev, monkeypatch, rows, gates):
