@@ -783,6 +783,11 @@ def probe(dev, layers, M, shapes=EXPERT_SET):
     print("probe done")
 
 
+def tile_kernel(plan):
+    """The kernel behind a plan of a large-M GEMM."""
+    return "gemm_fp8_tall_kernel" if "x256 " in plan and "in registers" in plan else "gemm_fp8_big_kernel"
+
+
 def stamps_report(dev):
     """`--stamps`: the cycle budget of the GEMM kernels from inside (debug build of the library, whose kernels record the
     shader clock at the ends of their phases; csrc/stamps.h).  Per workload one launch with fresh weights; per phase the
@@ -792,6 +797,9 @@ def stamps_report(dev):
 
     big = ["start -> first stage published", "main loop", "split-K sums gathered", "epilogue arithmetic, tile staged",
            "stores issued", "stores through"]
+    # (one workgroup per CU takes tile after tile: of its last one)
+    tall = ["start, tiles before -> first stage published", "main loop but for two stages", "everyone there", "last two stages and epilogue",
+            "", "stores through"]
     small = ["start -> rows landed", "row scales known", "codes written", "MFMAs done", "partial sums exchanged",
              "epilogue, stores issued", "stores through"]
     work = [("prefill gate_up + GeGLU", 816, 32768, 2048, "geglu_tanh"), ("prefill down", 816, 2048, 16384, None),
@@ -824,7 +832,8 @@ def stamps_report(dev):
         ops.debug_stamps(0)
         r = rec.cpu().double()
         r = r[r[:, 0] > 0]
-        names = small if small_m else big
+        plan = ops_plan(M, N, K, epi) if small_m else ops.describe_plan(M, N, K, epi, weight_layout=wl)
+        names = small if small_m else tall if tile_kernel(plan) == "gemm_fp8_tall_kernel" else big
         last = ops.STAMP_WORDS - 3
         marks = [0] + [i for i in range(1, last) if bool((r[:, i] > 0).any())] + [last]
         clock = ((r[:, last] - r[:, 0]) / ((r[:, -1] - r[:, -2]).clamp_min(1) / 100e6) / 1e9).median().item()
@@ -834,7 +843,6 @@ def stamps_report(dev):
             d = (r[:, b] - r[:, a]).sort().values
             name = names[b - 1] if b != last else names[-1]
             cells.append(f"{name}: {d[len(d) // 2].item():.0f} ({d[len(d) // 10].item():.0f} .. {d[(9 * len(d)) // 10].item():.0f})")
-        plan = ops_plan(M, N, K, epi) if small_m else ops.describe_plan(M, N, K, epi, weight_layout=wl)
         print(f"| {label} {M} x {N} x {K} | {plan}, {len(r)} wavefronts | {clock:.2f} | {span:.1f} | " + "; ".join(cells) + " |")
         del lay, rec
 
@@ -1109,7 +1117,7 @@ def main() -> int:
                      for name, N, K, epi in PREFILL_SET}
         dom = per_shape["gate_up"]
         roofline_prefill = {
-            "bound": "mfma", "kernel": "gemm_fp8_big_kernel (gate_up 2048->32768 + GeGLU at M=816: " + dom["kernel"] + ")",
+            "bound": "mfma", "kernel": tile_kernel(dom["kernel"]) + " (gate_up 2048->32768 + GeGLU at M=816: " + dom["kernel"] + ")",
             "achieved": dom["TFLOP/s"], "peak": FP8_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(dom["TFLOP/s"] / FP8_PEAK_TFLOPS, 4), "us": dom["us"],
             "measured_peak_TFLOPs": measured["fp8_TFLOPs"] if measured else None,

@@ -1041,9 +1041,10 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     pl.depth = (pl.tile == 128 || pl.tile == 96) ? 4 : 2;
     bool to_224 = false;
     if (operand_w && forced < 0 && pl.tile != 224 && K >= 4096 && K % 512 == 0) {
-        // Weights in operand order: the 224 x 256 tile loads them straight into registers and hands its activation
-        // stages over without barriers, and from K = 4096 on the prologue and epilogue that nothing overlaps in it weigh
-        // less than what its main loop gains.  Taken when it has at least 160 tiles and fills its rounds of 256
+        // Weights in operand order: tiles of 224 x 256 load them straight into registers and hand their activation
+        // stages over without barriers (gemm_tall.hip).  The line was drawn with that kernel's predecessor, whose prologue and
+        // epilogue stood alone, and whose times these are; GEMMs on ready codes keep to it, a linear's staged codes get
+        // the height that the costs below choose.  Taken with at least 160 tiles that fill their rounds of 256
         // workgroups with useful rows and columns at least 0.8 times as well as the shape chosen above fills its own
         // (chosen above / this, us: 6528 x 2048 x 16384 173 / 154, 13056 x 2048 x 16384 340 / 300, 6528 x 2048 x 8192 93.9 /
         // 81.8, 1632 x 8192 x 8192 93.4 / 85.0, 6528 x 4096 x 4096 104 / 96, 13056 x 2048 x 4096 101 / 91, 3264 x 16384 x 4096 +
@@ -1084,7 +1085,7 @@ BigPlan big_plan(int M, int N, int K, int epilogue, bool operand_w) {
     }
     // Weights in operand order and a whole number of trips round the ring per K range: the wavefronts load their own
     // weight blocks straight into registers (PHYAI_FP8_BIG_DIRECT=0: stage them like the rest).  224 x 256 tiles: ring
-    // of four.  128 x 128 tiles with a ring of four LDS stages and a plain epilogue: wavefronts 1 x 4 with one column
+    // of four, gemm_tall.hip.  128 x 128 tiles with a ring of four LDS stages and a plain epilogue: wavefronts 1 x 4 with one column
     // block each and a ring of eight.  (Not the 96 x 128 tile: its main loop gains what its longer prologue - six
     // stage-loads requested up front, at what the CU's vector-memory path passes - loses: 816 x 2560 x 2048 10.0 ->
     // 10.1 us on the earlier loop.  Up to K = 2048 the ring of eight is level with staged weights, and the ring of four of

@@ -305,7 +305,8 @@ void gemm_fp8_tall_kernel(
         half(d, set, Yes{}, Yes{}, Yes{}, No{}, nothing);
     };
     // The loop over stage-loads names sets 0 .. 3 in turn and ends with sets 2 and 3.  Up to three stage-loads beyond a multiple of
-    // four come before it, each in set 1, the two behind it moving up.
+    // four come before it, each in set 1, the two behind it moving up.  (The move waits for weights that were asked for half a stage
+    // ago.  K = 128 mod 512 and the like gain as much over staged tiles as the rest all the same, 9.8 - 10.5 % in 500 linears.)
     auto turn = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -474,7 +475,9 @@ void gemm_fp8_tall_kernel(
     for (bool first = true;; first = false) {
         // Stage-load 0 and the activations up to stage-load CLAIM - 1 have landed (what progress word -1 stands for; the
         // stores of the tile before, younger than all of these, only make the wait stricter).  The first tile's stage-load 2
-        // is on its way; a later one's, whose place was still in use, is asked for beside the first MFMAs.
+        // has been asked for; a later one's, whose place was still in use, is asked for beside the first MFMAs.  (The two ways
+        // meet in one set of registers, for which the compiler waits: a first tile for those weights before its first MFMA,
+        // a later one for most of them before half 1.)
         if (first) wait_copies<COPIES + BL + CONSTS>();
         else wait_copies<BL + CONSTS>();
         if (lane == 0) progress[wave] = -1;

@@ -167,9 +167,9 @@ def test_operand_order_with_the_gated_residual(dev, M, N, K):
     assert torch.equal(_bits(lin_op), _bits(lin_rm)) and torch.equal(_bits(gemm_op), _bits(gemm_rm))
 
 
-# how the pipelined tile kernel takes weights in operand order: staged through LDS as they lie (and, for the
-# 224-row tile with K a multiple of 512, straight into registers); the same without the register path; gathered
-# row by row into the row-major staging layout
+# how the pipelined tile kernels take weights in operand order: staged through LDS as they lie (for 224 x 256 tiles with K a
+# multiple of 512 and, with 128 x 128 tiles, for some K straight into registers); the same without the register path;
+# gathered row by row into the row-major staging layout
 @pytest.mark.parametrize("mode", ["", "PHYAI_FP8_BIG_DIRECT=0", "PHYAI_FP8_BIG_GATHER=1"])
 @pytest.mark.parametrize("tile", ["256", "224", "192", "128", "128/2", "12864", "96"])
 @pytest.mark.parametrize("M,N,K,epi", [(816, 768, 1024, None), (513, 400, 1536, "gelu"), (816, 1024, 1152, "geglu_tanh"),
