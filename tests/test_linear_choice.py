@@ -116,9 +116,11 @@ def test_weights_stay_out_of_registers_where_that_is_asked_for(monkeypatch):
 
 
 @pytest.mark.parametrize("M,N,K,epi,tile", [
-    # 10 - 16 % slower in tall tiles
-    (5719, 14080, 1152, "swiglu", "192x128"), (5398, 17856, 768, GATED, "192x128"),
-    (8689, 11840, 896, "gelu_tanh", "192x128"), (5360, 32512, 512, "swiglu", "192x128"), (3694, 26880, 1408, "geglu_erf", "192x128"),
+    # slower in tall tiles, by 4 to 16 % as cards differ
+    (6741, 8960, 1408, GATED, "192x128"), (5398, 17856, 768, GATED, "192x128"), (6693, 15616, 768, GATED, "192x128"),
+    (8689, 11840, 896, "gelu_tanh", "192x128"), (5360, 32512, 512, "swiglu", "192x128"),
+    # faster in them, where less than 5.5 % in favour would not have it so
+    (2307, 26336, 640, "swiglu", "x256"), (4467, 23072, 896, "swiglu", "x256"), (3996, 15776, 768, GATED, "x256"),
     # 14 - 23 % faster in them
     (816, 32768, 2048, GATED, "208x256"), (4800, 8192, 2048, "gelu", "208x256"), (4800, 6144, 2048, None, "240x256"),
     (5000, 5120, 1280, None, "x256"), (3264, 2560, 2048, None, "144x256")])
