@@ -130,7 +130,7 @@ void gemm_fp8_tall_kernel(
     int ring = 0;
     auto stage_at = [&](int base, int d) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_readfirstlane(((base + d) & 3) * STAGE_BYTES); };
     // (SGPRs are short here: the compiler keeps some in VGPR lanes, the base pointers of copies among them, and reads them back right
-    // in front of a copy.  Hence kBaseSettles, and multiply_copy where copies are many.)
+    // in front of a copy.  Hence kBaseSettles, and an MFMA among the wait states where copies are many: multiply_copy and `tail`.)
     auto copy = [&](int d, int c, uint32_t at) __attribute__((always_inline)) { copy16_to_lds<kBaseSettles>(a_a + d * BIG_BK, aoff[c], wave_a + at + c * 1024); };
     auto load = [&](int d, int e, auto set) __attribute__((always_inline)) {
         bring[decltype(set)::value][e >> 1][e & 1] = *reinterpret_cast<const v4i*>(bsrc[e >> 1] + ((size_t)d << 11) + (e & 1) * 1024 + lane16);
@@ -238,10 +238,10 @@ void gemm_fp8_tall_kernel(
         const uint8_t* const base = a_a + d * BIG_BK;
         const uint32_t from = aoff[k], to = wave_a + at + k * 1024;
         if constexpr (decltype(first)::value)
-            asm volatile("s_mov_b32 m0, %5\n\ts_nop 2\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0\n\tglobal_load_lds_dwordx4 %3, %4"
+            asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %3, %4"
                          : "=a"(c) : "v"(w), "v"(x), "v"(from), "s"(base), "s"(to) : "memory", "m0");
         else
-            asm volatile("s_mov_b32 m0, %5\n\ts_nop 2\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
+            asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %3, %4"
                          : "+a"(c) : "v"(w), "v"(x), "v"(from), "s"(base), "s"(to) : "memory", "m0");
     };
     v8i fa[2][H0];
@@ -376,6 +376,14 @@ void gemm_fp8_tall_kernel(
         tall_each<8 * (R + 3)>([&](auto piece_) __attribute__((always_inline)) {
                 constexpr int piece = decltype(piece_)::value, r = piece / 8, e = piece % 8;
                 if constexpr (e == 0 && r >= 1 && r <= R) s = s_next;
+                // The request behind this piece (evenly over the pieces beside MFMAs).  If a copy's base has to be read back it is here:
+                // the MFMA and its s_nop are wait states enough.  (kBaseSettles, three more each time, beside work that is VALU bound:
+                // two projections of 13056 rows 1148 us, 1145 so, 1143 with none at all)
+                constexpr int n = piece * OPENING / (8 * R);
+                constexpr bool asks = r < R && (piece == 0 || n != (piece - 1) * OPENING / (8 * R)), copies = asks && n >= BL && n < BL + 2 * CA;
+                constexpr int of_load = n < BL + CA ? 0 : 1;
+                const uint8_t* base = a_a + of_load * BIG_BK;
+                if constexpr (copies) asm volatile("" : "+s"(base));
                 if constexpr (r < R) {
                     multiply(big_join(bring[2 + (e >> 2)][e & 3][0], bring[2 + (e >> 2)][e & 3][1]), e < 4 ? f0 : f1, acc[r][e & 3], No{});
                     if constexpr (e == 3 && r + 1 < R) f0 = frag(lo0, hi0, r + 1);
@@ -454,8 +462,10 @@ void gemm_fp8_tall_kernel(
                         *reinterpret_cast<uint2*>(at + ((2 * jj + (q >> 1)) ^ sw) * 16 + (q & 1) * 8) = w;
                     }
                 }
-                constexpr int n = piece * OPENING / (8 * R);   // (evenly over the pieces beside MFMAs)
-                if constexpr (r < R && (piece == 0 || n != (piece - 1) * OPENING / (8 * R))) {
+                if constexpr (copies) {
+                    constexpr int c = n - BL - of_load * CA;
+                    if (more) copy16_to_lds(base, aoff[c], wave_a + stage_at(next_ring, of_load) + c * 1024);
+                } else if constexpr (asks) {
                     if (more) opening(std::integral_constant<int, n>{}, next_const_at, next_ring);
                 }
                 __builtin_amdgcn_sched_barrier(0);
