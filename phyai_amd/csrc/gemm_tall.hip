@@ -15,7 +15,8 @@
 //  * the first MFMA of a sum takes zero in place of it: no accumulators are cleared;
 //  * requests are spread over all MFMAs of a stage (weights in its first half, activations in the second): in one half they
 //    kept the CU's address unit busy for longer than that (main loop of 208 rows 28.4 -> 27.3 k cycles).
-// 45 k cycles a tile at 224 rows (opening 0.4 k, main loop 29 k for 25.1 k of MFMAs, last two stages and epilogue 16 k).
+// 47 k cycles a tile at 224 rows, K = 2048, GeGLU: main loop 29.4 k for 25.1 k of MFMAs, last two stages and epilogue 15.4 k (9.4 k
+// without an activation, 28.3 k with GELU), 2 k from there to the next tile's first stage; the first tile's opening 6 - 10 k.
 // us of a GEMM on ready codes, the shape that was taken before / this kernel: 816 x 32768 x 2048 + GeGLU (208 rows) 60.5 / 52.3,
 // 13056 x 32768 x 2048 + GeGLU 752 / 706, 4800 x 6144 x 2048 (240) 58.4 / 48.1, 4800 x 8192 x 2048 + GELU (208) 92.8 / 87.4,
 // 4800 x 2048 x 8192 (160) 67 / 57.5, 4800 x 2048 x 2048 21.5 / 17.6, 3264 x 2560 x 2048 (144) 21.4 / 17.2, 6528 x 2048 x 2048
@@ -306,7 +307,7 @@ void gemm_fp8_tall_kernel(
     };
     // The loop over stage-loads names sets 0 .. 3 in turn and ends with sets 2 and 3.  Up to three stage-loads beyond a multiple of
     // four come before it, each in set 1, the two behind it moving up.  (The move waits for weights that were asked for half a stage
-    // ago.  K = 128 mod 512 and the like gain as much over staged tiles as the rest all the same, 9.8 - 10.5 % in 500 linears.)
+    // ago.  K = 128, 256, 384 mod 512 are 1.09, 1.09, 1.08 times as fast as staged tiles all the same, the rest 1.10, in 325 linears.)
     auto turn = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {

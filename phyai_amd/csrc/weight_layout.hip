@@ -1,7 +1,10 @@
 // Re-lays a row-major fp8 weight matrix into MFMA operand order (weight_layout.h), once per layer
-// after loading.  One thread moves four 16-byte chunks; consecutive threads write consecutive chunks
+// after loading.  One thread moves CHUNKS 16-byte chunks; consecutive threads write consecutive chunks
 // of the destination, so the writes are contiguous and the reads are 16-byte pieces of 16
-// neighbouring rows.  Bound by bytes (6.8 TB/s); four requests in flight per thread instead of one keep it there.
+// neighbouring rows.  Bound by bytes (6.8 TB/s).  Two chunks where the source is a second matrix (us with the copy in front
+// of it, 1 / 2 / 4: 4096 x 2688 15.2 / 11.1 / 14.8, 5504 x 2688 16.8 / 14.0 / 17.8, 8192 x 2048 18.3 / 15.6 / 18.9, 14336 x 2048 25.4 /
+// 23.6 / 24.1), four where large matrices are re-laid by halves (a whole load of 16384 x 2048 39.6 / 37.4 with two / four, 24576 x
+// 2048 55.7 / 54.0, 32768 x 2048 72.6 / 71.9).
 //
 // A plain matrix is re-laid in place: unit u (16 rows x K) holds the same bytes in both orders, so a workgroup takes them
 // into its registers, waits for everyone and writes them back - half the bytes of re-laying into a second matrix and
@@ -27,21 +30,22 @@ static bool launched(void (*kernel)(P...), unsigned blocks, unsigned threads, hi
 
 // Chunks [first * K, first * K + chunks) of the destination, i.e. units from `first` on (a unit is K chunks).  Gated: gate rows
 // from `gate`, up rows from `up`, both counted from column 0; plain: rows of the matrix at `gate`.
+template <int CHUNKS>
 __global__ __launch_bounds__(256) void weight_to_operand_order_kernel(const v4i* gate, const v4i* up, v4i* out,
                                                                       uint32_t first, uint32_t K, int gated, uint32_t chunks) {
     const uint32_t steps = K >> 7;
-    v4i v[4];
+    v4i v[CHUNKS];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t t = blockIdx.x * 1024 + j * 256 + threadIdx.x, i = t < chunks ? t : chunks - 1;
+    for (int j = 0; j < CHUNKS; ++j) {
+        const uint32_t t = blockIdx.x * (256 * CHUNKS) + j * 256 + threadIdx.x, i = t < chunks ? t : chunks - 1;
         const uint32_t r = i & 15, c = (i >> 4) & 7, us = i >> 7;   // us = u * steps + s
         const uint32_t u = first + us / steps, s = us % steps;
         const uint32_t row = gated ? 8 * u + 2 * (r >> 2) + (r & 1) : 16 * u + r;
         v[j] = (gated && (r & 2) ? up : gate)[(size_t)row * (K >> 4) + s * 8 + c];
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t i = blockIdx.x * 1024 + j * 256 + threadIdx.x;
+    for (int j = 0; j < CHUNKS; ++j) {
+        const uint32_t i = blockIdx.x * (256 * CHUNKS) + j * 256 + threadIdx.x;
         if (i < chunks) out[(size_t)first * K + i] = v[j];
     }
 }
@@ -89,15 +93,16 @@ int launch_weight_to_operand_order_inplace(void* w, int64_t N, int64_t K, hipStr
     return ok ? 0 : -3;
 }
 
+template <int CHUNKS>
 static bool launch_units(const v4i* gate, const v4i* up, v4i* out, uint32_t first, uint32_t end, uint32_t K, int gated, hipStream_t st) {
     const uint32_t chunks = (end - first) * K;
-    return launched(weight_to_operand_order_kernel, (chunks + 1023) / 1024, 256, st, gate, up, out, first, K, gated, chunks);
+    return launched(weight_to_operand_order_kernel<CHUNKS>, (chunks + 256 * CHUNKS - 1) / (256 * CHUNKS), 256, st, gate, up, out, first, K, gated, chunks);
 }
 
 int launch_weight_to_operand_order(const void* w, int64_t N, int64_t K, int gated, void* out, hipStream_t st) {
     if (N * K > 0x7FFFFFFFll) return -2;
     const v4i* rows = static_cast<const v4i*>(w);
-    return launch_units(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st) ? 0 : -3;
+    return launch_units<2>(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st) ? 0 : -3;
 }
 
 }  // namespace phyai
@@ -121,6 +126,6 @@ extern "C" int phyai_host_relay_gated(void* w, int64_t N, int64_t K, void* scrat
     const uint32_t k = (uint32_t)K, units = (uint32_t)(N / 16), half = (uint32_t)(N / 2 * K / 16);
     const uint32_t middle = units / 2, kept = middle * 8 * (k / 16);   // (N % 32 == 0: units is even)
     if (!launched(weight_save_kernel, (half + kept + 1023) / 1024, 256, st, m, up, half, kept)) return -2;
-    if (!launch_units(m, up, m, middle, units, k, 1, st)) return -2;
-    return launch_units(up + half, up, m, 0, middle, k, 1, st) ? 0 : -3;
+    if (!launch_units<4>(m, up, m, middle, units, k, 1, st)) return -2;
+    return launch_units<4>(up + half, up, m, 0, middle, k, 1, st) ? 0 : -3;
 }
