@@ -203,10 +203,20 @@ def test_nonfinite_affine_parts_give_the_canonical_nan(dev, hidden, adaptive):
     assert torch.equal(got[:, keep], plain[:, keep])
 
 
-@pytest.mark.parametrize("M,K", [(2047, 2048), (2048, 2048), (2048, 1040), (2050, 1168), (3, 4112), (3, 8192), (1535, 4112), (1536, 4112), (1537, 8192), (5, 8208), (2, 16384), (3300, 16000)])
+@pytest.mark.parametrize("M,K", [(2047, 2048), (2048, 2048), (2048, 1040), (2050, 1168), (3, 4112), (3, 8192), (5, 8208), (2, 16384), (3300, 16000)])
 def test_quantizer_at_the_edges_of_its_workgroup_shapes(dev, M, K):
     x = seeded((M, K), seed=M + K, scale=2.0)
     x[M - 1, K - 1] = 77.0
+    xq, xs = _ops().fp8_quant_rowwise(x.to(dev))
+    q, s = ref.quant_rowwise(x)
+    assert torch.equal(xs.cpu(), s) and torch.equal(xq.cpu().view(torch.uint8), q.view(torch.uint8))
+
+
+@pytest.mark.parametrize("M,K", [(1535, 4112), (1536, 4112), (1537, 8192)])
+def test_quantizer_of_long_rows_where_its_workgroups_shrink(dev, M, K):
+    """512 threads a row below 1536 rows, 256 from there on, both up to K = 8192."""
+    x = seeded((M, K), seed=M + K, scale=2.0)
+    x[0, 0], x[M - 1, K - 1] = -65.0, 77.0
     xq, xs = _ops().fp8_quant_rowwise(x.to(dev))
     q, s = ref.quant_rowwise(x)
     assert torch.equal(xs.cpu(), s) and torch.equal(xq.cpu().view(torch.uint8), q.view(torch.uint8))
