@@ -139,16 +139,17 @@ static int launch_quant_rows(const void* x, int64_t M, int64_t K, int64_t ld, vo
     // either way, and two wavefronts wait for each other less than four (us, 256 threads / 128: 816 x 2048 3.25 / 3.28, 3264 x 2048
     // 6.2 / 5.9, 13056 x 2048 13.9 / 13.4).  Long rows: 512 threads instead of 256 (50 x 16384 3.9 / 3.5, 816 x 16384
     // 9.5 / 9.3, 3264 x 16384 25.7 - 27.4 / 24.3 - 27.0, 13056 x 16384 95.0 / 94.1); 1024 are
-    // slower again with many of them (58.4 at 13056 x 8192, where 512 take 49).  Up to K = 8192 for few rows only (50 x 8192 2.8 / 2.6, 256 x
+    // slower again with many of them (58.4 at 13056 x 8192, where 512 take 49).  Up to K = 5632 for few rows only (50 x 8192 2.8 / 2.6, 256 x
     // 5120 3.15 / 2.98, 777 x 5504 4.4 / 4.2): with many the second half of a workgroup waits for a short rest of the row (1600 x
-    // 4304 5.7 / 6.1, 4000 x 5504 13.4 / 14.0, 8000 x 5120 23.0 / 24.1; level at K = 8192).
+    // 4304 5.7 / 6.1, 3264 x 4608 9.3 / 9.4, 4800 x 4608 13.9 / 14.5, 8000 x 5120 22.9 / 23.6; level at K = 5632, and beyond, where it
+    // has half a row, 1600 x 7168 7.55 / 7.17, 4800 x 8064 22.6 / 22.1, 13056 x 8192 51.8 / 51.2).
     if (K <= 512) PHYAI_QL(64, 1);
     else if (K <= 1024) PHYAI_QL(128, 1);
     else if (K <= 2048 && M >= 2048) PHYAI_QL(128, 2);
     else if (K <= 2048) PHYAI_QL(256, 1);
     else if (K <= 4096) PHYAI_QL(256, 2);
-    else if (K <= 8192 && M < 1536) PHYAI_QL(512, 2);
-    else if (K <= 8192) PHYAI_QL(256, 4);
+    else if (K <= 5632 && M >= 1536) PHYAI_QL(256, 4);
+    else if (K <= 8192) PHYAI_QL(512, 2);
     else if (K <= 16384) PHYAI_QL(512, 4);
     else if (K <= 32768) PHYAI_QL(256, 16);
     else hipLaunchKernelGGL((quant_rows_loop_kernel<MODE>), grid, dim3(256), 0, st, xp, ld, k, (int)ldq, qp, scale);

@@ -212,9 +212,9 @@ def test_quantizer_at_the_edges_of_its_workgroup_shapes(dev, M, K):
     assert torch.equal(xs.cpu(), s) and torch.equal(xq.cpu().view(torch.uint8), q.view(torch.uint8))
 
 
-@pytest.mark.parametrize("M,K", [(1535, 4112), (1536, 4112), (1537, 8192)])
+@pytest.mark.parametrize("M,K", [(1535, 4112), (1536, 4112), (1537, 5632), (1536, 5648), (1537, 8192)])
 def test_quantizer_of_long_rows_where_its_workgroups_shrink(dev, M, K):
-    """512 threads a row below 1536 rows, 256 from there on, both up to K = 8192."""
+    """256 threads a row from 1536 rows on up to K = 5632, 512 otherwise up to K = 8192."""
     x = seeded((M, K), seed=M + K, scale=2.0)
     x[0, 0], x[M - 1, K - 1] = -65.0, 77.0
     xq, xs = _ops().fp8_quant_rowwise(x.to(dev))
