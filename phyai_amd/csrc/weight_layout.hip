@@ -1,10 +1,12 @@
 // Re-lays a row-major fp8 weight matrix into MFMA operand order (weight_layout.h), once per layer
 // after loading.  One thread moves CHUNKS 16-byte chunks; consecutive threads write consecutive chunks
 // of the destination, so the writes are contiguous and the reads are 16-byte pieces of 16
-// neighbouring rows.  Bound by bytes (6.8 TB/s).  Two chunks where the source is a second matrix (us with the copy in front
-// of it, 1 / 2 / 4: 4096 x 2688 15.2 / 11.1 / 14.8, 5504 x 2688 16.8 / 14.0 / 17.8, 8192 x 2048 18.3 / 15.6 / 18.9, 14336 x 2048 25.4 /
-// 23.6 / 24.1), four where large matrices are re-laid by halves (a whole load of 16384 x 2048 39.6 / 37.4 with two / four, 24576 x
-// 2048 55.7 / 54.0, 32768 x 2048 72.6 / 71.9).
+// neighbouring rows.  Bound by bytes (6.8 TB/s).  Two chunks where the source is a second matrix below 20 MB, whose workgroups
+// would be few (us, start of a load with the copy in front of it, 1 / 2 / 4: 4096 x 2688 15.2 / 11.1 / 14.8, 5504 x 2688 16.8 / 14.0 / 17.8,
+// 8192 x 2048 18.3 / 15.6 / 18.9), otherwise four (2 / 4: 14336 x 2048 23.6 / 24.1 with the copy; without one 13.7 / 13.2, 10240 x
+// 2048 8.31 / 8.26, 11776 x 2048 gated 11.6 / 10.6, 2048 x 16384 14.0 / 13.6, 32768 x 2048 26.1 / 24.9, 16384 x 8192 level), as where
+// large matrices are re-laid by halves (a whole load of 16384 x 2048 39.6 / 37.4, 24576 x 2048 55.7 / 54.0, 32768 x 2048 72.6 /
+// 71.9).
 //
 // A plain matrix is re-laid in place: unit u (16 rows x K) holds the same bytes in both orders, so a workgroup takes them
 // into its registers, waits for everyone and writes them back - half the bytes of re-laying into a second matrix and
@@ -18,6 +20,8 @@
 #include "weight_layout.h"
 
 namespace phyai {
+
+constexpr int64_t kFewChunks = 20 << 20;   // bytes of a matrix below which a thread moves two chunks, not four
 
 // The launch's own status.  hipGetLastError() may return an older error of the thread, and a caller that went another way for
 // it would re-lay the matrix a second time.
@@ -102,7 +106,8 @@ static bool launch_units(const v4i* gate, const v4i* up, v4i* out, uint32_t firs
 int launch_weight_to_operand_order(const void* w, int64_t N, int64_t K, int gated, void* out, hipStream_t st) {
     if (N * K > 0x7FFFFFFFll) return -2;
     const v4i* rows = static_cast<const v4i*>(w);
-    return launch_units<2>(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st) ? 0 : -3;
+    const auto launch = N * K < kFewChunks ? launch_units<2> : launch_units<4>;
+    return launch(rows, rows + N / 2 * K / 16, static_cast<v4i*>(out), 0, (uint32_t)(N / 16), (uint32_t)K, gated, st) ? 0 : -3;
 }
 
 }  // namespace phyai

@@ -73,6 +73,19 @@ def test_gated_relay_in_its_own_storage(dev, N, K):
     assert (around[:1024] == 0x5A).all() and (around[1024 + N * K:] == 0x5A).all()
 
 
+@pytest.mark.parametrize("N,K,gated", [(10240, 2048, True), (10240, 2048, False), (10208, 2048, True), (10224, 2048, False), (1712, 12160, False),
+                                       (1728, 12160, True)])
+def test_relay_at_the_edge_of_its_chunks_a_thread(dev, N, K, gated):
+    """20 MB: two chunks a thread below, four from there on, the last workgroup full or not; nothing beside the output is written."""
+    ops = _ops()
+    w = torch.randint(0, 256, (N, K), generator=torch.Generator().manual_seed(N + K), dtype=torch.uint8)
+    around = torch.full((N * K + 2048,), 0x5A, dtype=torch.uint8, device=dev)
+    mine = around[1024:1024 + N * K].view(N, K)
+    ops.fp8_weight_to_operand_order(w.to(dev).view(torch.float8_e4m3fn), gated=gated, out=mine.view(torch.float8_e4m3fn))
+    assert torch.equal(mine.cpu(), _operand_order_on_cpu(w, gated))
+    assert (around[:1024] == 0x5A).all() and (around[1024 + N * K:] == 0x5A).all()
+
+
 @pytest.mark.parametrize("N,K,gated", [(64, 256, False), (64, 256, True), (32768, 1024, True)])
 def test_relay_beside_an_older_error_of_the_thread(dev, N, K, gated):
     """An error that another HIP call left pending is not this one's: the matrix is re-laid, once, and the error is still there."""
